@@ -27,7 +27,7 @@ struct CellQ {
   double xi, hs, h, hu, hv, zb, u, v, s, p;
 };
 
-__host__ __device__ __forceinline__ CellQ make_cellq(double xi, double hs, double qx, double qy, double zb, double half_g,
+__device__ __forceinline__ CellQ make_cellq(double xi, double hs, double qx, double qy, double zb, double half_g,
                                             double hsmall) {
   CellQ c;
   c.xi = xi;
@@ -42,9 +42,10 @@ __host__ __device__ __forceinline__ CellQ make_cellq(double xi, double hs, doubl
   c.hu = hu;
   c.hv = hv;
   c.zb = zb;
-  c.u = hu / h;
-  c.v = hv / h;
-  c.s = sqrt(h + EPS);
+  const double rh = rcp_est(h);
+  c.u = div_est(hu, h, rh);
+  c.v = div_est(hv, h, rh);
+  c.s = sqrt_pos(h + EPS);
   c.p = half_g * ((xi + EPS) * (xi + EPS) + 2.0 * xi * hs);
   return c;
 }
@@ -52,7 +53,7 @@ __host__ __device__ __forceinline__ CellQ make_cellq(double xi, double hs, doubl
 // Flux through the face (A | B), normal n pointing from A to B.
 // fa = flux seen from A; when BOTH, fb = flux seen from B (normal -n).
 template <bool BOTH>
-__host__ __device__ __forceinline__ void roe_pair(const CellQ& A, const CellQ& B, double nx, double ny, double g,
+__device__ __forceinline__ void roe_pair(const CellQ& A, const CellQ& B, double nx, double ny, double g,
                                          double half_g, double hmin, double fa[3], double fb[3]) {
   if (A.h <= hmin && B.h <= hmin) {  // :16-22
     fa[0] = fa[1] = fa[2] = 0.0;
@@ -80,19 +81,21 @@ __host__ __device__ __forceinline__ void roe_pair(const CellQ& A, const CellQ& B
   }
   const double hRoe = (hA + hB) * 0.5;
   const double sAB = sA + sB;
-  const double uRoe = (sA * uA + sB * uB) / sAB;
-  const double vRoe = (sA * vA + sB * vB) / sAB;
+  const double ys = rcp_est(sAB);
+  const double uRoe = div_est(sA * uA + sB * uB, sAB, ys);
+  const double vRoe = div_est(sA * vA + sB * vB, sAB, ys);
   const double unRoe = uRoe * nx + vRoe * ny;
-  const double cRoe = sqrt(g * hRoe + EPS);
-  const double o = 0.5 / cRoe;
+  double r2c;
+  const double cRoe = sqrt_est(g * hRoe + EPS, r2c);
+  const double o = __builtin_fma(__builtin_fma(-cRoe, r2c, 0.5), 2.0 * r2c, r2c);  // 0.5 / cRoe
   const double d0 = B.xi - A.xi, d1 = huB - huA, d2 = hvB - hvA;
   const double w0 = (-(uRoe * ny - vRoe * nx)) * d0 + ny * d1 + (-nx) * d2;
   const double w1 = (unRoe * o + 0.5) * d0 + (-nx * o) * d1 + (-ny * o) * d2;
   const double w2 = (-unRoe * o + 0.5) * d0 + (nx * o) * d1 + (ny * o) * d2;
-  const double a0 = sqrt(unRoe * unRoe + EPS) * w0;
+  const double a0 = sqrt_pos(unRoe * unRoe + EPS) * w0;
   const double um = unRoe - cRoe, up = unRoe + cRoe;
-  const double a1 = sqrt(um * um + EPS) * w1;
-  const double a2 = sqrt(up * up + EPS) * w2;
+  const double a1 = sqrt_pos(um * um + EPS) * w1;
+  const double a2 = sqrt_pos(up * up + EPS) * w2;
   const double r0 = a1 + a2;
   const double T0 = ny * a0, T1 = (uRoe - cRoe * nx) * a1, T2 = (uRoe + cRoe * nx) * a2;
   const double U0 = (-nx) * a0, U1 = (vRoe - cRoe * ny) * a1, U2 = (vRoe + cRoe * ny) * a2;

@@ -42,7 +42,6 @@
 #include "hg_lux.hpp"
 #include "hgswe.h"
 
-using hg::Side;
 using hg::StepArgs;
 
 static thread_local std::string g_create_err;  // per caller thread, like the contexts
@@ -168,6 +167,60 @@ __device__ __forceinline__ void store_state(double* p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A boundary face's ghost state (bc_2D.jl:640-834) as the flux reads it,
+// formed from its internal cell's flux inputs A (Manning n: n_i).  tot_f: the
+// conveyance of an inlet-Q ghost's inlet when the kernel formed it itself
+// (fused), else it is read from a.totalA.  Args: the step kernels' blocks.
+template <class Args>
+__device__ __forceinline__ hg::CellQ ghost_cellq(const Args& a, const hg::CellQ& A, double n_i, int gi, double nx,
+                                                 double ny, bool fused, double tot_f) {
+  const double hsmall = a.hsmall;
+  double h, qx, qy;
+  switch (a.g_kind[gi]) {
+    case HG_BC_INLETQ: {
+      const int b = a.g_bc[gi];
+      const double w = (A.h > hsmall) ? 1.0 : 0.0;
+      const double v = a.inletQ[b] / (fused ? tot_f : a.totalA[b]) * a.g_L23[gi] / n_i;
+      h = A.h;
+      qx = -A.h * v * nx * w;
+      qy = -A.h * v * ny * w;
+      break;
+    }
+    case HG_BC_EXITH: {
+      const double hx = a.exitWSE[a.g_bc[gi]] - A.zb;
+      h = (hx > hsmall) ? hx : hsmall;
+      qx = A.hu;
+      qy = A.hv;
+      break;
+    }
+    case HG_BC_WALL:
+      h = A.h;
+      qx = -A.hu;
+      qy = -A.hv;
+      break;
+    default: {  // HG_BC_SYMM
+      const double vdn = A.hu * nx + A.hv * ny;
+      h = A.h;
+      qx = A.hu - 2.0 * vdn * nx;
+      qy = A.hv - 2.0 * vdn * ny;
+      break;
+    }
+  }
+  hg::CellQ B;
+  B.hs = a.g_hstill[gi];
+  B.xi = h - B.hs;
+  B.h = h;
+  B.hu = qx;
+  B.hv = qy;
+  B.zb = a.g_zb[gi];
+  const double rh = hg::rcp_est(h);
+  B.u = hg::div_est(qx, h, rh);
+  B.v = hg::div_est(qy, h, rh);
+  B.s = hg::sqrt_pos(h + hg::EPS);
+  B.p = a.half_g * ((B.xi + hg::EPS) * (B.xi + hg::EPS) + 2.0 * B.xi * B.hs);
+  return B;
+}
+
 // Fused RHS (+ Euler step and dry clamp when STEP).  One work-item per cell.
 template <bool STEP>
 __global__ __launch_bounds__(kBlock) void k_swe_step(StepArgs a0) {
@@ -179,75 +232,30 @@ __global__ __launch_bounds__(kBlock) void k_swe_step(StepArgs a0) {
   const double hsmall = a.hsmall;
   const double xi = a.xi[i], hs = a.hstill[i];
   const double qx0 = a.qx[i], qy0 = a.qy[i];
-  double h = xi + hs, qx = qx0, qy = qy0;  // semi_discretize_swe_2D.jl:101-106
-  if (h <= hsmall) {
-    h = hsmall;
-    qx = 0.0;
-    qy = 0.0;
-  }
   const double zb = a.zb[i];
   const double nman = a.n[i];
-  const Side Ls{xi, hs, h, qx, qy, zb};
+  const hg::CellQ me = hg::make_cellq(xi, hs, qx0, qy0, zb, a.half_g, hsmall);
+  const double h = me.h, qx = me.hu, qy = me.hv;
   double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
   const int d = a.deg[i];
   for (int k = 0; k < d; ++k) {
     const int s = k * a.N + i;
     const int j = a.nbr[s];
     const double nx = a.fnx[s], ny = a.fny[s], L = a.flen[s];
-    Side Rs;
-    if (j >= 0) {
-      const double xj = a.xi[j], hsj = a.hstill[j];
-      double hj = xj + hsj, qxj = a.qx[j], qyj = a.qy[j];
-      if (hj <= hsmall) {
-        hj = hsmall;
-        qxj = 0.0;
-        qyj = 0.0;
-      }
-      Rs = Side{xj, hsj, hj, qxj, qyj, a.zb[j]};
-    } else {  // ghost (bc_2D.jl:640-834), internal cell = this cell
-      const int gi = ~j;
-      double hg, qxg, qyg;
-      switch (a.g_kind[gi]) {
-        case HG_BC_INLETQ: {
-          const int b = a.g_bc[gi];
-          const double w = (h > hsmall) ? 1.0 : 0.0;
-          const double v = a.inletQ[b] / a.totalA[b] * a.g_L23[gi] / nman;
-          hg = h;
-          qxg = -h * v * nx * w;
-          qyg = -h * v * ny * w;
-          break;
-        }
-        case HG_BC_EXITH: {
-          const double hx = a.exitWSE[a.g_bc[gi]] - zb;
-          hg = (hx > hsmall) ? hx : hsmall;
-          qxg = qx;
-          qyg = qy;
-          break;
-        }
-        case HG_BC_WALL:
-          hg = h;
-          qxg = -qx;
-          qyg = -qy;
-          break;
-        default: {  // HG_BC_SYMM
-          const double vdn = qx * nx + qy * ny;
-          hg = h;
-          qxg = qx - 2.0 * vdn * nx;
-          qyg = qy - 2.0 * vdn * ny;
-          break;
-        }
-      }
-      const double hsg = a.g_hstill[gi];
-      Rs = Side{hg - hsg, hsg, hg, qxg, qyg, a.g_zb[gi]};
-    }
-    double f0, f1, f2;
-    hg::roe_flux(Ls, Rs, nx, ny, a.g, a.half_g, hsmall, f0, f1, f2);
-    acc0 = acc0 + f0 * L;
-    acc1 = acc1 + f1 * L;
-    acc2 = acc2 + f2 * L;
+    hg::CellQ B;
+    if (j >= 0)
+      B = hg::make_cellq(a.xi[j], a.hstill[j], a.qx[j], a.qy[j], a.zb[j], a.half_g, hsmall);
+    else
+      B = ghost_cellq(a, me, nman, ~j, nx, ny, false, 0.0);
+    double f[3], fb[3];
+    hg::roe_pair<false>(me, B, nx, ny, a.g, a.half_g, hsmall, f, fb);
+    acc0 = acc0 + f[0] * L;
+    acc1 = acc1 + f[1] * L;
+    acc2 = acc2 + f[2] * L;
   }
   const double A = a.area[i];
-  const double r0 = -acc0 / A, r1 = -acc1 / A, r2 = -acc2 / A;
+  const double rA = hg::rcp_est(A);
+  const double r0 = hg::div_est(-acc0, A, rA), r1 = hg::div_est(-acc1, A, rA), r2 = hg::div_est(-acc2, A, rA);
   double s1 = 0.0, s2 = 0.0;
   if (h > hsmall) {  // :463-475
     double fx, fy;
@@ -437,50 +445,8 @@ __global__ __launch_bounds__(T) void k_swe_tile(hg::TileArgs a0) {
       B.s = C[8 * T + ib]; B.p = C[9 * T + ib];
     } else if (type == 1) {
       B = hg::make_cellq(jxi, jhs, jqx, jqy, jzb, a.half_g, hsmall);
-    } else {  // ghost (bc_2D.jl:640-834); its internal cell is A
-      const int gi = rec.ref;
-      double hg_, qxg, qyg;
-      switch (a.g_kind[gi]) {
-        case HG_BC_INLETQ: {
-          const int b = a.g_bc[gi];
-          const double w = (A.h > hsmall) ? 1.0 : 0.0;
-          const double tot = (a.n_inlet > 0) ? tA[(code >> 14) & (kTileInlets - 1)] : a.totalA[b];
-          const double v = a.inletQ[b] / tot * a.g_L23[gi] / a.n[t * T + ia];
-          hg_ = A.h;
-          qxg = -A.h * v * nx * w;
-          qyg = -A.h * v * ny * w;
-          break;
-        }
-        case HG_BC_EXITH: {
-          const double hx = a.exitWSE[a.g_bc[gi]] - A.zb;
-          hg_ = (hx > hsmall) ? hx : hsmall;
-          qxg = A.hu;
-          qyg = A.hv;
-          break;
-        }
-        case HG_BC_WALL:
-          hg_ = A.h;
-          qxg = -A.hu;
-          qyg = -A.hv;
-          break;
-        default: {
-          const double vdn = A.hu * nx + A.hv * ny;
-          hg_ = A.h;
-          qxg = A.hu - 2.0 * vdn * nx;
-          qyg = A.hv - 2.0 * vdn * ny;
-          break;
-        }
-      }
-      B.hs = a.g_hstill[gi];
-      B.xi = hg_ - B.hs;
-      B.h = hg_;
-      B.hu = qxg;
-      B.hv = qyg;
-      B.zb = a.g_zb[gi];
-      B.u = qxg / hg_;
-      B.v = qyg / hg_;
-      B.s = sqrt(hg_ + hg::EPS);
-      B.p = a.half_g * ((B.xi + hg::EPS) * (B.xi + hg::EPS) + 2.0 * B.xi * B.hs);
+    } else {  // ghost; its internal cell is A
+      B = ghost_cellq(a, A, a.n[t * T + ia], rec.ref, nx, ny, a.n_inlet > 0, tA[(code >> 14) & (kTileInlets - 1)]);
     }
     double fa[3], fb[3];
     hg::roe_pair<true>(A, B, nx, ny, a.g, a.half_g, hsmall, fa, fb);
@@ -499,7 +465,8 @@ __global__ __launch_bounds__(T) void k_swe_tile(hg::TileArgs a0) {
       acc2 = acc2 + FL[(2 * MD + k) * T + li];
     }
   }
-  const double r0 = -acc0 / A_i, r1 = -acc1 / A_i, r2 = -acc2 / A_i;
+  const double rA = hg::rcp_est(A_i);
+  const double r0 = hg::div_est(-acc0, A_i, rA), r1 = hg::div_est(-acc1, A_i, rA), r2 = hg::div_est(-acc2, A_i, rA);
   double s1 = 0.0, s2 = 0.0;
   const double h = me.h;
   if (h > hsmall) {
