@@ -346,6 +346,14 @@ struct hg_ctx {
   bool deg_full = false;  // every cell has tileMD faces: the tile kernels need not read deg
   int32_t xcd_chunk = 0;  // identity block -> tile mapping by default (the autotuner re-checks)
   int32_t ncu = 256;      // compute units of the device
+  int32_t max_items = 0;  // work items of the fullest tile
+  // resident runs (k_swe_run): work-groups the device holds at once (0: not
+  // asked yet), off for good once a wait ran out, the exchange ring and its
+  // control word
+  int32_t res_cap = 0;
+  bool res_off = false, res_split = false;
+  unsigned long long* res_ring = nullptr;
+  int32_t* res_ctl = nullptr;
   // the reverse step's tiling (its own tile size; the step kernel's items
   // when those have it, else its own copy built on first use)
   int32_t adj_T_req = 0;  // hg_set_adjoint_tile (0: the library's choice)

@@ -123,6 +123,21 @@ int upload(hg_ctx* ctx, T* dst, const T* src, size_t n) {
 // --------------------------------------------------------------- kernels ---
 
 
+// acc + the first cnt lanes' terms of this wave, one after the other (lanes
+// from cnt on hold +0.0; the terms are not negative, so the zeros that fill
+// the last group of eight change nothing).  A lane read costs two scalar
+// moves; a lane exchange through LDS per term instead took 8.8 us, not 6.9, for
+// a resident step of a 96k-cell channel whose inlet has 69 faces.
+__device__ __forceinline__ double wave_left_fold(double acc, double term, int cnt) {
+  const long long v = __double_as_longlong(term);
+  const int lo = int(v), hi = int(v >> 32);
+  for (int k = 0; k < cnt; k += 8)
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      acc = acc + __hiloint2double(__builtin_amdgcn_readlane(hi, k + u), __builtin_amdgcn_readlane(lo, k + u));
+  return acc;
+}
+
 // Inlet conveyance (bc_2D.jl:640-680): total_A_b = sum over the inlet's
 // faces, in NodeString order, of ((L^(5/3) h_c) / n_c) * wet_c.  The terms
 // are formed in parallel, the sum is a left fold by one lane (the
@@ -167,27 +182,41 @@ __device__ __forceinline__ void store_state(double* p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// A boundary face's ghost state (bc_2D.jl:640-834) as the flux reads it,
-// formed from its internal cell's flux inputs A (Manning n: n_i).  tot_f: the
-// conveyance of an inlet-Q ghost's inlet when the kernel formed it itself
-// (fused), else it is read from a.totalA.  Args: the step kernels' blocks.
+// What a boundary face's ghost state reads besides its cell and the inlet's
+// conveyance: p is the inlet's discharge or the outlet's stage.
+struct GhostFace {
+  int kind, bc;
+  double hs, zb, p, L23;
+};
 template <class Args>
-__device__ __forceinline__ hg::CellQ ghost_cellq(const Args& a, const hg::CellQ& A, double n_i, int gi, double nx,
-                                                 double ny, bool fused, double tot_f) {
-  const double hsmall = a.hsmall;
+__device__ __forceinline__ GhostFace ghost_face(const Args& a, int gi) {
+  GhostFace g;
+  g.kind = a.g_kind[gi];
+  g.bc = a.g_bc[gi];
+  g.hs = a.g_hstill[gi];
+  g.zb = a.g_zb[gi];
+  g.L23 = a.g_L23[gi];
+  g.p = g.kind == HG_BC_INLETQ ? a.inletQ[g.bc] : g.kind == HG_BC_EXITH ? a.exitWSE[g.bc] : 0.0;
+  return g;
+}
+
+// A boundary face's ghost state (bc_2D.jl:640-834) as the flux reads it,
+// formed from its internal cell's flux inputs A (Manning n: n_i); tot: the
+// conveyance of an inlet-Q ghost's inlet.
+__device__ __forceinline__ hg::CellQ ghost_cellq(const GhostFace& g, const hg::CellQ& A, double n_i, double nx,
+                                                 double ny, double tot, double half_g, double hsmall) {
   double h, qx, qy;
-  switch (a.g_kind[gi]) {
+  switch (g.kind) {
     case HG_BC_INLETQ: {
-      const int b = a.g_bc[gi];
       const double w = (A.h > hsmall) ? 1.0 : 0.0;
-      const double v = a.inletQ[b] / (fused ? tot_f : a.totalA[b]) * a.g_L23[gi] / n_i;
+      const double v = g.p / tot * g.L23 / n_i;
       h = A.h;
       qx = -A.h * v * nx * w;
       qy = -A.h * v * ny * w;
       break;
     }
     case HG_BC_EXITH: {
-      const double hx = a.exitWSE[a.g_bc[gi]] - A.zb;
+      const double hx = g.p - A.zb;
       h = (hx > hsmall) ? hx : hsmall;
       qx = A.hu;
       qy = A.hv;
@@ -207,17 +236,17 @@ __device__ __forceinline__ hg::CellQ ghost_cellq(const Args& a, const hg::CellQ&
     }
   }
   hg::CellQ B;
-  B.hs = a.g_hstill[gi];
+  B.hs = g.hs;
   B.xi = h - B.hs;
   B.h = h;
   B.hu = qx;
   B.hv = qy;
-  B.zb = a.g_zb[gi];
+  B.zb = g.zb;
   const double rh = hg::rcp_est(h);
   B.u = hg::div_est(qx, h, rh);
   B.v = hg::div_est(qy, h, rh);
   B.s = hg::sqrt_pos(h + hg::EPS);
-  B.p = a.half_g * ((B.xi + hg::EPS) * (B.xi + hg::EPS) + 2.0 * B.xi * B.hs);
+  B.p = half_g * ((B.xi + hg::EPS) * (B.xi + hg::EPS) + 2.0 * B.xi * B.hs);
   return B;
 }
 
@@ -245,8 +274,10 @@ __global__ __launch_bounds__(kBlock) void k_swe_step(StepArgs a0) {
     hg::CellQ B;
     if (j >= 0)
       B = hg::make_cellq(a.xi[j], a.hstill[j], a.qx[j], a.qy[j], a.zb[j], a.half_g, hsmall);
-    else
-      B = ghost_cellq(a, me, nman, ~j, nx, ny, false, 0.0);
+    else {
+      const GhostFace gf = ghost_face(a, ~j);
+      B = ghost_cellq(gf, me, nman, nx, ny, gf.kind == HG_BC_INLETQ ? a.totalA[gf.bc] : 0.0, a.half_g, hsmall);
+    }
     double f[3], fb[3];
     hg::roe_pair<false>(me, B, nx, ny, a.g, a.half_g, hsmall, f, fb);
     acc0 = acc0 + f[0] * L;
@@ -400,11 +431,7 @@ __global__ __launch_bounds__(T) void k_swe_tile(hg::TileArgs a0) {
           const double w = (h > hsmall) ? 1.0 : 0.0;
           term = a.in_L53[f] * h / a.n[c] * w;
         }
-        const int cnt = min(64, f1 - base);
-        for (int k = 0; k < cnt; ++k) {
-          const double tk = __shfl(term, k, 64);
-          acc = (base + k == f0) ? tk : acc + tk;
-        }
+        acc = wave_left_fold(acc, term, min(64, f1 - base));
       }
       if (li == 0) {
         tA[sl - s0] = acc;
@@ -446,7 +473,11 @@ __global__ __launch_bounds__(T) void k_swe_tile(hg::TileArgs a0) {
     } else if (type == 1) {
       B = hg::make_cellq(jxi, jhs, jqx, jqy, jzb, a.half_g, hsmall);
     } else {  // ghost; its internal cell is A
-      B = ghost_cellq(a, A, a.n[t * T + ia], rec.ref, nx, ny, a.n_inlet > 0, tA[(code >> 14) & (kTileInlets - 1)]);
+      const GhostFace gf = ghost_face(a, rec.ref);
+      const double tot = gf.kind != HG_BC_INLETQ ? 0.0
+                         : a.n_inlet > 0         ? tA[(code >> 14) & (kTileInlets - 1)]
+                                                 : a.totalA[gf.bc];
+      B = ghost_cellq(gf, A, a.n[t * T + ia], nx, ny, tot, a.half_g, hsmall);
     }
     double fa[3], fb[3];
     hg::roe_pair<true>(A, B, nx, ny, a.g, a.half_g, hsmall, fa, fb);
@@ -499,6 +530,289 @@ __global__ __launch_bounds__(T) void k_swe_tile(hg::TileArgs a0) {
     a.xo[i] = d0;
     a.qxo[i] = d1;
     a.qyo[i] = d2;
+  }
+}
+
+// ---- resident run: many steps of a small mesh in one launch.
+// A step of a mesh of up to about 130,000 cells is one dependent chain --
+// launch, cell loads, items, neighbours, two barriers -- of 7 us and more,
+// however few cells it has; the chip is mostly idle.  Here every tile keeps
+// its cells, their constants and its work items in registers for the whole
+// run, and only the cells that another tile reads travel through memory.
+// Per step: 1,000 quads 7.4 -> 2.5 us; a closed 59k-triangle mesh about 7 ->
+// 3.7 us; channels, whose inlet tiles also wait for all of the inlet's cells
+// and fold their conveyance, 3.5 us at 1,300 cells, 4.0 at 20k, 6.5 at 96k
+// (8.7 us with one launch per step) and 6.8 at 126k.  Larger meshes do not fit
+// on the chip in this form.
+//
+// Exchange: a published cell's new state goes to slot (s + 1) % 4 of a ring of
+// four states, whose entries hold kResEmpty (a signalling NaN no arithmetic
+// produces) until then; a reader polls the values themselves, each a relaxed
+// agent-scope access, so one memory trip carries data and readiness.  When a
+// tile publishes state s + 1 it has read its neighbours' state s, hence they
+// have read its state s - 1 (face and inlet neighbours are mutual): it resets
+// that slot, which state s + 3 takes, and the wait before publishing s + 2
+// completes the reset before any reader can poll for s + 3.
+//
+// All tiles must be on the device together: the host launches no more
+// work-groups than fit, and every wait is bounded (kResTicks); a wait that
+// runs out raises ctl[0], every tile then leaves, and the host repeats the
+// steps with one launch each (the input state is not written).
+//
+// The first T work-items own the cells; the cross-tile items go to others, so
+// a poll is not queued behind the publishing stores; the last wave forms the
+// inlet conveyances; the cells' friction is formed while the faces are
+// waited for.  Each work-item takes at most one item: tiles of triangles hold
+// up to 256, others up to 320 (fuller tiles are not run this way).  SPLIT
+// (few tiles): the cells' work-items take no items, so the friction is off the
+// step's critical path; else they take the items that the rest leave.
+constexpr unsigned long long kResEmpty = 0x7ff4c0de5ea1ed01ull;
+constexpr long long kResTicks = 100000000;  // wall_clock64 ticks (100 MHz): 1 s
+constexpr int kResT = 128;                  // cells per tile
+constexpr int64_t kResSteps = 4096;         // steps per launch
+
+struct ResArgs {
+  unsigned long long* ring;  // [4][3][N]
+  int32_t* ctl;              // [0]: a wait ran out
+  int64_t ns;
+  const int32_t* nbr;        // ELL, for the published cells
+  // optional record of the run (the adjoint's forward sweep): states 0 .. ns
+  // ([ns + 1][3][N]; state 0 is there already), clamps [ns][N], conveyances
+  double* rec;
+  uint8_t* rec_clamp;
+  double* rec_totalA;
+  int32_t n_inlet_all;
+};
+
+__device__ __forceinline__ unsigned long long res_peek(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void res_put(unsigned long long* p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The NC values p, p + stride, ...: waits until none is empty.  False when
+// the wait ran out here or elsewhere.
+template <int NC>
+__device__ __forceinline__ bool res_poll(const unsigned long long* p, int64_t stride, int32_t* ctl, double (&v)[NC]) {
+  long long t0 = 0;
+  for (int n = 0;; ++n) {
+    unsigned long long u[NC];
+    bool ready = true;
+    for (int c = 0; c < NC; ++c) u[c] = res_peek(p + c * stride);
+    for (int c = 0; c < NC; ++c) ready = ready && u[c] != kResEmpty;
+    if (ready) {
+      for (int c = 0; c < NC; ++c) v[c] = __longlong_as_double((long long)u[c]);
+      return true;
+    }
+    if ((n & 63) == 63) {
+      const long long t = wall_clock64();
+      if (n == 63) t0 = t;
+      if (t - t0 > kResTicks) __hip_atomic_store(ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__hip_atomic_load(ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        for (int c = 0; c < NC; ++c) v[c] = 0.0;
+        return false;
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_res_init(int64_t n, unsigned long long* ring, int32_t* ctl) {
+  const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (i < n) ring[i] = kResEmpty;
+  if (i == 0) *ctl = 0;
+}
+
+constexpr int res_items(int MD) { return MD == 3 ? 256 : 320; }
+constexpr int res_threads(int MD, bool split) { return res_items(MD) + (split ? kResT : 0); }
+constexpr int kResIn = 128;  // inlet faces whose constants a tile keeps in LDS
+
+template <int MD, bool SPLIT>
+__global__ __launch_bounds__(res_threads(MD, SPLIT), SPLIT ? 3 : 4) void k_swe_run(hg::TileArgs a, ResArgs R) {
+  constexpr int T = kResT, NT = res_threads(MD, SPLIT);
+  extern __shared__ double lds[];
+  double* C = lds;                // 10 x T cell quantities
+  double* FL = lds + 10 * T;      // 3 x MD x T face contributions
+  double* tA = FL + 3 * MD * T;   // conveyance of the tile's inlets (kTileInlets)
+  double* in_c = tA + kTileInlets;  // 3 x kResIn: L^(5/3), h_still, n of the first inlet's faces
+  int32_t* in_i = reinterpret_cast<int32_t*>(in_c + 3 * kResIn);  // and their cells
+  int32_t* stop = in_i + kResIn;
+  const int t = blockIdx.x, tid = threadIdx.x, i = t * T + tid;
+  const bool own = tid < T && i < a.N;
+  const int64_t N = a.N;
+  const double hsmall = a.hsmall;
+  double xi = 0.0, qx = 0.0, qy = 0.0, hs = 0.0, zb = 0.0, n = 0.0, S0x = 0.0, S0y = 0.0, A = 1.0, dti = a.dt;
+  int d = 0;
+  bool pub = false;  // read by another tile, or an inlet cell
+  if (own) {
+    xi = a.xi[i]; qx = a.qx[i]; qy = a.qy[i];
+    hs = a.hstill[i]; zb = a.zb[i]; n = a.n[i]; S0x = a.S0x[i]; S0y = a.S0y[i]; A = a.area[i];
+    d = a.deg ? a.deg[i] : MD;
+    if (a.dtc) dti = a.dtc[i];
+    for (int k = 0; k < d; ++k) {
+      const int j = R.nbr[k * N + i];
+      pub = pub || (j >= 0 ? j / T != t : a.g_kind[~j] == HG_BC_INLETQ);
+    }
+  }
+  // this work-item's item (the cross-tile ones are the first of the list)
+  const int it = a.items.off[t] + (SPLIT ? tid - T : (tid + NT - T) % NT);
+  const bool has = it >= a.items.off[t] && it < a.items.off[t + 1];
+  hg::ItemRec rec{};
+  if (has) rec = load_item(a.items, it, a.items.x0[t]);
+  const int code = rec.code;
+  const int ia = code & 1023, ka = (code >> 10) & 15, ib = (code >> 14) & 1023, kb = (code >> 24) & 15;
+  const int type = has ? (code >> 28) & 3 : 3;
+  GhostFace gf{};  // the other side's constants: a cross-tile neighbour's h_still and zb, or the ghost's
+  double gn = 1.0;
+  if (type == 1) {
+    gf.hs = a.hstill[rec.ref];
+    gf.zb = a.zb[rec.ref];
+  } else if (type == 2) {
+    gf = ghost_face(a, rec.ref);
+    gn = a.n[t * T + ia];
+  }
+  const int in0 = a.n_inlet > 0 ? a.tile_in_off[t] : 0, in1 = a.n_inlet > 0 ? a.tile_in_off[t + 1] : 0;
+  int bl0 = 0, fl0 = 0, fl1 = 0;  // the tile's first inlet
+  if (in1 > in0) {
+    bl0 = a.tile_in_list[in0];
+    fl0 = a.in_off[bl0];
+    fl1 = a.in_off[bl0 + 1];
+    for (int f = tid; f < min(kResIn, fl1 - fl0); f += NT) {
+      const int c = a.in_cell[fl0 + f];
+      in_i[f] = c;
+      in_c[f] = a.in_L53[fl0 + f];
+      in_c[kResIn + f] = a.hstill[c];
+      in_c[2 * kResIn + f] = a.n[c];
+    }
+  }
+  if (tid == 0) *stop = 0;
+  __syncthreads();
+
+  for (int64_t s = 0; s < R.ns; ++s) {
+    const unsigned long long* slot = R.ring + (s & 3) * 3 * N;
+    hg::CellQ me{};
+    if (own) {
+      me = hg::make_cellq(xi, hs, qx, qy, zb, a.half_g, hsmall);
+      C[0 * T + tid] = me.xi; C[1 * T + tid] = me.hs; C[2 * T + tid] = me.h; C[3 * T + tid] = me.hu;
+      C[4 * T + tid] = me.hv; C[5 * T + tid] = me.zb; C[6 * T + tid] = me.u; C[7 * T + tid] = me.v;
+      C[8 * T + tid] = me.s; C[9 * T + tid] = me.p;
+    }
+    if (in1 > in0 && tid >= NT - 64) {  // inlet conveyances (as in k_swe_tile)
+      const int l = tid & 63;
+      for (int sl = in0; sl < in1; ++sl) {
+        const int b = sl == in0 ? bl0 : a.tile_in_list[sl];
+        const int f0 = sl == in0 ? fl0 : a.in_off[b], f1 = sl == in0 ? fl1 : a.in_off[b + 1];
+        double acc = 0.0;
+        bool ok = true;
+        for (int base = f0; base < f1; base += 128) {  // two faces per lane in flight
+          double term[2] = {0.0, 0.0};
+          const bool kept = sl == in0 && base == f0;
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            const int f = base + 64 * r + l, k = 64 * r + l;
+            if (f >= f1) continue;
+            const int c = kept ? in_i[k] : a.in_cell[f];
+            double x[1];
+            if (s == 0)
+              x[0] = a.xi[c];
+            else if (!res_poll<1>(slot + c, N, R.ctl, x))
+              ok = false;
+            double h = x[0] + (kept ? in_c[kResIn + k] : a.hstill[c]);
+            if (h <= hsmall) h = hsmall;
+            const double w = (h > hsmall) ? 1.0 : 0.0;
+            term[r] = (kept ? in_c[k] : a.in_L53[f]) * h / (kept ? in_c[2 * kResIn + k] : a.n[c]) * w;
+          }
+          acc = wave_left_fold(acc, term[0], min(64, f1 - base));
+          if (f1 - base > 64) acc = wave_left_fold(acc, term[1], min(64, f1 - base - 64));
+        }
+        if (__ballot(!ok)) {
+          *stop = 1;
+        } else if (l == 0) {
+          tA[sl - in0] = acc;
+          if (R.rec_totalA) R.rec_totalA[s * R.n_inlet_all + b] = acc;  // every tile of inlet b writes the same value
+          if (!(acc > 1e-10)) a.flag[0] = 1;
+        }
+      }
+    }
+    __syncthreads();
+    if (has) {
+      hg::CellQ P, Q;
+      P.xi = C[0 * T + ia]; P.hs = C[1 * T + ia]; P.h = C[2 * T + ia]; P.hu = C[3 * T + ia];
+      P.hv = C[4 * T + ia]; P.zb = C[5 * T + ia]; P.u = C[6 * T + ia]; P.v = C[7 * T + ia];
+      P.s = C[8 * T + ia]; P.p = C[9 * T + ia];
+      if (type == 0) {
+        Q.xi = C[0 * T + ib]; Q.hs = C[1 * T + ib]; Q.h = C[2 * T + ib]; Q.hu = C[3 * T + ib];
+        Q.hv = C[4 * T + ib]; Q.zb = C[5 * T + ib]; Q.u = C[6 * T + ib]; Q.v = C[7 * T + ib];
+        Q.s = C[8 * T + ib]; Q.p = C[9 * T + ib];
+      } else if (type == 1) {
+        const int j = rec.ref;
+        double v[3];
+        if (s == 0) {
+          v[0] = a.xi[j]; v[1] = a.qx[j]; v[2] = a.qy[j];
+        } else if (!res_poll<3>(slot + j, N, R.ctl, v)) {
+          *stop = 1;
+        }
+        Q = hg::make_cellq(v[0], gf.hs, v[1], v[2], gf.zb, a.half_g, hsmall);
+      } else {
+        const double tot = gf.kind == HG_BC_INLETQ ? tA[(code >> 14) & (kTileInlets - 1)] : 0.0;
+        Q = ghost_cellq(gf, P, gn, rec.nx, rec.ny, tot, a.half_g, hsmall);
+      }
+      double fa[3], fb[3];
+      hg::roe_pair<true>(P, Q, rec.nx, rec.ny, a.g, a.half_g, hsmall, fa, fb);
+      if (type == 0)
+        for (int c = 0; c < 3; ++c) FL[(c * MD + kb) * T + ib] = fb[c] * rec.len;
+      for (int c = 0; c < 3; ++c) FL[(c * MD + ka) * T + ia] = fa[c] * rec.len;
+    }
+    double s1 = 0.0, s2 = 0.0;
+    if (own && me.h > hsmall) {
+      double fx, fy;
+      hg::friction(a.g, a.kn2, hsmall, me.h, me.hu, me.hv, n, fx, fy);
+      s1 = a.g * xi * S0x - fx;
+      s2 = a.g * xi * S0y - fy;
+    }
+    const double rA = hg::rcp_est(A);
+    __syncthreads();
+    if (*stop) return;  // the same for the whole tile: set before the barrier only
+    if (!own) continue;
+    double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
+    for (int k = 0; k < MD; ++k) {  // local face order
+      if (k < d) {
+        acc0 = acc0 + FL[(0 * MD + k) * T + tid];
+        acc1 = acc1 + FL[(1 * MD + k) * T + tid];
+        acc2 = acc2 + FL[(2 * MD + k) * T + tid];
+      }
+    }
+    xi = xi + dti * (hg::div_est(-acc0, A, rA) + 0.0);
+    qx = qx + dti * (hg::div_est(-acc1, A, rA) + s1);
+    qy = qy + dti * (hg::div_est(-acc2, A, rA) + s2);
+    const bool dry = xi < hsmall;
+    if (dry) {
+      xi = hsmall;
+      qx = 0.0;
+      qy = 0.0;
+    }
+    if (pub && s + 1 < R.ns) {
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the last step's reset is done (lgkmcnt, expcnt not waited on)
+      unsigned long long* o = R.ring + ((s + 1) & 3) * 3 * N + i;
+      unsigned long long* e = R.ring + ((s + 3) & 3) * 3 * N + i;
+      res_put(o, __double_as_longlong(xi));
+      res_put(o + N, __double_as_longlong(qx));
+      res_put(o + 2 * N, __double_as_longlong(qy));
+      for (int c = 0; c < 3; ++c) res_put(e + c * N, kResEmpty);
+    }
+    if (!(isfinite(xi) && isfinite(qx) && isfinite(qy))) a.flag[1] = 1;  // checked after the stepping call
+    if (R.rec) {
+      double* q = R.rec + (s + 1) * 3 * N + i;
+      q[0] = xi;
+      q[N] = qx;
+      q[2 * N] = qy;
+      R.rec_clamp[s * N + i] = dry ? 1 : 0;
+    }
+  }
+  if (own) {
+    a.xo[i] = xi;
+    a.qxo[i] = qx;
+    a.qyo[i] = qy;
   }
 }
 
@@ -2209,6 +2523,11 @@ int free_items(hg_ctx* ctx, hg::ItemTable& d) {
   return rc;
 }
 
+size_t res_lds_bytes(int MD) {
+  return size_t(10 * kResT + 3 * MD * kResT + kTileInlets + 3 * kResIn) * sizeof(double) +
+         (kResIn + 1) * sizeof(int32_t);
+}
+
 size_t tile_lds_bytes(int T, int maxdeg) {
   return size_t(10 * T + 3 * maxdeg * T + kTileInlets) * sizeof(double);
 }
@@ -2557,6 +2876,96 @@ int enqueue_step_p(hg_ctx* ctx, const double* const in[3], double* const out[3],
       hipLaunchKernelGGL(k_swe_step<false>, dim3(grid_of(ctx->N)), dim3(kBlock), 0, ctx->stream, a);
   }
   HG_TRY(hipGetLastError());
+  return HG_OK;
+}
+
+// ---- resident run, host side
+
+// Work-groups of resident runs in flight on each device over the process's
+// contexts: a run is started only while all of them fit together.
+std::mutex g_res_mu;
+int g_res_groups[kMaxDevices] = {};
+
+// Tiles of a resident run that the device surely holds at once.  A tile's
+// waves need not spread evenly over a CU's four SIMDs (two tiles of six waves
+// each were not resident together where three waves fit per SIMD), so each
+// tile counts with its fullest SIMD.
+template <int MD, bool SPLIT>
+int res_capacity(hg_ctx* ctx) {
+  constexpr int waves = res_threads(MD, SPLIT) / 64, per_simd = SPLIT ? 3 : 4;
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_swe_run<MD, SPLIT>, 64 * waves, res_lds_bytes(MD)) !=
+      hipSuccess)
+    return 0;
+  return std::min(per_cu, per_simd / ((waves + 3) / 4)) * ctx->ncu;
+}
+
+template <int MD, bool SPLIT>
+void launch_run(hg_ctx* ctx, const hg::TileArgs& a, const ResArgs& R) {
+  hipLaunchKernelGGL((k_swe_run<MD, SPLIT>), dim3(ctx->ntiles), dim3(res_threads(MD, SPLIT)), res_lds_bytes(MD),
+                     ctx->stream, a, R);
+}
+
+// Whether nsteps steps may run resident: one field, the default tiling of
+// small meshes, at most one item per work-item and 64 inlets per tile, a
+// roughness that does not change with the state, and steps enough to pay for
+// the ring's initialisation.
+bool res_usable(hg_ctx* ctx, int64_t nsteps) {
+  return ctx->tiled && !ctx->res_off && ctx->K == 1 && nsteps >= 4 && ctx->tileT == kResT && ctx->tileMD <= 4 &&
+         ctx->max_items <= res_items(ctx->tileMD) && (ctx->n_inlet == 0 || ctx->fuse_inlet) && !ctx->ude_prec &&
+         ctx->nlaw.kind == hg::NLAW_OFF && ctx->lux.choice == hg::LUX_OFF && ctx->device < kMaxDevices;
+}
+
+// nsteps steps from state arrays `in` to `out` (not the same), optionally
+// recorded.  *done: false when the run was not started or a wait ran out
+// (nothing the caller reads has been written then).  Synchronizes.
+int res_run(hg_ctx* ctx, const double* const in[3], double* const out[3], double dt, int64_t nsteps, double* rec,
+            uint8_t* rec_clamp, double* rec_totalA, bool* done) {
+  *done = false;
+  const bool tri = ctx->tileMD == 3;
+  if (!ctx->res_cap) {
+    ctx->res_cap = tri ? res_capacity<3, true>(ctx) : res_capacity<4, true>(ctx);
+    ctx->res_split = ctx->ntiles <= ctx->res_cap;
+    if (!ctx->res_split) ctx->res_cap = tri ? res_capacity<3, false>(ctx) : res_capacity<4, false>(ctx);
+    if (ctx->res_cap < ctx->ntiles) {
+      ctx->res_off = true;
+      return HG_OK;
+    }
+  }
+  if (!ctx->res_ring) {
+    int rc = dalloc(ctx, &ctx->res_ring, size_t(12) * ctx->N);
+    if (!rc) rc = dalloc(ctx, &ctx->res_ctl, 1);
+    if (rc) return rc;
+  }
+  {
+    std::lock_guard<std::mutex> g(g_res_mu);
+    if (g_res_groups[ctx->device] + ctx->ntiles > ctx->res_cap) return HG_OK;
+    g_res_groups[ctx->device] += ctx->ntiles;
+  }
+  const int64_t nring = int64_t(12) * ctx->N;
+  hipLaunchKernelGGL(k_res_init, dim3(grid_of(nring)), dim3(kBlock), 0, ctx->stream, nring, ctx->res_ring,
+                     ctx->res_ctl);
+  hg::TileArgs a = make_tile_args_p(ctx, in, out, dt);
+  ResArgs R{ctx->res_ring, ctx->res_ctl, nsteps, ctx->nbr, rec, rec_clamp, rec_totalA, ctx->n_inlet};
+  if (tri)
+    ctx->res_split ? launch_run<3, true>(ctx, a, R) : launch_run<3, false>(ctx, a, R);
+  else
+    ctx->res_split ? launch_run<4, true>(ctx, a, R) : launch_run<4, false>(ctx, a, R);
+  int32_t ran_out = 0;
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(&ran_out, ctx->res_ctl, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  {
+    std::lock_guard<std::mutex> g(g_res_mu);
+    g_res_groups[ctx->device] -= ctx->ntiles;
+  }
+  HG_TRY(e);
+  if (ran_out) {  // the device was shared with something else: one launch per step from here on
+    ctx->res_off = true;
+    return HG_OK;
+  }
+  *done = true;
   return HG_OK;
 }
 
@@ -2939,9 +3348,22 @@ int forward_checkpointed(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck) {
       if (rc) return rc;
     }
   }
+  const int64_t ns = nsteps - (nseg - 1) * kck;
+  bool done = false;
+  if (res_usable(ctx, ns) && ns <= kResSteps) {
+    const double* in[3] = {ctx->st[ctx->cur][0], ctx->st[ctx->cur][1], ctx->st[ctx->cur][2]};
+    for (int c = 0; c < 3; ++c)
+      HG_TRY(hipMemcpyAsync(seg_state(ctx, 0, c, 0), in[c], N * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
+    int rc = res_run(ctx, in, ctx->st[1 - ctx->cur], dt, ns, ctx->adj_seg[0], ctx->adj_mask[0], seg_totalA(ctx, 0, 0),
+                     &done);
+    if (rc) return rc;
+    if (done) {
+      ctx->cur = 1 - ctx->cur;
+      return HG_OK;
+    }
+  }
   int rc = recompute_segment(ctx, dt, nsteps, kck, nseg - 1, 0, ctx->stream);
   if (rc) return rc;
-  const int64_t ns = nsteps - (nseg - 1) * kck;
   for (int c = 0; c < 3; ++c)
     HG_TRY(hipMemcpyAsync(ctx->st[0][c], seg_state(ctx, ns, c, 0), N * sizeof(double), hipMemcpyDeviceToDevice,
                           ctx->stream));
@@ -3434,6 +3856,8 @@ int setup_tiles(hg_ctx* ctx, int T) {
   ctx->tileT = T;
   ctx->ntiles = int32_t(ntiles);
   ctx->fuse_inlet = ctx->n_inlet > 0 && tb.max_inlets <= kTileInlets;
+  ctx->max_items = 0;
+  for (int64_t t = 0; t < ntiles; ++t) ctx->max_items = std::max(ctx->max_items, tb.off[t + 1] - tb.off[t]);
   return HG_OK;
 }
 
@@ -3462,6 +3886,16 @@ int ensure_graph(hg_ctx* ctx, double dt) {
 
 // Advance the device state nsteps (no host sync at the end).
 int advance_async(hg_ctx* ctx, double dt, int64_t nsteps) {
+  while (res_usable(ctx, nsteps)) {  // a small mesh: runs of steps in one launch each
+    const int64_t ns = std::min<int64_t>(nsteps, kResSteps);
+    const double* in[3] = {ctx->st[ctx->cur][0], ctx->st[ctx->cur][1], ctx->st[ctx->cur][2]};
+    bool done = false;
+    int rc = res_run(ctx, in, ctx->st[1 - ctx->cur], dt, ns, nullptr, nullptr, nullptr, &done);
+    if (rc) return rc;
+    if (!done) break;
+    ctx->cur = 1 - ctx->cur;
+    nsteps -= ns;
+  }
   if (nsteps <= 0) return HG_OK;
   if (ctx->cur == 1) {
     int rc = enqueue_step(ctx, 1, 0, dt, true);

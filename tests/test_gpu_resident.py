@@ -1,0 +1,144 @@
+"""Resident runs (many steps of a small mesh in one launch) against the
+per-cell kernel, one launch per step, bit for bit: the two form every value
+with the same operations in the same order, so the tolerance is zero.
+
+Sizes around one tile of 128 cells and several tiles, triangles, quads and a
+mix, closed domains and inlets (within one tile, over several, two on one
+cell), wet / dry fronts, per-instance time steps, recorded runs, and contexts
+on several threads that do not fit on the device together.
+"""
+import threading
+
+import numpy as np
+import pytest
+
+from hgswe import capi, cases
+from hgswe import mesh as hm
+
+pytestmark = pytest.mark.gpu
+
+
+def channel(n, seed=3, **kw):
+    return cases.channel(n, seed=seed, Lx=max(30.0, 0.25 * n ** 0.5 * 10), Ly=max(6.0, 0.025 * n ** 0.5 * 10),
+                         Q_in=2.0, n_bumps=2, **kw)
+
+
+def mixed(n_quads, seed):
+    nx = max(2, int(round((4.0 * n_quads) ** 0.5)))
+    xy, quads, side = cases.rect_quads(10.0 * nx, 10.0 * max(1, n_quads // nx), nx, max(1, n_quads // nx))
+    rng = np.random.default_rng(seed)
+    cells = []
+    for a, b, c, d in quads:
+        cells += [[a, b, c, -1], [a, c, d, -1]] if rng.random() < 0.5 else [[a, b, c, d]]
+    m = hm.build_mesh(xy, np.array(cells), {1: side["left"], 2: side["right"], 3: side["bottom"], 4: side["top"]},
+                      {1: "INLET-Q", 2: "EXIT-H", 3: "WALL", 4: "SYMM"})
+    zb = 0.2 * rng.random(m.n_cells)
+    zg, S0x, S0y = hm.bed_data(m, zb)
+    h = 2.0 + 0.2 * rng.random(m.n_cells)
+    hs = np.full(m.n_cells, 0.3)
+    c = cases.Case(name="mixed", mesh=m, hstill=hs, hstill_ghost=hs[m.ghost_cell], zb=zb, zb_ghost=zg, S0x=S0x, S0y=S0y,
+                   n=rng.uniform(0.02, 0.05, m.n_cells), inletQ=np.array([3.0]), exitWSE=np.array([2.1]),
+                   Q0=np.concatenate([h - hs, np.zeros(2 * m.n_cells)]), dt=0.0, nsteps=0)
+    c.dt = cases.cfl_dt(c, 0.3)
+    return c
+
+
+def check(c, steps, ctx=None, dts=None):
+    ctx, ref = ctx or capi.Context(c), capi.Context(c, cell_kernel=True)
+    if dts is not None:
+        ctx.batch_set_dt(dts)
+        ref.batch_set_dt(dts)
+    a, b = ctx.step(c.Q0, c.dt, steps), ref.step(c.Q0, c.dt, steps)
+    assert np.all(np.isfinite(b)) and (c.N == 1 or not np.array_equal(b, c.Q0))
+    assert np.array_equal(a, b)
+    return ctx
+
+
+@pytest.mark.parametrize("nx,ny", [(1, 1), (4, 3), (16, 8), (43, 3), (32, 4), (100, 10)])
+@pytest.mark.parametrize("steps", [4, 5, 6, 7, 33])
+def test_closed_quads(nx, ny, steps):
+    check(cases.dam_break(nx=nx, ny=ny), steps)
+
+
+@pytest.mark.parametrize("n", [40, 126, 260, 1100, 9000, 40000])
+def test_channel_triangles(n):
+    c = channel(n)
+    ctx = check(c, 40)
+    ctx.upload(c.Q0)  # in pieces: each run starts from the other state buffer
+    for k in (7, 4, 3, 26):
+        ctx.advance(c.dt, k)
+    assert np.array_equal(ctx.download(), ctx.step(c.Q0, c.dt, 40))
+
+
+@pytest.mark.parametrize("n", [30, 400, 3000])
+def test_mixed_mesh(n):
+    check(mixed(n, n), 30)
+
+
+def test_no_renumbering():
+    """Cells in a random order: tiles of up to three cross-tile faces per cell are run with one launch per step."""
+    c = channel(800)
+    check(c, 20, ctx=capi.Context(c, reorder=False))
+
+
+def test_wet_dry_fronts():
+    c = cases.channel(6_000, seed=12, Lx=1500.0, Ly=150.0, Q_in=60.0)
+    x = c.mesh.centroid[:, 0]
+    Q = c.Q0.copy()
+    Q[:c.N] = np.where(x < 500.0, np.maximum(c.h_small, 2.2 - c.zb), c.h_small) - c.hstill
+    check(c.copy_fields(Q0=Q, dt=cases.cfl_dt(c, 0.4, Q)), 60)
+
+
+def test_batch_with_own_time_steps():
+    parts = [channel(n, seed=n) for n in (90, 700, 300)]
+    c = cases.concat(parts)
+    check(c, 25, dts=[p.dt * f for p, f in zip(parts, (0.5, 0.8, 0.9))])
+    check(c, 25)
+
+
+@pytest.mark.parametrize("kck", [0, 20, 7])
+def test_recorded_run(kck):
+    """The gradient through a recorded resident run is the one through single launches."""
+    c = channel(2500)
+    probe = np.arange(0, c.N, 50, dtype=np.int32)
+    target = (c.Q0[:c.N] + c.hstill + c.zb)[probe] + 0.01
+    other = capi.Context(c)
+    other.set_tile_config(256)  # not the resident tiling
+    a = capi.Context(c).grad_probes(c.Q0, c.dt, 20, kck, probe, target)
+    b = other.grad_probes(c.Q0, c.dt, 20, 5, probe, target)
+    assert a[0] == b[0]
+    for x, y in zip(a[1:], b[1:]):
+        assert np.array_equal(x, y)
+
+
+def test_errors_are_reported():
+    c = channel(1100)
+    Q = c.Q0.copy()
+    Q[:c.N] = c.h_small - c.hstill  # a dry inlet has no conveyance
+    with pytest.raises(capi.HGError) as e:
+        capi.Context(c).step(Q, c.dt, 10)
+    assert e.value.code == capi.HG_ERR_CONVEYANCE
+    Q = c.Q0.copy()
+    Q[c.N // 2] = np.nan
+    ctx = capi.Context(c)
+    with pytest.raises(capi.HGError) as e:
+        ctx.step(Q, c.dt, 10)
+    assert e.value.code == capi.HG_ERR_NONFINITE
+    assert np.array_equal(ctx.step(c.Q0, c.dt, 10), capi.Context(c, cell_kernel=True).step(c.Q0, c.dt, 10))
+
+
+def test_threads_share_the_device():
+    """Three contexts on three threads, more tiles than the device holds at once: those that do not fit step with
+    single launches, and every result is the one of a run alone."""
+    c = channel(90_000)
+    ref = capi.Context(c).step(c.Q0, c.dt, 60)
+    out = [None] * 3
+
+    def work(k):
+        ctx = capi.Context(c)
+        out[k] = [ctx.step(c.Q0, c.dt, 60) for _ in range(4)]
+
+    th = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    [t.start() for t in th]
+    [t.join() for t in th]
+    assert all(np.array_equal(q, ref) for qs in out for q in qs)
