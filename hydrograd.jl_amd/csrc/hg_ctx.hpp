@@ -354,6 +354,9 @@ struct hg_ctx {
   bool res_off = false, res_split = false;
   unsigned long long* res_ring = nullptr;
   int32_t* res_ctl = nullptr;
+  int32_t adj_res_cap = 0;  // the same for the reverse run, its rings and the sums it writes
+  unsigned long long* adj_ring = nullptr;
+  double* adj_sums = nullptr;
   // the reverse step's tiling (its own tile size; the step kernel's items
   // when those have it, else its own copy built on first use)
   int32_t adj_T_req = 0;  // hg_set_adjoint_tile (0: the library's choice)

@@ -1055,7 +1055,7 @@ __device__ __forceinline__ void adj_ghost_route(const hg::AdjArgs& a, const hg::
       U.h += hgb + Bb.hu * (-v * nx * w) + Bb.hv * (-v * ny * w);
       const double vb = Bb.hu * (-me.h * nx * w) + Bb.hv * (-me.h * ny * w);
       nb += vb * (-v / n_i);
-      a.vbar[gi] = vb;
+      store_state(a.vbar + gi, vb);  // at device scope: other tiles of a resident run poll it
       break;
     }
     case HG_BC_EXITH: {  // h_g = max(h_small, WSE - zb_cell), q_g = q
@@ -1508,6 +1508,271 @@ __global__ __launch_bounds__(T, 3) void k_adj_tile(hg::AdjArgs a0) {
   ca.y2 = STEP ? dti * lt2 : lt2;
   // the slots carry xi + h already (h-bar only where the cell is wet)
   adj_finish_store<STEP>(a, i, ca, fin, uxh, 0.0, uqx, uqy, nb, zbb);
+}
+
+// Reverse mode of a resident run: R.ns steps of k_adj_tile and k_inlet_adj in
+// one launch over tiles of 128 cells, with the values they form, in their
+// order (same bits).  A tile keeps its cells' cotangents and sums in
+// registers and reads ahead the recorded state of the next step; the border
+// cells' cotangents and the inlet ghosts' velocity cotangents travel through
+// rings as the forward run's states do (see k_swe_run).  Sums are written to
+// arrays of their own (o_*), which the host takes over when the run is done.
+// One launch per step took 8.5 us for the tiles and 2.6 us for the inlets, of
+// which about 3 us and 1 us were launch and first loads; a step takes 4.6 us
+// here on 1,000 quads, 6.0 on a 1,300-cell channel (its inlet tiles exchange
+// twice per step) and 6.4 on 59k triangles.  Up to 512 tiles: the registers
+// that hold the cells allow two tiles per CU.
+struct AdjRunArgs {
+  unsigned long long* ring;   // [4][3][N] cotangents
+  unsigned long long* vring;  // [4][G] inlet ghost velocity cotangents
+  int32_t* ctl;
+  int64_t ns, G;
+  const double* rec;          // [ns][3][N] states
+  const uint8_t* rec_clamp;   // [ns][N]
+  const double* rec_totalA;   // [ns][n_inlet]
+  int32_t n_inlet;
+  const int32_t* tile_in_off;
+  const int32_t* tile_in_list;
+  const int32_t* in_off;
+  const hg::InletFaceRec* in_rec;
+  const double* Qbar;
+  double *o_nbar, *o_zbbar, *o_S0bar, *o_Qbar;
+};
+
+template <int MD>
+__global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(hg::AdjArgs a, AdjRunArgs R) {
+  constexpr int T = kResT, NT = res_items(MD);
+  extern __shared__ double lds[];
+  double* C = lds;                                         // kAdjRows x T
+  double* S = lds + kAdjRows * T;                          // 4 x MD x T
+  double* sA = S + 4 * MD * T;                             // 256
+  double* sQ = sA + 256;                                   // 256
+  double* qa = sQ + 256;                                   // kTileInlets: the inlets' discharge cotangents
+  int32_t* Xm = reinterpret_cast<int32_t*>(qa + kTileInlets);  // T
+  int32_t* stop = Xm + T;
+  const int t = blockIdx.x, tid = threadIdx.x, i = t * T + tid;
+  const bool own = tid < T && i < a.N;
+  const int64_t N = a.N;
+  const double hsmall = a.hsmall;
+  double hs = 0.0, zb = 0.0, n = 0.0, S0x = 0.0, S0y = 0.0, A = 1.0, dti = a.dt;
+  double l0 = 0.0, l1 = 0.0, l2 = 0.0, nbar = 0.0, zbbar = 0.0, S0bx = 0.0, S0by = 0.0;
+  int d = 0;
+  bool pub = false;  // read by another tile
+  if (own) {
+    hs = a.hstill[i]; zb = a.zb[i]; n = a.n[i]; S0x = a.S0x[i]; S0y = a.S0y[i]; A = a.area[i];
+    d = a.deg ? a.deg[i] : MD;
+    if (a.dtc) dti = a.dtc[i];
+    l0 = a.lx[i]; l1 = a.lqx[i]; l2 = a.lqy[i];
+    if (a.nbar) nbar = a.nbar[i];
+    if (a.zbbar) {
+      zbbar = a.zbbar[i];
+      S0bx = a.S0bar[i];
+      S0by = a.S0bar[N + i];
+    }
+    for (int k = 0; k < d; ++k) {
+      const int j = a.nbr[k * N + i];
+      pub = pub || (j >= 0 && j / T != t);
+    }
+  }
+  const int it = a.items.off[t] + (tid + NT - T) % NT;
+  const bool has = it < a.items.off[t + 1];
+  hg::ItemRec rec{};
+  if (has) rec = load_item(a.items, it, a.items.x0[t]);
+  const int type = has ? (rec.code >> 28) & 3 : 3;
+  NbrRaw nr{};
+  if (type == 1) {
+    nr.hs = a.hstill[rec.ref]; nr.zb = a.zb[rec.ref]; nr.area = a.area[rec.ref];
+    nr.dt = a.dtc ? a.dtc[rec.ref] : a.dt;
+  }
+  const bool in_ghost = type == 2 && a.g_kind[rec.ref] == HG_BC_INLETQ;
+  const int in0 = R.n_inlet > 0 ? R.tile_in_off[t] : 0, in1 = R.n_inlet > 0 ? R.tile_in_off[t + 1] : 0;
+  int my_sl = -1, my_f = -1;  // an inlet cell's inlet and first face there
+  for (int sl = in0; sl < in1; ++sl) {
+    const int b = R.tile_in_list[sl];
+    for (int f = R.in_off[b]; f < R.in_off[b + 1]; ++f)
+      if (own && R.in_rec[f].cell == i && R.in_rec[f].first) {
+        my_sl = sl;
+        my_f = f;
+      }
+    if (tid == 0) qa[sl - in0] = R.Qbar[b];
+  }
+  if (tid == 0) *stop = 0;
+  // the recorded state of the step (own cell, and a cross-tile neighbour's), read one step ahead
+  double px = 0.0, pqx = 0.0, pqy = 0.0, jx = 0.0, jqx = 0.0, jqy = 0.0;
+  uint8_t pm = 0, jm = 0;
+  auto read_ahead = [&](int64_t k) {
+    const double* q = R.rec + k * 3 * N;
+    const uint8_t* m = R.rec_clamp + k * N;
+    if (own) {
+      px = q[i]; pqx = q[N + i]; pqy = q[2 * N + i];
+      pm = m[i];
+    }
+    if (type == 1) {
+      jx = q[rec.ref]; jqx = q[N + rec.ref]; jqy = q[2 * N + rec.ref];
+      jm = m[rec.ref];
+    }
+  };
+  read_ahead(R.ns - 1);
+
+  for (int64_t r = 0; r < R.ns; ++r) {
+    const int64_t k = R.ns - 1 - r;  // the step that is reversed
+    const unsigned long long* slot = R.ring + (r & 3) * 3 * N;
+    a.totalA = R.rec_totalA ? R.rec_totalA + k * R.n_inlet : nullptr;
+    a.vbar = reinterpret_cast<double*>(R.vring + (r & 3) * R.G);
+    hg::CellQ me{};
+    double y0 = 0.0, y1 = 0.0, y2 = 0.0;
+    if (pm) l0 = l1 = l2 = 0.0;
+    nr.xi = jx; nr.qx = jqx; nr.qy = jqy;
+    nr.clamped = jm;
+    if (own) {
+      double rh, r2s;
+      me = adj_cellq(px, hs, pqx, pqy, zb, a.half_g, hsmall, rh, r2s);
+      const double rA = 1.0 / A;
+      y0 = dti * l0;
+      y1 = dti * l1;
+      y2 = dti * l2;
+      C[0 * T + tid] = me.xi; C[1 * T + tid] = me.hs; C[2 * T + tid] = me.hu; C[3 * T + tid] = me.hv;
+      C[4 * T + tid] = me.zb; C[5 * T + tid] = me.u; C[6 * T + tid] = me.v; C[7 * T + tid] = me.s;
+      C[8 * T + tid] = y0 * rA;
+      C[9 * T + tid] = y1 * rA;
+      C[10 * T + tid] = y2 * rA;
+      C[11 * T + tid] = rh;
+      C[12 * T + tid] = r2s;
+      for (int c = 0; c < MD; ++c) S[(3 * MD + c) * T + tid] = 0.0;
+      Xm[tid] = 0;
+    }
+    if (k > 0) read_ahead(k - 1);
+    __syncthreads();
+    if (has) {
+      if (type == 1) {
+        const int j = rec.ref;
+        double v[3];
+        if (r == 0) {
+          v[0] = a.lx[j]; v[1] = a.lqx[j]; v[2] = a.lqy[j];
+        } else if (!res_poll<3>(slot + j, N, R.ctl, v)) {
+          *stop = 1;
+        }
+        nr.m0 = v[0]; nr.m1 = v[1]; nr.m2 = v[2];
+      }
+      if (in_ghost) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): its last reset is done before it publishes again
+      adj_item<true, T, MD>(a, t, C, S, Xm, rec, nr);
+      if (in_ghost) res_put(R.vring + ((r + 2) & 3) * R.G + rec.ref, kResEmpty);
+    }
+    // the source term's cotangents, while the faces are waited for
+    double sxi = 0.0, sh = 0.0, sqx = 0.0, sqy = 0.0, sn = 0.0, sS0x = 0.0, sS0y = 0.0;
+    const bool wet = me.h > hsmall;
+    if (own && wet)
+      hg::source_vjp(a.g, a.kn2, hsmall, me.xi, me.h, me.hu, me.hv, n, S0x, S0y, y1, y2, sxi, sh, sqx, sqy, sn, sS0x,
+                     sS0y);
+    __syncthreads();
+    if (*stop) return;
+    if (own) {
+      double uxh = 0.0, uqx = 0.0, uqy = 0.0, nb = 0.0, zbb = 0.0;
+      const int xm = Xm[tid];
+      for (int c = 0; c < MD; ++c) {  // local face order
+        if (c < d) {
+          uxh += S[(0 * MD + c) * T + tid];
+          uqx += S[(1 * MD + c) * T + tid];
+          uqy += S[(2 * MD + c) * T + tid];
+          const double e = S[(3 * MD + c) * T + tid];
+          if ((xm >> c) & 1)
+            zbb += e;
+          else
+            nb += e;
+        }
+      }
+      nb += sn;
+      double ox = uxh + sxi, oqx = 0.0, oqy = 0.0;
+      if (wet) {
+        ox += sh;
+        oqx = uqx + sqx;
+        oqy = uqy + sqy;
+      }
+      l0 = ox + l0;
+      l1 = oqx + l1;
+      l2 = oqy + l2;
+      nbar = nbar + nb;
+      zbbar = zbbar + zbb;
+      S0bx = S0bx + sS0x;
+      S0by = S0by + sS0y;
+    }
+    // inlet conveyance adjoint (as k_inlet_adj)
+    for (int sl = in0; sl < in1; ++sl) {
+      const int b = R.tile_in_list[sl];
+      const int f0 = R.in_off[b], f1 = R.in_off[b + 1];
+      const double Ai = a.totalA[b], Qb = a.inletQ[b];
+      if (tid < 256) {
+        double pa = 0.0, pq = 0.0;
+        for (int f = f0 + tid; f < f1; f += 256) {
+          const hg::InletFaceRec fr = R.in_rec[f];
+          double vb[1];
+          if (!res_poll<1>(R.vring + (r & 3) * R.G + fr.ghost, 0, R.ctl, vb)) *stop = 1;
+          const double nc = a.n[fr.cell];
+          const double v = Qb / Ai * fr.L23 / nc;
+          pa += vb[0] * (-v / Ai);
+          pq += vb[0] * (fr.L23 / (Ai * nc));
+        }
+        sA[tid] = pa;
+        sQ[tid] = pq;
+      }
+      __syncthreads();
+      if (*stop) return;
+      if (tid < 128) {
+        sA[tid] += sA[tid + 128];
+        sQ[tid] += sQ[tid + 128];
+      }
+      __syncthreads();
+      if (tid < 64) {
+        double xa = sA[tid] + sA[tid + 64], xq = sQ[tid] + sQ[tid + 64];
+        for (int w = 32; w > 0; w >>= 1) {
+          xa = xa + __shfl_xor(xa, w, 64);
+          xq = xq + __shfl_xor(xq, w, 64);
+        }
+        if (tid == 0) {
+          sA[0] = xa;
+          qa[sl - in0] = qa[sl - in0] + xq;
+        }
+      }
+      __syncthreads();
+      if (my_sl == sl) {
+        const double h0 = me.xi + hs;
+        if (h0 > hsmall) {
+          const double Ab = sA[0];
+          for (int f = my_f; f >= 0;) {
+            const hg::InletFaceRec fr = R.in_rec[f];
+            l0 += Ab * fr.L53 / n;
+            nbar += Ab * (-fr.L53 * h0 / (n * n));
+            f = fr.next;
+          }
+        }
+      }
+      __syncthreads();  // sA / sQ reuse
+    }
+    if (own && pub && r + 1 < R.ns) {
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the last step's reset is done
+      unsigned long long* o = R.ring + ((r + 1) & 3) * 3 * N + i;
+      unsigned long long* e = R.ring + ((r + 3) & 3) * 3 * N + i;
+      res_put(o, __double_as_longlong(l0));
+      res_put(o + N, __double_as_longlong(l1));
+      res_put(o + 2 * N, __double_as_longlong(l2));
+      for (int c = 0; c < 3; ++c) res_put(e + c * N, kResEmpty);
+    }
+  }
+  if (own) {
+    a.ox[i] = l0;
+    a.oqx[i] = l1;
+    a.oqy[i] = l2;
+    if (R.o_nbar) R.o_nbar[i] = nbar;
+    if (R.o_zbbar) {
+      R.o_zbbar[i] = zbbar;
+      R.o_S0bar[i] = S0bx;
+      R.o_S0bar[N + i] = S0by;
+    }
+  }
+  for (int sl = in0 + tid; sl < in1; sl += NT) {  // by the tile of the inlet's first face
+    const int b = R.tile_in_list[sl];
+    if (R.in_rec[R.in_off[b]].cell / T == t) R.o_Qbar[b] = qa[sl - in0];
+  }
 }
 
 // Inlet conveyance adjoint (bc_2D.jl:640-694): v_f = (Q_b / A_b) L^(2/3) / n
@@ -2906,6 +3171,20 @@ void launch_run(hg_ctx* ctx, const hg::TileArgs& a, const ResArgs& R) {
                      ctx->stream, a, R);
 }
 
+size_t adj_run_lds_bytes(int MD) {
+  return size_t((kAdjRows + 4 * MD) * kResT + 512 + kTileInlets) * sizeof(double) + (kResT + 1) * sizeof(int32_t);
+}
+
+template <int MD>
+int adj_run_capacity(hg_ctx* ctx) {
+  constexpr int waves = res_items(MD) / 64;
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_adj_run<MD>, 64 * waves, adj_run_lds_bytes(MD)) !=
+      hipSuccess)
+    return 0;
+  return std::min(per_cu, 2 / ((waves + 3) / 4)) * ctx->ncu;  // see res_capacity
+}
+
 // Whether nsteps steps may run resident: one field, the default tiling of
 // small meshes, at most one item per work-item and 64 inlets per tile, a
 // roughness that does not change with the state, and steps enough to pay for
@@ -2914,6 +3193,35 @@ bool res_usable(hg_ctx* ctx, int64_t nsteps) {
   return ctx->tiled && !ctx->res_off && ctx->K == 1 && nsteps >= 4 && ctx->tileT == kResT && ctx->tileMD <= 4 &&
          ctx->max_items <= res_items(ctx->tileMD) && (ctx->n_inlet == 0 || ctx->fuse_inlet) && !ctx->ude_prec &&
          ctx->nlaw.kind == hg::NLAW_OFF && ctx->lux.choice == hg::LUX_OFF && ctx->device < kMaxDevices;
+}
+
+// Takes this context's tiles out of the device's room (of `cap` work-groups),
+// or false when they do not fit beside the runs in flight.
+bool res_claim(hg_ctx* ctx, int cap) {
+  std::lock_guard<std::mutex> g(g_res_mu);
+  if (g_res_groups[ctx->device] + ctx->ntiles > cap) return false;
+  g_res_groups[ctx->device] += ctx->ntiles;
+  return true;
+}
+
+// After the launch of a resident run: waits for it and gives its room back;
+// *done: every tile finished.
+int res_finish(hg_ctx* ctx, bool* done) {
+  int32_t ran_out = 0;
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(&ran_out, ctx->res_ctl, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  {
+    std::lock_guard<std::mutex> g(g_res_mu);
+    g_res_groups[ctx->device] -= ctx->ntiles;
+  }
+  HG_TRY(e);
+  if (ran_out)  // the device was shared with something else: one launch per step from here on
+    ctx->res_off = true;
+  else
+    *done = true;
+  return HG_OK;
 }
 
 // nsteps steps from state arrays `in` to `out` (not the same), optionally
@@ -2937,11 +3245,7 @@ int res_run(hg_ctx* ctx, const double* const in[3], double* const out[3], double
     if (!rc) rc = dalloc(ctx, &ctx->res_ctl, 1);
     if (rc) return rc;
   }
-  {
-    std::lock_guard<std::mutex> g(g_res_mu);
-    if (g_res_groups[ctx->device] + ctx->ntiles > ctx->res_cap) return HG_OK;
-    g_res_groups[ctx->device] += ctx->ntiles;
-  }
+  if (!res_claim(ctx, ctx->res_cap)) return HG_OK;
   const int64_t nring = int64_t(12) * ctx->N;
   hipLaunchKernelGGL(k_res_init, dim3(grid_of(nring)), dim3(kBlock), 0, ctx->stream, nring, ctx->res_ring,
                      ctx->res_ctl);
@@ -2951,22 +3255,7 @@ int res_run(hg_ctx* ctx, const double* const in[3], double* const out[3], double
     ctx->res_split ? launch_run<3, true>(ctx, a, R) : launch_run<3, false>(ctx, a, R);
   else
     ctx->res_split ? launch_run<4, true>(ctx, a, R) : launch_run<4, false>(ctx, a, R);
-  int32_t ran_out = 0;
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(&ran_out, ctx->res_ctl, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  {
-    std::lock_guard<std::mutex> g(g_res_mu);
-    g_res_groups[ctx->device] -= ctx->ntiles;
-  }
-  HG_TRY(e);
-  if (ran_out) {  // the device was shared with something else: one launch per step from here on
-    ctx->res_off = true;
-    return HG_OK;
-  }
-  *done = true;
-  return HG_OK;
+  return res_finish(ctx, done);
 }
 
 // ---- adjoint host side
@@ -3400,6 +3689,70 @@ int recompute_segment(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck, int64
   });
 }
 
+// The ns steps recorded in segment buffer b reversed in one resident run, from
+// the cotangent in adj_lam[lam0] to adj_lam[1 - lam0] (*done as for res_run;
+// the sums are taken over only then).
+int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done) {
+  *done = false;
+  if (!res_usable(ctx, ns) || ns > kResSteps || !ctx->inlets_disjoint || ctx->adj_T != kResT) return HG_OK;
+  const bool tri = ctx->tileMD == 3;
+  if (!ctx->adj_res_cap) ctx->adj_res_cap = std::max(1, tri ? adj_run_capacity<3>(ctx) : adj_run_capacity<4>(ctx));
+  if (ctx->adj_res_cap < ctx->ntiles) return HG_OK;
+  const int64_t N = ctx->N, G = std::max<int64_t>(ctx->G, 1), nring = 12 * N + 4 * G;
+  if (!ctx->adj_ring) {
+    int rc = dalloc(ctx, &ctx->adj_ring, size_t(nring));
+    if (!rc) rc = dalloc(ctx, &ctx->adj_sums, size_t(4) * N + std::max<int32_t>(ctx->n_inlet, 1));
+    if (!rc && !ctx->res_ctl) rc = dalloc(ctx, &ctx->res_ctl, 1);
+    if (rc) return rc;
+  }
+  if (!res_claim(ctx, ctx->adj_res_cap)) return HG_OK;
+  hipLaunchKernelGGL(k_res_init, dim3(grid_of(nring)), dim3(kBlock), 0, ctx->stream, nring, ctx->adj_ring,
+                     ctx->res_ctl);
+  const double* q[3] = {seg_state(ctx, 0, 0, b), seg_state(ctx, 0, 1, b), seg_state(ctx, 0, 2, b)};
+  double *L = ctx->adj_lam[lam0], *O = ctx->adj_lam[1 - lam0], *sums = ctx->adj_sums;
+  const double* lam[3] = {L, L + N, L + 2 * N};
+  double* out[3] = {O, O + N, O + 2 * N};
+  hg::AdjArgs a = make_adj_args(ctx, q, lam, nullptr, out, dt);
+  a.nbar = ctx->adj_want_n ? ctx->adj_nbar : nullptr;
+  if (ctx->deg_full) a.deg = nullptr;
+  a.items = ctx->adj_items;
+  AdjRunArgs R{};
+  R.ring = ctx->adj_ring;
+  R.vring = ctx->adj_ring + 12 * N;
+  R.ctl = ctx->res_ctl;
+  R.ns = ns;
+  R.G = G;
+  R.rec = ctx->adj_seg[b];
+  R.rec_clamp = ctx->adj_mask[b];
+  R.rec_totalA = seg_totalA(ctx, 0, b);
+  R.n_inlet = ctx->n_inlet;
+  R.tile_in_off = ctx->tile_in_off;
+  R.tile_in_list = ctx->tile_in_list;
+  R.in_off = ctx->in_off;
+  R.in_rec = ctx->in_rec;
+  R.Qbar = ctx->adj_Qbar;
+  R.o_nbar = ctx->adj_want_n ? sums : nullptr;
+  R.o_zbbar = ctx->adj_want_zb ? sums + N : nullptr;
+  R.o_S0bar = sums + 2 * N;
+  R.o_Qbar = sums + 4 * N;
+  if (tri)
+    hipLaunchKernelGGL(k_adj_run<3>, dim3(ctx->ntiles), dim3(res_items(3)), adj_run_lds_bytes(3), ctx->stream, a, R);
+  else
+    hipLaunchKernelGGL(k_adj_run<4>, dim3(ctx->ntiles), dim3(res_items(4)), adj_run_lds_bytes(4), ctx->stream, a, R);
+  int rc = res_finish(ctx, done);
+  if (rc || !*done) return rc;
+  auto take = [&](double* dst, const double* src, int64_t n) {
+    return n > 0 ? hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream) : hipSuccess;
+  };
+  if (R.o_nbar) HG_TRY(take(ctx->adj_nbar, R.o_nbar, N));
+  if (R.o_zbbar) {
+    HG_TRY(take(ctx->adj_zbbar, R.o_zbbar, N));
+    HG_TRY(take(ctx->adj_S0bar, R.o_S0bar, 2 * N));
+  }
+  HG_TRY(take(ctx->adj_Qbar, R.o_Qbar, ctx->n_inlet));
+  return HG_OK;
+}
+
 // Reverse sweep over the checkpointed trajectory; lam (device, 3 x N) holds
 // the cotangent of the final state on entry and of the initial state on exit.
 // Segment s - 1 is recomputed on the second stream into the other segment
@@ -3409,6 +3762,15 @@ int recompute_segment(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck, int64
 int reverse_sweep(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck, int& lam_cur) {
   const int64_t N = ctx->N;
   const int64_t nseg = (nsteps + kck - 1) / kck;
+  if (nseg == 1) {  // the whole run is recorded: a small mesh reverses it in one launch
+    bool done = false;
+    const int rc = adj_res_run(ctx, dt, nsteps, 0, lam_cur, &done);
+    if (rc) return rc;
+    if (done) {
+      lam_cur = 1 - lam_cur;
+      return HG_OK;
+    }
+  }
   const bool overlap = !ctx->ude_prec && ctx->nlaw.kind == hg::NLAW_OFF && ctx->lux.choice == hg::LUX_OFF;
   const hipStream_t rs = overlap ? ctx->stream2 : ctx->stream;
   if (overlap) {  // the recompute stream starts after everything already on the context stream

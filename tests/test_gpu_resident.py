@@ -142,3 +142,70 @@ def test_threads_share_the_device():
     [t.start() for t in th]
     [t.join() for t in th]
     assert all(np.array_equal(q, ref) for qs in out for q in qs)
+
+
+def two_inlets(n_quads=300):
+    """Two inlets on opposite ends of a closed channel (each over several tiles of a larger mesh)."""
+    nx = max(4, int(round(n_quads ** 0.5)))
+    xy, quads, side = cases.rect_quads(20.0 * nx, 20.0 * nx, nx, nx)
+    m = hm.build_mesh(xy, quads, {1: side["left"], 2: side["right"], 3: side["bottom"], 4: side["top"]},
+                      {1: "INLET-Q", 2: "INLET-Q", 3: "EXIT-H", 4: "WALL"})
+    zb = 0.1 * np.random.default_rng(5).random(m.n_cells)
+    zg, S0x, S0y = hm.bed_data(m, zb)
+    hs = np.full(m.n_cells, 0.3)
+    c = cases.Case(name="two_inlets", mesh=m, hstill=hs, hstill_ghost=hs[m.ghost_cell], zb=zb, zb_ghost=zg, S0x=S0x,
+                   S0y=S0y, n=np.full(m.n_cells, 0.03), inletQ=np.array([20.0, 30.0]), exitWSE=np.array([2.0]),
+                   Q0=np.concatenate([2.0 - zb - hs, np.zeros(2 * m.n_cells)]), dt=0.0, nsteps=0)
+    c.dt = cases.cfl_dt(c, 0.3)
+    return c
+
+
+def wet_dry():
+    c = cases.channel(6_000, seed=12, Lx=1500.0, Ly=150.0, Q_in=60.0)
+    x = c.mesh.centroid[:, 0]
+    Q = c.Q0.copy()
+    Q[:c.N] = np.where(x < 500.0, np.maximum(c.h_small, 2.2 - c.zb), c.h_small) - c.hstill
+    return c.copy_fields(Q0=Q, dt=cases.cfl_dt(c, 0.4, Q))
+
+
+REVERSE = {"one_tile": lambda: cases.dam_break(nx=16, ny=8), "tile_and_one": lambda: cases.dam_break(nx=43, ny=3),
+           "quads": lambda: cases.dam_break(nx=100, ny=10), "tiny_channel": lambda: channel(40),
+           "channel": lambda: channel(9000), "mixed": lambda: mixed(900, 2), "wet_dry": wet_dry,
+           "two_inlets": two_inlets, "two_inlets_large": lambda: two_inlets(8000),
+           "batch": lambda: cases.concat([channel(n, seed=n) for n in (90, 700, 300)])}
+
+
+@pytest.mark.parametrize("name", sorted(REVERSE))
+@pytest.mark.parametrize("steps", [4, 5, 30])
+def test_reverse_run(name, steps):
+    """The reverse sweep in one launch against one launch per step (another tile size), every cotangent, bit for bit."""
+    c = REVERSE[name]()
+    single = capi.Context(c)
+    single.set_tile_config(256)
+    ctx = capi.Context(c)
+    lam = np.random.default_rng(steps).normal(size=3 * c.N)
+    a, b = ctx.adjoint(c.Q0, c.dt, steps, 0, lam), single.adjoint(c.Q0, c.dt, steps, 0, lam)
+    assert np.all(np.isfinite(b[0])) and np.any(b[1])
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+    for wrt in (("n",), ("zb",), ("Q",), ()):  # the sums nobody asks for are left out
+        QN = ctx.adjoint_forward(c.Q0, c.dt, steps, 0)
+        assert np.array_equal(QN, single.step(c.Q0, c.dt, steps))
+        got = ctx.adjoint_reverse(lam, wrt=wrt)
+        assert np.array_equal(got[0], b[0])
+        for k, w in enumerate(("n", "zb", "Q")):
+            assert got[k + 1] is None if w not in wrt else np.array_equal(got[k + 1], b[k + 1])
+
+
+def test_reverse_run_with_own_time_steps():
+    parts = [channel(n, seed=n) for n in (90, 700, 300)]
+    c = cases.concat(parts)
+    out = []
+    for size in (0, 256):
+        ctx = capi.Context(c)
+        if size:
+            ctx.set_tile_config(size)
+        ctx.batch_set_dt([p.dt * f for p, f in zip(parts, (0.5, 0.8, 0.9))])
+        out.append(ctx.adjoint(c.Q0, c.dt, 12, 0, np.linspace(-1, 1, 3 * c.N)))
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
