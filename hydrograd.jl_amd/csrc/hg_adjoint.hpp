@@ -23,13 +23,13 @@ struct ExtBar {
   double xi, h, hu, hv, u, v, s, p;
 };
 
-__host__ __device__ __forceinline__ void ext_zero(ExtBar& e) { e.xi = e.h = e.hu = e.hv = e.u = e.v = e.s = e.p = 0.0; }
+__device__ __forceinline__ void ext_zero(ExtBar& e) { e.xi = e.h = e.hu = e.hv = e.u = e.v = e.s = e.p = 0.0; }
 
 // u = hu/h, v = hv/h, s = sqrt(h + eps), p = 0.5 g ((xi+eps)^2 + 2 xi hs):
 // fold the derived cotangents into (xi, h, hu, hv).
 // rh = 1 / h and r2s = 0.5 / s are the side's own reciprocals (a tiled
 // kernel forms them once per cell).
-__host__ __device__ __forceinline__ SideBar ext_to_side_r(const ExtBar& e, const CellQ& c, double rh, double r2s,
+__device__ __forceinline__ SideBar ext_to_side_r(const ExtBar& e, const CellQ& c, double rh, double r2s,
                                                           double half_g) {
   SideBar s;
   s.hu = e.hu + e.u * rh;
@@ -39,12 +39,12 @@ __host__ __device__ __forceinline__ SideBar ext_to_side_r(const ExtBar& e, const
   return s;
 }
 
-__host__ __device__ __forceinline__ SideBar ext_to_side(const ExtBar& e, const CellQ& c, double half_g) {
+__device__ __forceinline__ SideBar ext_to_side(const ExtBar& e, const CellQ& c, double half_g) {
   return ext_to_side_r(e, c, 1.0 / c.h, 0.5 / c.s, half_g);
 }
 
 // Physical flux of one side (hu, hv, u, v, p), reverse.
-__host__ __device__ __forceinline__ void phys_vjp(double hu, double hv, double u, double v, double nx, double ny,
+__device__ __forceinline__ void phys_vjp(double hu, double hv, double u, double v, double nx, double ny,
                                                   const double fb[3], ExtBar& e) {
   const double un = nx * u + ny * v;
   e.hu += fb[0] * nx + fb[1] * un;
@@ -59,7 +59,7 @@ __host__ __device__ __forceinline__ void phys_vjp(double hu, double hv, double u
 // and derived quantities (unfolded; ext_to_side folds them).  A and B are
 // the flux inputs (clamped depth, masked discharge, derived u, v, s, p) as
 // make_cellq forms them.  Every field of ea and eb is assigned.
-__host__ __device__ __forceinline__ void roe_vjp_ext(const CellQ& A, const CellQ& B, double nx, double ny, double g,
+__device__ __forceinline__ void roe_vjp_ext(const CellQ& A, const CellQ& B, double nx, double ny, double g,
                                                      double half_g, double hmin, const double Fb[3], ExtBar& ea,
                                                      ExtBar& eb) {
   if (A.h <= hmin && B.h <= hmin) {
@@ -163,7 +163,7 @@ __host__ __device__ __forceinline__ void roe_vjp_ext(const CellQ& A, const CellQ
 }
 
 // The same, folded: cotangents of both sides' (xi, h, hu, hv).
-__host__ __device__ inline void roe_vjp(const CellQ& A, const CellQ& B, double nx, double ny, double g, double half_g,
+__device__ inline void roe_vjp(const CellQ& A, const CellQ& B, double nx, double ny, double g, double half_g,
                                         double hmin, const double Fb[3], SideBar& Ab, SideBar& Bb) {
   ExtBar ea, eb;
   roe_vjp_ext(A, B, nx, ny, g, half_g, hmin, Fb, ea, eb);
@@ -176,7 +176,7 @@ __host__ __device__ inline void roe_vjp(const CellQ& A, const CellQ& B, double n
 // A's raw and derived quantities are ADDED to e (unfolded; ext_to_side folds
 // a cell's sum once).  Same branches and routing as roe_vjp; B's own
 // cotangent is never formed.
-__host__ __device__ __forceinline__ void roe_vjp_a(const CellQ& A, const CellQ& B, double nx, double ny, double g,
+__device__ __forceinline__ void roe_vjp_a(const CellQ& A, const CellQ& B, double nx, double ny, double g,
                                                    double half_g, double hmin, const double Fb[3], ExtBar& e) {
   if (A.h <= hmin && B.h <= hmin) return;
   int mode = 0;  // 0 general, 1 B mirrored from A, 2 A mirrored from B
@@ -265,7 +265,7 @@ __host__ __device__ __forceinline__ void roe_vjp_a(const CellQ& A, const CellQ& 
 // 474-475, 544-547): src = g xi S0 - friction.  y1, y2 are the cotangents of
 // the x / y momentum RHS; outputs add to the cotangents of xi, h, hu, hv,
 // n, S0x, S0y.
-__host__ __device__ __forceinline__ void source_vjp(double g, double kn2, double hsmall, double xi, double h,
+__device__ __forceinline__ void source_vjp(double g, double kn2, double hsmall, double xi, double h,
                                                     double qx, double qy, double n, double S0x, double S0y, double y1,
                                                     double y2, double& xib, double& hb, double& qxb, double& qyb,
                                                     double& nb, double& S0xb, double& S0yb) {
@@ -290,7 +290,7 @@ __host__ __device__ __forceinline__ void source_vjp(double g, double kn2, double
 
 // VJP of the momentum source with FlowResistance friction m q / |q|_eps
 // (semi_discretize_swe_2D.jl:474-475, 521-531); mb += d/dm.  No depth term.
-__host__ __device__ __forceinline__ void source_vjp_mag(double g, double xi, double qx, double qy, double m,
+__device__ __forceinline__ void source_vjp_mag(double g, double xi, double qx, double qy, double m,
                                                         double S0x, double S0y, double y1, double y2, double& xib,
                                                         double& qxb, double& qyb, double& mb, double& S0xb,
                                                         double& S0yb) {

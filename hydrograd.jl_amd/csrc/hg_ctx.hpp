@@ -269,6 +269,8 @@ struct LuxNet {
   double eps;                // LayerNorm epsilon
 };
 
+struct Tsit5State;
+
 template <class T>
 struct DBuf {  // owning device buffer
   T* p = nullptr;
@@ -347,14 +349,21 @@ struct hg_ctx {
   int32_t xcd_chunk = 0;  // identity block -> tile mapping by default (the autotuner re-checks)
   int32_t ncu = 256;      // compute units of the device
   int32_t max_items = 0;  // work items of the fullest tile
-  // resident runs (k_swe_run): work-groups the device holds at once (0: not
-  // asked yet), off for good once a wait ran out, the exchange ring and its
-  // control word
-  int32_t res_cap = 0;
-  bool res_off = false, res_split = false;
+  // resident runs (hg_resident.hpp): tiles the device holds at once of each
+  // variant ([split][n mode][dual]; -1: not asked yet), off for good once a
+  // wait ran out, this run's share of the device, the exchange ring and its
+  // control word; the same for the reverse run, its rings and the sums it
+  // writes, and for Tsit5, its state between launches and its frames
+  int32_t res_cap[2][3][2] = {{{-1, -1}, {-1, -1}, {-1, -1}}, {{-1, -1}, {-1, -1}, {-1, -1}}};
+  bool res_off = false;
+  int32_t res_share = 0;
   unsigned long long* res_ring = nullptr;
+  size_t res_ring_n = 0;
   int32_t* res_ctl = nullptr;
-  int32_t adj_res_cap = 0;  // the same for the reverse run, its rings and the sums it writes
+  int32_t adj_res_cap = -1, tsit5_cap[3] = {-1, -1, -1};
+  hg::Tsit5State* rk_state = nullptr;
+  double* rk_frames = nullptr;
+  size_t rk_frames_n = 0;
   unsigned long long* adj_ring = nullptr;
   double* adj_sums = nullptr;
   // the reverse step's tiling (its own tile size; the step kernel's items

@@ -6,6 +6,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "hg_device.hpp"
+
 namespace hg {
 
 struct Dual1 {
@@ -31,13 +33,14 @@ __host__ __device__ __forceinline__ Dual1 operator*(const Dual1& a, const Dual1&
 __host__ __device__ __forceinline__ Dual1 operator/(const Dual1& a, const Dual1& b) {
   return Dual1(a.v / b.v, (a.d * b.v - a.v * b.d) / (b.v * b.v));
 }
-__host__ __device__ __forceinline__ Dual1 operator+(const Dual1& a, double b) { return a + Dual1(b); }
-__host__ __device__ __forceinline__ Dual1 operator+(double a, const Dual1& b) { return Dual1(a) + b; }
-__host__ __device__ __forceinline__ Dual1 operator-(const Dual1& a, double b) { return a - Dual1(b); }
-__host__ __device__ __forceinline__ Dual1 operator-(double a, const Dual1& b) { return Dual1(a) - b; }
-__host__ __device__ __forceinline__ Dual1 operator*(const Dual1& a, double b) { return a * Dual1(b); }
-__host__ __device__ __forceinline__ Dual1 operator*(double a, const Dual1& b) { return Dual1(a) * b; }
-__host__ __device__ __forceinline__ Dual1 operator/(const Dual1& a, double b) { return a / Dual1(b); }
+// A constant carries no tangent.
+__host__ __device__ __forceinline__ Dual1 operator+(const Dual1& a, double b) { return Dual1(a.v + b, a.d); }
+__host__ __device__ __forceinline__ Dual1 operator+(double a, const Dual1& b) { return Dual1(a + b.v, b.d); }
+__host__ __device__ __forceinline__ Dual1 operator-(const Dual1& a, double b) { return Dual1(a.v - b, a.d); }
+__host__ __device__ __forceinline__ Dual1 operator-(double a, const Dual1& b) { return Dual1(a - b.v, -b.d); }
+__host__ __device__ __forceinline__ Dual1 operator*(const Dual1& a, double b) { return Dual1(a.v * b, a.d * b); }
+__host__ __device__ __forceinline__ Dual1 operator*(double a, const Dual1& b) { return Dual1(a * b.v, a * b.d); }
+__host__ __device__ __forceinline__ Dual1 operator/(const Dual1& a, double b) { return Dual1(a.v / b, a.d / b); }
 __host__ __device__ __forceinline__ Dual1 operator/(double a, const Dual1& b) { return Dual1(a) / b; }
 
 __host__ __device__ __forceinline__ bool operator<(const Dual1& a, const Dual1& b) { return a.v < b.v; }
@@ -47,11 +50,29 @@ __host__ __device__ __forceinline__ bool operator<(const Dual1& a, double b) { r
 __host__ __device__ __forceinline__ bool operator<=(const Dual1& a, double b) { return a.v <= b; }
 __host__ __device__ __forceinline__ bool operator>(const Dual1& a, double b) { return a.v > b; }
 
-__host__ __device__ __forceinline__ Dual1 sqrt(const Dual1& a) {
-  const double r = ::sqrt(a.v);
-  return Dual1(r, a.d / (2.0 * r));
+// The shared-part quotients and roots of hg_device.hpp: y = 1 / b.v, and the
+// root's derivative from the same 0.5 / sqrt.
+__device__ __forceinline__ double rcp_est(const Dual1& b) { return rcp_est(b.v); }
+__device__ __forceinline__ Dual1 div_est(const Dual1& a, const Dual1& b, double y) {
+  const double v = div_est(a.v, b.v, y);
+  return Dual1(v, (a.d - v * b.d) * y);
 }
-__host__ __device__ __forceinline__ Dual1 cbrt(const Dual1& a) {
+__device__ __forceinline__ Dual1 div_est(const Dual1& a, double b, double y) {
+  return Dual1(div_est(a.v, b, y), a.d * y);
+}
+__device__ __forceinline__ Dual1 sqrt_half_rcp(const Dual1& x, Dual1& o) {
+  double ov;
+  const double s = sqrt_half_rcp(x.v, ov);
+  const double sd = x.d * ov;
+  o = Dual1(ov, -2.0 * (ov * ov) * sd);
+  return Dual1(s, sd);
+}
+__device__ __forceinline__ Dual1 sqrt_pos(const Dual1& x) {
+  double ov;
+  const double s = sqrt_half_rcp(x.v, ov);
+  return Dual1(s, x.d * ov);
+}
+__device__ __forceinline__ Dual1 cbrt_of(const Dual1& a) {
   const double r = ::cbrt(a.v);
   return Dual1(r, a.d * (r / (3.0 * a.v)));
 }

@@ -108,7 +108,7 @@ __device__ __forceinline__ Dual1 sigmoid_t(const Dual1& x) {
   return Dual1(s, s * (1.0 - s) * x.d);
 }
 __device__ __forceinline__ double sqrt_t(double x) { return ::sqrt(x); }
-__device__ __forceinline__ Dual1 sqrt_t(const Dual1& x) { return hg::sqrt(x); }
+__device__ __forceinline__ Dual1 sqrt_t(const Dual1& x) { return sqrt_pos(x); }
 
 // Hidden layer l on input x (width win): pre-activation z, activation a,
 // normalised xh = (a - mean) / s.

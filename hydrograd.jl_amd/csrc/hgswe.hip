@@ -35,14 +35,38 @@
 #include "hg_ctx.hpp"
 #include "hg_device.hpp"
 #include "hg_roe_pair.hpp"
+#include "hg_adj_tile.hpp"
 #include "hg_adjoint.hpp"
 #include "hg_ude.hpp"
-#include "hg_dual.hpp"  // after the double paths: its sqrt / cbrt overloads must stay out of them
+#include "hg_dual.hpp"
 #include "hg_nlaw.hpp"
 #include "hg_lux.hpp"
+#include "hg_resident.hpp"
+#include "hg_tile.hpp"
+#include "hg_tsit5.hpp"
 #include "hgswe.h"
 
 using hg::StepArgs;
+using hg::adj_cellq;
+using hg::adj_ghost_route;
+using hg::adj_ghost_state;
+using hg::adj_item;
+using hg::ghost_cellq;
+using hg::ghost_face;
+using hg::GhostAdj;
+using hg::GhostFace;
+using hg::GhostFaceT;
+using hg::kAdjRows;
+using hg::kResT;
+using hg::kResSteps;
+using hg::kTileInlets;
+using hg::lds_cellq;
+using hg::load_item;
+using hg::nbr_load;
+using hg::NbrRaw;
+using hg::res_items;
+using hg::store_state;
+using hg::wave_left_fold;
 
 static thread_local std::string g_create_err;  // per caller thread, like the contexts
 
@@ -77,7 +101,6 @@ constexpr int kBlock = 256;
 constexpr int kRewarmSteps = 1024;  // graph-replayed steps the autotuner ends with (a multiple of kGraphSteps)
 constexpr int kGraphSteps = 16;  // steps per captured graph (even: the graph returns to buffer 0)
 constexpr int kXCD = 8;         // MI355X: 8 accelerator complex dies, one L2 each
-constexpr int kTileInlets = 64;  // inlet boundaries one tile may touch when the conveyance is fused
 
 template <class T>
 int dalloc(hg_ctx* ctx, T** p, size_t n) {
@@ -123,21 +146,6 @@ int upload(hg_ctx* ctx, T* dst, const T* src, size_t n) {
 // --------------------------------------------------------------- kernels ---
 
 
-// acc + the first cnt lanes' terms of this wave, one after the other (lanes
-// from cnt on hold +0.0; the terms are not negative, so the zeros that fill
-// the last group of eight change nothing).  A lane read costs two scalar
-// moves; a lane exchange through LDS per term instead took 8.8 us, not 6.9, for
-// a resident step of a 96k-cell channel whose inlet has 69 faces.
-__device__ __forceinline__ double wave_left_fold(double acc, double term, int cnt) {
-  const long long v = __double_as_longlong(term);
-  const int lo = int(v), hi = int(v >> 32);
-  for (int k = 0; k < cnt; k += 8)
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      acc = acc + __hiloint2double(__builtin_amdgcn_readlane(hi, k + u), __builtin_amdgcn_readlane(lo, k + u));
-  return acc;
-}
-
 // Inlet conveyance (bc_2D.jl:640-680): total_A_b = sum over the inlet's
 // faces, in NodeString order, of ((L^(5/3) h_c) / n_c) * wet_c.  The terms
 // are formed in parallel, the sum is a left fold by one lane (the
@@ -171,83 +179,6 @@ __global__ __launch_bounds__(kBlock) void k_inlet_conveyance(hg::InletArgs a) {
     a.totalA[b] = acc;
     if (!(acc > 1e-10)) a.flag[0] = 1;
   }
-}
-
-// The new state of a step, stored as a relaxed store at device (agent)
-// scope: the same vector store with the device-scope cache policy bit
-// (sc1).  The next step's kernel reads these values, from any XCD; on the
-// 1M-cell channel the step kernel measured about 1 % faster with it than
-// with plain stores (the stored values are the same).
-__device__ __forceinline__ void store_state(double* p, double v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// What a boundary face's ghost state reads besides its cell and the inlet's
-// conveyance: p is the inlet's discharge or the outlet's stage.
-struct GhostFace {
-  int kind, bc;
-  double hs, zb, p, L23;
-};
-template <class Args>
-__device__ __forceinline__ GhostFace ghost_face(const Args& a, int gi) {
-  GhostFace g;
-  g.kind = a.g_kind[gi];
-  g.bc = a.g_bc[gi];
-  g.hs = a.g_hstill[gi];
-  g.zb = a.g_zb[gi];
-  g.L23 = a.g_L23[gi];
-  g.p = g.kind == HG_BC_INLETQ ? a.inletQ[g.bc] : g.kind == HG_BC_EXITH ? a.exitWSE[g.bc] : 0.0;
-  return g;
-}
-
-// A boundary face's ghost state (bc_2D.jl:640-834) as the flux reads it,
-// formed from its internal cell's flux inputs A (Manning n: n_i); tot: the
-// conveyance of an inlet-Q ghost's inlet.
-__device__ __forceinline__ hg::CellQ ghost_cellq(const GhostFace& g, const hg::CellQ& A, double n_i, double nx,
-                                                 double ny, double tot, double half_g, double hsmall) {
-  double h, qx, qy;
-  switch (g.kind) {
-    case HG_BC_INLETQ: {
-      const double w = (A.h > hsmall) ? 1.0 : 0.0;
-      const double v = g.p / tot * g.L23 / n_i;
-      h = A.h;
-      qx = -A.h * v * nx * w;
-      qy = -A.h * v * ny * w;
-      break;
-    }
-    case HG_BC_EXITH: {
-      const double hx = g.p - A.zb;
-      h = (hx > hsmall) ? hx : hsmall;
-      qx = A.hu;
-      qy = A.hv;
-      break;
-    }
-    case HG_BC_WALL:
-      h = A.h;
-      qx = -A.hu;
-      qy = -A.hv;
-      break;
-    default: {  // HG_BC_SYMM
-      const double vdn = A.hu * nx + A.hv * ny;
-      h = A.h;
-      qx = A.hu - 2.0 * vdn * nx;
-      qy = A.hv - 2.0 * vdn * ny;
-      break;
-    }
-  }
-  hg::CellQ B;
-  B.hs = g.hs;
-  B.xi = h - B.hs;
-  B.h = h;
-  B.hu = qx;
-  B.hv = qy;
-  B.zb = g.zb;
-  const double rh = hg::rcp_est(h);
-  B.u = hg::div_est(qx, h, rh);
-  B.v = hg::div_est(qy, h, rh);
-  B.s = hg::sqrt_pos(h + hg::EPS);
-  B.p = half_g * ((B.xi + hg::EPS) * (B.xi + hg::EPS) + 2.0 * B.xi * B.hs);
-  return B;
 }
 
 // Fused RHS (+ Euler step and dry clamp when STEP).  One work-item per cell.
@@ -334,18 +265,6 @@ __global__ __launch_bounds__(kBlock) void k_swe_step(StepArgs a0) {
 //     the source terms and applies the Euler update and dry clamp.
 // T (cells per tile) and MD (slots per cell) are compile-time constants so
 // every LDS address is a base register plus an immediate offset.
-// Work item it of a tile whose items before ix0 carry a ref (see ItemTable).
-__device__ __forceinline__ hg::ItemRec load_item(const hg::ItemTable& tb, int it, int ix0) {
-  hg::ItemRec r;
-  r.code = tb.code[it];
-  r.ref = it < ix0 ? tb.ref[it] : 0;
-  const hg::ItemGeo g = tb.geo[it];
-  r.nx = g.nx;
-  r.ny = g.ny;
-  r.len = g.len;
-  return r;
-}
-
 // This work-group's tile t and field fld (the launch covers every tile of
 // each of K fields; see k_swe_tile).
 __device__ __forceinline__ void tile_of_block(int K, int xcd_chunk, int& t, int& fld) {
@@ -533,289 +452,6 @@ __global__ __launch_bounds__(T) void k_swe_tile(hg::TileArgs a0) {
   }
 }
 
-// ---- resident run: many steps of a small mesh in one launch.
-// A step of a mesh of up to about 130,000 cells is one dependent chain --
-// launch, cell loads, items, neighbours, two barriers -- of 7 us and more,
-// however few cells it has; the chip is mostly idle.  Here every tile keeps
-// its cells, their constants and its work items in registers for the whole
-// run, and only the cells that another tile reads travel through memory.
-// Per step: 1,000 quads 7.4 -> 2.5 us; a closed 59k-triangle mesh about 7 ->
-// 3.7 us; channels, whose inlet tiles also wait for all of the inlet's cells
-// and fold their conveyance, 3.5 us at 1,300 cells, 4.0 at 20k, 6.5 at 96k
-// (8.7 us with one launch per step) and 6.8 at 126k.  Larger meshes do not fit
-// on the chip in this form.
-//
-// Exchange: a published cell's new state goes to slot (s + 1) % 4 of a ring of
-// four states, whose entries hold kResEmpty (a signalling NaN no arithmetic
-// produces) until then; a reader polls the values themselves, each a relaxed
-// agent-scope access, so one memory trip carries data and readiness.  When a
-// tile publishes state s + 1 it has read its neighbours' state s, hence they
-// have read its state s - 1 (face and inlet neighbours are mutual): it resets
-// that slot, which state s + 3 takes, and the wait before publishing s + 2
-// completes the reset before any reader can poll for s + 3.
-//
-// All tiles must be on the device together: the host launches no more
-// work-groups than fit, and every wait is bounded (kResTicks); a wait that
-// runs out raises ctl[0], every tile then leaves, and the host repeats the
-// steps with one launch each (the input state is not written).
-//
-// The first T work-items own the cells; the cross-tile items go to others, so
-// a poll is not queued behind the publishing stores; the last wave forms the
-// inlet conveyances; the cells' friction is formed while the faces are
-// waited for.  Each work-item takes at most one item: tiles of triangles hold
-// up to 256, others up to 320 (fuller tiles are not run this way).  SPLIT
-// (few tiles): the cells' work-items take no items, so the friction is off the
-// step's critical path; else they take the items that the rest leave.
-constexpr unsigned long long kResEmpty = 0x7ff4c0de5ea1ed01ull;
-constexpr long long kResTicks = 100000000;  // wall_clock64 ticks (100 MHz): 1 s
-constexpr int kResT = 128;                  // cells per tile
-constexpr int64_t kResSteps = 4096;         // steps per launch
-
-struct ResArgs {
-  unsigned long long* ring;  // [4][3][N]
-  int32_t* ctl;              // [0]: a wait ran out
-  int64_t ns;
-  const int32_t* nbr;        // ELL, for the published cells
-  // optional record of the run (the adjoint's forward sweep): states 0 .. ns
-  // ([ns + 1][3][N]; state 0 is there already), clamps [ns][N], conveyances
-  double* rec;
-  uint8_t* rec_clamp;
-  double* rec_totalA;
-  int32_t n_inlet_all;
-};
-
-__device__ __forceinline__ unsigned long long res_peek(const unsigned long long* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void res_put(unsigned long long* p, unsigned long long v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// The NC values p, p + stride, ...: waits until none is empty.  False when
-// the wait ran out here or elsewhere.
-template <int NC>
-__device__ __forceinline__ bool res_poll(const unsigned long long* p, int64_t stride, int32_t* ctl, double (&v)[NC]) {
-  long long t0 = 0;
-  for (int n = 0;; ++n) {
-    unsigned long long u[NC];
-    bool ready = true;
-    for (int c = 0; c < NC; ++c) u[c] = res_peek(p + c * stride);
-    for (int c = 0; c < NC; ++c) ready = ready && u[c] != kResEmpty;
-    if (ready) {
-      for (int c = 0; c < NC; ++c) v[c] = __longlong_as_double((long long)u[c]);
-      return true;
-    }
-    if ((n & 63) == 63) {
-      const long long t = wall_clock64();
-      if (n == 63) t0 = t;
-      if (t - t0 > kResTicks) __hip_atomic_store(ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (__hip_atomic_load(ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-        for (int c = 0; c < NC; ++c) v[c] = 0.0;
-        return false;
-      }
-    }
-  }
-}
-
-__global__ __launch_bounds__(kBlock) void k_res_init(int64_t n, unsigned long long* ring, int32_t* ctl) {
-  const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (i < n) ring[i] = kResEmpty;
-  if (i == 0) *ctl = 0;
-}
-
-constexpr int res_items(int MD) { return MD == 3 ? 256 : 320; }
-constexpr int res_threads(int MD, bool split) { return res_items(MD) + (split ? kResT : 0); }
-constexpr int kResIn = 128;  // inlet faces whose constants a tile keeps in LDS
-
-template <int MD, bool SPLIT>
-__global__ __launch_bounds__(res_threads(MD, SPLIT), SPLIT ? 3 : 4) void k_swe_run(hg::TileArgs a, ResArgs R) {
-  constexpr int T = kResT, NT = res_threads(MD, SPLIT);
-  extern __shared__ double lds[];
-  double* C = lds;                // 10 x T cell quantities
-  double* FL = lds + 10 * T;      // 3 x MD x T face contributions
-  double* tA = FL + 3 * MD * T;   // conveyance of the tile's inlets (kTileInlets)
-  double* in_c = tA + kTileInlets;  // 3 x kResIn: L^(5/3), h_still, n of the first inlet's faces
-  int32_t* in_i = reinterpret_cast<int32_t*>(in_c + 3 * kResIn);  // and their cells
-  int32_t* stop = in_i + kResIn;
-  const int t = blockIdx.x, tid = threadIdx.x, i = t * T + tid;
-  const bool own = tid < T && i < a.N;
-  const int64_t N = a.N;
-  const double hsmall = a.hsmall;
-  double xi = 0.0, qx = 0.0, qy = 0.0, hs = 0.0, zb = 0.0, n = 0.0, S0x = 0.0, S0y = 0.0, A = 1.0, dti = a.dt;
-  int d = 0;
-  bool pub = false;  // read by another tile, or an inlet cell
-  if (own) {
-    xi = a.xi[i]; qx = a.qx[i]; qy = a.qy[i];
-    hs = a.hstill[i]; zb = a.zb[i]; n = a.n[i]; S0x = a.S0x[i]; S0y = a.S0y[i]; A = a.area[i];
-    d = a.deg ? a.deg[i] : MD;
-    if (a.dtc) dti = a.dtc[i];
-    for (int k = 0; k < d; ++k) {
-      const int j = R.nbr[k * N + i];
-      pub = pub || (j >= 0 ? j / T != t : a.g_kind[~j] == HG_BC_INLETQ);
-    }
-  }
-  // this work-item's item (the cross-tile ones are the first of the list)
-  const int it = a.items.off[t] + (SPLIT ? tid - T : (tid + NT - T) % NT);
-  const bool has = it >= a.items.off[t] && it < a.items.off[t + 1];
-  hg::ItemRec rec{};
-  if (has) rec = load_item(a.items, it, a.items.x0[t]);
-  const int code = rec.code;
-  const int ia = code & 1023, ka = (code >> 10) & 15, ib = (code >> 14) & 1023, kb = (code >> 24) & 15;
-  const int type = has ? (code >> 28) & 3 : 3;
-  GhostFace gf{};  // the other side's constants: a cross-tile neighbour's h_still and zb, or the ghost's
-  double gn = 1.0;
-  if (type == 1) {
-    gf.hs = a.hstill[rec.ref];
-    gf.zb = a.zb[rec.ref];
-  } else if (type == 2) {
-    gf = ghost_face(a, rec.ref);
-    gn = a.n[t * T + ia];
-  }
-  const int in0 = a.n_inlet > 0 ? a.tile_in_off[t] : 0, in1 = a.n_inlet > 0 ? a.tile_in_off[t + 1] : 0;
-  int bl0 = 0, fl0 = 0, fl1 = 0;  // the tile's first inlet
-  if (in1 > in0) {
-    bl0 = a.tile_in_list[in0];
-    fl0 = a.in_off[bl0];
-    fl1 = a.in_off[bl0 + 1];
-    for (int f = tid; f < min(kResIn, fl1 - fl0); f += NT) {
-      const int c = a.in_cell[fl0 + f];
-      in_i[f] = c;
-      in_c[f] = a.in_L53[fl0 + f];
-      in_c[kResIn + f] = a.hstill[c];
-      in_c[2 * kResIn + f] = a.n[c];
-    }
-  }
-  if (tid == 0) *stop = 0;
-  __syncthreads();
-
-  for (int64_t s = 0; s < R.ns; ++s) {
-    const unsigned long long* slot = R.ring + (s & 3) * 3 * N;
-    hg::CellQ me{};
-    if (own) {
-      me = hg::make_cellq(xi, hs, qx, qy, zb, a.half_g, hsmall);
-      C[0 * T + tid] = me.xi; C[1 * T + tid] = me.hs; C[2 * T + tid] = me.h; C[3 * T + tid] = me.hu;
-      C[4 * T + tid] = me.hv; C[5 * T + tid] = me.zb; C[6 * T + tid] = me.u; C[7 * T + tid] = me.v;
-      C[8 * T + tid] = me.s; C[9 * T + tid] = me.p;
-    }
-    if (in1 > in0 && tid >= NT - 64) {  // inlet conveyances (as in k_swe_tile)
-      const int l = tid & 63;
-      for (int sl = in0; sl < in1; ++sl) {
-        const int b = sl == in0 ? bl0 : a.tile_in_list[sl];
-        const int f0 = sl == in0 ? fl0 : a.in_off[b], f1 = sl == in0 ? fl1 : a.in_off[b + 1];
-        double acc = 0.0;
-        bool ok = true;
-        for (int base = f0; base < f1; base += 128) {  // two faces per lane in flight
-          double term[2] = {0.0, 0.0};
-          const bool kept = sl == in0 && base == f0;
-#pragma unroll
-          for (int r = 0; r < 2; ++r) {
-            const int f = base + 64 * r + l, k = 64 * r + l;
-            if (f >= f1) continue;
-            const int c = kept ? in_i[k] : a.in_cell[f];
-            double x[1];
-            if (s == 0)
-              x[0] = a.xi[c];
-            else if (!res_poll<1>(slot + c, N, R.ctl, x))
-              ok = false;
-            double h = x[0] + (kept ? in_c[kResIn + k] : a.hstill[c]);
-            if (h <= hsmall) h = hsmall;
-            const double w = (h > hsmall) ? 1.0 : 0.0;
-            term[r] = (kept ? in_c[k] : a.in_L53[f]) * h / (kept ? in_c[2 * kResIn + k] : a.n[c]) * w;
-          }
-          acc = wave_left_fold(acc, term[0], min(64, f1 - base));
-          if (f1 - base > 64) acc = wave_left_fold(acc, term[1], min(64, f1 - base - 64));
-        }
-        if (__ballot(!ok)) {
-          *stop = 1;
-        } else if (l == 0) {
-          tA[sl - in0] = acc;
-          if (R.rec_totalA) R.rec_totalA[s * R.n_inlet_all + b] = acc;  // every tile of inlet b writes the same value
-          if (!(acc > 1e-10)) a.flag[0] = 1;
-        }
-      }
-    }
-    __syncthreads();
-    if (has) {
-      hg::CellQ P, Q;
-      P.xi = C[0 * T + ia]; P.hs = C[1 * T + ia]; P.h = C[2 * T + ia]; P.hu = C[3 * T + ia];
-      P.hv = C[4 * T + ia]; P.zb = C[5 * T + ia]; P.u = C[6 * T + ia]; P.v = C[7 * T + ia];
-      P.s = C[8 * T + ia]; P.p = C[9 * T + ia];
-      if (type == 0) {
-        Q.xi = C[0 * T + ib]; Q.hs = C[1 * T + ib]; Q.h = C[2 * T + ib]; Q.hu = C[3 * T + ib];
-        Q.hv = C[4 * T + ib]; Q.zb = C[5 * T + ib]; Q.u = C[6 * T + ib]; Q.v = C[7 * T + ib];
-        Q.s = C[8 * T + ib]; Q.p = C[9 * T + ib];
-      } else if (type == 1) {
-        const int j = rec.ref;
-        double v[3];
-        if (s == 0) {
-          v[0] = a.xi[j]; v[1] = a.qx[j]; v[2] = a.qy[j];
-        } else if (!res_poll<3>(slot + j, N, R.ctl, v)) {
-          *stop = 1;
-        }
-        Q = hg::make_cellq(v[0], gf.hs, v[1], v[2], gf.zb, a.half_g, hsmall);
-      } else {
-        const double tot = gf.kind == HG_BC_INLETQ ? tA[(code >> 14) & (kTileInlets - 1)] : 0.0;
-        Q = ghost_cellq(gf, P, gn, rec.nx, rec.ny, tot, a.half_g, hsmall);
-      }
-      double fa[3], fb[3];
-      hg::roe_pair<true>(P, Q, rec.nx, rec.ny, a.g, a.half_g, hsmall, fa, fb);
-      if (type == 0)
-        for (int c = 0; c < 3; ++c) FL[(c * MD + kb) * T + ib] = fb[c] * rec.len;
-      for (int c = 0; c < 3; ++c) FL[(c * MD + ka) * T + ia] = fa[c] * rec.len;
-    }
-    double s1 = 0.0, s2 = 0.0;
-    if (own && me.h > hsmall) {
-      double fx, fy;
-      hg::friction(a.g, a.kn2, hsmall, me.h, me.hu, me.hv, n, fx, fy);
-      s1 = a.g * xi * S0x - fx;
-      s2 = a.g * xi * S0y - fy;
-    }
-    const double rA = hg::rcp_est(A);
-    __syncthreads();
-    if (*stop) return;  // the same for the whole tile: set before the barrier only
-    if (!own) continue;
-    double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
-    for (int k = 0; k < MD; ++k) {  // local face order
-      if (k < d) {
-        acc0 = acc0 + FL[(0 * MD + k) * T + tid];
-        acc1 = acc1 + FL[(1 * MD + k) * T + tid];
-        acc2 = acc2 + FL[(2 * MD + k) * T + tid];
-      }
-    }
-    xi = xi + dti * (hg::div_est(-acc0, A, rA) + 0.0);
-    qx = qx + dti * (hg::div_est(-acc1, A, rA) + s1);
-    qy = qy + dti * (hg::div_est(-acc2, A, rA) + s2);
-    const bool dry = xi < hsmall;
-    if (dry) {
-      xi = hsmall;
-      qx = 0.0;
-      qy = 0.0;
-    }
-    if (pub && s + 1 < R.ns) {
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the last step's reset is done (lgkmcnt, expcnt not waited on)
-      unsigned long long* o = R.ring + ((s + 1) & 3) * 3 * N + i;
-      unsigned long long* e = R.ring + ((s + 3) & 3) * 3 * N + i;
-      res_put(o, __double_as_longlong(xi));
-      res_put(o + N, __double_as_longlong(qx));
-      res_put(o + 2 * N, __double_as_longlong(qy));
-      for (int c = 0; c < 3; ++c) res_put(e + c * N, kResEmpty);
-    }
-    if (!(isfinite(xi) && isfinite(qx) && isfinite(qy))) a.flag[1] = 1;  // checked after the stepping call
-    if (R.rec) {
-      double* q = R.rec + (s + 1) * 3 * N + i;
-      q[0] = xi;
-      q[N] = qx;
-      q[2 * N] = qy;
-      R.rec_clamp[s * N + i] = dry ? 1 : 0;
-    }
-  }
-  if (own) {
-    a.xo[i] = xi;
-    a.qxo[i] = qx;
-    a.qyo[i] = qy;
-  }
-}
-
 // update_bed_data (process_bed_2D.jl:46-66): zb_ghost and S0 from zb.
 __global__ __launch_bounds__(kBlock) void k_bed_data(int N, int G, const double* zb, const int32_t* deg,
                                                     const int32_t* nbr, const double* fnx, const double* fny,
@@ -981,102 +617,6 @@ __device__ __forceinline__ CellAdj cell_adj(const hg::AdjArgs& a, int i) {
   c.y1 = STEP ? dti * c.lt1 : c.lt1;
   c.y2 = STEP ? dti * c.lt2 : c.lt2;
   return c;
-}
-
-// A boundary face's ghost state (bc_2D.jl:640-834) formed from its cell's
-// flux inputs `me`, and what the routing of its cotangent back to the cell
-// needs (the ghost's kind; inlet-Q: the ghost velocity v and wet flag w).
-struct GhostAdj {
-  int kind, bc;
-  double v, w;
-};
-
-__device__ __forceinline__ hg::CellQ adj_ghost_state(const hg::AdjArgs& a, const hg::CellQ& me, double n_i, int gi,
-                                                     double nx, double ny, GhostAdj& gs) {
-  const double hsmall = a.hsmall;
-  gs.kind = a.g_kind[gi];
-  gs.bc = a.g_bc[gi];
-  gs.v = 0.0;
-  gs.w = 0.0;
-  double hgh, qxg, qyg;
-  switch (gs.kind) {
-    case HG_BC_INLETQ: {
-      gs.w = (me.h > hsmall) ? 1.0 : 0.0;
-      gs.v = a.inletQ[gs.bc] / a.totalA[gs.bc] * a.g_L23[gi] / n_i;
-      hgh = me.h;
-      qxg = -me.h * gs.v * nx * gs.w;
-      qyg = -me.h * gs.v * ny * gs.w;
-      break;
-    }
-    case HG_BC_EXITH: {
-      const double hx = a.exitWSE[gs.bc] - me.zb;
-      hgh = (hx > hsmall) ? hx : hsmall;
-      qxg = me.hu;
-      qyg = me.hv;
-      break;
-    }
-    case HG_BC_WALL:
-      hgh = me.h;
-      qxg = -me.hu;
-      qyg = -me.hv;
-      break;
-    default: {
-      const double vdn = me.hu * nx + me.hv * ny;
-      hgh = me.h;
-      qxg = me.hu - 2.0 * vdn * nx;
-      qyg = me.hv - 2.0 * vdn * ny;
-      break;
-    }
-  }
-  hg::CellQ B;
-  B.hs = a.g_hstill[gi];
-  B.xi = hgh - B.hs;
-  B.h = hgh;
-  B.hu = qxg;
-  B.hv = qyg;
-  B.zb = a.g_zb[gi];
-  B.u = qxg / hgh;
-  B.v = qyg / hgh;
-  B.s = sqrt(hgh + hg::EPS);
-  B.p = a.half_g * ((B.xi + hg::EPS) * (B.xi + hg::EPS) + 2.0 * B.xi * B.hs);
-  return B;
-}
-
-// Routes the ghost's cotangent Bb back through its boundary rule: adds to
-// the cell's U, and its n / exit-H bed cotangents; writes the inlet ghost's
-// velocity cotangent for the inlet conveyance adjoint.
-__device__ __forceinline__ void adj_ghost_route(const hg::AdjArgs& a, const hg::CellQ& me, double n_i, int gi,
-                                                const GhostAdj& gs, const hg::SideBar& Bb, double nx, double ny,
-                                                hg::SideBar& U, double& nb, double& zbb) {
-  const double hgb = Bb.h + Bb.xi;  // xi_g = h_g - hstill_g
-  switch (gs.kind) {
-    case HG_BC_INLETQ: {  // h_g = h, q_g = -h v n w, v = (Q / A) L^(2/3) / n
-      const double v = gs.v, w = gs.w;
-      U.h += hgb + Bb.hu * (-v * nx * w) + Bb.hv * (-v * ny * w);
-      const double vb = Bb.hu * (-me.h * nx * w) + Bb.hv * (-me.h * ny * w);
-      nb += vb * (-v / n_i);
-      store_state(a.vbar + gi, vb);  // at device scope: other tiles of a resident run poll it
-      break;
-    }
-    case HG_BC_EXITH: {  // h_g = max(h_small, WSE - zb_cell), q_g = q
-      if (a.exitWSE[gs.bc] - me.zb > a.hsmall) zbb -= hgb;
-      U.hu += Bb.hu;
-      U.hv += Bb.hv;
-      break;
-    }
-    case HG_BC_WALL:
-      U.h += hgb;
-      U.hu -= Bb.hu;
-      U.hv -= Bb.hv;
-      break;
-    default: {
-      const double vdnb = -2.0 * (Bb.hu * nx + Bb.hv * ny);
-      U.h += hgb;
-      U.hu += Bb.hu + vdnb * nx;
-      U.hv += Bb.hv + vdnb * ny;
-      break;
-    }
-  }
 }
 
 // The VJP of the boundary face in slot s (cell i = s % N, local face
@@ -1251,156 +791,8 @@ __device__ __forceinline__ void adj_cell_finish(const hg::AdjArgs& a, int i, con
 // LDS: (13 + 4 MD) doubles and one int per cell, 51 KiB for 256 triangles:
 // three work-groups per CU, as many as the registers allow.  (At 53 KiB and
 // more per work-group only two of them run on a CU at once on MI355X.)
-constexpr int kAdjRows = 13;  // CellQ without h and p (8), z (3), 1 / h, 0.5 / s
-
 size_t adj_tile_lds_bytes(int T, int MD) {
   return size_t(kAdjRows * T + 4 * MD * T) * sizeof(double) + size_t(T) * sizeof(int32_t);
-}
-
-// Rows: 0 xi, 1 h_still, 2 hu, 3 hv, 4 zb, 5 u, 6 v, 7 s, 8-10 z, 11 1 / h,
-// 12 0.5 / s.  The depth and the pressure are re-formed where read, with
-// make_cellq's operations.
-template <int T>
-__device__ __forceinline__ hg::CellQ lds_cellq(const double* C, int r, double half_g, double hsmall) {
-  hg::CellQ q;
-  q.xi = C[0 * T + r]; q.hs = C[1 * T + r]; q.hu = C[2 * T + r]; q.hv = C[3 * T + r];
-  q.zb = C[4 * T + r]; q.u = C[5 * T + r]; q.v = C[6 * T + r]; q.s = C[7 * T + r];
-  double h = q.xi + q.hs;
-  if (h <= hsmall) h = hsmall;
-  q.h = h;
-  q.p = half_g * ((q.xi + hg::EPS) * (q.xi + hg::EPS) + 2.0 * q.xi * q.hs);
-  return q;
-}
-
-// A cell's flux inputs as the tiled reverse step forms them, for the tile's
-// own cells and for cross-tile neighbours alike (so a face's VJP has the same
-// bits whichever work-group evaluates it): make_cellq's clamp and pressure,
-// with u and v from one reciprocal of h and sqrt(h + eps) and its reciprocal
-// from one rsqrt.  rh = 1 / h, r2s = 0.5 / sqrt(h + eps).
-__device__ __forceinline__ hg::CellQ adj_cellq(double xi, double hs, double qx, double qy, double zb, double half_g,
-                                               double hsmall, double& rh, double& r2s) {
-  hg::CellQ c;
-  c.xi = xi;
-  c.hs = hs;
-  double h = xi + hs, hu = qx, hv = qy;
-  if (h <= hsmall) {
-    h = hsmall;
-    hu = 0.0;
-    hv = 0.0;
-  }
-  c.h = h;
-  c.hu = hu;
-  c.hv = hv;
-  c.zb = zb;
-  rh = 1.0 / h;
-  c.u = hu * rh;
-  c.v = hv * rh;
-  const double he = h + hg::EPS;
-  const double rs = rsqrt(he);
-  c.s = he * rs;
-  r2s = 0.5 * rs;
-  c.p = half_g * ((xi + hg::EPS) * (xi + hg::EPS) + 2.0 * xi * hs);
-  return c;
-}
-
-// A cross-tile neighbour's raw data as a work item of the tiled reverse step
-// reads it.
-struct NbrRaw {
-  double xi, hs, qx, qy, zb, m0, m1, m2, dt, area;
-  uint8_t clamped;
-};
-
-template <bool STEP>
-__device__ __forceinline__ NbrRaw nbr_load(const hg::AdjArgs& a, int j) {
-  NbrRaw r;
-  r.xi = a.xi[j]; r.hs = a.hstill[j]; r.qx = a.qx[j]; r.qy = a.qy[j]; r.zb = a.zb[j];
-  r.m0 = a.lx[j]; r.m1 = a.lqx[j]; r.m2 = a.lqy[j];
-  r.clamped = (STEP && a.mask) ? a.mask[j] : uint8_t(0);
-  r.dt = a.dtc ? a.dtc[j] : a.dt;
-  r.area = a.area[j];
-  return r;
-}
-
-// One work item of the tiled reverse step (see k_adj_tile); nr is the
-// neighbour of a cross-tile item.
-template <bool STEP, int T, int MD>
-__device__ __forceinline__ void adj_item(const hg::AdjArgs& a, int t, const double* C, double* S, int32_t* Xm,
-                                         const hg::ItemRec& rec, const NbrRaw& nr) {
-  const double hsmall = a.hsmall, half_g = a.half_g;
-  const int code = rec.code;
-  const int ia = code & 1023, ka = (code >> 10) & 15;
-  const int ib = (code >> 14) & 1023, kb = (code >> 24) & 15;
-  const int type = (code >> 28) & 3;
-  const double nx = rec.nx, ny = rec.ny, L = rec.len;
-  // P / Q: the evaluation's first / second side (normal from P)
-  const bool sw = type != 2 && !(nx > 0.0 || (nx == 0.0 && ny > 0.0));
-  const double ex = sw ? -nx : nx, ey = sw ? -ny : ny;
-  hg::CellQ P, Q;
-  double zP0, zP1, zP2, zQ0, zQ1, zQ2, rhP, rhQ, r2P, r2Q;
-  int ip = ia, kp = ka, iq = ia, kq = ka;  // LDS slots of P and Q (type 0); the tile's cell otherwise
-  GhostAdj gs{};
-  double n_a = 0.0;
-  if (type == 0) {
-    if (sw) { ip = ib; kp = kb; } else { iq = ib; kq = kb; }
-    P = lds_cellq<T>(C, ip, half_g, hsmall);
-    Q = lds_cellq<T>(C, iq, half_g, hsmall);
-    zP0 = C[8 * T + ip]; zP1 = C[9 * T + ip]; zP2 = C[10 * T + ip];
-    zQ0 = C[8 * T + iq]; zQ1 = C[9 * T + iq]; zQ2 = C[10 * T + iq];
-    rhP = C[11 * T + ip]; r2P = C[12 * T + ip];
-    rhQ = C[11 * T + iq]; r2Q = C[12 * T + iq];
-  } else {
-    const hg::CellQ Lc = lds_cellq<T>(C, ia, half_g, hsmall);
-    const double zL0 = C[8 * T + ia], zL1 = C[9 * T + ia], zL2 = C[10 * T + ia];
-    const double rhL = C[11 * T + ia], r2L = C[12 * T + ia];
-    hg::CellQ G;
-    double zG0 = 0.0, zG1 = 0.0, zG2 = 0.0;
-    double rhG, r2G;
-    if (type == 1) {  // cross-tile neighbour
-      G = adj_cellq(nr.xi, nr.hs, nr.qx, nr.qy, nr.zb, half_g, hsmall, rhG, r2G);
-      double m0 = nr.m0, m1 = nr.m1, m2 = nr.m2;
-      if (nr.clamped) m0 = m1 = m2 = 0.0;
-      const double rAj = 1.0 / nr.area;
-      zG0 = (STEP ? nr.dt * m0 : m0) * rAj;
-      zG1 = (STEP ? nr.dt * m1 : m1) * rAj;
-      zG2 = (STEP ? nr.dt * m2 : m2) * rAj;
-    } else {  // ghost (no cotangent of its own)
-      n_a = a.n[t * T + ia];
-      G = adj_ghost_state(a, Lc, n_a, rec.ref, nx, ny, gs);
-      rhG = 1.0 / G.h;
-      r2G = 0.5 / G.s;
-    }
-    P = sw ? G : Lc;
-    Q = sw ? Lc : G;
-    zP0 = sw ? zG0 : zL0; zP1 = sw ? zG1 : zL1; zP2 = sw ? zG2 : zL2;
-    zQ0 = sw ? zL0 : zG0; zQ1 = sw ? zL1 : zG1; zQ2 = sw ? zL2 : zG2;
-    rhP = sw ? rhG : rhL; r2P = sw ? r2G : r2L;
-    rhQ = sw ? rhL : rhG; r2Q = sw ? r2L : r2G;
-  }
-  const double c[3] = {L * zQ0 - L * zP0, L * zQ1 - L * zP1, L * zQ2 - L * zP2};
-  hg::ExtBar eP, eQ;
-  hg::roe_vjp_ext(P, Q, ex, ey, a.g, half_g, hsmall, c, eP, eQ);
-  hg::SideBar sP = hg::ext_to_side_r(eP, P, rhP, r2P, half_g);
-  const hg::SideBar sQ = hg::ext_to_side_r(eQ, Q, rhQ, r2Q, half_g);
-  if (type == 2) {
-    double nb = 0.0, zbb = 0.0;
-    adj_ghost_route(a, P, n_a, rec.ref, gs, sQ, nx, ny, sP, nb, zbb);
-    if (gs.kind == HG_BC_EXITH) {
-      S[(3 * MD + ka) * T + ia] = zbb;
-      atomicOr(&Xm[ia], 1 << ka);
-    } else {
-      S[(3 * MD + ka) * T + ia] = nb;
-    }
-  }
-  if (type == 0 || !sw) {
-    S[(0 * MD + kp) * T + ip] = (P.h > hsmall) ? sP.xi + sP.h : sP.xi;
-    S[(1 * MD + kp) * T + ip] = sP.hu;
-    S[(2 * MD + kp) * T + ip] = sP.hv;
-  }
-  if (type == 0 || sw) {
-    S[(0 * MD + kq) * T + iq] = (Q.h > hsmall) ? sQ.xi + sQ.h : sQ.xi;
-    S[(1 * MD + kq) * T + iq] = sQ.hu;
-    S[(2 * MD + kq) * T + iq] = sQ.hv;
-  }
 }
 
 template <bool STEP, int T, int MD>
@@ -1508,271 +900,6 @@ __global__ __launch_bounds__(T, 3) void k_adj_tile(hg::AdjArgs a0) {
   ca.y2 = STEP ? dti * lt2 : lt2;
   // the slots carry xi + h already (h-bar only where the cell is wet)
   adj_finish_store<STEP>(a, i, ca, fin, uxh, 0.0, uqx, uqy, nb, zbb);
-}
-
-// Reverse mode of a resident run: R.ns steps of k_adj_tile and k_inlet_adj in
-// one launch over tiles of 128 cells, with the values they form, in their
-// order (same bits).  A tile keeps its cells' cotangents and sums in
-// registers and reads ahead the recorded state of the next step; the border
-// cells' cotangents and the inlet ghosts' velocity cotangents travel through
-// rings as the forward run's states do (see k_swe_run).  Sums are written to
-// arrays of their own (o_*), which the host takes over when the run is done.
-// One launch per step took 8.5 us for the tiles and 2.6 us for the inlets, of
-// which about 3 us and 1 us were launch and first loads; a step takes 4.6 us
-// here on 1,000 quads, 6.0 on a 1,300-cell channel (its inlet tiles exchange
-// twice per step) and 6.4 on 59k triangles.  Up to 512 tiles: the registers
-// that hold the cells allow two tiles per CU.
-struct AdjRunArgs {
-  unsigned long long* ring;   // [4][3][N] cotangents
-  unsigned long long* vring;  // [4][G] inlet ghost velocity cotangents
-  int32_t* ctl;
-  int64_t ns, G;
-  const double* rec;          // [ns][3][N] states
-  const uint8_t* rec_clamp;   // [ns][N]
-  const double* rec_totalA;   // [ns][n_inlet]
-  int32_t n_inlet;
-  const int32_t* tile_in_off;
-  const int32_t* tile_in_list;
-  const int32_t* in_off;
-  const hg::InletFaceRec* in_rec;
-  const double* Qbar;
-  double *o_nbar, *o_zbbar, *o_S0bar, *o_Qbar;
-};
-
-template <int MD>
-__global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(hg::AdjArgs a, AdjRunArgs R) {
-  constexpr int T = kResT, NT = res_items(MD);
-  extern __shared__ double lds[];
-  double* C = lds;                                         // kAdjRows x T
-  double* S = lds + kAdjRows * T;                          // 4 x MD x T
-  double* sA = S + 4 * MD * T;                             // 256
-  double* sQ = sA + 256;                                   // 256
-  double* qa = sQ + 256;                                   // kTileInlets: the inlets' discharge cotangents
-  int32_t* Xm = reinterpret_cast<int32_t*>(qa + kTileInlets);  // T
-  int32_t* stop = Xm + T;
-  const int t = blockIdx.x, tid = threadIdx.x, i = t * T + tid;
-  const bool own = tid < T && i < a.N;
-  const int64_t N = a.N;
-  const double hsmall = a.hsmall;
-  double hs = 0.0, zb = 0.0, n = 0.0, S0x = 0.0, S0y = 0.0, A = 1.0, dti = a.dt;
-  double l0 = 0.0, l1 = 0.0, l2 = 0.0, nbar = 0.0, zbbar = 0.0, S0bx = 0.0, S0by = 0.0;
-  int d = 0;
-  bool pub = false;  // read by another tile
-  if (own) {
-    hs = a.hstill[i]; zb = a.zb[i]; n = a.n[i]; S0x = a.S0x[i]; S0y = a.S0y[i]; A = a.area[i];
-    d = a.deg ? a.deg[i] : MD;
-    if (a.dtc) dti = a.dtc[i];
-    l0 = a.lx[i]; l1 = a.lqx[i]; l2 = a.lqy[i];
-    if (a.nbar) nbar = a.nbar[i];
-    if (a.zbbar) {
-      zbbar = a.zbbar[i];
-      S0bx = a.S0bar[i];
-      S0by = a.S0bar[N + i];
-    }
-    for (int k = 0; k < d; ++k) {
-      const int j = a.nbr[k * N + i];
-      pub = pub || (j >= 0 && j / T != t);
-    }
-  }
-  const int it = a.items.off[t] + (tid + NT - T) % NT;
-  const bool has = it < a.items.off[t + 1];
-  hg::ItemRec rec{};
-  if (has) rec = load_item(a.items, it, a.items.x0[t]);
-  const int type = has ? (rec.code >> 28) & 3 : 3;
-  NbrRaw nr{};
-  if (type == 1) {
-    nr.hs = a.hstill[rec.ref]; nr.zb = a.zb[rec.ref]; nr.area = a.area[rec.ref];
-    nr.dt = a.dtc ? a.dtc[rec.ref] : a.dt;
-  }
-  const bool in_ghost = type == 2 && a.g_kind[rec.ref] == HG_BC_INLETQ;
-  const int in0 = R.n_inlet > 0 ? R.tile_in_off[t] : 0, in1 = R.n_inlet > 0 ? R.tile_in_off[t + 1] : 0;
-  int my_sl = -1, my_f = -1;  // an inlet cell's inlet and first face there
-  for (int sl = in0; sl < in1; ++sl) {
-    const int b = R.tile_in_list[sl];
-    for (int f = R.in_off[b]; f < R.in_off[b + 1]; ++f)
-      if (own && R.in_rec[f].cell == i && R.in_rec[f].first) {
-        my_sl = sl;
-        my_f = f;
-      }
-    if (tid == 0) qa[sl - in0] = R.Qbar[b];
-  }
-  if (tid == 0) *stop = 0;
-  // the recorded state of the step (own cell, and a cross-tile neighbour's), read one step ahead
-  double px = 0.0, pqx = 0.0, pqy = 0.0, jx = 0.0, jqx = 0.0, jqy = 0.0;
-  uint8_t pm = 0, jm = 0;
-  auto read_ahead = [&](int64_t k) {
-    const double* q = R.rec + k * 3 * N;
-    const uint8_t* m = R.rec_clamp + k * N;
-    if (own) {
-      px = q[i]; pqx = q[N + i]; pqy = q[2 * N + i];
-      pm = m[i];
-    }
-    if (type == 1) {
-      jx = q[rec.ref]; jqx = q[N + rec.ref]; jqy = q[2 * N + rec.ref];
-      jm = m[rec.ref];
-    }
-  };
-  read_ahead(R.ns - 1);
-
-  for (int64_t r = 0; r < R.ns; ++r) {
-    const int64_t k = R.ns - 1 - r;  // the step that is reversed
-    const unsigned long long* slot = R.ring + (r & 3) * 3 * N;
-    a.totalA = R.rec_totalA ? R.rec_totalA + k * R.n_inlet : nullptr;
-    a.vbar = reinterpret_cast<double*>(R.vring + (r & 3) * R.G);
-    hg::CellQ me{};
-    double y0 = 0.0, y1 = 0.0, y2 = 0.0;
-    if (pm) l0 = l1 = l2 = 0.0;
-    nr.xi = jx; nr.qx = jqx; nr.qy = jqy;
-    nr.clamped = jm;
-    if (own) {
-      double rh, r2s;
-      me = adj_cellq(px, hs, pqx, pqy, zb, a.half_g, hsmall, rh, r2s);
-      const double rA = 1.0 / A;
-      y0 = dti * l0;
-      y1 = dti * l1;
-      y2 = dti * l2;
-      C[0 * T + tid] = me.xi; C[1 * T + tid] = me.hs; C[2 * T + tid] = me.hu; C[3 * T + tid] = me.hv;
-      C[4 * T + tid] = me.zb; C[5 * T + tid] = me.u; C[6 * T + tid] = me.v; C[7 * T + tid] = me.s;
-      C[8 * T + tid] = y0 * rA;
-      C[9 * T + tid] = y1 * rA;
-      C[10 * T + tid] = y2 * rA;
-      C[11 * T + tid] = rh;
-      C[12 * T + tid] = r2s;
-      for (int c = 0; c < MD; ++c) S[(3 * MD + c) * T + tid] = 0.0;
-      Xm[tid] = 0;
-    }
-    if (k > 0) read_ahead(k - 1);
-    __syncthreads();
-    if (has) {
-      if (type == 1) {
-        const int j = rec.ref;
-        double v[3];
-        if (r == 0) {
-          v[0] = a.lx[j]; v[1] = a.lqx[j]; v[2] = a.lqy[j];
-        } else if (!res_poll<3>(slot + j, N, R.ctl, v)) {
-          *stop = 1;
-        }
-        nr.m0 = v[0]; nr.m1 = v[1]; nr.m2 = v[2];
-      }
-      if (in_ghost) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): its last reset is done before it publishes again
-      adj_item<true, T, MD>(a, t, C, S, Xm, rec, nr);
-      if (in_ghost) res_put(R.vring + ((r + 2) & 3) * R.G + rec.ref, kResEmpty);
-    }
-    // the source term's cotangents, while the faces are waited for
-    double sxi = 0.0, sh = 0.0, sqx = 0.0, sqy = 0.0, sn = 0.0, sS0x = 0.0, sS0y = 0.0;
-    const bool wet = me.h > hsmall;
-    if (own && wet)
-      hg::source_vjp(a.g, a.kn2, hsmall, me.xi, me.h, me.hu, me.hv, n, S0x, S0y, y1, y2, sxi, sh, sqx, sqy, sn, sS0x,
-                     sS0y);
-    __syncthreads();
-    if (*stop) return;
-    if (own) {
-      double uxh = 0.0, uqx = 0.0, uqy = 0.0, nb = 0.0, zbb = 0.0;
-      const int xm = Xm[tid];
-      for (int c = 0; c < MD; ++c) {  // local face order
-        if (c < d) {
-          uxh += S[(0 * MD + c) * T + tid];
-          uqx += S[(1 * MD + c) * T + tid];
-          uqy += S[(2 * MD + c) * T + tid];
-          const double e = S[(3 * MD + c) * T + tid];
-          if ((xm >> c) & 1)
-            zbb += e;
-          else
-            nb += e;
-        }
-      }
-      nb += sn;
-      double ox = uxh + sxi, oqx = 0.0, oqy = 0.0;
-      if (wet) {
-        ox += sh;
-        oqx = uqx + sqx;
-        oqy = uqy + sqy;
-      }
-      l0 = ox + l0;
-      l1 = oqx + l1;
-      l2 = oqy + l2;
-      nbar = nbar + nb;
-      zbbar = zbbar + zbb;
-      S0bx = S0bx + sS0x;
-      S0by = S0by + sS0y;
-    }
-    // inlet conveyance adjoint (as k_inlet_adj)
-    for (int sl = in0; sl < in1; ++sl) {
-      const int b = R.tile_in_list[sl];
-      const int f0 = R.in_off[b], f1 = R.in_off[b + 1];
-      const double Ai = a.totalA[b], Qb = a.inletQ[b];
-      if (tid < 256) {
-        double pa = 0.0, pq = 0.0;
-        for (int f = f0 + tid; f < f1; f += 256) {
-          const hg::InletFaceRec fr = R.in_rec[f];
-          double vb[1];
-          if (!res_poll<1>(R.vring + (r & 3) * R.G + fr.ghost, 0, R.ctl, vb)) *stop = 1;
-          const double nc = a.n[fr.cell];
-          const double v = Qb / Ai * fr.L23 / nc;
-          pa += vb[0] * (-v / Ai);
-          pq += vb[0] * (fr.L23 / (Ai * nc));
-        }
-        sA[tid] = pa;
-        sQ[tid] = pq;
-      }
-      __syncthreads();
-      if (*stop) return;
-      if (tid < 128) {
-        sA[tid] += sA[tid + 128];
-        sQ[tid] += sQ[tid + 128];
-      }
-      __syncthreads();
-      if (tid < 64) {
-        double xa = sA[tid] + sA[tid + 64], xq = sQ[tid] + sQ[tid + 64];
-        for (int w = 32; w > 0; w >>= 1) {
-          xa = xa + __shfl_xor(xa, w, 64);
-          xq = xq + __shfl_xor(xq, w, 64);
-        }
-        if (tid == 0) {
-          sA[0] = xa;
-          qa[sl - in0] = qa[sl - in0] + xq;
-        }
-      }
-      __syncthreads();
-      if (my_sl == sl) {
-        const double h0 = me.xi + hs;
-        if (h0 > hsmall) {
-          const double Ab = sA[0];
-          for (int f = my_f; f >= 0;) {
-            const hg::InletFaceRec fr = R.in_rec[f];
-            l0 += Ab * fr.L53 / n;
-            nbar += Ab * (-fr.L53 * h0 / (n * n));
-            f = fr.next;
-          }
-        }
-      }
-      __syncthreads();  // sA / sQ reuse
-    }
-    if (own && pub && r + 1 < R.ns) {
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the last step's reset is done
-      unsigned long long* o = R.ring + ((r + 1) & 3) * 3 * N + i;
-      unsigned long long* e = R.ring + ((r + 3) & 3) * 3 * N + i;
-      res_put(o, __double_as_longlong(l0));
-      res_put(o + N, __double_as_longlong(l1));
-      res_put(o + 2 * N, __double_as_longlong(l2));
-      for (int c = 0; c < 3; ++c) res_put(e + c * N, kResEmpty);
-    }
-  }
-  if (own) {
-    a.ox[i] = l0;
-    a.oqx[i] = l1;
-    a.oqy[i] = l2;
-    if (R.o_nbar) R.o_nbar[i] = nbar;
-    if (R.o_zbbar) {
-      R.o_zbbar[i] = zbbar;
-      R.o_S0bar[i] = S0bx;
-      R.o_S0bar[N + i] = S0by;
-    }
-  }
-  for (int sl = in0 + tid; sl < in1; sl += NT) {  // by the tile of the inlet's first face
-    const int b = R.tile_in_list[sl];
-    if (R.in_rec[R.in_off[b]].cell / T == t) R.o_Qbar[b] = qa[sl - in0];
-  }
 }
 
 // Inlet conveyance adjoint (bc_2D.jl:640-694): v_f = (Q_b / A_b) L^(2/3) / n
@@ -2453,24 +1580,8 @@ __global__ __launch_bounds__(64) void k_mfma_probe(const T* A, const T* B, T* D)
   for (int r = 0; r < 4; ++r) D[M::row(kq, r) * 16 + col] = acc[r];
 }
 
-// ---- Tsit5: Tsitouras' 5(4) Runge-Kutta pair (Ch. Tsitouras, Comput. Math.
-// Appl. 62 (2011) 770-775), first-same-as-last, the adaptive integrator the
-// reference's examples run through OrdinaryDiffEq (Tsit5()).
-namespace tsit5 {
-constexpr double c[7] = {0.0, 0.161, 0.327, 0.9, 0.9800255409045097, 1.0, 1.0};
-constexpr double a[7][6] = {
-    {0.0, 0.0, 0.0, 0.0, 0.0, 0.0},
-    {0.161, 0.0, 0.0, 0.0, 0.0, 0.0},
-    {-0.008480655492356989, 0.335480655492357, 0.0, 0.0, 0.0, 0.0},
-    {2.897153057105493, -6.359448489975075, 4.3622954328695815, 0.0, 0.0, 0.0},
-    {5.325864828439257, -11.748883564062828, 7.4955393428898365, -0.09249506636175525, 0.0, 0.0},
-    {5.86145544294642, -12.92096931784711, 8.159367898576159, -0.071584973281401, -0.028269050394068383, 0.0},
-    {0.09646076681806523, 0.01, 0.4798896504144996, 1.379008574103742, -3.290069515436081, 2.324710524099774}};
-// b = a[6] (fifth order, b7 = 0); btilde = b - bhat (bhat: the embedded fourth-order weights)
-constexpr double btilde[7] = {-0.00178001105222577714, -0.0008164344596567469, 0.007880878010261995,
-                              -0.1447110071732629,     0.5823571654525552,    -0.45808210592918697,
-                              0.015151515151515152};
-}  // namespace tsit5
+// ---- Tsit5 (hg_tsit5.hpp): stage combinations and the error norm
+namespace tsit5 = hg::tsit5;
 
 struct RkArgs {
   int64_t n;             // 3N
@@ -2576,76 +1687,35 @@ __global__ __launch_bounds__(kBlock) void k_swe_step_jvp(JvpArgs J) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.N) return;
   const double hsmall = a.hsmall;
-  const Dual1 xi = ldd(a.xi, J.dxi, i);
-  const double hs = a.hstill[i];
-  const Dual1 qx0 = ldd(a.qx, J.dqx, i), qy0 = ldd(a.qy, J.dqy, i);
-  Dual1 h = xi + hs, qx = qx0, qy = qy0;  // semi_discretize_swe_2D.jl:101-106
-  if (h <= hsmall) {
-    h = Dual1(hsmall);
-    qx = Dual1(0.0);
-    qy = Dual1(0.0);
-  }
-  const Dual1 zb = ldd(a.zb, J.dzb, i);
+  const Dual1 xi = ldd(a.xi, J.dxi, i), qx0 = ldd(a.qx, J.dqx, i), qy0 = ldd(a.qy, J.dqy, i);
   const Dual1 nman = ldd(a.n, J.dn, i);
-  const hg::SideT<Dual1> Ls{xi, Dual1(hs), h, qx, qy, zb};
+  const hg::CellQT<Dual1> me = hg::make_cellq(xi, a.hstill[i], qx0, qy0, ldd(a.zb, J.dzb, i), a.half_g, hsmall);
+  const Dual1 h = me.h, qx = me.hu, qy = me.hv;
   Dual1 acc0(0.0), acc1(0.0), acc2(0.0);
   const int d = a.deg[i];
   for (int k = 0; k < d; ++k) {
     const int s = k * a.N + i;
     const int j = a.nbr[s];
     const double nx = a.fnx[s], ny = a.fny[s], L = a.flen[s];
-    hg::SideT<Dual1> Rs;
+    hg::CellQT<Dual1> B;
     if (j >= 0) {
-      const Dual1 xj = ldd(a.xi, J.dxi, j);
-      const double hsj = a.hstill[j];
-      Dual1 hj = xj + hsj, qxj = ldd(a.qx, J.dqx, j), qyj = ldd(a.qy, J.dqy, j);
-      if (hj <= hsmall) {
-        hj = Dual1(hsmall);
-        qxj = Dual1(0.0);
-        qyj = Dual1(0.0);
+      B = hg::make_cellq(ldd(a.xi, J.dxi, j), a.hstill[j], ldd(a.qx, J.dqx, j), ldd(a.qy, J.dqy, j),
+                         ldd(a.zb, J.dzb, j), a.half_g, hsmall);
+    } else {
+      GhostFaceT<Dual1> gf = ghost_face<Dual1>(a, ~j);
+      if (J.dg_zb) gf.zb.d = J.dg_zb[~j];
+      Dual1 tot(0.0);
+      if (gf.kind == HG_BC_INLETQ) {
+        if (J.dinletQ) gf.p.d = J.dinletQ[gf.bc];
+        tot = ldd(a.totalA, J.dtotalA, gf.bc);
       }
-      Rs = hg::SideT<Dual1>{xj, Dual1(hsj), hj, qxj, qyj, ldd(a.zb, J.dzb, j)};
-    } else {  // ghost (bc_2D.jl:640-834), internal cell = this cell
-      const int gi = ~j;
-      Dual1 hgh, qxg, qyg;
-      switch (a.g_kind[gi]) {
-        case HG_BC_INLETQ: {
-          const int b = a.g_bc[gi];
-          const double w = (h > hsmall) ? 1.0 : 0.0;
-          const Dual1 v = ldd(a.inletQ, J.dinletQ, b) / ldd(a.totalA, J.dtotalA, b) * a.g_L23[gi] / nman;
-          hgh = h;
-          qxg = -h * v * nx * w;
-          qyg = -h * v * ny * w;
-          break;
-        }
-        case HG_BC_EXITH: {
-          const Dual1 hx = a.exitWSE[a.g_bc[gi]] - zb;
-          hgh = (hx > hsmall) ? hx : Dual1(hsmall);
-          qxg = qx;
-          qyg = qy;
-          break;
-        }
-        case HG_BC_WALL:
-          hgh = h;
-          qxg = -qx;
-          qyg = -qy;
-          break;
-        default: {  // HG_BC_SYMM
-          const Dual1 vdn = qx * nx + qy * ny;
-          hgh = h;
-          qxg = qx - 2.0 * vdn * nx;
-          qyg = qy - 2.0 * vdn * ny;
-          break;
-        }
-      }
-      const double hsg = a.g_hstill[gi];
-      Rs = hg::SideT<Dual1>{hgh - hsg, Dual1(hsg), hgh, qxg, qyg, ldd(a.g_zb, J.dg_zb, gi)};
+      B = ghost_cellq(gf, me, nman, nx, ny, tot, a.half_g, hsmall);
     }
-    Dual1 f0, f1, f2;
-    hg::roe_flux(Ls, Rs, nx, ny, a.g, a.half_g, hsmall, f0, f1, f2);
-    acc0 = acc0 + f0 * L;
-    acc1 = acc1 + f1 * L;
-    acc2 = acc2 + f2 * L;
+    Dual1 f[3], fb[3];
+    hg::roe_pair<false>(me, B, nx, ny, a.g, a.half_g, hsmall, f, fb);
+    acc0 = acc0 + f[0] * L;
+    acc1 = acc1 + f[1] * L;
+    acc2 = acc2 + f[2] * L;
   }
   const double A = a.area[i];
   const Dual1 r0 = -acc0 / A, r1 = -acc1 / A, r2 = -acc2 / A;
@@ -2786,11 +1856,6 @@ int free_items(hg_ctx* ctx, hg::ItemTable& d) {
   if (!rc) rc = dfree(ctx, d.ref);
   if (!rc) rc = dfree(ctx, d.geo);
   return rc;
-}
-
-size_t res_lds_bytes(int MD) {
-  return size_t(10 * kResT + 3 * MD * kResT + kTileInlets + 3 * kResIn) * sizeof(double) +
-         (kResIn + 1) * sizeof(int32_t);
 }
 
 size_t tile_lds_bytes(int T, int maxdeg) {
@@ -3146,75 +2211,90 @@ int enqueue_step_p(hg_ctx* ctx, const double* const in[3], double* const out[3],
 
 // ---- resident run, host side
 
-// Work-groups of resident runs in flight on each device over the process's
-// contexts: a run is started only while all of them fit together.
+// Shares of each device (of kResRoom) that resident runs in flight take, over
+// the process's contexts: a run is started only while all of them fit together.
+constexpr int kResRoom = 1 << 20;
 std::mutex g_res_mu;
-int g_res_groups[kMaxDevices] = {};
+int g_res_room[kMaxDevices] = {};
 
-// Tiles of a resident run that the device surely holds at once.  A tile's
-// waves need not spread evenly over a CU's four SIMDs (two tiles of six waves
-// each were not resident together where three waves fit per SIMD), so each
-// tile counts with its fullest SIMD.
-template <int MD, bool SPLIT>
-int res_capacity(hg_ctx* ctx) {
-  constexpr int waves = res_threads(MD, SPLIT) / 64, per_simd = SPLIT ? 3 : 4;
-  int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_swe_run<MD, SPLIT>, 64 * waves, res_lds_bytes(MD)) !=
-      hipSuccess)
-    return 0;
-  return std::min(per_cu, per_simd / ((waves + 3) / 4)) * ctx->ncu;
+// Whether nsteps steps (or right-hand sides) may run resident, and as which
+// variant: one field, the default tiling of small meshes, at most one item
+// per work-item and 64 inlets per tile, n from the field, a law or a network
+// of at most four units per layer, and steps enough to pay for the ring's
+// initialisation.
+bool res_kind(hg_ctx* ctx, int64_t nsteps, bool dual, hg::ResKind& k) {
+  if (!ctx->tiled || ctx->res_off || ctx->K != 1 || nsteps < 4 || ctx->tileT != kResT || ctx->tileMD > 4 ||
+      ctx->max_items > res_items(ctx->tileMD) || (ctx->n_inlet > 0 && !ctx->fuse_inlet) || ctx->ude_prec ||
+      ctx->device >= kMaxDevices)
+    return false;
+  k.md = ctx->tileMD;
+  k.nmode = ctx->nlaw.kind != hg::NLAW_OFF ? hg::RES_N_LAW : ctx->lux.choice ? hg::RES_N_NET : hg::RES_N_FIELD;
+  k.dual = dual;
+  if (k.nmode == hg::RES_N_NET && ctx->lux_mw != 4) return false;
+  for (bool split : {true, false}) {
+    k.split = split;
+    int32_t& cap = ctx->res_cap[split][k.nmode][dual];
+    if (cap < 0) cap = hg::res_capacity(k, ctx->ncu);
+    if (ctx->ntiles <= cap) return true;
+  }
+  return false;
 }
 
-template <int MD, bool SPLIT>
-void launch_run(hg_ctx* ctx, const hg::TileArgs& a, const ResArgs& R) {
-  hipLaunchKernelGGL((k_swe_run<MD, SPLIT>), dim3(ctx->ntiles), dim3(res_threads(MD, SPLIT)), res_lds_bytes(MD),
-                     ctx->stream, a, R);
+// What the variants read of the closure in force.
+hg::ResArgs res_args(hg_ctx* ctx, int64_t nsteps) {
+  hg::ResArgs R{};
+  R.ring = ctx->res_ring;
+  R.ctl = ctx->res_ctl;
+  R.ns = nsteps;
+  R.nbr = ctx->nbr;
+  R.n_inlet = ctx->n_inlet;
+  R.law = ctx->nlaw;
+  R.net = ctx->lux;
+  R.net_w = ctx->lux_w;
+  R.ks = ctx->nlaw.kind == hg::NLAW_H_UMAG_KS              ? ctx->nlaw_ks
+         : ctx->lux.choice == hg::LUX_MANNING_H_UMAG_KS ? ctx->lux_ks
+                                                        : nullptr;
+  return R;
 }
 
-size_t adj_run_lds_bytes(int MD) {
-  return size_t((kAdjRows + 4 * MD) * kResT + 512 + kTileInlets) * sizeof(double) + (kResT + 1) * sizeof(int32_t);
+// The exchange ring for `words` values per cell and slot, behind it the
+// tiles' error sums.
+int ensure_res_ring(hg_ctx* ctx, int words) {
+  const size_t need = size_t(4) * words * ctx->N + 4 * hg::kResRed;
+  int rc = 0;
+  if (need > ctx->res_ring_n) {
+    rc = dfree(ctx, ctx->res_ring);
+    ctx->res_ring_n = 0;
+    if (!rc) rc = dalloc(ctx, &ctx->res_ring, need);
+    if (!rc) ctx->res_ring_n = need;
+  }
+  if (!rc && !ctx->res_ctl) rc = dalloc(ctx, &ctx->res_ctl, 1);
+  return rc;
 }
 
-template <int MD>
-int adj_run_capacity(hg_ctx* ctx) {
-  constexpr int waves = res_items(MD) / 64;
-  int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_adj_run<MD>, 64 * waves, adj_run_lds_bytes(MD)) !=
-      hipSuccess)
-    return 0;
-  return std::min(per_cu, 2 / ((waves + 3) / 4)) * ctx->ncu;  // see res_capacity
-}
-
-// Whether nsteps steps may run resident: one field, the default tiling of
-// small meshes, at most one item per work-item and 64 inlets per tile, a
-// roughness that does not change with the state, and steps enough to pay for
-// the ring's initialisation.
-bool res_usable(hg_ctx* ctx, int64_t nsteps) {
-  return ctx->tiled && !ctx->res_off && ctx->K == 1 && nsteps >= 4 && ctx->tileT == kResT && ctx->tileMD <= 4 &&
-         ctx->max_items <= res_items(ctx->tileMD) && (ctx->n_inlet == 0 || ctx->fuse_inlet) && !ctx->ude_prec &&
-         ctx->nlaw.kind == hg::NLAW_OFF && ctx->lux.choice == hg::LUX_OFF && ctx->device < kMaxDevices;
-}
-
-// Takes this context's tiles out of the device's room (of `cap` work-groups),
-// or false when they do not fit beside the runs in flight.
+// Takes this context's tiles out of the device's room, or false when they do
+// not fit beside the runs in flight.  Runs of different kernels may share the
+// device, so each claims the share of it that its tiles are of its own
+// kernel's capacity `cap`.
 bool res_claim(hg_ctx* ctx, int cap) {
+  const int share = int((int64_t(ctx->ntiles) * kResRoom + cap - 1) / cap);
   std::lock_guard<std::mutex> g(g_res_mu);
-  if (g_res_groups[ctx->device] + ctx->ntiles > cap) return false;
-  g_res_groups[ctx->device] += ctx->ntiles;
+  if (g_res_room[ctx->device] + share > kResRoom) return false;
+  g_res_room[ctx->device] += share;
+  ctx->res_share = share;
   return true;
 }
 
-// After the launch of a resident run: waits for it and gives its room back;
+// After the launch of a resident run (e: its status): waits for it and gives its room back;
 // *done: every tile finished.
-int res_finish(hg_ctx* ctx, bool* done) {
+int res_finish(hg_ctx* ctx, hipError_t e, bool* done) {
   int32_t ran_out = 0;
-  hipError_t e = hipGetLastError();
   if (e == hipSuccess)
     e = hipMemcpyAsync(&ran_out, ctx->res_ctl, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   {
     std::lock_guard<std::mutex> g(g_res_mu);
-    g_res_groups[ctx->device] -= ctx->ntiles;
+    g_res_room[ctx->device] -= ctx->res_share;
   }
   HG_TRY(e);
   if (ran_out)  // the device was shared with something else: one launch per step from here on
@@ -3224,38 +2304,30 @@ int res_finish(hg_ctx* ctx, bool* done) {
   return HG_OK;
 }
 
-// nsteps steps from state arrays `in` to `out` (not the same), optionally
-// recorded.  *done: false when the run was not started or a wait ran out
+// nsteps steps of variant k from state arrays `in` to `out` (not the same),
+// optionally recorded, or with tangents (T: their buffers and those of the
+// parameters).  *done: false when the run was not started or a wait ran out
 // (nothing the caller reads has been written then).  Synchronizes.
-int res_run(hg_ctx* ctx, const double* const in[3], double* const out[3], double dt, int64_t nsteps, double* rec,
-            uint8_t* rec_clamp, double* rec_totalA, bool* done) {
+int res_run(hg_ctx* ctx, const hg::ResKind& k, const double* const in[3], double* const out[3], double dt,
+            int64_t nsteps, double* rec, uint8_t* rec_clamp, double* rec_totalA, const hg::ResArgs* T, bool* done) {
   *done = false;
-  const bool tri = ctx->tileMD == 3;
-  if (!ctx->res_cap) {
-    ctx->res_cap = tri ? res_capacity<3, true>(ctx) : res_capacity<4, true>(ctx);
-    ctx->res_split = ctx->ntiles <= ctx->res_cap;
-    if (!ctx->res_split) ctx->res_cap = tri ? res_capacity<3, false>(ctx) : res_capacity<4, false>(ctx);
-    if (ctx->res_cap < ctx->ntiles) {
-      ctx->res_off = true;
-      return HG_OK;
-    }
+  const int words = k.dual ? 6 : 3;
+  int rc = ensure_res_ring(ctx, words);
+  if (rc) return rc;
+  if (!res_claim(ctx, ctx->res_cap[k.split][k.nmode][k.dual])) return HG_OK;
+  hg::ResArgs R = res_args(ctx, nsteps);
+  R.rec = rec;
+  R.rec_clamp = rec_clamp;
+  R.rec_totalA = rec_totalA;
+  if (T) {
+    R.dxi = T->dxi; R.dqx = T->dqx; R.dqy = T->dqy;
+    R.dxo = T->dxo; R.dqxo = T->dqxo; R.dqyo = T->dqyo;
+    R.dn = T->dn; R.dzb = T->dzb; R.dS0x = T->dS0x; R.dS0y = T->dS0y;
+    R.dg_zb = T->dg_zb; R.dinletQ = T->dinletQ; R.net_dw = T->net_dw;
   }
-  if (!ctx->res_ring) {
-    int rc = dalloc(ctx, &ctx->res_ring, size_t(12) * ctx->N);
-    if (!rc) rc = dalloc(ctx, &ctx->res_ctl, 1);
-    if (rc) return rc;
-  }
-  if (!res_claim(ctx, ctx->res_cap)) return HG_OK;
-  const int64_t nring = int64_t(12) * ctx->N;
-  hipLaunchKernelGGL(k_res_init, dim3(grid_of(nring)), dim3(kBlock), 0, ctx->stream, nring, ctx->res_ring,
-                     ctx->res_ctl);
-  hg::TileArgs a = make_tile_args_p(ctx, in, out, dt);
-  ResArgs R{ctx->res_ring, ctx->res_ctl, nsteps, ctx->nbr, rec, rec_clamp, rec_totalA, ctx->n_inlet};
-  if (tri)
-    ctx->res_split ? launch_run<3, true>(ctx, a, R) : launch_run<3, false>(ctx, a, R);
-  else
-    ctx->res_split ? launch_run<4, true>(ctx, a, R) : launch_run<4, false>(ctx, a, R);
-  return res_finish(ctx, done);
+  hipError_t e = hg::res_init(ctx->stream, int64_t(4) * words * ctx->N, ctx->res_ring, ctx->res_ctl);
+  if (e == hipSuccess) e = hg::launch_run(ctx->stream, k, ctx->ntiles, make_tile_args_p(ctx, in, out, dt), R);
+  return res_finish(ctx, e, done);
 }
 
 // ---- adjoint host side
@@ -3639,12 +2711,13 @@ int forward_checkpointed(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck) {
   }
   const int64_t ns = nsteps - (nseg - 1) * kck;
   bool done = false;
-  if (res_usable(ctx, ns) && ns <= kResSteps) {
+  hg::ResKind k;
+  if (ns <= kResSteps && res_kind(ctx, ns, false, k)) {
     const double* in[3] = {ctx->st[ctx->cur][0], ctx->st[ctx->cur][1], ctx->st[ctx->cur][2]};
     for (int c = 0; c < 3; ++c)
       HG_TRY(hipMemcpyAsync(seg_state(ctx, 0, c, 0), in[c], N * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-    int rc = res_run(ctx, in, ctx->st[1 - ctx->cur], dt, ns, ctx->adj_seg[0], ctx->adj_mask[0], seg_totalA(ctx, 0, 0),
-                     &done);
+    int rc = res_run(ctx, k, in, ctx->st[1 - ctx->cur], dt, ns, ctx->adj_seg[0], ctx->adj_mask[0],
+                     seg_totalA(ctx, 0, 0), nullptr, &done);
     if (rc) return rc;
     if (done) {
       ctx->cur = 1 - ctx->cur;
@@ -3694,9 +2767,11 @@ int recompute_segment(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck, int64
 // the sums are taken over only then).
 int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done) {
   *done = false;
-  if (!res_usable(ctx, ns) || ns > kResSteps || !ctx->inlets_disjoint || ctx->adj_T != kResT) return HG_OK;
-  const bool tri = ctx->tileMD == 3;
-  if (!ctx->adj_res_cap) ctx->adj_res_cap = std::max(1, tri ? adj_run_capacity<3>(ctx) : adj_run_capacity<4>(ctx));
+  hg::ResKind k;
+  if (!res_kind(ctx, ns, false, k) || k.nmode != hg::RES_N_FIELD || ns > kResSteps || !ctx->inlets_disjoint ||
+      ctx->adj_T != kResT)
+    return HG_OK;
+  if (ctx->adj_res_cap < 0) ctx->adj_res_cap = hg::adj_run_capacity(ctx->tileMD, ctx->ncu);
   if (ctx->adj_res_cap < ctx->ntiles) return HG_OK;
   const int64_t N = ctx->N, G = std::max<int64_t>(ctx->G, 1), nring = 12 * N + 4 * G;
   if (!ctx->adj_ring) {
@@ -3706,8 +2781,6 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
     if (rc) return rc;
   }
   if (!res_claim(ctx, ctx->adj_res_cap)) return HG_OK;
-  hipLaunchKernelGGL(k_res_init, dim3(grid_of(nring)), dim3(kBlock), 0, ctx->stream, nring, ctx->adj_ring,
-                     ctx->res_ctl);
   const double* q[3] = {seg_state(ctx, 0, 0, b), seg_state(ctx, 0, 1, b), seg_state(ctx, 0, 2, b)};
   double *L = ctx->adj_lam[lam0], *O = ctx->adj_lam[1 - lam0], *sums = ctx->adj_sums;
   const double* lam[3] = {L, L + N, L + 2 * N};
@@ -3716,7 +2789,7 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
   a.nbar = ctx->adj_want_n ? ctx->adj_nbar : nullptr;
   if (ctx->deg_full) a.deg = nullptr;
   a.items = ctx->adj_items;
-  AdjRunArgs R{};
+  hg::AdjRunArgs R{};
   R.ring = ctx->adj_ring;
   R.vring = ctx->adj_ring + 12 * N;
   R.ctl = ctx->res_ctl;
@@ -3735,11 +2808,9 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
   R.o_zbbar = ctx->adj_want_zb ? sums + N : nullptr;
   R.o_S0bar = sums + 2 * N;
   R.o_Qbar = sums + 4 * N;
-  if (tri)
-    hipLaunchKernelGGL(k_adj_run<3>, dim3(ctx->ntiles), dim3(res_items(3)), adj_run_lds_bytes(3), ctx->stream, a, R);
-  else
-    hipLaunchKernelGGL(k_adj_run<4>, dim3(ctx->ntiles), dim3(res_items(4)), adj_run_lds_bytes(4), ctx->stream, a, R);
-  int rc = res_finish(ctx, done);
+  hipError_t e = hg::res_init(ctx->stream, nring, ctx->adj_ring, ctx->res_ctl);
+  if (e == hipSuccess) e = hg::launch_adj_run(ctx->stream, ctx->tileMD, ctx->ntiles, a, R);
+  int rc = res_finish(ctx, e, done);
   if (rc || !*done) return rc;
   auto take = [&](double* dst, const double* src, int64_t n) {
     return n > 0 ? hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream) : hipSuccess;
@@ -4248,11 +3319,11 @@ int ensure_graph(hg_ctx* ctx, double dt) {
 
 // Advance the device state nsteps (no host sync at the end).
 int advance_async(hg_ctx* ctx, double dt, int64_t nsteps) {
-  while (res_usable(ctx, nsteps)) {  // a small mesh: runs of steps in one launch each
+  for (hg::ResKind k; res_kind(ctx, nsteps, false, k);) {  // a small mesh: runs of steps in one launch each
     const int64_t ns = std::min<int64_t>(nsteps, kResSteps);
     const double* in[3] = {ctx->st[ctx->cur][0], ctx->st[ctx->cur][1], ctx->st[ctx->cur][2]};
     bool done = false;
-    int rc = res_run(ctx, in, ctx->st[1 - ctx->cur], dt, ns, nullptr, nullptr, nullptr, &done);
+    int rc = res_run(ctx, k, in, ctx->st[1 - ctx->cur], dt, ns, nullptr, nullptr, nullptr, nullptr, &done);
     if (rc) return rc;
     if (!done) break;
     ctx->cur = 1 - ctx->cur;
@@ -5588,9 +4659,31 @@ int hg_jvp(hg_ctx* ctx, const double* Q0, const double* dQ0, const double* param
   int cur = 0;
   double* Tb[2] = {T0, T1};
   const bool law = ctx->nlaw.kind != hg::NLAW_OFF;
+  int64_t t0 = 0;
+  // a small mesh: runs of steps in one launch each
+  for (hg::ResKind k; !(lux_fr && pn) && res_kind(ctx, nsteps - t0, true, k);) {
+    const int64_t ns = std::min<int64_t>(nsteps - t0, kResSteps);
+    const double* in[3] = {ctx->st[cur][0], ctx->st[cur][1], ctx->st[cur][2]};
+    hg::ResArgs D{};
+    D.dxi = Tb[cur]; D.dqx = Tb[cur] + N; D.dqy = Tb[cur] + 2 * N;
+    D.dxo = Tb[1 - cur]; D.dqxo = Tb[1 - cur] + N; D.dqyo = Tb[1 - cur] + 2 * N;
+    D.dn = pn;
+    D.dzb = pzb;
+    D.dS0x = pzb ? dS0x : nullptr;
+    D.dS0y = pzb ? dS0y : nullptr;
+    D.dg_zb = pzb ? dgzb : nullptr;
+    D.dinletQ = pQ;
+    D.net_dw = pw;
+    bool done = false;
+    rc = res_run(ctx, k, in, ctx->st[1 - cur], dt, ns, nullptr, nullptr, nullptr, &D, &done);
+    if (rc) return rc;
+    if (!done) break;
+    cur = 1 - cur;
+    t0 += ns;
+  }
   if (law || (lux && !lux_fr)) pn = dn;  // the law's or network's tangent of n, rewritten every step
   double* dfm = lux_fr ? dn : nullptr;     // the network's tangent of the friction magnitude
-  for (int64_t t = 0; t < nsteps; ++t) {
+  for (int64_t t = t0; t < nsteps; ++t) {
     const double* in[3] = {ctx->st[cur][0], ctx->st[cur][1], ctx->st[cur][2]};
     double* out[3] = {ctx->st[1 - cur][0], ctx->st[1 - cur][1], ctx->st[1 - cur][2]};
     if (law) {
@@ -5641,6 +4734,80 @@ int hg_jvp(hg_ctx* ctx, const double* Q0, const double* dQ0, const double* param
   if (!rc) rc = check_flags(ctx);
   return rc;
 }
+
+}  // extern "C"
+
+// hg_tsit5_solve on a small mesh: from the state in slot 0, all trial steps on
+// the device (at most kResTrials per launch), frames in one transfer.  *done:
+// false when it was not started or a wait ran out.
+static int tsit5_resident(hg_ctx* ctx, double t0, double t1, int64_t n_save, double abstol, double reltol, double dt0,
+                          double* Qsave, int64_t* stats, bool* done) {
+  *done = false;
+  hg::ResKind k;
+  const int64_t N = ctx->N, n3 = 3 * N;
+  const size_t frames = size_t(n_save + 1) * n3;
+  if (!res_kind(ctx, 4, false, k) || n_save >= (int64_t(1) << 30) || frames > (size_t(1) << 27)) return HG_OK;
+  int32_t& cap = ctx->tsit5_cap[k.nmode];
+  if (cap < 0) cap = hg::tsit5_capacity(k.md, k.nmode, ctx->ncu);
+  if (ctx->ntiles > cap) return HG_OK;
+  int rc = ensure_res_ring(ctx, 3);
+  if (!rc && !ctx->rk_state) rc = dalloc(ctx, &ctx->rk_state, 2);
+  if (!rc && frames > ctx->rk_frames_n) {
+    rc = dfree(ctx, ctx->rk_frames);
+    ctx->rk_frames_n = 0;
+    if (!rc) rc = dalloc(ctx, &ctx->rk_frames, frames);
+    if (!rc) ctx->rk_frames_n = frames;
+  }
+  if (rc) return rc;
+  if (!rc) rc = clear_flags(ctx);
+  hg::Tsit5Args P{};
+  P.t0 = t0;
+  P.t1 = t1;
+  P.abstol = abstol;
+  P.reltol = reltol;
+  P.n_save = n_save;
+  P.trials = hg::kResTrials;
+  P.max_steps = 100000000;
+  P.dt0 = dt0;
+  P.k0 = ctx->rk;
+  P.y = ctx->rk + 7 * n3;
+  P.red = ctx->res_ring + 12 * N;
+  P.frames = ctx->rk_frames;
+  P.perm = ctx->d_perm;
+  hg::Tsit5State st{};
+  for (int launch = 0; !st.done && st.code == HG_OK; ++launch) {
+    const double* in[3] = {launch ? P.y : ctx->st[0][0], launch ? P.y + N : ctx->st[0][1],
+                           launch ? P.y + 2 * N : ctx->st[0][2]};
+    P.in = launch ? ctx->rk_state + ((launch - 1) & 1) : nullptr;
+    P.out = ctx->rk_state + (launch & 1);
+    if (!res_claim(ctx, cap)) return HG_OK;
+    hipError_t e = hg::res_init(ctx->stream, 12 * N + 4 * hg::kResRed, ctx->res_ring, ctx->res_ctl);
+    if (e == hipSuccess)
+      e = hg::launch_tsit5(ctx->stream, k.md, k.nmode, ctx->ntiles, make_tile_args_p(ctx, in, ctx->st[1], 0.0),
+                           res_args(ctx, 0), P);
+    if (e == hipSuccess) e = hipMemcpyAsync(&st, P.out, sizeof(st), hipMemcpyDeviceToHost, ctx->stream);
+    bool ran = false;
+    rc = res_finish(ctx, e, &ran);
+    if (rc || !ran) return rc;
+  }
+  *done = true;
+  rc = device_to_host(ctx, Qsave, ctx->rk_frames, size_t(st.frame) * n3);  // the frames that were reached
+  if (rc) return rc;
+  if (st.code == HG_ERR_NONFINITE)
+    ctx->err = "hg_tsit5_solve: non-finite error estimate";
+  else if (st.code != HG_OK)
+    ctx->err = st.sub == 1 ? "hg_tsit5_solve: step size underflow" : "hg_tsit5_solve: too many steps";
+  if (st.code != HG_OK) return st.code;
+  rc = check_flags(ctx);
+  if (stats) {
+    stats[0] = st.accepted;
+    stats[1] = st.rejected;
+    stats[2] = st.nrhs;
+  }
+  return rc;
+}
+
+extern "C" {
 
 int hg_tsit5_tableau(double* c, double* a, double* btilde) {
   for (int i = 0; i < 7; ++i) {
@@ -5703,6 +4870,11 @@ int hg_tsit5_solve(hg_ctx* ctx, const double* Q0, const double* params, int64_t 
     return state_out(ctx, src, Qsave + idx * n3);
   };
   rc = state_in(ctx, Q0, 0);
+  {
+    bool done = false;
+    if (!rc) rc = tsit5_resident(ctx, t0, t1, n_save, abstol, reltol, dt0, Qsave, stats, &done);
+    if (rc || done) return rc;
+  }
   for (int c3 = 0; c3 < 3 && !rc; ++c3)
     if (hipMemcpyAsync(y + c3 * N, ctx->st[0][c3], N * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream) !=
         hipSuccess)

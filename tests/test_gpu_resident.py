@@ -209,3 +209,126 @@ def test_reverse_run_with_own_time_steps():
         out.append(ctx.adjoint(c.Q0, c.dt, 12, 0, np.linspace(-1, 1, 3 * c.N)))
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+# ---- forward mode, laws and networks, and Tsit5 ----
+LAWS = {"field": None, "sigmoid": dict(kind="sigmoid", n_lower=0.02, n_upper=0.06, k=2.0, h_mid=1.5),
+        "power_law": dict(kind="power_law", n_lower=0.02, n_upper=0.05, k=0.4),
+        "h_Umag_ks": dict(kind="h_Umag_ks"), "ManningN_h": 1, "ManningN_h_Umag_ks": 3, "FlowResistance": 2}
+
+
+def moving(c):
+    """The case with water moving everywhere (the h_Umag_ks law has no value at rest)."""
+    Q = c.Q0.copy()
+    Q[c.N:] = 0.1 * np.random.default_rng(8).uniform(0.5, 1.5, 2 * c.N)
+    return c.copy_fields(Q0=Q)
+
+
+def with_law(ctx, c, law, seed=4):
+    """Turns the named law or network on; returns the network's weights (None for a law)."""
+    rng = np.random.default_rng(seed)
+    ks = rng.uniform(0.02, 0.1, c.N)
+    spec = LAWS[law]
+    if spec is None:
+        return None
+    if isinstance(spec, dict):
+        ctx.set_n_law(**spec, ks=ks if law == "h_Umag_ks" else None)
+        return None
+    bounds = (1e-3, 1e-2) if law == "FlowResistance" else (0.02, 0.06)
+    net = capi.lux_net(law, [3, 4], ["tanh", "softplus"], bounds, (0.1, 4.0), (0.0, 2.0), (0.0, 0.2))
+    w = 0.5 * rng.normal(size=capi.lux_n_params(net))
+    ctx.set_lux_ude(net, w, ks=ks if law == "ManningN_h_Umag_ks" else None)
+    return w
+
+
+@pytest.mark.parametrize("law", sorted(LAWS))
+@pytest.mark.parametrize("name", ["tiny_channel", "channel", "mixed", "two_inlets", "quads"])
+def test_state_dependent_roughness(name, law):
+    c = moving(REVERSE[name]())
+    ctx, single = capi.Context(c), capi.Context(c)
+    single.set_tile_config(256)
+    for k in (ctx, single):
+        with_law(k, c, law)
+    for steps in (4, 21):
+        assert np.array_equal(ctx.step(c.Q0, c.dt, steps), single.step(c.Q0, c.dt, steps))
+
+
+@pytest.mark.parametrize("law", ["field", "sigmoid", "h_Umag_ks", "ManningN_h", "FlowResistance"])
+@pytest.mark.parametrize("name", sorted(REVERSE))
+def test_forward_mode(name, law):
+    """Value: the step's bits.  Tangent: the per-cell dual kernel's, which sums a cell's faces in the same order and
+    forms them with the same operations; the compiler may pick the two sides' sums differently, so a few ulp of the
+    largest tangent per step: 24 steps x 100 operations x 2^-53 is 3e-13."""
+    c = moving(REVERSE[name]()) if name != "wet_dry" else REVERSE[name]()
+    if name == "wet_dry" and law == "h_Umag_ks":
+        pytest.skip("the law has no value at rest")
+    kinds = [capi.HG_PARAM_NONE, capi.HG_PARAM_ZB]
+    if law == "field":
+        kinds += [capi.HG_PARAM_N_CELL] + ([capi.HG_PARAM_Q] if c.mesh.n_inlet else [])
+    if law in ("ManningN_h", "FlowResistance"):
+        kinds += [capi.HG_PARAM_UDE]
+    rng = np.random.default_rng(11)
+    d0 = 1e-2 * rng.normal(size=3 * c.N)
+    for kind in kinds:
+        out = []
+        for size in (0, 256):
+            ctx = capi.Context(c)
+            if size:
+                ctx.set_tile_config(size)
+            w = with_law(ctx, c, law)
+            ctx.set_active_param(kind)
+            p = {capi.HG_PARAM_NONE: None, capi.HG_PARAM_ZB: c.zb, capi.HG_PARAM_N_CELL: c.n,
+                 capi.HG_PARAM_Q: c.inletQ, capi.HG_PARAM_UDE: w}[kind]
+            dp = None if p is None else np.random.default_rng(12).normal(size=np.size(p)) * 1e-3
+            out.append(ctx.jvp(c.Q0, c.dt, 24, dQ0=d0, params=p, dparams=dp))
+            assert np.array_equal(out[-1][0], ctx.step(c.Q0, c.dt, 24, params=p))
+        (Q, dQ), (R, dR) = out
+        assert np.array_equal(Q, R)
+        assert np.all(np.isfinite(dR)) and np.max(np.abs(dQ - dR)) <= 3e-13 * np.max(np.abs(dR)), kind
+
+
+@pytest.mark.parametrize("law", ["field", "sigmoid", "ManningN_h"])
+@pytest.mark.parametrize("name", ["one_tile", "tile_and_one", "quads", "channel", "mixed", "two_inlets"])
+def test_tsit5(name, law):
+    """The error norm's sum over the cells is grouped by tiles, so the step sizes differ by a few ulp from those of
+    single launches; how far that carries depends on the flow, so the bound is measured: ten times what a change of
+    the first step by two ulp does to the single-launch run itself (or 1e-13).  Over a short run most steps are set
+    by the frames, not the error: 1e-13.  (FlowResistance friction is stiff at rest: its step sizes sit at the
+    stability limit and no run of it is stable under such a change; its RHS is the Euler runs' above.)"""
+    c = REVERSE[name]()
+    T = 60 * cases.cfl_dt(c, 0.4)
+
+    def run(size, T, first):
+        ctx = capi.Context(c)
+        if size:
+            ctx.set_tile_config(size)
+        with_law(ctx, c, law)
+        return ctx.tsit5(c.Q0, 0.0, T, 7, dt0=0.01 * T * first, reltol=1e-4)
+
+    short = 0.2 * T
+    (F, n), (G, m) = run(0, short, 1.0), run(256, short, 1.0)
+    assert n == m and n[0] >= 7
+    assert np.array_equal(F[0], c.Q0)
+    assert np.max(np.abs(F - G)) <= 1e-13 * np.max(np.abs(G))
+    (F, n), (G, m), (H, k) = run(0, T, 1.0), run(256, T, 1.0), run(256, T, 1.0 + 2.0 ** -51)
+    assert n == m or m != k
+    for f, g, h in zip(F, G, H):
+        assert np.max(np.abs(f - g)) <= max(1e-13 * np.max(np.abs(G)), 10 * np.max(np.abs(h - g)))
+
+
+def test_tsit5_many_steps():
+    """More trial steps than one launch takes, and the errors of the single-launch path."""
+    c = cases.dam_break(nx=40, ny=5)
+    a, b = capi.Context(c), capi.Context(c)
+    b.set_tile_config(256)
+    T = 120.0
+    (F, n), (G, m) = [x.tsit5(c.Q0, 0.0, T, 3, abstol=1e-13, reltol=1e-12, dt0=1e-3) for x in (a, b)]
+    assert n[0] + n[1] > 1024 and m[0] + m[1] > 1024
+    assert np.max(np.abs(F - G)) <= 1e-9 * np.max(np.abs(G))  # both are within 1e-11 of the solution
+    Q = c.Q0.copy()
+    Q[3] = np.nan
+    for ctx in (a, b):
+        with pytest.raises(capi.HGError) as e:
+            ctx.tsit5(Q, 0.0, 1.0, 2)
+        assert e.value.code == capi.HG_ERR_NONFINITE
+        assert np.array_equal(ctx.tsit5(c.Q0, 0.0, 1.0, 2)[0][0], c.Q0)
