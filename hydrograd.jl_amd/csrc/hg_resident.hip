@@ -619,7 +619,11 @@ __global__ __launch_bounds__(res_threads(MD, true), 2) void k_tsit5_run(TileArgs
 // here on 1,000 quads, 6.0 on a 1,300-cell channel (its inlet tiles exchange
 // twice per step) and 6.4 on 59k triangles.  Up to 512 tiles: the registers
 // that hold the cells allow two tiles per CU.
-template <int MD>
+constexpr int adj_run_base_doubles(int MD) {  // without the network's values
+  return (kAdjRows + 4 * MD) * kResT + 512 + kTileInlets + (kResT + 2) / 2;
+}
+
+template <int MD, int NM>
 __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunArgs R) {
   constexpr int T = kResT, NT = res_items(MD);
   extern __shared__ double lds[];
@@ -634,6 +638,14 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
   const bool own = tid < T && i < a.N;
   const int64_t N = a.N;
   const double hsmall = a.hsmall;
+  // the network: per weight and cell, its derivative at the step and the run's sum
+  const int NP = NM == RES_N_NET ? R.net.P : 0;
+  double* J = lds + adj_run_base_doubles(MD) + tid;
+  double* Wsum = J + NP * T;
+  const bool mag = NM == RES_N_NET && R.net.choice == LUX_FLOW_RESISTANCE;  // the output is the friction magnitude
+  if (own)
+    for (int p = 0; p < NP; ++p) Wsum[p * T] = 0.0;
+  const double ksc = NM && R.ks && own ? R.ks[i] : 1.0;
   double hs = 0.0, zb = 0.0, n = 0.0, S0x = 0.0, S0y = 0.0, A = 1.0, dti = a.dt;
   double l0 = 0.0, l1 = 0.0, l2 = 0.0, nbar = 0.0, zbbar = 0.0, S0bx = 0.0, S0by = 0.0;
   int d = 0;
@@ -678,7 +690,7 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
   }
   if (tid == 0) *stop = 0;
   // the recorded state of the step (own cell, and a cross-tile neighbour's), read one step ahead
-  double px = 0.0, pqx = 0.0, pqy = 0.0, jx = 0.0, jqx = 0.0, jqy = 0.0;
+  double px = 0.0, pqx = 0.0, pqy = 0.0, jx = 0.0, jqx = 0.0, jqy = 0.0, pn = 0.0;
   uint8_t pm = 0, jm = 0;
   auto read_ahead = [&](int64_t k) {
     const double* q = R.rec + k * 3 * N;
@@ -686,6 +698,7 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
     if (own) {
       px = q[i]; pqx = q[N + i]; pqy = q[2 * N + i];
       pm = m[i];
+      if (NM) pn = R.rec_n[k * N + i];
     }
     if (type == 1) {
       jx = q[rec.ref]; jqx = q[N + rec.ref]; jqy = q[2 * N + rec.ref];
@@ -701,6 +714,15 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
     a.vbar = reinterpret_cast<double*>(R.vring + (r & 3) * R.G);
     CellQ me{};
     double y0 = 0.0, y1 = 0.0, y2 = 0.0;
+    const double sx1 = pqx, sx2 = pqy;  // the raw discharge of the step's state
+    double ncl = 0.0;  // the law's or network's value of this step
+    if (NM) {
+      ncl = pn;
+      if (!mag) {
+        n = pn;
+        a.n = R.rec_n + k * N;
+      }
+    }
     if (pm) l0 = l1 = l2 = 0.0;
     nr.xi = jx; nr.qx = jqx; nr.qy = jqy;
     nr.clamped = jm;
@@ -741,11 +763,50 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
     // the source term's cotangents, while the faces are waited for
     double sxi = 0.0, sh = 0.0, sqx = 0.0, sqy = 0.0, sn = 0.0, sS0x = 0.0, sS0y = 0.0;
     const bool wet = me.h > hsmall;
-    if (own && wet)
-      source_vjp(a.g, a.kn2, hsmall, me.xi, me.h, me.hu, me.hv, n, S0x, S0y, y1, y2, sxi, sh, sqx, sqy, sn, sS0x,
-                     sS0y);
+    if (own && wet) {
+      if (NM == RES_N_NET && mag)
+        source_vjp_mag(a.g, me.xi, me.hu, me.hv, ncl, S0x, S0y, y1, y2, sxi, sqx, sqy, sn, sS0x, sS0y);
+      else
+        source_vjp(a.g, a.kn2, hsmall, me.xi, me.h, me.hu, me.hv, n, S0x, S0y, y1, y2, sxi, sh, sqx, sqy, sn, sS0x,
+                   sS0y);
+    }
+    // the closure's derivatives by the cell's state, and by the weights
+    double cs[3] = {0.0, 0.0, 0.0};
+    if (NM && own) {
+      const double q[3] = {me.xi, sx1, sx2};
+      const int ns = NM == RES_N_LAW ? (R.law.kind == NLAW_H_UMAG_KS ? 3 : 1) : (R.net.choice == LUX_MANNING_H ? 1 : 3);
+      double df[3] = {0.0, 0.0, 0.0};
+      if (NM == RES_N_NET) {
+        double f[3];
+        lux_features<double>(R.net, q[0], q[1], q[2], hs, hsmall, ksc, f);
+        if (R.net.n_hidden == 1)
+          (void)lux_jacobian<4, 1>(R.net, R.net_w, f, J, T, df);
+        else
+          (void)lux_jacobian<4, 2>(R.net, R.net_w, f, J, T, df);
+      }
+      for (int c = 0; c < ns; ++c) {
+        const Dual1 x0(q[0], c == 0 ? 1.0 : 0.0), x1(q[1], c == 1 ? 1.0 : 0.0), x2(q[2], c == 2 ? 1.0 : 0.0);
+        double v;
+        if (NM == RES_N_LAW) {
+          Dual1 h, U;
+          nlaw_features<Dual1>(R.law, x0, x1, x2, hs, hsmall, h, U);
+          v = nlaw_eval<Dual1, false>(R.law, h, U, ksc, nullptr, nullptr, nullptr).d;
+        } else {
+          Dual1 fd[3];
+          lux_features<Dual1>(R.net, x0, x1, x2, hs, hsmall, ksc, fd);
+          v = df[0] * fd[0].d + df[1] * fd[1].d + df[2] * fd[2].d;
+        }
+        if (c == 0)
+          cs[0] = v;
+        else if (c == 1)
+          cs[1] = v;
+        else
+          cs[2] = v;
+      }
+    }
     __syncthreads();
     if (*stop) return;
+    double ob = 0.0;
     if (own) {
       double uxh = 0.0, uqx = 0.0, uqy = 0.0, nb = 0.0, zbb = 0.0;
       const int xm = Xm[tid];
@@ -761,7 +822,11 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
             nb += e;
         }
       }
-      nb += sn;
+      double mb = 0.0;
+      if (NM == RES_N_NET && mag)
+        mb = sn;
+      else
+        nb += sn;
       double ox = uxh + sxi, oqx = 0.0, oqy = 0.0;
       if (wet) {
         ox += sh;
@@ -771,7 +836,8 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
       l0 = ox + l0;
       l1 = oqx + l1;
       l2 = oqy + l2;
-      nbar = nbar + nb;
+      ob = mag ? mb : nb;  // this step's cotangent of the closure's output
+      if (!NM || mag) nbar = nbar + nb;
       zbbar = zbbar + zbb;
       S0bx = S0bx + sS0x;
       S0by = S0by + sS0y;
@@ -821,12 +887,18 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
           for (int f = my_f; f >= 0;) {
             const InletFaceRec fr = R.in_rec[f];
             l0 += Ab * fr.L53 / n;
-            nbar += Ab * (-fr.L53 * h0 / (n * n));
+            ob += (NM && !mag) ? Ab * (-fr.L53 * h0 / (n * n)) : 0.0;
+            if (!NM || mag) nbar += Ab * (-fr.L53 * h0 / (n * n));
             f = fr.next;
           }
         }
       }
       __syncthreads();  // sA / sQ reuse
+    }
+    if (NM && own && ob != 0.0) {
+      l0 += ob * cs[0];
+      l1 += ob * cs[1];
+      l2 += ob * cs[2];
     }
     if (own && pub && r + 1 < R.ns) {
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the last step's reset is done
@@ -836,6 +908,10 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
       res_put(o + N, __double_as_longlong(l1));
       res_put(o + 2 * N, __double_as_longlong(l2));
       for (int c = 0; c < 3; ++c) res_put(e + c * N, kResEmpty);
+    }
+    if (NM == RES_N_NET && own) {
+#pragma unroll 8
+      for (int p = 0; p < NP; ++p) Wsum[p * T] += ob * J[p * T];
     }
   }
   if (own) {
@@ -849,15 +925,23 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
       R.o_S0bar[N + i] = S0by;
     }
   }
+  if (NM == RES_N_NET) {  // the tile's sum of each weight's cotangent, by a fixed tree
+    __syncthreads();
+    const double* W0 = lds + adj_run_base_doubles(MD) + NP * T;
+    for (int p = tid / 64; p < NP; p += NT / 64) {
+      const int l = tid & 63;
+      double v = (t * T + l < a.N ? W0[p * T + l] : 0.0) + (t * T + 64 + l < a.N ? W0[p * T + 64 + l] : 0.0);
+      for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w, 64);
+      if (l == 0) R.o_wpart[int64_t(p) * gridDim.x + t] = v;
+    }
+  }
   for (int sl = in0 + tid; sl < in1; sl += NT) {  // by the tile of the inlet's first face
     const int b = R.tile_in_list[sl];
     if (R.in_rec[R.in_off[b]].cell / T == t) R.o_Qbar[b] = qa[sl - in0];
   }
 }
 
-size_t adj_run_lds_bytes(int MD) {
-  return size_t((kAdjRows + 4 * MD) * kResT + 512 + kTileInlets) * sizeof(double) + (kResT + 1) * sizeof(int32_t);
-}
+size_t adj_run_lds_bytes(int MD, int P) { return (size_t(adj_run_base_doubles(MD)) + 2 * size_t(P) * kResT) * sizeof(double); }
 
 // Tiles per CU: a tile's waves need not spread evenly over the four SIMDs (two
 // tiles of six waves each were not resident together where three waves fit
@@ -914,6 +998,22 @@ void with_tsit5(int md, int nm, F&& f) {
 #undef HG_TSIT5_MD
 }
 
+template <int MD, int NM>
+struct AdjVariant {
+  static int cap(int P, int ncu) {
+    return capacity(k_adj_run<MD, NM>, res_items(MD), adj_run_lds_bytes(MD, P), 2, ncu);
+  }
+  static void launch(hipStream_t st, int P, int ntiles, const AdjArgs& a, const AdjRunArgs& R) {
+    hipLaunchKernelGGL((k_adj_run<MD, NM>), dim3(ntiles), dim3(res_items(MD)), adj_run_lds_bytes(MD, P), st, a, R);
+  }
+};
+template <class F>
+void with_adj_run(int md, int nm, F&& f) {
+#define HG_ADJ_MD(NM) (md == 3 ? f(AdjVariant<3, NM>()) : f(AdjVariant<4, NM>()))
+  nm == 0 ? HG_ADJ_MD(0) : nm == 1 ? HG_ADJ_MD(1) : HG_ADJ_MD(2);
+#undef HG_ADJ_MD
+}
+
 }  // namespace
 
 int res_capacity(const ResKind& k, int ncu) {
@@ -922,9 +1022,10 @@ int res_capacity(const ResKind& k, int ncu) {
   return c;
 }
 
-int adj_run_capacity(int md, int ncu) {
-  return md == 3 ? capacity(k_adj_run<3>, res_items(3), adj_run_lds_bytes(3), 2, ncu)
-                 : capacity(k_adj_run<4>, res_items(4), adj_run_lds_bytes(4), 2, ncu);
+int adj_run_capacity(int md, int nmode, int net_P, int ncu) {
+  int c = 0;
+  with_adj_run(md, nmode, [&](auto v) { c = v.cap(nmode == RES_N_NET ? net_P : 0, ncu); });
+  return c;
 }
 
 int tsit5_capacity(int md, int nmode, int ncu) {
@@ -943,11 +1044,8 @@ hipError_t launch_run(hipStream_t stream, const ResKind& k, int ntiles, const Ti
   return hipGetLastError();
 }
 
-hipError_t launch_adj_run(hipStream_t stream, int md, int ntiles, const AdjArgs& a, const AdjRunArgs& R) {
-  if (md == 3)
-    hipLaunchKernelGGL(k_adj_run<3>, dim3(ntiles), dim3(res_items(3)), adj_run_lds_bytes(3), stream, a, R);
-  else
-    hipLaunchKernelGGL(k_adj_run<4>, dim3(ntiles), dim3(res_items(4)), adj_run_lds_bytes(4), stream, a, R);
+hipError_t launch_adj_run(hipStream_t stream, int md, int nmode, int ntiles, const AdjArgs& a, const AdjRunArgs& R) {
+  with_adj_run(md, nmode, [&](auto v) { v.launch(stream, nmode == RES_N_NET ? R.net.P : 0, ntiles, a, R); });
   return hipGetLastError();
 }
 

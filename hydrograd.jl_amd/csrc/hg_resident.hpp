@@ -82,6 +82,14 @@ struct AdjRunArgs {
   const InletFaceRec* in_rec;
   const double* Qbar;
   double *o_nbar, *o_zbbar, *o_S0bar, *o_Qbar;
+  // with a law or network: what the forward run recorded of it ([ns][N]), the
+  // closure (as in ResArgs), and the tiles' weight cotangents ([P][ntiles])
+  const double* rec_n;
+  NLaw law;
+  LuxNet net;
+  const double* ks;
+  const double* net_w;
+  double* o_wpart;
 };
 
 // The kernel variants.  split: the cells' work-items take no items (few tiles).
@@ -95,12 +103,14 @@ struct ResKind {
 // Tiles of such a run that the device surely holds at once (0: there is no
 // such variant).
 int res_capacity(const ResKind& k, int ncu);
-int adj_run_capacity(int md, int ncu);
+int adj_run_capacity(int md, int nmode, int net_P, int ncu);
+// Weights and hidden layers a resident reverse run can hold (2 LDS values per weight and cell).
+constexpr int kAdjRunMaxP = 56, kAdjRunMaxHidden = 2;
 int tsit5_capacity(int md, int nmode, int ncu);
 
 hipError_t res_init(hipStream_t stream, int64_t n, unsigned long long* ring, int32_t* ctl);
 hipError_t launch_run(hipStream_t stream, const ResKind& k, int ntiles, const TileArgs& a, const ResArgs& R);
-hipError_t launch_adj_run(hipStream_t stream, int md, int ntiles, const AdjArgs& a, const AdjRunArgs& R);
+hipError_t launch_adj_run(hipStream_t stream, int md, int nmode, int ntiles, const AdjArgs& a, const AdjRunArgs& R);
 hipError_t launch_tsit5(hipStream_t stream, int md, int nmode, int ntiles, const TileArgs& a, const ResArgs& R,
                         const Tsit5Args& P);
 

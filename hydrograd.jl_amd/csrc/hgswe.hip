@@ -2309,7 +2309,8 @@ int res_finish(hg_ctx* ctx, hipError_t e, bool* done) {
 // parameters).  *done: false when the run was not started or a wait ran out
 // (nothing the caller reads has been written then).  Synchronizes.
 int res_run(hg_ctx* ctx, const hg::ResKind& k, const double* const in[3], double* const out[3], double dt,
-            int64_t nsteps, double* rec, uint8_t* rec_clamp, double* rec_totalA, const hg::ResArgs* T, bool* done) {
+            int64_t nsteps, double* rec, uint8_t* rec_clamp, double* rec_totalA, double* rec_n, const hg::ResArgs* T,
+            bool* done) {
   *done = false;
   const int words = k.dual ? 6 : 3;
   int rc = ensure_res_ring(ctx, words);
@@ -2319,6 +2320,7 @@ int res_run(hg_ctx* ctx, const hg::ResKind& k, const double* const in[3], double
   R.rec = rec;
   R.rec_clamp = rec_clamp;
   R.rec_totalA = rec_totalA;
+  R.rec_n = rec_n;
   if (T) {
     R.dxi = T->dxi; R.dqx = T->dqx; R.dqy = T->dqy;
     R.dxo = T->dxo; R.dqxo = T->dqxo; R.dqyo = T->dqyo;
@@ -2335,6 +2337,7 @@ int advance_async(hg_ctx* ctx, double dt, int64_t nsteps);
 int advance_timed(hg_ctx* ctx, double dt, int64_t nsteps, double* kernel_ms);
 int drop_graph(hg_ctx* ctx);
 int ensure_adj_tiles(hg_ctx* ctx);
+bool adj_res_usable(hg_ctx* ctx, int64_t ns, hg::ResKind& k);
 
 // Launches the cached graph of `key` on `stream`, capturing it first from
 // enqueue() (which enqueues on ctx->stream, pointed at `stream` meanwhile;
@@ -2712,14 +2715,29 @@ int forward_checkpointed(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck) {
   const int64_t ns = nsteps - (nseg - 1) * kck;
   bool done = false;
   hg::ResKind k;
+  ctx->rec_resident = false;
   if (ns <= kResSteps && res_kind(ctx, ns, false, k)) {
+    hg::ResKind ka;
+    double* rec_n = nullptr;  // what a resident reversal reads of a law or network
+    if (nseg == 1 && k.nmode != hg::RES_N_FIELD && adj_res_usable(ctx, ns, ka)) {
+      if (size_t(ns) > ctx->adj_nseg_cap[0]) {
+        int rc = drop_graph(ctx);
+        if (!rc) rc = dfree(ctx, ctx->adj_nseg[0]);
+        ctx->adj_nseg_cap[0] = 0;
+        if (!rc) rc = dalloc(ctx, &ctx->adj_nseg[0], size_t(ns) * N);
+        if (rc) return rc;
+        ctx->adj_nseg_cap[0] = size_t(ns);
+      }
+      rec_n = ctx->adj_nseg[0];
+    }
     const double* in[3] = {ctx->st[ctx->cur][0], ctx->st[ctx->cur][1], ctx->st[ctx->cur][2]};
     for (int c = 0; c < 3; ++c)
       HG_TRY(hipMemcpyAsync(seg_state(ctx, 0, c, 0), in[c], N * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
     int rc = res_run(ctx, k, in, ctx->st[1 - ctx->cur], dt, ns, ctx->adj_seg[0], ctx->adj_mask[0],
-                     seg_totalA(ctx, 0, 0), nullptr, &done);
+                     seg_totalA(ctx, 0, 0), rec_n, nullptr, &done);
     if (rc) return rc;
     if (done) {
+      ctx->rec_resident = true;
       ctx->cur = 1 - ctx->cur;
       return HG_OK;
     }
@@ -2762,17 +2780,23 @@ int recompute_segment(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck, int64
   });
 }
 
+// Whether a recorded run of ns steps can be reversed resident.
+bool adj_res_usable(hg_ctx* ctx, int64_t ns, hg::ResKind& k) {
+  if (!res_kind(ctx, ns, false, k) || ns > kResSteps || !ctx->inlets_disjoint || ctx->adj_T != kResT) return false;
+  if (k.nmode == hg::RES_N_NET && (ctx->lux.P > hg::kAdjRunMaxP || ctx->lux.n_hidden > hg::kAdjRunMaxHidden))
+    return false;
+  int32_t& cap = ctx->adj_res_cap[k.nmode];  // asked again when a network is set
+  if (cap < 0) cap = hg::adj_run_capacity(ctx->tileMD, k.nmode, ctx->lux.P, ctx->ncu);
+  return ctx->ntiles <= cap;
+}
+
 // The ns steps recorded in segment buffer b reversed in one resident run, from
 // the cotangent in adj_lam[lam0] to adj_lam[1 - lam0] (*done as for res_run;
 // the sums are taken over only then).
 int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done) {
   *done = false;
   hg::ResKind k;
-  if (!res_kind(ctx, ns, false, k) || k.nmode != hg::RES_N_FIELD || ns > kResSteps || !ctx->inlets_disjoint ||
-      ctx->adj_T != kResT)
-    return HG_OK;
-  if (ctx->adj_res_cap < 0) ctx->adj_res_cap = hg::adj_run_capacity(ctx->tileMD, ctx->ncu);
-  if (ctx->adj_res_cap < ctx->ntiles) return HG_OK;
+  if (!ctx->rec_resident || !adj_res_usable(ctx, ns, k)) return HG_OK;
   const int64_t N = ctx->N, G = std::max<int64_t>(ctx->G, 1), nring = 12 * N + 4 * G;
   if (!ctx->adj_ring) {
     int rc = dalloc(ctx, &ctx->adj_ring, size_t(nring));
@@ -2780,13 +2804,19 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
     if (!rc && !ctx->res_ctl) rc = dalloc(ctx, &ctx->res_ctl, 1);
     if (rc) return rc;
   }
-  if (!res_claim(ctx, ctx->adj_res_cap)) return HG_OK;
+  const int P = k.nmode == hg::RES_N_NET ? ctx->lux.P : 0;
+  if (P && !ctx->adj_wpart) {
+    int rc = dalloc(ctx, &ctx->adj_wpart, size_t(hg::kAdjRunMaxP) * ctx->ntiles);
+    if (rc) return rc;
+  }
+  if (!res_claim(ctx, ctx->adj_res_cap[k.nmode])) return HG_OK;
   const double* q[3] = {seg_state(ctx, 0, 0, b), seg_state(ctx, 0, 1, b), seg_state(ctx, 0, 2, b)};
   double *L = ctx->adj_lam[lam0], *O = ctx->adj_lam[1 - lam0], *sums = ctx->adj_sums;
   const double* lam[3] = {L, L + N, L + 2 * N};
   double* out[3] = {O, O + N, O + 2 * N};
   hg::AdjArgs a = make_adj_args(ctx, q, lam, nullptr, out, dt);
-  a.nbar = ctx->adj_want_n ? ctx->adj_nbar : nullptr;
+  const bool sum_n = ctx->adj_want_n && (k.nmode == hg::RES_N_FIELD || ctx->lux.choice == hg::LUX_FLOW_RESISTANCE);
+  a.nbar = sum_n ? ctx->adj_nbar : nullptr;
   if (ctx->deg_full) a.deg = nullptr;
   a.items = ctx->adj_items;
   hg::AdjRunArgs R{};
@@ -2804,12 +2834,21 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
   R.in_off = ctx->in_off;
   R.in_rec = ctx->in_rec;
   R.Qbar = ctx->adj_Qbar;
-  R.o_nbar = ctx->adj_want_n ? sums : nullptr;
+  R.o_nbar = sum_n ? sums : nullptr;
   R.o_zbbar = ctx->adj_want_zb ? sums + N : nullptr;
   R.o_S0bar = sums + 2 * N;
   R.o_Qbar = sums + 4 * N;
+  if (k.nmode != hg::RES_N_FIELD) {
+    const hg::ResArgs A = res_args(ctx, ns);
+    R.rec_n = ctx->adj_nseg[b];
+    R.law = A.law;
+    R.net = A.net;
+    R.ks = A.ks;
+    R.net_w = A.net_w;
+    R.o_wpart = ctx->adj_wpart;
+  }
   hipError_t e = hg::res_init(ctx->stream, nring, ctx->adj_ring, ctx->res_ctl);
-  if (e == hipSuccess) e = hg::launch_adj_run(ctx->stream, ctx->tileMD, ctx->ntiles, a, R);
+  if (e == hipSuccess) e = hg::launch_adj_run(ctx->stream, ctx->tileMD, k.nmode, ctx->ntiles, a, R);
   int rc = res_finish(ctx, e, done);
   if (rc || !*done) return rc;
   auto take = [&](double* dst, const double* src, int64_t n) {
@@ -2821,6 +2860,11 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
     HG_TRY(take(ctx->adj_S0bar, R.o_S0bar, 2 * N));
   }
   HG_TRY(take(ctx->adj_Qbar, R.o_Qbar, ctx->n_inlet));
+  if (P) {
+    hipLaunchKernelGGL(k_ude_wsum, dim3(P), dim3(kBlock), 0, ctx->stream, ctx->ntiles, nullptr, ctx->adj_wpart,
+                       int64_t(ctx->ntiles), int64_t(1), ctx->lux_wbar);
+    HG_TRY(hipGetLastError());
+  }
   return HG_OK;
 }
 
@@ -3323,7 +3367,7 @@ int advance_async(hg_ctx* ctx, double dt, int64_t nsteps) {
     const int64_t ns = std::min<int64_t>(nsteps, kResSteps);
     const double* in[3] = {ctx->st[ctx->cur][0], ctx->st[ctx->cur][1], ctx->st[ctx->cur][2]};
     bool done = false;
-    int rc = res_run(ctx, k, in, ctx->st[1 - ctx->cur], dt, ns, nullptr, nullptr, nullptr, nullptr, &done);
+    int rc = res_run(ctx, k, in, ctx->st[1 - ctx->cur], dt, ns, nullptr, nullptr, nullptr, nullptr, nullptr, &done);
     if (rc) return rc;
     if (!done) break;
     ctx->cur = 1 - ctx->cur;
@@ -4499,6 +4543,7 @@ int hg_set_lux_ude(hg_ctx* ctx, const hg_lux_net* net, const double* params, con
   for (int l = 0; l < L.n_hidden; ++l) maxw = std::max(maxw, int(L.width[l]));
   ctx->lux_mw = maxw <= 4 ? 4 : hg::kLuxMaxW;
   ctx->lux = L;
+  ctx->adj_res_cap[hg::RES_N_NET] = -1;  // its LDS depends on the number of weights
   return HG_OK;
 }
 
@@ -4675,7 +4720,7 @@ int hg_jvp(hg_ctx* ctx, const double* Q0, const double* dQ0, const double* param
     D.dinletQ = pQ;
     D.net_dw = pw;
     bool done = false;
-    rc = res_run(ctx, k, in, ctx->st[1 - cur], dt, ns, nullptr, nullptr, nullptr, &D, &done);
+    rc = res_run(ctx, k, in, ctx->st[1 - cur], dt, ns, nullptr, nullptr, nullptr, nullptr, &D, &done);
     if (rc) return rc;
     if (!done) break;
     cur = 1 - cur;

@@ -332,3 +332,31 @@ def test_tsit5_many_steps():
             ctx.tsit5(Q, 0.0, 1.0, 2)
         assert e.value.code == capi.HG_ERR_NONFINITE
         assert np.array_equal(ctx.tsit5(c.Q0, 0.0, 1.0, 2)[0][0], c.Q0)
+
+
+@pytest.mark.parametrize("law", ["sigmoid", "power_law", "h_Umag_ks", "ManningN_h", "ManningN_h_Umag_ks",
+                                 "FlowResistance", "one_layer", "three_layers"])
+@pytest.mark.parametrize("name", ["tiny_channel", "channel", "mixed", "two_inlets", "quads", "batch"])
+def test_reverse_run_with_closure(name, law):
+    """Every cotangent, those of the network's weights among them, against single launches.  The closure's
+    derivatives are formed once per step and scaled, and the weight sums are grouped by tiles: 12 steps of about 1,000
+    operations give 12 x 1000 x 2^-53 = 1.3e-12 of the largest component, times ten for sums of both signs.  (A network
+    of three hidden layers is not held resident in reverse: its forward run is, and feeds the single launches.)"""
+    c = moving(REVERSE[name]())
+    lam = np.random.default_rng(1).normal(size=3 * c.N)
+    out = []
+    for size in (0, 256):
+        ctx = capi.Context(c)
+        if size:
+            ctx.set_tile_config(size)
+        net = law in ("one_layer", "three_layers")
+        if net:
+            hidden, acts = ([4], ["sigmoid"]) if law == "one_layer" else ([3, 2, 4], ["tanh", "leakyrelu", "softplus"])
+            n = capi.lux_net("ManningN_h", hidden, acts, (0.02, 0.06), (0.1, 4.0))
+            ctx.set_lux_ude(n, 0.5 * np.random.default_rng(2).normal(size=capi.lux_n_params(n)))
+        else:
+            net = with_law(ctx, c, law) is not None
+        out.append(list(ctx.adjoint(c.Q0, c.dt, 12, 0, lam)) + ([ctx.lux_grad()] if net else []))
+    for x, y in zip(*out):
+        assert np.all(np.isfinite(y))
+        assert np.max(np.abs(x - y), initial=0.0) <= 1.3e-11 * np.max(np.abs(y), initial=0.0)
