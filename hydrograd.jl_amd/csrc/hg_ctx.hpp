@@ -336,8 +336,11 @@ struct hg_ctx {
   hg::InletFaceRec* in_rec = nullptr;
   bool inlets_disjoint = true;  // no cell sits on two inlets: the inlet adjoint runs one work-group per inlet
   double *inletQ = nullptr, *inletQ0 = nullptr, *exitWSE = nullptr, *totalA = nullptr;
-  int32_t* flags = nullptr;  // device address of flags_host: [0] conveyance error, [1] non-finite state
+  int32_t* flags = nullptr;  // device address of flags_host: [0] conveyance error, [1] non-finite state, [2] a resident run's wait ran out
   volatile int32_t* flags_host = nullptr;  // pinned, coherent host memory: cleared and read by the host
+  char* pin = nullptr;   // pinned block of small transfers (pin_take), in the flags' allocation
+  size_t pin_n = 0, pin_used = 0;
+  bool base_dirty = true;  // the working copies of zb, n, S0, zb_ghost, inletQ may differ from the fields
   int32_t* zone = nullptr;
   // tiled kernel data
   bool tiled = false;
@@ -385,7 +388,8 @@ struct hg_ctx {
   // host <-> device transfers in caller order: a 3N staging buffer and the
   // permutation (library cell i is caller cell perm[i]) on the device
   double* stage = nullptr;
-  int32_t* d_perm = nullptr;
+  int32_t* d_perm = nullptr;  // library cell -> caller cell
+  int32_t* d_inv = nullptr;   // caller cell -> library cell
   // probe-loss buffers of hg_grad_probes (capacity probe_cap probes)
   int32_t* probe_i = nullptr;
   double* probe_d = nullptr;
@@ -469,7 +473,7 @@ struct hg_ctx {
 
   // events attached to timed step dispatches (hg_advance_timed), reused
   std::vector<hipEvent_t> ev_pool;
-  hipEvent_t ev_xfer[2] = {nullptr, nullptr};  // chunk events of the pinned host transfers
+  hipEvent_t ev_xfer[4] = {nullptr, nullptr, nullptr, nullptr};  // chunk events of the pinned host transfers
 
   // cached graph of kGraphSteps steps (buffer 0 -> ... -> buffer 0) per dt
   hipGraphExec_t gexec = nullptr;

@@ -387,7 +387,10 @@ struct ResTile {
     }
     const double rA = rcp_est(A);
     __syncthreads();
-    if (*stop) return false;  // the same for the whole tile: set before the barrier only
+    if (*stop) {  // the same for the whole tile: set before the barrier only
+      if (tid == 0) a.flag[2] = 1;
+      return false;
+    }
     if (!own) return true;
     T acc0(0.0), acc1(0.0), acc2(0.0);
     for (int k = 0; k < MD; ++k) {  // local face order
@@ -564,7 +567,10 @@ __global__ __launch_bounds__(res_threads(MD, true), 2) void k_tsit5_run(TileArgs
     if (tid < nt && !res_poll<1>(P.red + (q & 3) * kResRed + tid, 0, R.ctl, part)) *rt.stop = 1;
     if (tid < kResRed) red[tid] = part[0];
     __syncthreads();
-    if (*rt.stop) return;
+    if (*rt.stop) {
+      if (tid == 0) a.flag[2] = 1;
+      return;
+    }
     double ss = 0.0;
     for (int w = 0; w < kResRed; w += 64) ss += red[w + (tid & 63)];
     for (int w = 32; w > 0; w >>= 1) ss += __shfl_xor(ss, w, 64);
@@ -805,7 +811,10 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
       }
     }
     __syncthreads();
-    if (*stop) return;
+    if (*stop) {
+      if (tid == 0) R.flag[2] = 1;
+      return;
+    }
     double ob = 0.0;
     if (own) {
       double uxh = 0.0, uqx = 0.0, uqy = 0.0, nb = 0.0, zbb = 0.0;
@@ -862,7 +871,10 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
         sQ[tid] = pq;
       }
       __syncthreads();
-      if (*stop) return;
+      if (*stop) {
+        if (tid == 0) R.flag[2] = 1;
+        return;
+      }
       if (tid < 128) {
         sA[tid] += sA[tid + 128];
         sQ[tid] += sQ[tid + 128];

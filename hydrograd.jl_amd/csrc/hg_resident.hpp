@@ -71,6 +71,7 @@ struct AdjRunArgs {
   unsigned long long* ring;   // [4][3][N] cotangents
   unsigned long long* vring;  // [4][G] inlet ghost velocity cotangents
   int32_t* ctl;
+  int32_t* flag;              // the host's error flags
   int64_t ns, G;
   const double* rec;          // [ns][3][N] states
   const uint8_t* rec_clamp;   // [ns][N]

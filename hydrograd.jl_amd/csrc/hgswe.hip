@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -100,6 +101,11 @@ double* g_scratch_dev[kMaxDevices] = {};
 constexpr int kBlock = 256;
 constexpr int kRewarmSteps = 1024;  // graph-replayed steps the autotuner ends with (a multiple of kGraphSteps)
 constexpr int kGraphSteps = 16;  // steps per captured graph (even: the graph returns to buffer 0)
+// Largest state and cotangent together (bytes) that go through a context's
+// pinned block, by a host RHS both ways: 19,530 cells (0.9 MiB) 62 us through
+// the block and 79 through the process's chunks, 39,248 (1.8 MiB) 97 and 105,
+// 78,244 (3.6 MiB) 186 and 147.
+constexpr size_t kPinSmall = size_t(2) << 20;
 constexpr int kXCD = 8;         // MI355X: 8 accelerator complex dies, one L2 each
 
 template <class T>
@@ -135,11 +141,45 @@ int dfree(hg_ctx* ctx, T*& p) {
   return HG_OK;
 }
 
+// A piece of the context's pinned host block, or NULL when it is larger than
+// that.  Pieces are handed out one after the other; when the block is used up
+// the stream is synchronized first, after which every earlier piece has been
+// read or written.
+char* pin_take(hg_ctx* ctx, size_t bytes) {
+  bytes = (bytes + 63) & ~size_t(63);
+  if (!ctx->pin || bytes > ctx->pin_n) return nullptr;
+  if (ctx->pin_used + bytes > ctx->pin_n) {
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return nullptr;
+    ctx->pin_used = 0;
+  }
+  char* const p = ctx->pin + ctx->pin_used;
+  ctx->pin_used += bytes;
+  return p;
+}
+
+// Host array -> device array, in stream order; src may be reused on return.
 template <class T>
 int upload(hg_ctx* ctx, T* dst, const T* src, size_t n) {
   if (n == 0) return HG_OK;
+  if (char* p = pin_take(ctx, n * sizeof(T))) {
+    std::memcpy(p, src, n * sizeof(T));
+    HG_TRY(hipMemcpyAsync(dst, p, n * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
+    return HG_OK;
+  }
   HG_TRY(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
   HG_TRY(hipStreamSynchronize(ctx->stream));
+  return HG_OK;
+}
+
+// Device array -> host array; synchronous.
+template <class T>
+int download(hg_ctx* ctx, T* dst, const T* src, size_t n) {
+  if (n == 0) return HG_OK;
+  char* p = pin_take(ctx, n * sizeof(T));
+  HG_TRY(hipMemcpyAsync(p ? static_cast<void*>(p) : dst, src, n * sizeof(T), hipMemcpyDeviceToHost, ctx->stream));
+  HG_TRY(hipStreamSynchronize(ctx->stream));
+  if (p) std::memcpy(dst, p, n * sizeof(T));
+  ctx->pin_used = 0;
   return HG_OK;
 }
 
@@ -521,32 +561,53 @@ __global__ __launch_bounds__(kBlock) void k_min_parts(int n, const double* part,
   if (threadIdx.x == 0) out[0] = scale * red[0];
 }
 
-// Caller order -> library order: d_c[i] = src[c N + perm[i]] for the
-// ncomp (1 or 3) components.
-__global__ __launch_bounds__(kBlock) void k_perm_in(int64_t N, int ncomp, const int32_t* __restrict__ perm,
-                                                   const double* __restrict__ src, double* d0, double* d1,
-                                                   double* d2) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  const int64_t p = perm[i];
-  d0[i] = src[p];
-  if (ncomp > 1) {
-    d1[i] = src[N + p];
-    d2[i] = src[2 * N + p];
+// Up to ten arrays copied (or, without a source, cleared) in one launch.
+struct ArrayList {
+  double* dst[10];
+  const double* src[10];
+  int64_t n[10];
+  int count = 0;
+  void add(double* d, const double* s, int64_t len) {
+    if (len > 0) {
+      dst[count] = d;
+      src[count] = s;
+      n[count++] = len;
+    }
+  }
+};
+__global__ __launch_bounds__(kBlock) void k_arrays(ArrayList a) {
+  const int y = blockIdx.y;
+  for (int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x; i < a.n[y]; i += int64_t(gridDim.x) * kBlock)
+    a.dst[y][i] = a.src[y] ? a.src[y][i] : 0.0;
+}
+
+// Values off ... off+len of a caller array of components of N values each ->
+// library order: d_c[inv[j]] = value j of component c (up to three).  The
+// caller's order is the one read in sequence: src is host memory more often
+// than not.
+__global__ __launch_bounds__(kBlock) void k_perm_in(int64_t off, int64_t len, int64_t N,
+                                                   const int32_t* __restrict__ inv, const double* __restrict__ src,
+                                                   double* d0, double* d1, double* d2) {
+  for (int64_t k = int64_t(blockIdx.x) * kBlock + threadIdx.x; k < len; k += int64_t(gridDim.x) * kBlock) {
+    const int64_t g = off + k, j = g < N ? g : g < 2 * N ? g - N : g - 2 * N;
+    double* const d = g < N ? d0 : g < 2 * N ? d1 : d2;
+    d[inv[j]] = src[k];
   }
 }
 
-// Library order -> caller order: dst[c N + perm[i]] = s_c[i].
-__global__ __launch_bounds__(kBlock) void k_perm_out(int64_t N, int ncomp, const int32_t* __restrict__ perm,
-                                                    const double* s0, const double* s1, const double* s2,
-                                                    double* __restrict__ dst) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  const int64_t p = perm[i];
-  dst[p] = s0[i];
-  if (ncomp > 1) {
-    dst[N + p] = s1[i];
-    dst[2 * N + p] = s2[i];
+// The same values the other way, dst[k] = s_c[inv[j]]; without inv, s0[off + k].
+__global__ __launch_bounds__(kBlock) void k_perm_out(int64_t off, int64_t len, int64_t N,
+                                                    const int32_t* __restrict__ inv, const double* s0,
+                                                    const double* s1, const double* s2, double* __restrict__ dst) {
+  for (int64_t k = int64_t(blockIdx.x) * kBlock + threadIdx.x; k < len; k += int64_t(gridDim.x) * kBlock) {
+    const int64_t g = off + k;
+    if (!inv) {
+      dst[k] = s0[g];
+      continue;
+    }
+    const int64_t j = g < N ? g : g < 2 * N ? g - N : g - 2 * N;
+    const double* const s = g < N ? s0 : g < 2 * N ? s1 : s2;
+    dst[k] = s[inv[j]];
   }
 }
 
@@ -2005,6 +2066,15 @@ hg::InletArgs inlet_args(hg_ctx* ctx, int src) {
 
 int grid_of(int64_t n) { return int((n + kBlock - 1) / kBlock); }
 
+int launch_arrays(hg_ctx* ctx, const ArrayList& a) {
+  if (!a.count) return HG_OK;
+  int64_t longest = 0;
+  for (int k = 0; k < a.count; ++k) longest = std::max(longest, a.n[k]);
+  hipLaunchKernelGGL(k_arrays, dim3(std::min(grid_of(longest), 1024), a.count), dim3(kBlock), 0, ctx->stream, a);
+  HG_TRY(hipGetLastError());
+  return HG_OK;
+}
+
 // Tile kernel instances: T in {128, 256, 512} cells per tile (one work-item
 // per cell), MD = 3 (triangles), 4 (quads or mixed), 8 (up to octagons).
 template <int T, int MD>
@@ -2288,19 +2358,19 @@ bool res_claim(hg_ctx* ctx, int cap) {
 // After the launch of a resident run (e: its status): waits for it and gives its room back;
 // *done: every tile finished.
 int res_finish(hg_ctx* ctx, hipError_t e, bool* done) {
-  int32_t ran_out = 0;
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(&ran_out, ctx->res_ctl, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   {
     std::lock_guard<std::mutex> g(g_res_mu);
     g_res_room[ctx->device] -= ctx->res_share;
   }
   HG_TRY(e);
-  if (ran_out)  // the device was shared with something else: one launch per step from here on
+  ctx->pin_used = 0;
+  if (ctx->flags_host[2]) {  // the device was shared with something else: one launch per step from here on
+    ctx->flags_host[2] = 0;
     ctx->res_off = true;
-  else
+  } else {
     *done = true;
+  }
   return HG_OK;
 }
 
@@ -2655,23 +2725,23 @@ int finish_adjoint(hg_ctx* ctx) {
 }
 
 int zero_adj_accumulators(hg_ctx* ctx) {
+  ArrayList z;
   if (ctx->ude_prec) {
-    HG_TRY(hipMemsetAsync(ctx->ude_wbar, 0, size_t(ctx->ude_nsets) * hg::kUdeW * sizeof(double), ctx->stream));
-    HG_TRY(hipMemsetAsync(ctx->ude_wpart, 0, size_t(hg::kUdeW) * ctx->ude_nslots * sizeof(double), ctx->stream));
+    z.add(ctx->ude_wbar, nullptr, int64_t(ctx->ude_nsets) * hg::kUdeW);
+    z.add(ctx->ude_wpart, nullptr, int64_t(hg::kUdeW) * ctx->ude_nslots);
   }
   if (ctx->lux.choice) {
-    HG_TRY(hipMemsetAsync(ctx->lux_wbar, 0, ctx->lux.P * sizeof(double), ctx->stream));
-    HG_TRY(hipMemsetAsync(ctx->lux_wpart, 0, size_t(ctx->lux.P) * lux_vjp_blocks(ctx) * sizeof(double),
-                          ctx->stream));
+    z.add(ctx->lux_wbar, nullptr, ctx->lux.P);
+    z.add(ctx->lux_wpart, nullptr, int64_t(ctx->lux.P) * lux_vjp_blocks(ctx));
   }
   if (ctx->adj_want_zb) {
-    HG_TRY(hipMemsetAsync(ctx->adj_S0bar, 0, 2 * ctx->N * sizeof(double), ctx->stream));
-    HG_TRY(hipMemsetAsync(ctx->adj_zbbar, 0, ctx->N * sizeof(double), ctx->stream));
+    z.add(ctx->adj_S0bar, nullptr, 2 * ctx->N);
+    z.add(ctx->adj_zbbar, nullptr, ctx->N);
   }
-  if (ctx->adj_want_n) HG_TRY(hipMemsetAsync(ctx->adj_nbar, 0, ctx->N * sizeof(double), ctx->stream));
-  HG_TRY(hipMemsetAsync(ctx->adj_Qbar, 0, std::max<int32_t>(ctx->n_inlet, 1) * sizeof(double), ctx->stream));
-  HG_TRY(hipMemsetAsync(ctx->adj_vbar, 0, std::max<int64_t>(ctx->G, 1) * sizeof(double), ctx->stream));
-  return HG_OK;
+  if (ctx->adj_want_n) z.add(ctx->adj_nbar, nullptr, ctx->N);
+  z.add(ctx->adj_Qbar, nullptr, std::max<int32_t>(ctx->n_inlet, 1));
+  z.add(ctx->adj_vbar, nullptr, std::max<int64_t>(ctx->G, 1));
+  return launch_arrays(ctx, z);
 }
 
 int perm_out(hg_ctx* ctx, const double* const s[3], int ncomp, double* dst);
@@ -2703,16 +2773,18 @@ int recompute_segment(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck, int64
 int forward_checkpointed(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck) {
   const int64_t N = ctx->N;
   const int64_t nseg = (nsteps + kck - 1) / kck;
-  for (int64_t sgi = 0; sgi < nseg; ++sgi) {
+  const int64_t ns = nsteps - (nseg - 1) * kck;
+  auto checkpoint = [&](int64_t sgi) -> int {
     for (int c = 0; c < 3; ++c)
       HG_TRY(hipMemcpyAsync(ctx->adj_ckpt + (sgi * 3 + c) * N, ctx->st[ctx->cur][c], N * sizeof(double),
                             hipMemcpyDeviceToDevice, ctx->stream));
-    if (sgi + 1 < nseg) {
-      int rc = advance_async(ctx, dt, kck);
-      if (rc) return rc;
-    }
+    return HG_OK;
+  };
+  for (int64_t sgi = 0; sgi + 1 < nseg; ++sgi) {
+    int rc = checkpoint(sgi);
+    if (!rc) rc = advance_async(ctx, dt, kck);
+    if (rc) return rc;
   }
-  const int64_t ns = nsteps - (nseg - 1) * kck;
   bool done = false;
   hg::ResKind k;
   ctx->rec_resident = false;
@@ -2731,9 +2803,14 @@ int forward_checkpointed(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck) {
       rec_n = ctx->adj_nseg[0];
     }
     const double* in[3] = {ctx->st[ctx->cur][0], ctx->st[ctx->cur][1], ctx->st[ctx->cur][2]};
-    for (int c = 0; c < 3; ++c)
-      HG_TRY(hipMemcpyAsync(seg_state(ctx, 0, c, 0), in[c], N * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-    int rc = res_run(ctx, k, in, ctx->st[1 - ctx->cur], dt, ns, ctx->adj_seg[0], ctx->adj_mask[0],
+    ArrayList copy;  // the recorded run's first state, and the segment's checkpoint
+    for (int c = 0; c < 3; ++c) {
+      copy.add(seg_state(ctx, 0, c, 0), in[c], N);
+      copy.add(ctx->adj_ckpt + ((nseg - 1) * 3 + c) * N, in[c], N);
+    }
+    int rc = launch_arrays(ctx, copy);
+    if (rc) return rc;
+    rc = res_run(ctx, k, in, ctx->st[1 - ctx->cur], dt, ns, ctx->adj_seg[0], ctx->adj_mask[0],
                      seg_totalA(ctx, 0, 0), rec_n, nullptr, &done);
     if (rc) return rc;
     if (done) {
@@ -2742,7 +2819,8 @@ int forward_checkpointed(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck) {
       return HG_OK;
     }
   }
-  int rc = recompute_segment(ctx, dt, nsteps, kck, nseg - 1, 0, ctx->stream);
+  int rc = checkpoint(nseg - 1);
+  if (!rc) rc = recompute_segment(ctx, dt, nsteps, kck, nseg - 1, 0, ctx->stream);
   if (rc) return rc;
   for (int c = 0; c < 3; ++c)
     HG_TRY(hipMemcpyAsync(ctx->st[0][c], seg_state(ctx, ns, c, 0), N * sizeof(double), hipMemcpyDeviceToDevice,
@@ -2820,6 +2898,7 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
   if (ctx->deg_full) a.deg = nullptr;
   a.items = ctx->adj_items;
   hg::AdjRunArgs R{};
+  R.flag = ctx->flags;
   R.ring = ctx->adj_ring;
   R.vring = ctx->adj_ring + 12 * N;
   R.ctl = ctx->res_ctl;
@@ -2851,15 +2930,15 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
   if (e == hipSuccess) e = hg::launch_adj_run(ctx->stream, ctx->tileMD, k.nmode, ctx->ntiles, a, R);
   int rc = res_finish(ctx, e, done);
   if (rc || !*done) return rc;
-  auto take = [&](double* dst, const double* src, int64_t n) {
-    return n > 0 ? hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream) : hipSuccess;
-  };
-  if (R.o_nbar) HG_TRY(take(ctx->adj_nbar, R.o_nbar, N));
+  ArrayList take;
+  if (R.o_nbar) take.add(ctx->adj_nbar, R.o_nbar, N);
   if (R.o_zbbar) {
-    HG_TRY(take(ctx->adj_zbbar, R.o_zbbar, N));
-    HG_TRY(take(ctx->adj_S0bar, R.o_S0bar, 2 * N));
+    take.add(ctx->adj_zbbar, R.o_zbbar, N);
+    take.add(ctx->adj_S0bar, R.o_S0bar, 2 * N);
   }
-  HG_TRY(take(ctx->adj_Qbar, R.o_Qbar, ctx->n_inlet));
+  take.add(ctx->adj_Qbar, R.o_Qbar, ctx->n_inlet);
+  rc = launch_arrays(ctx, take);
+  if (rc) return rc;
   if (P) {
     hipLaunchKernelGGL(k_ude_wsum, dim3(P), dim3(kBlock), 0, ctx->stream, ctx->ntiles, nullptr, ctx->adj_wpart,
                        int64_t(ctx->ntiles), int64_t(1), ctx->lux_wbar);
@@ -2939,8 +3018,8 @@ int reverse_sweep(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck, int& lam_
 // The error flags live in pinned, coherent host memory that the kernels
 // write only on an error: clearing and reading them takes no copy on the
 // stream.  Every call that clears them has no kernel of its own in flight
-// (each entry point ends synchronized), and the stream is synchronized
-// before they are read.
+// that writes them (each entry point that starts one ends synchronized), and
+// the stream is synchronized before they are read.
 int clear_flags(hg_ctx* ctx) {
   for (int k = 0; k < 4; ++k) ctx->flags_host[k] = 0;
   return HG_OK;
@@ -2966,72 +3045,97 @@ int check_flags(hg_ctx* ctx) {
 // Host 3N state (caller order) -> device state `slot` (library order).
 // The staging buffer and device permutation of the transfers below
 // (allocated on first use).
-// ---- host <-> device copies of caller arrays.  A caller's array is
-// ordinary (pageable) host memory, which the DMA engine reads or writes only
-// through the runtime's own staging, slowly for device -> host.  Instead the
-// array moves in 4 MiB chunks through two pinned buffers: host threads copy
-// one chunk between the caller's array and a pinned buffer while the DMA
-// engine moves the other.  The pinned buffers and the threads are the
-// process's, shared by every context (one transfer at a time).
+// ---- host <-> device copies of caller arrays.  A caller's array is ordinary
+// (pageable) host memory, which the GPU cannot address.  It goes through
+// pinned memory, which the permutation kernels read and write directly: they
+// reach the link's 55 GB/s, and against a DMA into a staging array this saves
+// the array's second pass and some 10 us for each copy started.  An array
+// that fits takes a piece of the context's own block: one kernel each way,
+// and no wait before the kernels that follow (138 -> 27 us for a host RHS of
+// 1,000 cells).  A larger one moves in 2 MiB chunks through four pinned
+// buffers of the process: host threads, woken once per transfer, copy the
+// chunks that the calling thread opens to them, while kernels move the others
+// (a host RHS of 1M cells, 24 MB each way: 1310 -> 1120 us, of which the link
+// needs 870).  One such transfer at a time.
 
-constexpr size_t kXferChunk = size_t(1) << 19;  // doubles per chunk (4 MiB)
+constexpr size_t kXferChunk = size_t(1) << 18;  // doubles per chunk (2 MiB)
+constexpr size_t kXferBufs = 4;
 
-// memcpy split over a fixed set of host threads (the caller takes part 0).
-struct HostCopyPool {
-  std::vector<std::thread> th;
-  std::mutex m;
-  std::condition_variable go, done;
+struct HostXfer {
+  std::mutex m;  // one transfer at a time
+  double* pin[kXferBufs] = {};
+  pid_t pid = 0;  // the process that made the threads (a forked child makes its own)
+  bool ok = false;
+  int parts = 0;  // threads, each with its part of every chunk
+  // the transfer in progress
+  std::mutex jm;
+  std::condition_variable go;
   uint64_t gen = 0;
-  int left = 0, parts = 1;
-  char* dst = nullptr;
-  const char* src = nullptr;
-  size_t bytes = 0;
-  explicit HostCopyPool(int workers) : parts(workers + 1) {
-    for (int k = 1; k <= workers; ++k) th.emplace_back([this, k] { worker(k); });
+  bool to_pin = false;
+  char* user = nullptr;
+  size_t bytes = 0, nch = 0;
+  std::atomic<size_t> open{0};           // chunks that may be copied
+  std::atomic<int> done[kXferBufs] = {};  // parts of the buffer's chunk that are
+  std::atomic<int> running{0};
+
+  void copy_part(size_t c, int p) const {
+    const size_t off = c * kXferChunk * sizeof(double), len = std::min(kXferChunk * sizeof(double), bytes - off);
+    const size_t per = ((len + size_t(parts) - 1) / size_t(parts) + 63) & ~size_t(63);
+    const size_t a = std::min(len, per * size_t(p)), b = std::min(len, a + per);
+    char* const buf = reinterpret_cast<char*>(pin[c % kXferBufs]) + a;
+    if (b <= a) return;
+    if (to_pin)
+      std::memcpy(buf, user + off + a, b - a);
+    else
+      std::memcpy(user + off + a, buf, b - a);
   }
-  void part(int p) const {
-    const size_t per = ((bytes + size_t(parts) - 1) / size_t(parts) + 63) & ~size_t(63);
-    const size_t a = std::min(bytes, per * size_t(p)), b = std::min(bytes, a + per);
-    if (b > a) std::memcpy(dst + a, src + a, b - a);
+  template <class F>
+  static void spin(F&& ready) {
+    for (int k = 0; !ready(); ++k)
+      if (k > 256) std::this_thread::yield();
   }
-  void worker(int p) {
-    uint64_t seen = 0;
-    std::unique_lock<std::mutex> lk(m);
+  void worker(int p, uint64_t seen) {
     for (;;) {
-      go.wait(lk, [&] { return gen != seen; });
-      seen = gen;
-      lk.unlock();
-      part(p);
-      lk.lock();
-      if (--left == 0) done.notify_one();
+      {
+        std::unique_lock<std::mutex> lk(jm);
+        go.wait(lk, [&] { return gen != seen; });
+        seen = gen;
+      }
+      for (size_t c = 0; c < nch; ++c) {
+        spin([&] { return open.load(std::memory_order_acquire) > c; });
+        copy_part(c, p);
+        done[c % kXferBufs].fetch_add(1, std::memory_order_release);
+      }
+      running.fetch_sub(1, std::memory_order_release);
     }
   }
-  void copy(void* d, const void* s, size_t n) {
+  void start(bool in, void* host, size_t n) {
+    for (auto& d : done) d.store(0, std::memory_order_relaxed);
+    open.store(0, std::memory_order_relaxed);
+    running.store(parts, std::memory_order_relaxed);
     {
-      std::lock_guard<std::mutex> g(m);
-      dst = static_cast<char*>(d);
-      src = static_cast<const char*>(s);
-      bytes = n;
-      left = parts - 1;
+      std::lock_guard<std::mutex> g(jm);
+      to_pin = in;
+      user = static_cast<char*>(host);
+      bytes = n * sizeof(double);
+      nch = (n + kXferChunk - 1) / kXferChunk;
       ++gen;
     }
     go.notify_all();
-    part(0);
-    std::unique_lock<std::mutex> lk(m);
-    done.wait(lk, [&] { return left == 0; });
+  }
+  void wait_done(size_t c) {
+    spin([&] { return done[c % kXferBufs].load(std::memory_order_acquire) == parts; });
+  }
+  void open_to(size_t c) { open.store(c, std::memory_order_release); }
+  // Every part of every chunk copied (also after an error: nothing stays open).
+  void finish() {
+    open_to(nch);
+    spin([&] { return running.load(std::memory_order_acquire) == 0; });
   }
 };
 
-struct HostXfer {
-  std::mutex m;            // one transfer at a time
-  double* pin[2] = {nullptr, nullptr};
-  HostCopyPool* pool = nullptr;  // threads live until the process ends
-  pid_t pid = 0;                 // the process that made them (a forked child makes its own)
-  bool ok = false;
-};
-
 HostXfer& host_xfer() {
-  static HostXfer x;
+  static HostXfer& x = *new HostXfer();  // its threads run until the process ends
   return x;
 }
 
@@ -3039,19 +3143,24 @@ HostXfer& host_xfer() {
 // is not available (the plain copies are used then).
 bool host_xfer_ready(HostXfer& x) {
   if (x.ok && x.pid == getpid()) return true;
-  if (x.ok) {  // a fork: the parent's threads did not come along (its pool is left as it is)
-    x.pool = nullptr;
-    x.ok = false;
+  for (double*& p : x.pin)
+    if (!p && hipHostMalloc(reinterpret_cast<void**>(&p), kXferChunk * sizeof(double)) != hipSuccess) {
+      p = nullptr;
+      return false;
+    }
+  // (after a fork the parent's threads did not come along: the child makes its own)
+  const unsigned hw = std::thread::hardware_concurrency();
+  const int want = int(std::max(1u, std::min(8u, hw / 2)));
+  const uint64_t gen = x.gen;
+  x.parts = 0;
+  try {
+    for (int k = 0; k < want; ++k) {
+      std::thread([&x, k, gen] { x.worker(k, gen); }).detach();
+      x.parts = k + 1;
+    }
+  } catch (const std::exception&) {  // no more threads to be had: as many parts as there are
   }
-  if (!x.pin[0] && hipHostMalloc(reinterpret_cast<void**>(&x.pin[0]), kXferChunk * sizeof(double)) != hipSuccess)
-    x.pin[0] = nullptr;
-  if (!x.pin[1] && hipHostMalloc(reinterpret_cast<void**>(&x.pin[1]), kXferChunk * sizeof(double)) != hipSuccess)
-    x.pin[1] = nullptr;
-  if (!x.pin[0] || !x.pin[1]) return false;
-  if (!x.pool) {
-    const unsigned hw = std::thread::hardware_concurrency();
-    x.pool = new HostCopyPool(int(std::min(7u, hw > 1 ? hw / 2 : 0u)));
-  }
+  if (x.parts == 0) return false;
   x.pid = getpid();
   x.ok = true;
   return true;
@@ -3063,58 +3172,99 @@ int ensure_xfer_events(hg_ctx* ctx) {
   return HG_OK;
 }
 
-// n doubles: caller's host array src -> device dst (ctx->stream; returns
-// with the copies enqueued after the last host chunk was staged).
-int host_to_device(hg_ctx* ctx, double* dst, const double* src, size_t n) {
+int xfer_grid(size_t len) { return std::min(grid_of(int64_t(len)), 512); }
+
+// Large caller array (ncomp x N values) -> device arrays d[c] in library
+// order (ctx->stream; returns when the array has been read and moved).
+int host_to_device(hg_ctx* ctx, double* const d[3], const double* src, int ncomp) {
+  const size_t n = size_t(ncomp) * ctx->N;
+  auto put = [&](const double* from, size_t off, size_t len) {
+    hipLaunchKernelGGL(k_perm_in, dim3(xfer_grid(len)), dim3(kBlock), 0, ctx->stream, int64_t(off), int64_t(len),
+                       ctx->N, ctx->d_inv, from, d[0], d[1], d[2]);
+    return hipGetLastError();
+  };
   HostXfer& x = host_xfer();
   std::lock_guard<std::mutex> g(x.m);
   if (!host_xfer_ready(x)) {
-    HG_TRY(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    HG_TRY(hipMemcpyAsync(ctx->stage, src, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+    HG_TRY(put(ctx->stage, 0, n));
     HG_TRY(hipStreamSynchronize(ctx->stream));
     return HG_OK;
   }
   if (int rc = ensure_xfer_events(ctx)) return rc;
-  for (size_t off = 0, k = 0; off < n; off += kXferChunk, ++k) {
-    const int b = int(k & 1);
-    const size_t len = std::min(kXferChunk, n - off);
-    if (k >= 2) HG_TRY(hipEventSynchronize(ctx->ev_xfer[b]));  // the DMA that last read pin[b]
-    x.pool->copy(x.pin[b], src + off, len * sizeof(double));
-    HG_TRY(hipMemcpyAsync(dst + off, x.pin[b], len * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    HG_TRY(hipEventRecord(ctx->ev_xfer[b], ctx->stream));
+  x.start(true, const_cast<double*>(src), n);
+  hipError_t e = hipSuccess;
+  size_t opened = std::min(kXferBufs, x.nch);
+  x.open_to(opened);
+  for (size_t c = 0; c < x.nch && e == hipSuccess; ++c) {
+    // open the chunks whose buffers' kernels are done (chunk c's own if need be, waiting)
+    while (opened < x.nch && opened < c + kXferBufs) {
+      const hipEvent_t ev = ctx->ev_xfer[opened % kXferBufs];
+      if (opened < c + 1)
+        e = hipEventSynchronize(ev);
+      else if (hipEventQuery(ev) != hipSuccess)
+        break;
+      if (e != hipSuccess) break;
+      x.done[opened % kXferBufs].store(0, std::memory_order_relaxed);
+      x.open_to(++opened);
+    }
+    if (e != hipSuccess) break;
+    x.wait_done(c);
+    const size_t off = c * kXferChunk;
+    e = put(x.pin[c % kXferBufs], off, std::min(kXferChunk, n - off));
+    if (e == hipSuccess) e = hipEventRecord(ctx->ev_xfer[c % kXferBufs], ctx->stream);
   }
-  HG_TRY(hipStreamSynchronize(ctx->stream));  // the pinned buffers are free for the next transfer
+  x.finish();
+  const hipError_t es = hipStreamSynchronize(ctx->stream);  // the pinned buffers are free for the next transfer
+  HG_TRY(e);
+  HG_TRY(es);
   return HG_OK;
 }
 
-// n doubles: device src -> caller's host array dst, after the work already
-// on ctx->stream; synchronous.
-int device_to_host(hg_ctx* ctx, double* dst, const double* src, size_t n) {
+// n values of device arrays s[c] of N values each, by d_inv (without it, of
+// s[0]) -> caller's host array, after the work already on ctx->stream;
+// synchronous.  Without pinned memory, through ctx->stage in pieces.
+int device_to_host(hg_ctx* ctx, double* dst, const double* const s[3], const int32_t* inv, size_t n) {
+  auto put = [&](double* to, size_t off, size_t len) {
+    hipLaunchKernelGGL(k_perm_out, dim3(xfer_grid(len)), dim3(kBlock), 0, ctx->stream, int64_t(off), int64_t(len),
+                       ctx->N, inv, s[0], s[1], s[2], to);
+    return hipGetLastError();
+  };
   HostXfer& x = host_xfer();
   std::lock_guard<std::mutex> g(x.m);
   if (!host_xfer_ready(x)) {
-    HG_TRY(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HG_TRY(hipStreamSynchronize(ctx->stream));
+    const size_t piece = size_t(3) * ctx->N;
+    for (size_t off = 0; off < n; off += piece) {
+      const size_t len = std::min(piece, n - off);
+      HG_TRY(put(ctx->stage, off, len));
+      HG_TRY(hipMemcpyAsync(dst + off, ctx->stage, len * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+      HG_TRY(hipStreamSynchronize(ctx->stream));
+    }
     return HG_OK;
   }
   if (int rc = ensure_xfer_events(ctx)) return rc;
-  const size_t nch = (n + kXferChunk - 1) / kXferChunk;
-  auto issue = [&](size_t k) -> int {
-    const int b = int(k & 1);
-    const size_t off = k * kXferChunk, len = std::min(kXferChunk, n - off);
-    HG_TRY(hipMemcpyAsync(x.pin[b], src + off, len * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HG_TRY(hipEventRecord(ctx->ev_xfer[b], ctx->stream));
-    return HG_OK;
+  auto issue = [&](size_t c) {
+    const size_t off = c * kXferChunk;
+    const hipError_t e = put(x.pin[c % kXferBufs], off, std::min(kXferChunk, n - off));
+    return e == hipSuccess ? hipEventRecord(ctx->ev_xfer[c % kXferBufs], ctx->stream) : e;
   };
-  for (size_t k = 0; k < std::min<size_t>(2, nch); ++k)
-    if (int rc = issue(k)) return rc;
-  for (size_t k = 0; k < nch; ++k) {
-    const int b = int(k & 1);
-    const size_t off = k * kXferChunk, len = std::min(kXferChunk, n - off);
-    HG_TRY(hipEventSynchronize(ctx->ev_xfer[b]));
-    x.pool->copy(dst + off, x.pin[b], len * sizeof(double));
-    if (k + 2 < nch)
-      if (int rc = issue(k + 2)) return rc;
+  const size_t nch = (n + kXferChunk - 1) / kXferChunk;
+  hipError_t e = hipSuccess;
+  for (size_t c = 0; c < std::min(kXferBufs, nch) && e == hipSuccess; ++c) e = issue(c);
+  x.start(false, dst, n);
+  for (size_t c = 0; c < nch && e == hipSuccess; ++c) {
+    e = hipEventSynchronize(ctx->ev_xfer[c % kXferBufs]);
+    if (e != hipSuccess) break;
+    x.open_to(c + 1);
+    if (c >= 1 && c - 1 + kXferBufs < nch) {  // the previous chunk's buffer, once it is copied out
+      x.wait_done(c - 1);
+      x.done[(c - 1) % kXferBufs].store(0, std::memory_order_relaxed);
+      e = issue(c - 1 + kXferBufs);
+    }
   }
+  x.finish();
+  if (e != hipSuccess) (void)hipStreamSynchronize(ctx->stream);  // no kernel writes the buffers any more
+  HG_TRY(e);
   return HG_OK;
 }
 
@@ -3122,34 +3272,67 @@ int ensure_xfer(hg_ctx* ctx) {
   if (ctx->stage) return HG_OK;
   int rc = dalloc(ctx, &ctx->d_perm, size_t(ctx->N));
   if (!rc) rc = upload(ctx, ctx->d_perm, ctx->perm.data(), size_t(ctx->N));
+  if (!rc) rc = dalloc(ctx, &ctx->d_inv, size_t(ctx->N));
+  if (!rc) rc = upload(ctx, ctx->d_inv, ctx->iperm.data(), size_t(ctx->N));
   if (!rc) rc = dalloc(ctx, &ctx->stage, size_t(3) * ctx->N);
   return rc;
 }
 
 // Host array of ncomp x N values in caller order -> device arrays d[c] in
-// library order: one contiguous copy, then the permutation on the device.
+// library order.
 int perm_in(hg_ctx* ctx, const double* src, int ncomp, double* const d[3]) {
-  const int64_t N = ctx->N;
+  const int64_t n = int64_t(ncomp) * ctx->N;
   int rc = ensure_xfer(ctx);
-  if (rc) return rc;
-  rc = host_to_device(ctx, ctx->stage, src, size_t(ncomp) * N);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_perm_in, dim3(grid_of(N)), dim3(kBlock), 0, ctx->stream, N, ncomp, ctx->d_perm, ctx->stage,
-                     d[0], d[ncomp > 1 ? 1 : 0], d[ncomp > 1 ? 2 : 0]);
+  if (rc || n == 0) return rc;
+  char* const p = pin_take(ctx, size_t(n) * sizeof(double));
+  if (!p) return host_to_device(ctx, d, src, ncomp);
+  std::memcpy(p, src, size_t(n) * sizeof(double));
+  hipLaunchKernelGGL(k_perm_in, dim3(xfer_grid(size_t(n))), dim3(kBlock), 0, ctx->stream, int64_t(0), n, ctx->N,
+                     ctx->d_inv, reinterpret_cast<const double*>(p), d[0], d[1], d[2]);
   HG_TRY(hipGetLastError());
-  HG_TRY(hipStreamSynchronize(ctx->stream));
   return HG_OK;
 }
 
-// Device arrays s[c] in library order -> host array in caller order.
-int perm_out(hg_ctx* ctx, const double* const s[3], int ncomp, double* dst) {
+// Device arrays in library order -> host arrays in caller order: s[c] of ncomp
+// (1 or 3) components each, `count` of them with one wait when they are small.
+struct OutArray {
+  const double* s[3];
+  int ncomp;
+  double* dst;
+};
+
+int perm_out_all(hg_ctx* ctx, const OutArray* out, int count) {
   const int64_t N = ctx->N;
   int rc = ensure_xfer(ctx);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_perm_out, dim3(grid_of(N)), dim3(kBlock), 0, ctx->stream, N, ncomp, ctx->d_perm, s[0],
-                     s[ncomp > 1 ? 1 : 0], s[ncomp > 1 ? 2 : 0], ctx->stage);
-  HG_TRY(hipGetLastError());
-  return device_to_host(ctx, dst, ctx->stage, size_t(ncomp) * N);
+  size_t total = 0;
+  for (int k = 0; k < count; ++k) total += (size_t(out[k].ncomp) * N * sizeof(double) + 63) & ~size_t(63);
+  if (char* p = total ? pin_take(ctx, total) : nullptr) {
+    size_t off = 0;
+    for (int k = 0; k < count; ++k) {
+      const int64_t n = int64_t(out[k].ncomp) * N;
+      hipLaunchKernelGGL(k_perm_out, dim3(xfer_grid(size_t(n))), dim3(kBlock), 0, ctx->stream, int64_t(0), n, N,
+                         ctx->d_inv, out[k].s[0], out[k].s[1], out[k].s[2], reinterpret_cast<double*>(p + off));
+      HG_TRY(hipGetLastError());
+      off += (size_t(out[k].ncomp) * N * sizeof(double) + 63) & ~size_t(63);
+    }
+    HG_TRY(hipStreamSynchronize(ctx->stream));
+    off = 0;
+    for (int k = 0; k < count; ++k) {
+      std::memcpy(out[k].dst, p + off, size_t(out[k].ncomp) * N * sizeof(double));
+      off += (size_t(out[k].ncomp) * N * sizeof(double) + 63) & ~size_t(63);
+    }
+    ctx->pin_used = 0;
+    return HG_OK;
+  }
+  for (int k = 0; k < count && !rc; ++k)
+    rc = device_to_host(ctx, out[k].dst, out[k].s, ctx->d_inv, size_t(out[k].ncomp) * N);
+  return rc;
+}
+
+int perm_out(hg_ctx* ctx, const double* const s[3], int ncomp, double* dst) {
+  const OutArray o{{s[0], s[1], s[2]}, ncomp, dst};
+  return perm_out_all(ctx, &o, 1);
 }
 
 int state_in(hg_ctx* ctx, const double* Q, int slot) {
@@ -3173,8 +3356,8 @@ int mesh_cell_in(hg_ctx* ctx, double* dst, const double* src) {
   if (ctx->K == 1) return cell_in(ctx, dst, src);
   const int64_t Nm = ctx->Nm;
   HG_TRY(hipMemcpyAsync(ctx->stage, src, size_t(Nm) * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-  hipLaunchKernelGGL(k_perm_in, dim3(grid_of(Nm)), dim3(kBlock), 0, ctx->stream, Nm, 1, ctx->d_perm, ctx->stage, dst,
-                     dst, dst);
+  hipLaunchKernelGGL(k_perm_in, dim3(xfer_grid(size_t(Nm))), dim3(kBlock), 0, ctx->stream, int64_t(0), Nm, Nm,
+                     ctx->d_inv, ctx->stage, dst, dst, dst);
   HG_TRY(hipGetLastError());
   HG_TRY(hipStreamSynchronize(ctx->stream));
   return HG_OK;
@@ -3185,24 +3368,27 @@ int mesh_cell_in(hg_ctx* ctx, double* dst, const double* src) {
 // per call only).
 int restore_base(hg_ctx* ctx) {
   const int64_t Nm = ctx->Nm;  // the mesh's bed data (shared by the fields); n per field
-  HG_TRY(hipMemcpyAsync(ctx->zb, ctx->zb0, Nm * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-  HG_TRY(hipMemcpyAsync(ctx->n, ctx->n0, ctx->N * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-  HG_TRY(hipMemcpyAsync(ctx->S0x, ctx->S0x0, Nm * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-  HG_TRY(hipMemcpyAsync(ctx->S0y, ctx->S0y0, Nm * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-  if (ctx->Gm)
-    HG_TRY(hipMemcpyAsync(ctx->g_zb, ctx->g_zb0, ctx->Gm * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
-  if (ctx->n_inlet)
-    HG_TRY(hipMemcpyAsync(ctx->inletQ, ctx->inletQ0, ctx->n_inlet * sizeof(double), hipMemcpyDeviceToDevice,
-                          ctx->stream));
-  HG_TRY(hipStreamSynchronize(ctx->stream));
-  return HG_OK;
+  ArrayList c;
+  c.add(ctx->zb, ctx->zb0, Nm);
+  c.add(ctx->n, ctx->n0, ctx->N);
+  c.add(ctx->S0x, ctx->S0x0, Nm);
+  c.add(ctx->S0y, ctx->S0y0, Nm);
+  c.add(ctx->g_zb, ctx->g_zb0, ctx->Gm);
+  c.add(ctx->inletQ, ctx->inletQ0, ctx->n_inlet);
+  return launch_arrays(ctx, c);
 }
 
 // Apply params_vector per the active parameter (semi_discretize_swe_2D.jl:114-199).
 int apply_params(hg_ctx* ctx, const double* params, int64_t np) {
   const int64_t N = ctx->N;
-  int rc0 = restore_base(ctx);
-  if (rc0) return rc0;
+  // parameters override the working copies, and a closure rewrites n: without
+  // either since the last restore, the copies are still the fields
+  const bool changes = ctx->active != HG_PARAM_NONE || ctx->ude_prec || ctx->nlaw.kind || ctx->lux.choice;
+  if (changes || ctx->base_dirty) {
+    int rc0 = restore_base(ctx);
+    if (rc0) return rc0;
+  }
+  ctx->base_dirty = changes;
   switch (ctx->active) {
     case HG_PARAM_NONE:
       break;
@@ -3249,7 +3435,6 @@ int apply_params(hg_ctx* ctx, const double* params, int64_t np) {
       ctx->err = "unknown active parameter";
       return HG_ERR_ARG;
   }
-  HG_TRY(hipStreamSynchronize(ctx->stream));
   return HG_OK;
 }
 
@@ -3657,18 +3842,24 @@ int create_impl(hg_ctx** out, const hg_mesh* m, const hg_bcs* b, const hg_consts
   if (!rc) rc = dalloc(ctx, &ctx->exitWSE, ctx->n_exit);
   if (!rc) rc = dalloc(ctx, &ctx->totalA, ctx->n_inlet);
   if (!rc) {
-    void* hp = nullptr;
-    if (hipHostMalloc(&hp, 4 * sizeof(int32_t), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
-      ctx->err = "hipHostMalloc (error flags) failed";
+    // one pinned, coherent block: the error flags, the Tsit5 state between
+    // launches, and the pieces of pin_take (small transfers, see perm_in)
+    const size_t small = size_t(6) * NT * sizeof(double);
+    ctx->pin_n = small <= kPinSmall ? 2 * small + 65536 : 65536;
+    constexpr size_t head = 1024;
+    static_assert(64 + 2 * sizeof(hg::Tsit5State) <= head, "the block's head");
+    void *hp = nullptr, *dp = nullptr;
+    if (hipHostMalloc(&hp, head + ctx->pin_n, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer(&dp, hp, 0) != hipSuccess || dp != hp) {
+      ctx->err = "hipHostMalloc (error flags and small transfers) failed";
+      if (hp) (void)hipHostFree(hp);
       rc = HG_ERR_HIP;
     } else {
+      std::memset(hp, 0, head);
       ctx->flags_host = static_cast<volatile int32_t*>(hp);
-      void* dp = nullptr;
-      if (hipHostGetDevicePointer(&dp, hp, 0) != hipSuccess) {
-        ctx->err = "hipHostGetDevicePointer (error flags) failed";
-        rc = HG_ERR_HIP;
-      }
-      ctx->flags = static_cast<int32_t*>(dp);
+      ctx->flags = static_cast<int32_t*>(hp);
+      ctx->rk_state = reinterpret_cast<hg::Tsit5State*>(static_cast<char*>(hp) + 64);
+      ctx->pin = static_cast<char*>(hp) + head;
     }
   }
   if (!rc) rc = dalloc(ctx, &ctx->zone, N);
@@ -3900,7 +4091,7 @@ int hg_destroy(hg_ctx* ctx) {
   for (auto& kv : ctx->seg_graphs) (void)hipGraphExecDestroy(kv.second);
   for (hipEvent_t e : ctx->ev_pool) (void)hipEventDestroy(e);
   for (hipEvent_t e : {ctx->ev_seg[0], ctx->ev_seg[1], ctx->ev_rev[0], ctx->ev_rev[1], ctx->ev_fwd, ctx->ev_xfer[0],
-                       ctx->ev_xfer[1]})
+                       ctx->ev_xfer[1], ctx->ev_xfer[2], ctx->ev_xfer[3]})
     if (e) (void)hipEventDestroy(e);
   if (ctx->stream2) {
     (void)hipStreamSynchronize(ctx->stream2);
@@ -3951,6 +4142,7 @@ int hg_set_fields(hg_ctx* ctx, const double* hstill, const double* hstill_ghost,
   if (!rc) rc = upload(ctx, ctx->exitWSE, exitWSE, ctx->n_exit);
   if (rc) return rc;
   ctx->fields_set = true;
+  ctx->base_dirty = true;
   return restore_base(ctx);
 }
 
@@ -4138,7 +4330,7 @@ int hg_cfl_dt_noalloc(hg_ctx* ctx, const double* Q, double cfl, double* dt) {
     return HG_ERR_ARG;
   }
   double* const sc = ctx->noalloc_scratch;
-  if (!sc || !ctx->stage || !ctx->d_perm) {
+  if (!sc || !ctx->stage || !ctx->d_inv) {
     ctx->err = "hg_cfl_dt_noalloc: context set-up incomplete";
     return HG_ERR_STATE;
   }
@@ -4146,8 +4338,8 @@ int hg_cfl_dt_noalloc(hg_ctx* ctx, const double* Q, double cfl, double* dt) {
   // (as hg_cfl_dt); partial minima in scratch[0, nb), the result in
   // scratch[kNoAllocParts].  Every slot read is written first by this call.
   HG_TRY(hipMemcpyAsync(ctx->stage, Q, size_t(3) * N * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-  hipLaunchKernelGGL(k_perm_in, dim3(grid_of(N)), dim3(kBlock), 0, ctx->stream, N, 3, ctx->d_perm, ctx->stage,
-                     ctx->st[0][0], ctx->st[0][1], ctx->st[0][2]);
+  hipLaunchKernelGGL(k_perm_in, dim3(xfer_grid(size_t(3) * N)), dim3(kBlock), 0, ctx->stream, int64_t(0), 3 * N, N,
+                     ctx->d_inv, ctx->stage, ctx->st[0][0], ctx->st[0][1], ctx->st[0][2]);
   ctx->cur = 0;
   hipLaunchKernelGGL(k_cfl, dim3(nb), dim3(kBlock), 0, ctx->stream, int(N), int(ctx->Nm), ctx->st[0][0], ctx->st[0][1],
                      ctx->st[0][2], ctx->hstill, ctx->deg, ctx->flen, ctx->area, ctx->c.g, ctx->c.h_small, sc);
@@ -4161,6 +4353,7 @@ int hg_cfl_dt_noalloc(hg_ctx* ctx, const double* Q, double cfl, double* dt) {
 int hg_set_ude(hg_ctx* ctx, int32_t n_sets, const double* weights, const int32_t* set_of_cell,
                int32_t precision) {
   if (!ctx) return HG_ERR_ARG;
+  ctx->base_dirty = true;  // the closure writes n
   ctx->adj_pending = false;  // a recorded forward sweep no longer matches
   HG_TRY(hipStreamSynchronize(ctx->stream));
   if (drop_graph(ctx)) return HG_ERR_HIP;  // captured steps may include (or lack) the closure
@@ -4307,6 +4500,7 @@ int hg_ude_grad(hg_ctx* ctx, double* w_bar) {
 
 int hg_set_n_law(hg_ctx* ctx, int32_t kind, const double* params, const double* ks) {
   if (!ctx) return HG_ERR_ARG;
+  ctx->base_dirty = true;  // the closure writes n
   ctx->adj_pending = false;  // a recorded forward sweep no longer matches
   if (kind != HG_NLAW_OFF && refuse_fields(ctx, "hg_set_n_law")) return HG_ERR_STATE;
   if (kind < HG_NLAW_OFF || kind > HG_NLAW_H_UMAG_KS) {
@@ -4479,6 +4673,7 @@ int64_t hg_lux_n_params(const hg_lux_net* net) {
 
 int hg_set_lux_ude(hg_ctx* ctx, const hg_lux_net* net, const double* params, const double* ks) {
   if (!ctx) return HG_ERR_ARG;
+  ctx->base_dirty = true;  // the closure writes n
   ctx->adj_pending = false;  // a recorded forward sweep no longer matches
   if (net && refuse_fields(ctx, "hg_set_lux_ude")) return HG_ERR_STATE;
   HG_TRY(hipStreamSynchronize(ctx->stream));
@@ -4569,10 +4764,7 @@ int hg_lux_grad(hg_ctx* ctx, double* params_bar) {
     ctx->err = "hg_lux_grad: the UDE network is off";
     return HG_ERR_STATE;
   }
-  HG_TRY(hipMemcpyAsync(params_bar, ctx->lux_wbar, size_t(ctx->lux.P) * sizeof(double), hipMemcpyDeviceToHost,
-                        ctx->stream));
-  HG_TRY(hipStreamSynchronize(ctx->stream));
-  return HG_OK;
+  return download(ctx, params_bar, ctx->lux_wbar, size_t(ctx->lux.P));
 }
 
 int hg_mfma_probe(int32_t precision, const double* A, const double* B, double* D) {
@@ -4796,7 +4988,6 @@ static int tsit5_resident(hg_ctx* ctx, double t0, double t1, int64_t n_save, dou
   if (cap < 0) cap = hg::tsit5_capacity(k.md, k.nmode, ctx->ncu);
   if (ctx->ntiles > cap) return HG_OK;
   int rc = ensure_res_ring(ctx, 3);
-  if (!rc && !ctx->rk_state) rc = dalloc(ctx, &ctx->rk_state, 2);
   if (!rc && frames > ctx->rk_frames_n) {
     rc = dfree(ctx, ctx->rk_frames);
     ctx->rk_frames_n = 0;
@@ -4830,13 +5021,18 @@ static int tsit5_resident(hg_ctx* ctx, double t0, double t1, int64_t n_save, dou
     if (e == hipSuccess)
       e = hg::launch_tsit5(ctx->stream, k.md, k.nmode, ctx->ntiles, make_tile_args_p(ctx, in, ctx->st[1], 0.0),
                            res_args(ctx, 0), P);
-    if (e == hipSuccess) e = hipMemcpyAsync(&st, P.out, sizeof(st), hipMemcpyDeviceToHost, ctx->stream);
     bool ran = false;
     rc = res_finish(ctx, e, &ran);
     if (rc || !ran) return rc;
+    st = ctx->rk_state[launch & 1];
   }
   *done = true;
-  rc = device_to_host(ctx, Qsave, ctx->rk_frames, size_t(st.frame) * n3);  // the frames that were reached
+  const size_t got = size_t(st.frame) * n3;  // the frames that were reached
+  const double* const src[3] = {ctx->rk_frames, nullptr, nullptr};
+  if (got * sizeof(double) <= ctx->pin_n)
+    rc = download(ctx, Qsave, ctx->rk_frames, got);
+  else
+    rc = device_to_host(ctx, Qsave, src, nullptr, got);
   if (rc) return rc;
   if (st.code == HG_ERR_NONFINITE)
     ctx->err = "hg_tsit5_solve: non-finite error estimate";
@@ -5229,19 +5425,13 @@ static int adj_upload_lam(hg_ctx* ctx, const double* hbar, double* dst) {
 static int adj_download(hg_ctx* ctx, const double* lam_dev, double* Q_bar, double* n_bar, double* zb_bar,
                         double* inletQ_bar) {
   const int64_t N = ctx->N;
-  int rc = 0;
-  if (Q_bar) {
-    double* src[3] = {const_cast<double*>(lam_dev), const_cast<double*>(lam_dev) + N,
-                      const_cast<double*>(lam_dev) + 2 * N};
-    rc = state_out(ctx, src, Q_bar);
-  }
-  if (!rc && n_bar) rc = cell_out(ctx, ctx->adj_nbar, n_bar);
-  if (!rc && zb_bar) rc = cell_out(ctx, ctx->adj_zbbar, zb_bar);
-  if (!rc && inletQ_bar && ctx->n_inlet) {
-    HG_TRY(hipMemcpyAsync(inletQ_bar, ctx->adj_Qbar, ctx->n_inlet * sizeof(double), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    HG_TRY(hipStreamSynchronize(ctx->stream));
-  }
+  OutArray out[3];
+  int k = 0;
+  if (Q_bar) out[k++] = OutArray{{lam_dev, lam_dev + N, lam_dev + 2 * N}, 3, Q_bar};
+  if (n_bar) out[k++] = OutArray{{ctx->adj_nbar, ctx->adj_nbar, ctx->adj_nbar}, 1, n_bar};
+  if (zb_bar) out[k++] = OutArray{{ctx->adj_zbbar, ctx->adj_zbbar, ctx->adj_zbbar}, 1, zb_bar};
+  int rc = k ? perm_out_all(ctx, out, k) : HG_OK;
+  if (!rc && inletQ_bar) rc = download(ctx, inletQ_bar, ctx->adj_Qbar, size_t(ctx->n_inlet));
   return rc;
 }
 
@@ -5277,6 +5467,8 @@ int hg_rhs_vjp(hg_ctx* ctx, const double* Q, const double* params, int64_t n_par
 int64_t auto_kck(hg_ctx* ctx, int64_t nsteps) {
   const double N = double(ctx->N);
   const double per_step = 24.0 * N + N + 8.0 * std::max<int32_t>(ctx->n_inlet, 1) + (ctx->ude_prec ? 8.0 * N : 0.0);
+  if (int64_t(ctx->adj_seg_cap[0]) >= nsteps && (!ctx->ude_prec || int64_t(ctx->adj_nseg_cap[0]) >= nsteps))
+    return nsteps;  // an earlier call took the room
   size_t fr = 0, tot = 0;
   double avail = 0.0;
   if (hipMemGetInfo(&fr, &tot) == hipSuccess) avail = double(fr);
@@ -5392,9 +5584,8 @@ int hg_grad_probes(hg_ctx* ctx, const double* Q0, const double* params, int64_t 
                        int(ctx->Nm), ctx->probe_i, ctx->probe_d, ctx->st[ctx->cur][0], ctx->hstill, ctx->zb,
                        ctx->probe_d + cap);
     HG_TRY(hipGetLastError());
-    HG_TRY(hipMemcpyAsync(r.data(), ctx->probe_d + cap, n_probe * sizeof(double), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    HG_TRY(hipStreamSynchronize(ctx->stream));
+    rc = download(ctx, r.data(), ctx->probe_d + cap, size_t(n_probe));
+    if (rc) return rc;
   }
   // the loss, and its cotangent of the final state: 2 r at each probe cell
   // (summed over repeated probes, in probe order), zero elsewhere
