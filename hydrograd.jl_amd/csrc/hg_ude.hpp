@@ -120,21 +120,41 @@ struct UdeArgs {
   double hsmall;
 };
 
+// What the features of one cell are formed from.
+struct UdeRaw {
+  double xi, hstill, qx, qy, zb;
+  int set;
+};
+
+__device__ __forceinline__ UdeRaw ude_raw(const UdeArgs& a, int i, bool wanted) {
+  UdeRaw r{0.0, 0.0, 0.0, 0.0, 0.0, 0};
+  if (wanted && i < a.N) {
+    const int m = i % a.Nm;
+    r.xi = a.xi[i];
+    r.hstill = a.hstill[m];
+    r.qx = a.qx[i];
+    r.qy = a.qy[i];
+    r.zb = a.zb[m];
+    if (a.set_of_cell) r.set = a.set_of_cell[i];
+  }
+  return r;
+}
+
 // Features of one cell (double), see the header comment.
-__device__ __forceinline__ void ude_features(const UdeArgs& a, int i, double& h, double& u, double& v, double& um,
-                                             bool& wet) {
-  const double xi = a.xi[i];
-  h = xi + a.hstill[i % a.Nm];
-  double hu = a.qx[i], hv = a.qy[i];
-  wet = h > a.hsmall;
+__device__ __forceinline__ void ude_features(const UdeRaw& r, double hsmall, double& h, double& u, double& v,
+                                             double& um, bool& wet) {
+  h = r.xi + r.hstill;
+  double hu = r.qx, hv = r.qy;
+  wet = h > hsmall;
   if (!wet) {
-    h = a.hsmall;
+    h = hsmall;
     hu = 0.0;
     hv = 0.0;
   }
-  u = hu / h;
-  v = hv / h;
-  um = sqrt(u * u + v * v + EPS);
+  const double rh = rcp_est(h);
+  u = div_est(hu, h, rh);
+  v = div_est(hv, h, rh);
+  um = sqrt_pos(u * u + v * v + EPS);
 }
 
 }  // namespace hg

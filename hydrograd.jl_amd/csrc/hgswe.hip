@@ -1153,75 +1153,85 @@ std::vector<int32_t> morton_perm(const std::vector<int64_t>& seg, const double* 
 
 // ---- UDE closure for Manning's n (matrix cores; one wave = 64 cells) ----
 
-// Hidden layers of 64 cells: features F[64][4] (column 3 = 1) -> A1 =
-// tanh(F [W1 | b1]^T) -> A2 = tanh(A1 W2^T + b2), each layer as 16-row blocks
-// of 16x16x4 matrix-core products (b2 as their initial accumulator); results
-// land in LDS row-major [cell][unit].
+// Activations lie in LDS as one row of 16 units per cell.  A row's stride of
+// 20 floats or 18 doubles keeps its 16-byte alignment and gives every access
+// below distinct banks: a wave's own rows (lane = cell, 16 lanes to a bank at
+// a stride of 16) and the 16 x 4 blocks of the matrix-core operands alike.
+// With it and the operands kept in registers (k_ude_vjp), 1.5M cells in 32
+// sets: k_ude_n 39 -> 36 us, k_ude_vjp 108 -> 91 us (its 100 matrix-core
+// products per 64 cells take 31 us of it, its vector instructions 36).
 template <class T>
-__device__ __forceinline__ void ude_hidden(const T* __restrict__ W, const T* F, T* A1, T* A2, int l) {
+constexpr int kUdeLd = sizeof(T) == 4 ? 20 : 18;
+
+// The cell of a 16-cell block in row i of its matrix-core products, chosen so
+// that lane (col, kq) receives in element r = 0..3 the result of cell
+// 4 r + kq of the block: as step k = 4 rb + r of a sum over the 64 cells takes
+// cells 4 k + kq, the received values are its operands as they are.
+template <class T>
+__device__ __forceinline__ int ude_row_cell(int i) {
+  return sizeof(T) == 4 ? 4 * (i & 3) + (i >> 2) : i;
+}
+
+// One weight set held in registers, laid out for the lane's share of the
+// matrix-core operands: b1 joins W1 as the column of the constant feature.
+template <class T>
+struct UdeRegs {
+  T w1, w2[4], b2;
+  __device__ __forceinline__ void load(const T* __restrict__ W, int col, int kq) {
+    w1 = kq < 3 ? W[hg::kUdeW1 + col * 3 + kq] : W[hg::kUdeB1 + col];  // [W1 | b1][j][k]
+    for (int kc = 0; kc < 4; ++kc) w2[kc] = W[hg::kUdeW2 + col * 16 + 4 * kc + kq];  // W2[j][4 kc + k]
+    b2 = W[hg::kUdeB2 + col];
+  }
+};
+
+// Hidden layers of the first ROWS cells (32 or 64) of a chunk: features
+// F[64][4] (column 3 = 1) -> A1 = tanh(F [W1 | b1]^T) -> A2 = tanh(A1 W2^T +
+// b2), each layer as 16-row blocks of 16x16x4 matrix-core products (b2 as
+// their initial accumulator); results land in LDS, and in the lane's a1, a2
+// (element r of block rb: unit col of cell 16 rb + 4 r + kq).  A1 and A2 may
+// be one array: a block's rows are read before they are written again.  A
+// cell's values do not depend on ROWS.
+template <class T, int ROWS = 64>
+__device__ __forceinline__ void ude_hidden(const UdeRegs<T>& R, const T* F, T* A1, T* A2, int l, T (&a1)[ROWS / 4],
+                                           T (&a2)[ROWS / 4]) {
   using M = hg::Mfma<T>;
-  const int col = l & 15, kq = l >> 4;
-  for (int rb = 0; rb < 4; ++rb) {
-    const T av = F[(16 * rb + col) * 4 + kq];                                    // F[16 rb + i][k]
-    const T bv = kq < 3 ? W[hg::kUdeW1 + col * 3 + kq] : W[hg::kUdeB1 + col];  // [W1 | b1][j][k]
+  constexpr int LD = kUdeLd<T>;
+  const int col = l & 15, kq = l >> 4, rc = ude_row_cell<T>(col);
+#pragma unroll
+  for (int rb = 0; rb < ROWS / 16; ++rb) {
     typename M::V acc = {T(0), T(0), T(0), T(0)};
-    acc = M::op(av, bv, acc);
-    for (int r = 0; r < 4; ++r) A1[(16 * rb + M::row(kq, r)) * 16 + col] = M::tanh_(acc[r]);
+    acc = M::op(F[(16 * rb + rc) * 4 + kq], R.w1, acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) A1[(16 * rb + 4 * r + kq) * LD + col] = a1[4 * rb + r] = M::tanh_(acc[r]);
   }
   hg::wave_sync();
-  const T b2 = W[hg::kUdeB2 + col];
-  for (int rb = 0; rb < 4; ++rb) {
-    typename M::V acc = {b2, b2, b2, b2};
-    for (int kc = 0; kc < 4; ++kc) {
-      const T av = A1[(16 * rb + col) * 16 + 4 * kc + kq];           // A1[16 rb + i][4 kc + k]
-      const T bv = W[hg::kUdeW2 + col * 16 + 4 * kc + kq];           // W2[j][4 kc + k]
-      acc = M::op(av, bv, acc);
-    }
-    for (int r = 0; r < 4; ++r) A2[(16 * rb + M::row(kq, r)) * 16 + col] = M::tanh_(acc[r]);
+#pragma unroll
+  for (int rb = 0; rb < ROWS / 16; ++rb) {
+    typename M::V acc = {R.b2, R.b2, R.b2, R.b2};
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc) acc = M::op(A1[(16 * rb + rc) * LD + 4 * kc + kq], R.w2[kc], acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) A2[(16 * rb + 4 * r + kq) * LD + col] = a2[4 * rb + r] = M::tanh_(acc[r]);
   }
   hg::wave_sync();
+}
+
+// A wave-uniform weight set, read through the scalar cache (constant while a
+// kernel that reads it runs).
+template <class T>
+using UdeConst = const __attribute__((address_space(4))) T*;
+template <class T>
+__device__ __forceinline__ UdeConst<T> ude_const(const T* W) {
+  return (UdeConst<T>)(reinterpret_cast<uintptr_t>(W));
 }
 
 // Output layer of cell l: z3 = b3 + sum_j A2[l][j] W3[j].
 template <class T>
-__device__ __forceinline__ T ude_out(const T* __restrict__ W, const T* A2, int l) {
+__device__ __forceinline__ T ude_out(UdeConst<T> W, const T* A2, int l) {
   T z3 = W[hg::kUdeB3];
-  for (int j = 0; j < 16; ++j) z3 = hg::Mfma<T>::fma_(A2[l * 16 + j], W[hg::kUdeW3 + j], z3);
+#pragma unroll
+  for (int j = 0; j < 16; ++j) z3 = hg::Mfma<T>::fma_(A2[l * kUdeLd<T> + j], W[hg::kUdeW3 + j], z3);
   return z3;
-}
-
-// One weight set held in registers, laid out for the lane's share of the
-// matrix-core operands (see ude_hidden) and for the output layer.
-template <class T>
-struct UdeRegs {
-  T w1, w2[4], b2, w3[16], b3;
-  __device__ __forceinline__ void load(const T* __restrict__ W, int col, int kq) {
-    w1 = kq < 3 ? W[hg::kUdeW1 + col * 3 + kq] : W[hg::kUdeB1 + col];  // [W1 | b1]
-    for (int kc = 0; kc < 4; ++kc) w2[kc] = W[hg::kUdeW2 + col * 16 + 4 * kc + kq];
-    b2 = W[hg::kUdeB2 + col];
-    for (int j = 0; j < 16; ++j) w3[j] = W[hg::kUdeW3 + j];
-    b3 = W[hg::kUdeB3];
-  }
-};
-
-// ude_hidden with the weights in registers, for the first ROWS cells (16,
-// 32, 48 or 64) of the chunk; each cell's values do not depend on ROWS.
-template <class T, int ROWS = 64>
-__device__ __forceinline__ void ude_hidden_r(const UdeRegs<T>& R, const T* F, T* A1, T* A2, int l) {
-  using M = hg::Mfma<T>;
-  const int col = l & 15, kq = l >> 4;
-  for (int rb = 0; rb < ROWS / 16; ++rb) {
-    typename M::V acc = {T(0), T(0), T(0), T(0)};
-    acc = M::op(F[(16 * rb + col) * 4 + kq], R.w1, acc);
-    for (int r = 0; r < 4; ++r) A1[(16 * rb + M::row(kq, r)) * 16 + col] = M::tanh_(acc[r]);
-  }
-  hg::wave_sync();
-  for (int rb = 0; rb < ROWS / 16; ++rb) {
-    typename M::V acc = {R.b2, R.b2, R.b2, R.b2};
-    for (int kc = 0; kc < 4; ++kc) acc = M::op(A1[(16 * rb + col) * 16 + 4 * kc + kq], R.w2[kc], acc);
-    for (int r = 0; r < 4; ++r) A2[(16 * rb + M::row(kq, r)) * 16 + col] = M::tanh_(acc[r]);
-  }
-  hg::wave_sync();
 }
 
 // n = 0.01 + softplus(MLP(features)) for every cell.  Each wave walks
@@ -1230,30 +1240,29 @@ __device__ __forceinline__ void ude_hidden_r(const UdeRegs<T>& R, const T* F, T*
 // use several sets takes one pass per set (the matrix-core products need one
 // set across the wave).
 template <class T, int WPB, int CH = 64>
-__global__ __launch_bounds__(64 * WPB) void k_ude_n(hg::UdeArgs a) {
+__global__ __launch_bounds__(64 * WPB, sizeof(T) == 4 ? 5 : 2) void k_ude_n(hg::UdeArgs a) {
   static_assert(CH == 32 || CH == 64, "chunk of 32 or 64 cells");
-  __shared__ T Fs[WPB][CH * 4];
-  __shared__ T A1s[WPB][CH * 16];
-  __shared__ T A2s[WPB][CH * 16];
+  __shared__ __align__(16) T Fs[WPB][CH * 4];
+  __shared__ __align__(16) T As[WPB][CH * kUdeLd<T>];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   const int col = l & 15, kq = l >> 4;
   T* F = Fs[w];
-  T* A1 = A1s[w];
-  T* A2 = A2s[w];
+  T* A = As[w];
   const int nchunks = (a.N + CH - 1) / CH;
   UdeRegs<T> R;
   int cur = -1;
-  for (int ch = blockIdx.x * WPB + w; ch < nchunks; ch += gridDim.x * WPB) {
+  const int stride = gridDim.x * WPB;
+  hg::UdeRaw nx = hg::ude_raw(a, (blockIdx.x * WPB + w) * CH + l, l < CH);
+  for (int ch = blockIdx.x * WPB + w; ch < nchunks; ch += stride) {
     const int i = ch * CH + l;
     const bool valid = l < CH && i < a.N;
-    double h = 0.0, u = 0.0, v = 0.0, um = 0.0, zb = 0.0;
+    const hg::UdeRaw raw = nx;
+    if (ch + stride < nchunks) nx = hg::ude_raw(a, i + stride * CH, l < CH);  // in flight over this chunk's passes
+    double h = 0.0, u = 0.0, v = 0.0, um = 0.0;
     bool wet = false;
-    int set = 0;
-    if (valid) {
-      hg::ude_features(a, i, h, u, v, um, wet);
-      zb = a.zb[i % a.Nm];
-      if (a.set_of_cell) set = a.set_of_cell[i];
-    }
+    const int set = raw.set;
+    const double zb = raw.zb;
+    if (valid) hg::ude_features(raw, a.hsmall, h, u, v, um, wet);
     if (l < CH) {  // F has CH rows
       F[l * 4 + 0] = T(h);
       F[l * 4 + 1] = T(um);
@@ -1271,13 +1280,10 @@ __global__ __launch_bounds__(64 * WPB) void k_ude_n(hg::UdeArgs a) {
         R.load(static_cast<const T*>(a.w) + size_t(s) * hg::kUdeW, col, kq);
         cur = s;
       }
-      ude_hidden_r<T, CH>(R, F, A1, A2, l);
-      if (mine) {
-        T z3 = R.b3;
-        for (int j = 0; j < 16; ++j) z3 = hg::Mfma<T>::fma_(A2[l * 16 + j], R.w3[j], z3);
-        a.n[i] = 0.01 + double(hg::softplus<T>(z3));
-      }
-      hg::wave_sync();  // the next pass rewrites A1, A2
+      T a1[CH / 4], a2[CH / 4];
+      ude_hidden<T, CH>(R, F, A, A, l, a1, a2);
+      if (mine) a.n[i] = 0.01 + double(hg::softplus<T>(ude_out<T>(ude_const(static_cast<const T*>(a.w) + size_t(s) * hg::kUdeW), A, l)));
+      hg::wave_sync();  // the next pass rewrites A
     }
   }
 }
@@ -1335,39 +1341,47 @@ __device__ __forceinline__ void ude_flush(double* __restrict__ wp, const typenam
 // as k_ude_n).  The weight cotangents are sums over cells on the matrix cores
 // (K = cells); consecutive passes of one set keep adding into the same
 // accumulators, which go into the (block, set) slot when the set changes and
-// at the end.  A chunk's inputs are read before its passes, its
-// state-cotangent values after them.  The backward activations overwrite the forward ones
-// once read: Z2 replaces A2, then Z1 replaces A1.
+// at the end.  Their operands are the activations and cotangents as the lane
+// received or formed them (ude_row_cell); LDS only carries what another lane
+// reads: each layer's rows for the next layer's products and for the cell's
+// own sums.  Z2 = z3bar W3 (1 - A2^2) replaces A2 there, Z1 = A1bar (1 - A1^2)
+// replaces A1.  The next chunk's inputs are in flight over a chunk's passes.
 template <class T>
 __global__ __launch_bounds__(64, sizeof(T) == 4 ? 3 : 1) void k_ude_vjp(hg::UdeArgs a) {
   using M = hg::Mfma<T>;
-  __shared__ T F[64 * 4];
-  __shared__ T A1[64 * 16];  // A1, then Z1 = A1bar (1 - A1^2)
-  __shared__ T A2[64 * 16];  // A2, then Z2 = z3bar W3 (1 - A2^2)
-  __shared__ T Z3[64];
+  constexpr int LD = kUdeLd<T>;
+  __shared__ __align__(16) T F[64 * 4];
+  __shared__ __align__(16) T A1[64 * LD];
+  __shared__ __align__(16) T A2[64 * LD];
+  __shared__ __align__(16) T Z3[64];
   const int l = threadIdx.x;
-  const int col = l & 15, kq = l >> 4;
+  const int col = l & 15, kq = l >> 4, rc = ude_row_cell<T>(col);
   const int nchunks = (a.N + 63) / 64;
   const int ch0 = int(blockIdx.x) * a.cpb, ch1 = min(nchunks, ch0 + a.cpb);
   typename M::V w1 = {T(0), T(0), T(0), T(0)}, w2 = w1, w3 = w1;
-  double b3 = 0.0;
+  double b3 = 0.0;    // this lane's share
   int acc_set = -1;  // set of the running accumulators (-1: none yet)
+  UdeRegs<T> R{};
+  T w2t[4] = {T(0), T(0), T(0), T(0)}, w3c = T(0);  // W2[4 kc + k][j], W3[j]
+  auto flush = [&] {
+    double b3s = b3;
+    for (int m = 32; m > 0; m >>= 1) b3s += __shfl_xor(b3s, m, 64);
+    ude_flush<T>(a.wpart + size_t(ude_slot(a, acc_set)) * hg::kUdeW, w1, w2, w3, b3s, l);
+  };
+  hg::UdeRaw nx = hg::ude_raw(a, ch0 * 64 + l, true);
   for (int ch = ch0; ch < ch1; ++ch) {
     const int i = ch * 64 + l;
     const bool valid = i < a.N;
-    double h = 0.0, u = 0.0, v = 0.0, um = 0.0, zb = 0.0;
-    T nb = T(0);
+    const hg::UdeRaw raw = nx;
+    const T nb = valid ? T(a.nbar[i]) : T(0);
+    if (ch + 1 < ch1) nx = hg::ude_raw(a, i + 64, true);
+    double h = 0.0, u = 0.0, v = 0.0, um = 0.0;
     bool wet = false;
-    int set = 0;
-    if (valid) {
-      hg::ude_features(a, i, h, u, v, um, wet);
-      zb = a.zb[i % a.Nm];
-      if (a.set_of_cell) set = a.set_of_cell[i];
-      nb = T(a.nbar[i]);
-    }
+    const int set = raw.set;
+    if (valid) hg::ude_features(raw, a.hsmall, h, u, v, um, wet);
     F[l * 4 + 0] = T(h);
     F[l * 4 + 1] = T(um);
-    F[l * 4 + 2] = T(zb);
+    F[l * 4 + 2] = T(raw.zb);
     F[l * 4 + 3] = T(1);  // the bias column of layer 1
     hg::wave_sync();
     T g0 = T(0), g1 = T(0), g2 = T(0);  // the cell's feature cotangents, from its set's pass
@@ -1377,91 +1391,84 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 3 : 1) void k_ude_vjp(hg::UdeA
       const int s = __builtin_amdgcn_readfirstlane(__shfl(set, lead, 64));  // wave-uniform: scalar weight loads
       const bool mine = valid && set == s;
       pending &= ~uint64_t(__ballot(mine));
+      const T* W = static_cast<const T*>(a.w) + size_t(s) * hg::kUdeW;
       if (s != acc_set) {
-        if (acc_set >= 0) ude_flush<T>(a.wpart + size_t(ude_slot(a, acc_set)) * hg::kUdeW, w1, w2, w3, b3, l);
+        if (acc_set >= 0) flush();
         w1 = typename M::V{T(0), T(0), T(0), T(0)};
         w2 = w1;
         w3 = w1;
         b3 = 0.0;
         acc_set = s;
+        R.load(W, col, kq);
+        for (int kc = 0; kc < 4; ++kc) w2t[kc] = W[hg::kUdeW2 + (4 * kc + kq) * 16 + col];
+        w3c = W[hg::kUdeW3 + col];
       }
-      const T* W = static_cast<const T*>(a.w) + size_t(s) * hg::kUdeW;
-      ude_hidden<T>(W, F, A1, A2, l);
+      T a1[16], a2[16];
+      ude_hidden<T>(R, F, A1, A2, l, a1, a2);
       // output layer and softplus, lane = cell; cells of other sets carry a zero cotangent
-      const T z3 = ude_out<T>(W, A2, l);
+      const UdeConst<T> Wc = ude_const(W);
+      const T z3 = ude_out<T>(Wc, A2, l);
       const T z3b = mine ? nb * hg::sigmoid<T>(z3) : T(0);
+      b3 += double(z3b);
       Z3[l] = z3b;
       hg::wave_sync();
       // Weight cotangents as sums over the cells on the matrix cores (K = cells):
       // w3 column 1: W3bar = A2^T Z3; column 0: b2bar = Z2^T 1; w2: W2bar = Z2^T A1;
-      // w1: [W1bar | b1bar] = Z1^T [F | 1]; b3bar = sum of Z3 by a fixed xor tree.
-      for (int kc = 0; kc < 16; ++kc) {
-        const int c = 4 * kc + kq;  // cell of this lane's K-row
-        w3 = M::op(A2[c * 16 + col], col == 1 ? Z3[c] : T(0), w3);
+      // w1: [W1bar | b1bar] = Z1^T [F | 1].
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const T zc = Z3[4 * k + kq];
+        w3 = M::op(a2[k], col == 1 ? zc : T(0), w3);
+        a2[k] = (zc * w3c) * M::fma_(-a2[k], a2[k], T(1));  // Z2
+        A2[(4 * k + kq) * LD + col] = a2[k];
       }
       hg::wave_sync();
-      for (int j = 0; j < 16; ++j) {  // Z2 over A2, own row
-        const T a2 = A2[l * 16 + j];
-        A2[l * 16 + j] = (z3b * W[hg::kUdeW3 + j]) * M::fma_(-a2, a2, T(1));
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        w2 = M::op(a2[k], a1[k], w2);
+        w3 = M::op(a2[k], T(col == 0), w3);
       }
-      hg::wave_sync();
-      const T* Z2 = A2;
-      for (int kc = 0; kc < 16; ++kc) {
-        const int c = 4 * kc + kq;
-        const T z2 = Z2[c * 16 + col];
-        w2 = M::op(z2, A1[c * 16 + col], w2);
-        w3 = M::op(z2, T(col == 0), w3);
-      }
-      // A1bar = Z2 W2 (rows = cells)
-      typename M::V ab[4];
-      for (int rb = 0; rb < 4; ++rb) {
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) {  // A1bar = Z2 W2 (rows = cells), then Z1 over A1
         typename M::V acc = {T(0), T(0), T(0), T(0)};
-        for (int kc = 0; kc < 4; ++kc) {
-          const T av = Z2[(16 * rb + col) * 16 + 4 * kc + kq];    // Z2[16 rb + i][4 kc + k]
-          const T bv = W[hg::kUdeW2 + (4 * kc + kq) * 16 + col];  // W2[4 kc + k][j]
-          acc = M::op(av, bv, acc);
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc) acc = M::op(A2[(16 * rb + rc) * LD + 4 * kc + kq], w2t[kc], acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int k = 4 * rb + r;
+          a1[k] = acc[r] * M::fma_(-a1[k], a1[k], T(1));
+          A1[(4 * k + kq) * LD + col] = a1[k];
         }
-        ab[rb] = acc;
       }
       hg::wave_sync();
-      for (int rb = 0; rb < 4; ++rb)  // Z1 = A1bar (1 - A1^2) over A1
-        for (int r = 0; r < 4; ++r) {
-          const int row = 16 * rb + M::row(kq, r);
-          const T a1 = A1[row * 16 + col];
-          A1[row * 16 + col] = ab[rb][r] * M::fma_(-a1, a1, T(1));
-        }
-      hg::wave_sync();
-      const T* Z1 = A1;
       // feature cotangents -> state cotangent (lane = cell)
       T fb0 = T(0), fb1 = T(0), fb2 = T(0);
+#pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const T z = Z1[l * 16 + j];
-        fb0 = M::fma_(z, W[hg::kUdeW1 + j * 3 + 0], fb0);
-        fb1 = M::fma_(z, W[hg::kUdeW1 + j * 3 + 1], fb1);
-        fb2 = M::fma_(z, W[hg::kUdeW1 + j * 3 + 2], fb2);
+        const T z = A1[l * LD + j];
+        fb0 = M::fma_(z, Wc[hg::kUdeW1 + j * 3 + 0], fb0);
+        fb1 = M::fma_(z, Wc[hg::kUdeW1 + j * 3 + 1], fb1);
+        fb2 = M::fma_(z, Wc[hg::kUdeW1 + j * 3 + 2], fb2);
       }
       if (mine) {
         g0 = fb0;
         g1 = fb1;
         g2 = fb2;
       }
-      for (int kc = 0; kc < 16; ++kc) {
-        const int c = 4 * kc + kq;
-        w1 = M::op(Z1[c * 16 + col], col < 3 ? F[c * 4 + col] : T(col == 3), w1);
-      }
-      double z3s = double(Z3[l]);
-      for (int m = 32; m > 0; m >>= 1) z3s += __shfl_xor(z3s, m, 64);
-      b3 += z3s;
+#pragma unroll
+      for (int k = 0; k < 16; ++k)
+        w1 = M::op(a1[k], col < 3 ? F[(4 * k + kq) * 4 + (col & 3)] : T(col == 3), w1);
       hg::wave_sync();  // the next pass rewrites A1, A2 and Z3
     }
     if (valid) {  // all four read before any is written: one round trip
       const double o0 = a.ox[i], o1 = a.oqx[i], o2 = a.oqy[i], oz = a.zbbar ? a.zbbar[i] : 0.0;
       double xib = 0.0, qxb = 0.0, qyb = 0.0;
       if (wet) {  // h = xi + h_still, |u| = sqrt(u^2 + v^2 + eps), u = q_x / h, v = q_y / h
-        const double ub = double(g1) * u / um, vb = double(g1) * v / um;
-        xib = double(g0) - (ub * u + vb * v) / h;
-        qxb = ub / h;
-        qyb = vb / h;
+        const double rum = hg::rcp_est(um), rh = hg::rcp_est(h);
+        const double ub = hg::div_est(double(g1) * u, um, rum), vb = hg::div_est(double(g1) * v, um, rum);
+        xib = double(g0) - hg::div_est(ub * u + vb * v, h, rh);
+        qxb = hg::div_est(ub, h, rh);
+        qyb = hg::div_est(vb, h, rh);
       }
       const double zbb = double(g2);
       a.ox[i] = o0 + xib;
@@ -1470,7 +1477,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 3 : 1) void k_ude_vjp(hg::UdeA
       if (a.zbbar) a.zbbar[i] = oz + zbb;
     }
   }
-  if (acc_set >= 0) ude_flush<T>(a.wpart + size_t(ude_slot(a, acc_set)) * hg::kUdeW, w1, w2, w3, b3, l);
+  if (acc_set >= 0) flush();
 }
 
 // wbar[s][k] += the sum of the slots of weight set s (set_start[s] ..
