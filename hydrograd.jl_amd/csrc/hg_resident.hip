@@ -124,15 +124,16 @@ template <class T, int MD, bool SPLIT, int NM>
 struct ResTile {
   static constexpr int TT = kResT, NT = res_threads(MD, SPLIT), W = Words<T>::W, NC = 3 * W;
   static constexpr int kRows = NM ? 10 : 9;  // xi, h, hu, hv, zb, u, v, s, p and, when it changes, n
+  static constexpr int kNet = NM == RES_N_NET ? W * kLuxPadN : 0;  // the network's weights (and tangents)
 
   static constexpr size_t lds_bytes() {
-    return size_t((kRows + 3 * MD) * W * TT + W * kTileInlets + (2 + W) * kResIn) * sizeof(double) +
+    return size_t((kRows + 3 * MD) * W * TT + W * kTileInlets + (2 + W) * kResIn + kNet) * sizeof(double) +
            (kResIn + 1) * sizeof(int32_t);
   }
 
   const TileArgs& a;
   const ResArgs& R;
-  double *C, *FL, *tA, *in_c;
+  double *C, *FL, *tA, *net, *in_c;
   int32_t *in_i, *stop;
   int t, tid, i, d, it_code, type, ref, in0, in1, bl0, fl0, fl1;
   bool own, pub, has;
@@ -166,7 +167,7 @@ struct ResTile {
     }
     T f[3];
     lux_features<T>(R.net, xi, qx, qy, hsc, a.hsmall, ksc, f);
-    return lux_eval<4, T>(R.net, R.net_w, f, R.net_dw);
+    return lux_eval<4, T>(R.net, LuxPad{net, net + kLuxPadN, R.net.n_hidden}, f);
   }
   __device__ __forceinline__ bool gives_n() const { return NM == RES_N_LAW || R.net.choice != LUX_FLOW_RESISTANCE; }
 
@@ -174,7 +175,8 @@ struct ResTile {
     C = lds;
     FL = C + kRows * W * TT;
     tA = FL + 3 * MD * W * TT;
-    in_c = tA + W * kTileInlets;
+    net = tA + W * kTileInlets;
+    in_c = net + kNet;
     in_i = reinterpret_cast<int32_t*>(in_c + (2 + W) * kResIn);
     stop = in_i + kResIn;
     t = blockIdx.x;
@@ -239,6 +241,10 @@ struct ResTile {
         in_c[kResIn + f] = a.hstill[c];
         for (int w = 0; w < W; ++w) in_c[(2 + w) * kResIn + f] = word(nc, w);
       }
+    }
+    if (NM == RES_N_NET) {
+      lux_pad_fill(R.net, R.net_w, net, tid, NT);
+      if (W > 1) lux_pad_fill(R.net, R.net_dw, net + kLuxPadN, tid, NT);
     }
     if (tid == 0) *stop = 0;
     __syncthreads();
@@ -628,30 +634,106 @@ __global__ __launch_bounds__(res_threads(MD, true), 2) void k_tsit5_run(TileArgs
 constexpr int adj_run_base_doubles(int MD) {  // without the network's values
   return (kAdjRows + 4 * MD) * kResT + 512 + kTileInlets + (kResT + 2) / 2;
 }
+template <int MD>
+__device__ __forceinline__ int32_t* adj_run_stop(double* lds) {
+  return reinterpret_cast<int32_t*>(lds + (kAdjRows + 4 * MD) * kResT + 512 + kTileInlets) + kResT;
+}
+// The network's derivatives are formed by a work-item of their own for each
+// cell, one step ahead of the cells' and faces' (adj_run_net).
+constexpr int adj_run_threads(int MD, int NM) { return res_items(MD) + (NM == RES_N_NET ? kResT : 0); }
+// LDS of the network: two values per weight and cell, four per cell, the padded weights.
+constexpr int adj_run_net_doubles(int P) { return 2 * P * kResT + 4 * kResT + kLuxPadN; }
 
+// The network's part of a resident reverse run, by the tile's last kResT
+// work-items (cell c): for every step, the derivatives of the network's output
+// by the weights (J, one value per weight and cell) and by the cell's state
+// (Cs), from the recorded state alone; then the sums over the steps of J times
+// the output's cotangent, which the cell's work-item leaves in Ob.  The forward
+// pass of the next step runs while the cells finish theirs.  Takes every
+// barrier that the tile's other work-items take.  A step of the [3, 3] network
+// on 180 cells takes 10.1 us, and took 12.9 with the derivatives formed by the
+// cells' own work-items between the faces and the sums.
+template <int NH>
+__device__ __forceinline__ bool adj_run_net(const AdjArgs& a, const AdjRunArgs& R, const LuxPad& pad, double* J,
+                                            double* Wsum, double* Cs, const double* Ob, const int32_t* stop, int i,
+                                            bool own, int n_in) {
+  constexpr int T = kResT;
+  const int64_t N = a.N;
+  const int ns = R.net.choice == LUX_MANNING_H ? 1 : 3, P = R.net.P;
+  const double hs = own ? a.hstill[i] : 0.0, ksc = R.ks && own ? R.ks[i] : 1.0;
+  double q[3] = {0.0, 0.0, 0.0}, nx[3] = {0.0, 0.0, 0.0};  // the step's recorded state, and the next one's
+  auto read_ahead = [&](int64_t k) {
+    if (own)
+      for (int c = 0; c < 3; ++c) nx[c] = R.rec[(k * 3 + c) * N + i];
+  };
+  LuxPass<4, NH> pass;
+  auto forward = [&] {
+    double f[3];
+    lux_features<double>(R.net, q[0], q[1], q[2], hs, a.hsmall, ksc, f);
+    lux_pass<4, NH>(R.net, pad, f, pass);
+  };
+  auto add = [&] {
+    const double ob = Ob[0];
+#pragma unroll 8
+    for (int p = 0; p < P; ++p) Wsum[p * T] += ob * J[p * T];
+  };
+  if (own)
+    for (int p = 0; p < P; ++p) Wsum[p * T] = 0.0;
+  __syncthreads();  // the padded weights
+  read_ahead(R.ns - 1);
+  for (int64_t r = -1; r < R.ns; ++r) {
+    if (r >= 0) __syncthreads();  // the last step's Ob is there, its Cs has been read
+    if (r >= 0 && own) {
+      if (r > 0) add();
+      double df[3];
+      lux_jacobian<4, NH>(R.net, pad, pass, J, T, df);
+      for (int c = 0; c < ns; ++c) {
+        const Dual1 x0(q[0], c == 0 ? 1.0 : 0.0), x1(q[1], c == 1 ? 1.0 : 0.0), x2(q[2], c == 2 ? 1.0 : 0.0);
+        Dual1 fd[3];
+        lux_features<Dual1>(R.net, x0, x1, x2, hs, a.hsmall, ksc, fd);
+        Cs[c * T] = df[0] * fd[0].d + df[1] * fd[1].d + df[2] * fd[2].d;
+      }
+      for (int c = ns; c < 3; ++c) Cs[c * T] = 0.0;
+    }
+    if (r >= 0) {
+      __syncthreads();
+      if (*stop) return false;
+    }
+    if (r + 1 < R.ns) {  // the next step's state and forward pass
+      for (int c = 0; c < 3; ++c) q[c] = nx[c];
+      if (r + 2 < R.ns) read_ahead(R.ns - 3 - r);
+      if (own) forward();
+    }
+    for (int k = 0; r >= 0 && k < n_in; ++k) {
+      __syncthreads();
+      if (*stop) return false;
+      for (int b = 0; b < 3; ++b) __syncthreads();
+    }
+  }
+  __syncthreads();  // the last Ob
+  if (own) add();
+  return true;
+}
+
+// The cells and faces of a tile, by its first res_items(MD) work-items; false
+// when a wait ran out.
 template <int MD, int NM>
-__global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunArgs R) {
+__device__ __forceinline__ bool adj_run_cells(AdjArgs a, const AdjRunArgs& R, double* lds) {
   constexpr int T = kResT, NT = res_items(MD);
-  extern __shared__ double lds[];
   double* C = lds;                                         // kAdjRows x T
   double* S = lds + kAdjRows * T;                          // 4 x MD x T
   double* sA = S + 4 * MD * T;                             // 256
   double* sQ = sA + 256;                                   // 256
   double* qa = sQ + 256;                                   // kTileInlets: the inlets' discharge cotangents
   int32_t* Xm = reinterpret_cast<int32_t*>(qa + kTileInlets);  // T
-  int32_t* stop = Xm + T;
+  int32_t* stop = adj_run_stop<MD>(lds);
   const int t = blockIdx.x, tid = threadIdx.x, i = t * T + tid;
   const bool own = tid < T && i < a.N;
   const int64_t N = a.N;
   const double hsmall = a.hsmall;
-  // the network: per weight and cell, its derivative at the step and the run's sum
-  const int NP = NM == RES_N_NET ? R.net.P : 0;
-  double* J = lds + adj_run_base_doubles(MD) + tid;
-  double* Wsum = J + NP * T;
   const bool mag = NM == RES_N_NET && R.net.choice == LUX_FLOW_RESISTANCE;  // the output is the friction magnitude
-  if (own)
-    for (int p = 0; p < NP; ++p) Wsum[p * T] = 0.0;
-  const double ksc = NM && R.ks && own ? R.ks[i] : 1.0;
+  double* const Cs = lds + adj_run_base_doubles(MD) + 2 * (NM == RES_N_NET ? R.net.P : 0) * T + tid;  // see adj_run_net
+  const double ksc = NM == RES_N_LAW && R.ks && own ? R.ks[i] : 1.0;
   double hs = 0.0, zb = 0.0, n = 0.0, S0x = 0.0, S0y = 0.0, A = 1.0, dti = a.dt;
   double l0 = 0.0, l1 = 0.0, l2 = 0.0, nbar = 0.0, zbbar = 0.0, S0bx = 0.0, S0by = 0.0;
   int d = 0;
@@ -712,6 +794,7 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
     }
   };
   read_ahead(R.ns - 1);
+  if (NM == RES_N_NET) __syncthreads();
 
   for (int64_t r = 0; r < R.ns; ++r) {
     const int64_t k = R.ns - 1 - r;  // the step that is reversed
@@ -776,32 +859,16 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
         source_vjp(a.g, a.kn2, hsmall, me.xi, me.h, me.hu, me.hv, n, S0x, S0y, y1, y2, sxi, sh, sqx, sqy, sn, sS0x,
                    sS0y);
     }
-    // the closure's derivatives by the cell's state, and by the weights
+    // the law's derivatives by the cell's state
     double cs[3] = {0.0, 0.0, 0.0};
-    if (NM && own) {
+    if (NM == RES_N_LAW && own) {
       const double q[3] = {me.xi, sx1, sx2};
-      const int ns = NM == RES_N_LAW ? (R.law.kind == NLAW_H_UMAG_KS ? 3 : 1) : (R.net.choice == LUX_MANNING_H ? 1 : 3);
-      double df[3] = {0.0, 0.0, 0.0};
-      if (NM == RES_N_NET) {
-        double f[3];
-        lux_features<double>(R.net, q[0], q[1], q[2], hs, hsmall, ksc, f);
-        if (R.net.n_hidden == 1)
-          (void)lux_jacobian<4, 1>(R.net, R.net_w, f, J, T, df);
-        else
-          (void)lux_jacobian<4, 2>(R.net, R.net_w, f, J, T, df);
-      }
+      const int ns = R.law.kind == NLAW_H_UMAG_KS ? 3 : 1;
       for (int c = 0; c < ns; ++c) {
         const Dual1 x0(q[0], c == 0 ? 1.0 : 0.0), x1(q[1], c == 1 ? 1.0 : 0.0), x2(q[2], c == 2 ? 1.0 : 0.0);
-        double v;
-        if (NM == RES_N_LAW) {
-          Dual1 h, U;
-          nlaw_features<Dual1>(R.law, x0, x1, x2, hs, hsmall, h, U);
-          v = nlaw_eval<Dual1, false>(R.law, h, U, ksc, nullptr, nullptr, nullptr).d;
-        } else {
-          Dual1 fd[3];
-          lux_features<Dual1>(R.net, x0, x1, x2, hs, hsmall, ksc, fd);
-          v = df[0] * fd[0].d + df[1] * fd[1].d + df[2] * fd[2].d;
-        }
+        Dual1 h, U;
+        nlaw_features<Dual1>(R.law, x0, x1, x2, hs, hsmall, h, U);
+        const double v = nlaw_eval<Dual1, false>(R.law, h, U, ksc, nullptr, nullptr, nullptr).d;
         if (c == 0)
           cs[0] = v;
         else if (c == 1)
@@ -813,7 +880,7 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
     __syncthreads();
     if (*stop) {
       if (tid == 0) R.flag[2] = 1;
-      return;
+      return false;
     }
     double ob = 0.0;
     if (own) {
@@ -873,7 +940,7 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
       __syncthreads();
       if (*stop) {
         if (tid == 0) R.flag[2] = 1;
-        return;
+        return false;
       }
       if (tid < 128) {
         sA[tid] += sA[tid + 128];
@@ -907,6 +974,10 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
       }
       __syncthreads();  // sA / sQ reuse
     }
+    if (NM == RES_N_NET && own) {
+      for (int c = 0; c < 3; ++c) cs[c] = Cs[c * T];
+      Cs[3 * T] = ob;
+    }
     if (NM && own && ob != 0.0) {
       l0 += ob * cs[0];
       l1 += ob * cs[1];
@@ -921,10 +992,6 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
       res_put(o + 2 * N, __double_as_longlong(l2));
       for (int c = 0; c < 3; ++c) res_put(e + c * N, kResEmpty);
     }
-    if (NM == RES_N_NET && own) {
-#pragma unroll 8
-      for (int p = 0; p < NP; ++p) Wsum[p * T] += ob * J[p * T];
-    }
   }
   if (own) {
     a.ox[i] = l0;
@@ -937,23 +1004,52 @@ __global__ __launch_bounds__(res_items(MD), 2) void k_adj_run(AdjArgs a, AdjRunA
       R.o_S0bar[N + i] = S0by;
     }
   }
-  if (NM == RES_N_NET) {  // the tile's sum of each weight's cotangent, by a fixed tree
-    __syncthreads();
-    const double* W0 = lds + adj_run_base_doubles(MD) + NP * T;
-    for (int p = tid / 64; p < NP; p += NT / 64) {
-      const int l = tid & 63;
-      double v = (t * T + l < a.N ? W0[p * T + l] : 0.0) + (t * T + 64 + l < a.N ? W0[p * T + 64 + l] : 0.0);
-      for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w, 64);
-      if (l == 0) R.o_wpart[int64_t(p) * gridDim.x + t] = v;
-    }
-  }
   for (int sl = in0 + tid; sl < in1; sl += NT) {  // by the tile of the inlet's first face
     const int b = R.tile_in_list[sl];
     if (R.in_rec[R.in_off[b]].cell / T == t) R.o_Qbar[b] = qa[sl - in0];
   }
+  if (NM == RES_N_NET) __syncthreads();
+  return true;
 }
 
-size_t adj_run_lds_bytes(int MD, int P) { return (size_t(adj_run_base_doubles(MD)) + 2 * size_t(P) * kResT) * sizeof(double); }
+template <int MD, int NM>
+__global__ __launch_bounds__(adj_run_threads(MD, NM), 2) void k_adj_run(AdjArgs a, AdjRunArgs R) {
+  extern __shared__ double lds[];
+  if constexpr (NM != RES_N_NET) {
+    (void)adj_run_cells<MD, NM>(a, R, lds);
+  } else {
+    constexpr int T = kResT, NT = res_items(MD);
+    const int t = blockIdx.x, tid = threadIdx.x, P = R.net.P;
+    double* const J = lds + adj_run_base_doubles(MD);
+    double* const Wsum = J + P * T;
+    double* const Cs = Wsum + P * T;
+    double* const net = Cs + 4 * T;
+    lux_pad_fill(R.net, R.net_w, net, tid, adj_run_threads(MD, NM));
+    if (tid >= NT) {
+      const int c = tid - NT, i = t * T + c;
+      const LuxPad pad{net, nullptr, R.net.n_hidden};
+      const int n_in = R.n_inlet > 0 ? R.tile_in_off[t + 1] - R.tile_in_off[t] : 0;
+      const int32_t* stop = adj_run_stop<MD>(lds);
+      const bool done = R.net.n_hidden == 1
+                            ? adj_run_net<1>(a, R, pad, J + c, Wsum + c, Cs + c, Cs + 3 * T + c, stop, i, i < a.N, n_in)
+                            : adj_run_net<2>(a, R, pad, J + c, Wsum + c, Cs + c, Cs + 3 * T + c, stop, i, i < a.N, n_in);
+      if (!done) return;
+    } else if (!adj_run_cells<MD, NM>(a, R, lds)) {
+      return;
+    }
+    __syncthreads();
+    for (int p = tid / 64; p < P; p += adj_run_threads(MD, NM) / 64) {  // the tile's sum per weight, by a fixed tree
+      const int l = tid & 63;
+      double v = (t * T + l < a.N ? Wsum[p * T + l] : 0.0) + (t * T + 64 + l < a.N ? Wsum[p * T + 64 + l] : 0.0);
+      for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w, 64);
+      if (l == 0) R.o_wpart[int64_t(p) * gridDim.x + t] = v;
+    }
+  }
+}
+
+size_t adj_run_lds_bytes(int MD, int P) {
+  return (size_t(adj_run_base_doubles(MD)) + (P ? adj_run_net_doubles(P) : 0)) * sizeof(double);
+}
 
 // Tiles per CU: a tile's waves need not spread evenly over the four SIMDs (two
 // tiles of six waves each were not resident together where three waves fit
@@ -1013,10 +1109,10 @@ void with_tsit5(int md, int nm, F&& f) {
 template <int MD, int NM>
 struct AdjVariant {
   static int cap(int P, int ncu) {
-    return capacity(k_adj_run<MD, NM>, res_items(MD), adj_run_lds_bytes(MD, P), 2, ncu);
+    return capacity(k_adj_run<MD, NM>, adj_run_threads(MD, NM), adj_run_lds_bytes(MD, P), 2, ncu);
   }
   static void launch(hipStream_t st, int P, int ntiles, const AdjArgs& a, const AdjRunArgs& R) {
-    hipLaunchKernelGGL((k_adj_run<MD, NM>), dim3(ntiles), dim3(res_items(MD)), adj_run_lds_bytes(MD, P), st, a, R);
+    hipLaunchKernelGGL((k_adj_run<MD, NM>), dim3(ntiles), dim3(adj_run_threads(MD, NM)), adj_run_lds_bytes(MD, P), st, a, R);
   }
 };
 template <class F>

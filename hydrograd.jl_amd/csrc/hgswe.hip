@@ -1573,7 +1573,7 @@ __global__ __launch_bounds__(kBlock) void k_lux_fwd(hg::LuxArgs a) {
   if (i >= a.N) return;
   double f[3];
   hg::lux_features<double>(a.net, a.xi[i], a.qx[i], a.qy[i], a.hstill[i], a.hsmall, hg::lux_ks(a, i), f);
-  a.out[i] = hg::lux_eval<MW>(a.net, a.w, f);
+  a.out[i] = hg::lux_eval<MW>(a.net, hg::LuxRaw{a.net, hg::lux_const(a.w), nullptr}, f);
 }
 
 // Forward mode: the network's output and its tangent along the state
@@ -1588,7 +1588,7 @@ __global__ __launch_bounds__(kBlock) void k_lux_jvp(hg::LuxArgs a, const double*
   Dual1 f[3];
   hg::lux_features<Dual1>(a.net, Dual1(a.xi[i], dxi[i]), Dual1(a.qx[i], dqx[i]), Dual1(a.qy[i], dqy[i]),
                           a.hstill[i], a.hsmall, hg::lux_ks(a, i), f);
-  const Dual1 o = hg::lux_eval<MW, Dual1>(a.net, a.w, f, dw);
+  const Dual1 o = hg::lux_eval<MW, Dual1>(a.net, hg::LuxRaw{a.net, hg::lux_const(a.w), hg::lux_const(dw)}, f);
   a.out[i] = o.v;
   dout[i] = o.d;
 }
@@ -1614,7 +1614,7 @@ __global__ __launch_bounds__(64) void k_lux_vjp(hg::LuxArgs a) {
       hg::lux_features<double>(a.net, a.xi[i], a.qx[i], a.qy[i], a.hstill[i], a.hsmall, hg::lux_ks(a, i), f);
     }
     double fb[3];
-    hg::lux_backward<MW>(a.net, a.w, f, ob, acc, lane, fb);
+    hg::lux_backward<MW>(a.net, hg::lux_const(a.w), f, ob, acc, lane, fb);
     if (valid && ob != 0.0) {
       using hg::Dual1;
       const int ns = a.net.choice == hg::LUX_MANNING_H ? 1 : 3;  // ManningN_h reads the depth only
