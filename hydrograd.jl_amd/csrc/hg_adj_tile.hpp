@@ -18,7 +18,8 @@ struct GhostAdj {
 };
 
 __device__ __forceinline__ CellQ adj_ghost_state(const AdjArgs& a, const CellQ& me, double n_i, int gi,
-                                                     double nx, double ny, GhostAdj& gs) {
+                                                     double nx, double ny, GhostAdj& gs, double& rh, double& r2s) {
+#pragma clang fp contract(on)
   const double hsmall = a.hsmall;
   gs.kind = a.g_kind[gi];
   gs.bc = a.g_bc[gi];
@@ -61,9 +62,12 @@ __device__ __forceinline__ CellQ adj_ghost_state(const AdjArgs& a, const CellQ& 
   B.hu = qxg;
   B.hv = qyg;
   B.zb = a.g_zb[gi];
-  B.u = qxg / hgh;
-  B.v = qyg / hgh;
-  B.s = sqrt(hgh + EPS);
+  rh = rcp_est(hgh);
+  const double he = hgh + EPS, rs = rsq_est(he);
+  B.u = qxg * rh;
+  B.v = qyg * rh;
+  B.s = he * rs;
+  r2s = 0.5 * rs;
   B.p = a.half_g * ((B.xi + EPS) * (B.xi + EPS) + 2.0 * B.xi * B.hs);
   return B;
 }
@@ -74,6 +78,7 @@ __device__ __forceinline__ CellQ adj_ghost_state(const AdjArgs& a, const CellQ& 
 __device__ __forceinline__ void adj_ghost_route(const AdjArgs& a, const CellQ& me, double n_i, int gi,
                                                 const GhostAdj& gs, const SideBar& Bb, double nx, double ny,
                                                 SideBar& U, double& nb, double& zbb) {
+#pragma clang fp contract(on)
   const double hgb = Bb.h + Bb.xi;  // xi_g = h_g - hstill_g
   switch (gs.kind) {
     case HG_BC_INLETQ: {  // h_g = h, q_g = -h v n w, v = (Q / A) L^(2/3) / n
@@ -112,6 +117,7 @@ constexpr int kAdjRows = 13;  // CellQ without h and p (8), z (3), 1 / h, 0.5 / 
 // make_cellq's operations.
 template <int T>
 __device__ __forceinline__ CellQ lds_cellq(const double* C, int r, double half_g, double hsmall) {
+#pragma clang fp contract(on)
   CellQ q;
   q.xi = C[0 * T + r]; q.hs = C[1 * T + r]; q.hu = C[2 * T + r]; q.hv = C[3 * T + r];
   q.zb = C[4 * T + r]; q.u = C[5 * T + r]; q.v = C[6 * T + r]; q.s = C[7 * T + r];
@@ -129,6 +135,7 @@ __device__ __forceinline__ CellQ lds_cellq(const double* C, int r, double half_g
 // from one rsqrt.  rh = 1 / h, r2s = 0.5 / sqrt(h + eps).
 __device__ __forceinline__ CellQ adj_cellq(double xi, double hs, double qx, double qy, double zb, double half_g,
                                                double hsmall, double& rh, double& r2s) {
+#pragma clang fp contract(on)
   CellQ c;
   c.xi = xi;
   c.hs = hs;
@@ -142,11 +149,11 @@ __device__ __forceinline__ CellQ adj_cellq(double xi, double hs, double qx, doub
   c.hu = hu;
   c.hv = hv;
   c.zb = zb;
-  rh = 1.0 / h;
+  rh = rcp_est(h);
   c.u = hu * rh;
   c.v = hv * rh;
   const double he = h + EPS;
-  const double rs = rsqrt(he);
+  const double rs = rsq_est(he);
   c.s = he * rs;
   r2s = 0.5 * rs;
   c.p = half_g * ((xi + EPS) * (xi + EPS) + 2.0 * xi * hs);
@@ -176,6 +183,7 @@ __device__ __forceinline__ NbrRaw nbr_load(const AdjArgs& a, int j) {
 template <bool STEP, int T, int MD>
 __device__ __forceinline__ void adj_item(const AdjArgs& a, int t, const double* C, double* S, int32_t* Xm,
                                          const ItemRec& rec, const NbrRaw& nr) {
+#pragma clang fp contract(on)
   const double hsmall = a.hsmall, half_g = a.half_g;
   const int code = rec.code;
   const int ia = code & 1023, ka = (code >> 10) & 15;
@@ -209,15 +217,13 @@ __device__ __forceinline__ void adj_item(const AdjArgs& a, int t, const double* 
       G = adj_cellq(nr.xi, nr.hs, nr.qx, nr.qy, nr.zb, half_g, hsmall, rhG, r2G);
       double m0 = nr.m0, m1 = nr.m1, m2 = nr.m2;
       if (nr.clamped) m0 = m1 = m2 = 0.0;
-      const double rAj = 1.0 / nr.area;
+      const double rAj = rcp_est(nr.area);
       zG0 = (STEP ? nr.dt * m0 : m0) * rAj;
       zG1 = (STEP ? nr.dt * m1 : m1) * rAj;
       zG2 = (STEP ? nr.dt * m2 : m2) * rAj;
     } else {  // ghost (no cotangent of its own)
       n_a = a.n[t * T + ia];
-      G = adj_ghost_state(a, Lc, n_a, rec.ref, nx, ny, gs);
-      rhG = 1.0 / G.h;
-      r2G = 0.5 / G.s;
+      G = adj_ghost_state(a, Lc, n_a, rec.ref, nx, ny, gs, rhG, r2G);
     }
     P = sw ? G : Lc;
     Q = sw ? Lc : G;

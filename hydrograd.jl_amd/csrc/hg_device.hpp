@@ -38,6 +38,14 @@ __device__ __forceinline__ double div_est(double a, double b, double y) {
   return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
 }
 
+// 1 / sqrt(x) for normal finite x > 0, within about an ulp: the hardware's
+// estimate y and, with e = 1 - x y^2, the series y (1 + e / 2 + 3 e^2 / 8).
+__device__ __forceinline__ double rsq_est(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-x * y, y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+
 // sqrt(x) for normal finite x > 0 (every caller adds eps to a square or a
 // depth, so x >= 2^-52); r2 = 0.5 / sqrt(x) to about 2^-46.
 __device__ __forceinline__ double sqrt_est(double x, double& r2) {

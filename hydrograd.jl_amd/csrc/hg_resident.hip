@@ -818,7 +818,7 @@ __device__ __forceinline__ bool adj_run_cells(AdjArgs a, const AdjRunArgs& R, do
     if (own) {
       double rh, r2s;
       me = adj_cellq(px, hs, pqx, pqy, zb, a.half_g, hsmall, rh, r2s);
-      const double rA = 1.0 / A;
+      const double rA = rcp_est(A);
       y0 = dti * l0;
       y1 = dti * l1;
       y2 = dti * l2;

@@ -693,7 +693,8 @@ __device__ __forceinline__ void adj_ghost_face(const hg::AdjArgs& a, const CellA
   nb = 0.0;
   zbb = 0.0;
   GhostAdj gs;
-  const hg::CellQ B = adj_ghost_state(a, ca.me, ca.n, gi, nx, ny, gs);
+  double rhB, r2B;  // formed with B; not used here
+  const hg::CellQ B = adj_ghost_state(a, ca.me, ca.n, gi, nx, ny, gs, rhB, r2B);
   const double c[3] = {fi * ca.y0, fi * ca.y1, fi * ca.y2};
   hg::SideBar Bb;
   hg::roe_vjp(ca.me, B, nx, ny, a.g, a.half_g, a.hsmall, c, U, Bb);
@@ -888,7 +889,7 @@ __global__ __launch_bounds__(T, 3) void k_adj_tile(hg::AdjArgs a0) {
     double l0 = a.lx[i], l1 = a.lqx[i], l2 = a.lqy[i];
     if (STEP && a.mask && a.mask[i]) l0 = l1 = l2 = 0.0;
     const double dti = a.dtc ? a.dtc[i] : a.dt;
-    const double rA = 1.0 / a.area[i];
+    const double rA = hg::rcp_est(a.area[i]);
     C[0 * T + li] = me.xi; C[1 * T + li] = me.hs; C[2 * T + li] = me.hu; C[3 * T + li] = me.hv;
     C[4 * T + li] = me.zb; C[5 * T + li] = me.u; C[6 * T + li] = me.v; C[7 * T + li] = me.s;
     C[8 * T + li] = (STEP ? dti * l0 : l0) * rA;
