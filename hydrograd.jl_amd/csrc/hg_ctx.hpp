@@ -349,7 +349,7 @@ struct hg_ctx {
   hg::ItemTable items{};  // the step kernel's work items
   int32_t tileMD = 3;
   bool deg_full = false;  // every cell has tileMD faces: the tile kernels need not read deg
-  int32_t xcd_chunk = 0;  // identity block -> tile mapping by default (the autotuner re-checks)
+  int32_t xcd_chunk = 0;  // block -> tile mapping: default_chunk, until set or tuned
   int32_t ncu = 256;      // compute units of the device
   int32_t max_items = 0;  // work items of the fullest tile
   // resident runs (hg_resident.hpp): tiles the device holds at once of each
