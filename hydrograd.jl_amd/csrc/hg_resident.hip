@@ -628,7 +628,7 @@ __global__ __launch_bounds__(res_threads(MD, true), 2) void k_tsit5_run(TileArgs
 // arrays of their own (o_*), which the host takes over when the run is done.
 // One launch per step took 8.5 us for the tiles and 2.6 us for the inlets, of
 // which about 3 us and 1 us were launch and first loads; a step takes 4.6 us
-// here on 1,000 quads, 6.0 on a 1,300-cell channel (its inlet tiles exchange
+// here on 1,000 quads, 5.8 on a 1,300-cell channel (its inlet tiles exchange
 // twice per step) and 6.4 on 59k triangles.  Up to 512 tiles: the registers
 // that hold the cells allow two tiles per CU.
 constexpr int adj_run_base_doubles(int MD) {  // without the network's values

@@ -240,6 +240,7 @@ int hg_time_advance(hg_ctx* ctx, double dt, int64_t nsteps, int32_t reps, double
  * per tile (128, 256 or 512; one work-item per cell) and the work-group to
  * tile mapping: xcd_chunk = 0 maps work-group b to tile b; G > 0 gives each
  * of the 8 XCDs runs of G consecutive tiles within windows of 8G tiles.
+ * A mesh starts with G of about 32 (less for several fields of one mesh).
  * Every shape gives bit-identical results.  (Small meshes, which start with
  * 128-cell tiles, advance many steps per launch while they keep that size.) */
 int hg_set_tile_config(hg_ctx* ctx, int32_t tile_cells, int32_t xcd_chunk);
