@@ -2576,13 +2576,15 @@ hg::AdjArgs make_adj_args(hg_ctx* ctx, const double* const q[3], const double* c
 }
 
 // The reverse step runs tiled wherever the step does.  Its tile size is its
-// own: 256 cells, or 128 when 256-cell tiles would give fewer than two
-// rounds of three work-groups per CU (its results do not depend on the
-// tiling).  It uses the step kernel's work items when they have that tile
+// own: 256 cells, or 128 when 256-cell tiles would give less than one round of
+// three work-groups per CU (its results do not depend on the tiling).  A
+// gradient's step pair on 98,840 triangles (387 tiles of 256) takes 20.4 us
+// with 128 and 21.1 with 256, on 197,802 (773 tiles) 35.2 and 34.5, on 296,208
+// 43.2 and 42.1.  It uses the step kernel's work items when they have that tile
 // size, else its own copy, built once.
 int ensure_adj_tiles(hg_ctx* ctx) {
   const int64_t blocks256 = (ctx->Nm + 255) / 256 * ctx->K;
-  int T = ctx->adj_T_req ? ctx->adj_T_req : (blocks256 >= int64_t(2) * 3 * ctx->ncu ? 256 : 128);
+  int T = ctx->adj_T_req ? ctx->adj_T_req : (blocks256 >= int64_t(3) * ctx->ncu ? 256 : 128);
   if (adj_tile_lds_bytes(T, ctx->tileMD) > ctx->lds_max) T = 128;
   if (T == ctx->tileT) {
     ctx->adj_T = T;

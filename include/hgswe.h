@@ -248,7 +248,7 @@ int hg_get_tile_config(hg_ctx* ctx, int32_t* tile_cells, int32_t* xcd_chunk);
 
 /* Tile size of the tiled reverse step (no reference counterpart): 128, 256
  * or 512 cells, or 0 (default) for the library's choice (256, or 128 when
- * the mesh has fewer than two rounds of three 256-cell work-groups per CU).
+ * the mesh has less than one round of three 256-cell work-groups per CU).
  * It shares the step kernel's block -> tile mapping.  Every size gives
  * bit-identical gradients. */
 int hg_set_adjoint_tile(hg_ctx* ctx, int32_t tile_cells);
