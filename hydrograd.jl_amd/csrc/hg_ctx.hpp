@@ -364,7 +364,7 @@ struct hg_ctx {
   size_t res_ring_n = 0;
   int32_t* res_ctl = nullptr;
   int32_t adj_res_cap[3] = {-1, -1, -1}, tsit5_cap[3] = {-1, -1, -1};
-  bool rec_resident = false;   // the last forward sweep recorded its last segment resident
+  bool rec_resident = false;   // the last forward sweep recorded all that a resident reversal reads of its last segment
   double* adj_wpart = nullptr;  // a resident reversal's weight cotangents per tile
   hg::Tsit5State* rk_state = nullptr;
   double* rk_frames = nullptr;

@@ -2598,6 +2598,7 @@ int ensure_adj_tiles(hg_ctx* ctx) {
                                ctx->h_gbc);
     HG_TRY(hipStreamSynchronize(ctx->stream));
     int rc = drop_graph(ctx);
+    ctx->adj_own_T = 0;
     if (!rc) rc = free_items(ctx, ctx->adj_own);
     if (!rc) rc = upload_items(ctx, tb, ctx->adj_own);
     if (rc) return rc;
@@ -2840,7 +2841,7 @@ int forward_checkpointed(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck) {
                      seg_totalA(ctx, 0, 0), rec_n, nullptr, &done);
     if (rc) return rc;
     if (done) {
-      ctx->rec_resident = true;
+      ctx->rec_resident = k.nmode == hg::RES_N_FIELD || rec_n;
       ctx->cur = 1 - ctx->cur;
       return HG_OK;
     }
@@ -2982,6 +2983,10 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
 int reverse_sweep(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck, int& lam_cur) {
   const int64_t N = ctx->N;
   const int64_t nseg = (nsteps + kck - 1) / kck;
+  if (ctx->tiled) {  // the mesh may have been tiled anew since the forward sweep: adj_items would name freed arrays
+    const int rc = ensure_adj_tiles(ctx);
+    if (rc) return rc;
+  }
   if (nseg == 1) {  // the whole run is recorded: a small mesh reverses it in one launch
     bool done = false;
     const int rc = adj_res_run(ctx, dt, nsteps, 0, lam_cur, &done);

@@ -1,0 +1,38 @@
+"""Which path a small mesh takes (resident runs or one launch per step) is a
+matter of speed: changes of tiling, inputs that a resident run does not hold
+and waits that run out leave the results as they are."""
+import numpy as np
+import pytest
+
+from hgswe import capi
+
+from test_gpu_resident import channel, moving, with_law
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("between", [("tile", 256), ("tile", 256, 128), ("tile", 512), ("adjoint", 256),
+                                     ("adjoint", 256, 0), ("tune",)])
+@pytest.mark.parametrize("law", ["field", "sigmoid", "ManningN_h"])
+def test_tiled_anew_between_the_sweeps(law, between):
+    """Between hg_adjoint_forward and hg_adjoint_reverse the mesh is tiled anew: the same cotangents (bit for bit with n
+    from the field; the closures' bound is that of test_reverse_run_with_closure)."""
+    c = moving(channel(1100))
+    lam = np.random.default_rng(1).normal(size=3 * c.N)
+    ref, ctx = capi.Context(c), capi.Context(c)
+    for k in (ref, ctx):
+        with_law(k, c, law)
+    want = ref.adjoint(c.Q0, c.dt, 12, 0, lam)
+    if between[0] == "adjoint":  # the forward sweep under the other size
+        ctx.set_adjoint_tile(between[1])
+    QN = ctx.adjoint_forward(c.Q0, c.dt, 12, 0)
+    assert np.array_equal(QN, ref.step(c.Q0, c.dt, 12))
+    for size in between[1:]:
+        (ctx.set_tile_config if between[0] == "tile" else ctx.set_adjoint_tile)(size)
+    if between[0] == "tune":
+        ctx.autotune(c.dt, 8)
+    for x, y in zip(ctx.adjoint_reverse(lam), want):
+        if law == "field":
+            assert np.array_equal(x, y)
+        else:
+            assert np.max(np.abs(x - y), initial=0.0) <= 1.3e-11 * np.max(np.abs(y), initial=0.0)
