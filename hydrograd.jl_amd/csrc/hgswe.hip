@@ -2313,13 +2313,15 @@ int g_res_room[kMaxDevices] = {};
 
 // Whether nsteps steps (or right-hand sides) may run resident, and as which
 // variant: one field, the default tiling of small meshes, at most one item
-// per work-item and 64 inlets per tile, n from the field, a law or a network
+// per work-item and 64 inlets per tile, every inlet ghost in its inlet's list
+// (a tile that reads an inlet is then read by the inlet's other tiles, which the
+// rings' slots are reused by), n from the field, a law or a network
 // of at most four units per layer, and steps enough to pay for the ring's
 // initialisation.
 bool res_kind(hg_ctx* ctx, int64_t nsteps, bool dual, hg::ResKind& k) {
   if (!ctx->tiled || ctx->res_off || ctx->K != 1 || nsteps < 4 || ctx->tileT != kResT || ctx->tileMD > 4 ||
-      ctx->max_items > res_items(ctx->tileMD) || (ctx->n_inlet > 0 && !ctx->fuse_inlet) || ctx->ude_prec ||
-      ctx->device >= kMaxDevices)
+      ctx->max_items > res_items(ctx->tileMD) || (ctx->n_inlet > 0 && !(ctx->fuse_inlet && ctx->inlets_listed)) ||
+      ctx->ude_prec || ctx->device >= kMaxDevices)
     return false;
   k.md = ctx->tileMD;
   k.nmode = ctx->nlaw.kind != hg::NLAW_OFF ? hg::RES_N_LAW : ctx->lux.choice ? hg::RES_N_NET : hg::RES_N_FIELD;
@@ -3946,6 +3948,10 @@ int create_impl(hg_ctx** out, const hg_mesh* m, const hg_bcs* b, const hg_consts
       recs[f] = hg::InletFaceRec{gi, in_cell[f], first[f], next[f], g_L23[gi], in_L53[f]};
     }
     rc = upload(ctx, ctx->in_rec, recs.data(), ctx->n_inlet_faces);
+    std::vector<uint8_t> listed(size_t(G), 0);
+    for (int32_t f = 0; f < ctx->n_inlet_faces; ++f) listed[b->inlet_ghost[f]] = 1;
+    for (int64_t gi = 0; gi < G; ++gi)
+      if (b->ghost_kind[gi] == HG_BC_INLETQ && !listed[gi]) ctx->inlets_listed = false;
     std::unordered_map<int32_t, int32_t> owner;  // cell -> the inlet it sits on
     ctx->inlets_disjoint = true;
     for (int bi = 0; bi < b->n_inlet && ctx->inlets_disjoint; ++bi)

@@ -1,12 +1,14 @@
 """Which path a small mesh takes (resident runs or one launch per step) is a
 matter of speed: changes of tiling, inputs that a resident run does not hold
 and waits that run out leave the results as they are."""
+import dataclasses
+
 import numpy as np
 import pytest
 
 from hgswe import capi
 
-from test_gpu_resident import channel, moving, with_law
+from test_gpu_resident import channel, moving, two_inlets, with_law
 
 pytestmark = pytest.mark.gpu
 
@@ -36,3 +38,22 @@ def test_tiled_anew_between_the_sweeps(law, between):
             assert np.array_equal(x, y)
         else:
             assert np.max(np.abs(x - y), initial=0.0) <= 1.3e-11 * np.max(np.abs(y), initial=0.0)
+
+
+@pytest.mark.parametrize("keep", [1, 20])
+def test_inlet_faces_left_out_of_the_list(keep):
+    """Ghosts of inlet kind that their inlet's list does not name read its conveyance without adding to it: the same
+    bits with and without a tiling that runs resident."""
+    c = two_inlets(8000)
+    m = c.mesh
+    lists = [m.inlet_ghost[m.inlet_off[b]:m.inlet_off[b + 1]] for b in range(m.n_inlet)]
+    assert all(len(x) > 40 for x in lists)
+    lists[0] = lists[0][:keep]
+    c = dataclasses.replace(c, mesh=dataclasses.replace(
+        m, inlet_off=np.array([0, keep, keep + len(lists[1])], dtype=np.int32), inlet_ghost=np.concatenate(lists)))
+    lam = np.random.default_rng(1).normal(size=3 * c.N)
+    ctx, single = capi.Context(c), capi.Context(c)
+    single.set_tile_config(256)
+    assert np.array_equal(ctx.step(c.Q0, c.dt, 30), single.step(c.Q0, c.dt, 30))
+    for x, y in zip(ctx.adjoint(c.Q0, c.dt, 30, 0, lam), single.adjoint(c.Q0, c.dt, 30, 0, lam)):
+        assert np.all(np.isfinite(y)) and np.array_equal(x, y)
