@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from hgswe import capi
+from hgswe import mesh as hm
 
 from test_gpu_resident import channel, moving, two_inlets, with_law
 
@@ -57,3 +58,33 @@ def test_inlet_faces_left_out_of_the_list(keep):
     assert np.array_equal(ctx.step(c.Q0, c.dt, 30), single.step(c.Q0, c.dt, 30))
     for x, y in zip(ctx.adjoint(c.Q0, c.dt, 30, 0, lam), single.adjoint(c.Q0, c.dt, 30, 0, lam)):
         assert np.all(np.isfinite(y)) and np.array_equal(x, y)
+
+
+def second_inlet_walled(c):
+    """The case with the faces of its second inlet as walls: that inlet is left without faces."""
+    m = c.mesh
+    off = int(m.inlet_off[1])
+    kind = m.ghost_kind.copy()
+    kind[m.inlet_ghost[off:]] = hm.BC_WALL
+    return dataclasses.replace(c, mesh=dataclasses.replace(
+        m, ghost_kind=kind, inlet_off=np.array([0, off, off], dtype=np.int32), inlet_ghost=m.inlet_ghost[:off]))
+
+
+@pytest.mark.parametrize("n", [30, 300, 2000])
+def test_inlet_without_faces(n):
+    """Its discharge enters nowhere: its cotangent is zero, and the others are the per-tile kernel's."""
+    both = two_inlets(n)
+    c = second_inlet_walled(both)
+    lam = np.random.default_rng(1).normal(size=3 * c.N)
+    single = capi.Context(c)
+    single.set_tile_config(256)
+    want = single.adjoint(c.Q0, c.dt, 12, 0, lam)
+    assert want[3][1] == 0.0
+    for _ in range(3):  # contexts whose second inlet has a cotangent leave it in the memory that the next one takes
+        used = capi.Context(both)
+        assert used.adjoint(both.Q0, both.dt, 12, 0, lam)[3][1] != 0.0
+        used.close()
+        ctx = capi.Context(c)
+        for x, y in zip(ctx.adjoint(c.Q0, c.dt, 12, 0, lam), want):
+            assert np.array_equal(x, y)
+        ctx.close()
