@@ -294,7 +294,8 @@ __device__ __forceinline__ void source_vjp(double g, double kn2, double hsmall, 
   const double sb = fxb * cc * qx + fyb * cc * qy;
   qxb += fxb * cc * s + sb * qx * rs;
   qyb += fyb * cc * s + sb * qy * rs;
-  nb += cb * 2.0 * g * n * rp;
+  const double nt = cb * 2.0 * g * n * rp;  // rounded before it is added: a caller may add it to nb later
+  nb += nt;
   hb += cb * (-7.0 / 3.0) * cc * rcp_est(x);
 }
 

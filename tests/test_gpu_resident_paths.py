@@ -88,3 +88,15 @@ def test_inlet_without_faces(n):
         for x, y in zip(ctx.adjoint(c.Q0, c.dt, 12, 0, lam), want):
             assert np.array_equal(x, y)
         ctx.close()
+
+
+@pytest.mark.parametrize("n", [300, 8000])
+def test_roughness_cotangent_of_inlet_cells(n):
+    """An inlet cell's n has a boundary and a friction term, which the two paths add at different places."""
+    c = two_inlets(n)
+    ctx, single = capi.Context(c), capi.Context(c)
+    single.set_tile_config(256)
+    for seed in range(8):
+        lam = np.random.default_rng(seed).normal(size=3 * c.N)
+        for x, y in zip(ctx.adjoint(c.Q0, c.dt, 12, 0, lam), single.adjoint(c.Q0, c.dt, 12, 0, lam)):
+            assert np.array_equal(x, y)
