@@ -4861,9 +4861,9 @@ int hg_jvp(hg_ctx* ctx, const double* Q0, const double* dQ0, const double* param
   const int64_t N = ctx->N, G = ctx->G;
   int rc = hg_set_params(ctx, params, n_params);
   if (rc) return rc;
-  if (!ctx->jvp) {  // tangents: state (2 x 3N), dn, dzb, dS0x, dS0y (N each), dg_zb (G), dinletQ, dtotalA
+  if (!ctx->jvp) {  // tangents: state (2 x 3N), dn, dzb, dS0x, dS0y, dfmag (N each), dg_zb (G), dinletQ, dtotalA
     const size_t nI = size_t(std::max<int32_t>(ctx->n_inlet, 1));
-    rc = dalloc(ctx, &ctx->jvp, size_t(10) * N + size_t(std::max<int64_t>(G, 1)) + 2 * nI);
+    rc = dalloc(ctx, &ctx->jvp, size_t(11) * N + size_t(std::max<int64_t>(G, 1)) + 2 * nI);
     if (rc) return rc;
   }
   double* T0 = ctx->jvp;
@@ -4872,7 +4872,8 @@ int hg_jvp(hg_ctx* ctx, const double* Q0, const double* dQ0, const double* param
   double* dzb = dn + N;
   double* dS0x = dzb + N;
   double* dS0y = dS0x + N;
-  double* dgzb = dS0y + N;
+  double* dfmag = dS0y + N;
+  double* dgzb = dfmag + N;
   double* dQin = dgzb + std::max<int64_t>(G, 1);
   double* dtot = dQin + std::max<int32_t>(ctx->n_inlet, 1);
   // tangents of the parameter fields (semi_discretize_swe_2D.jl:114-199)
@@ -4936,7 +4937,7 @@ int hg_jvp(hg_ctx* ctx, const double* Q0, const double* dQ0, const double* param
   const bool law = ctx->nlaw.kind != hg::NLAW_OFF;
   int64_t t0 = 0;
   // a small mesh: runs of steps in one launch each
-  for (hg::ResKind k; !(lux_fr && pn) && res_kind(ctx, nsteps - t0, true, k);) {
+  for (hg::ResKind k; res_kind(ctx, nsteps - t0, true, k);) {
     const int64_t ns = std::min<int64_t>(nsteps - t0, kResSteps);
     const double* in[3] = {ctx->st[cur][0], ctx->st[cur][1], ctx->st[cur][2]};
     hg::ResArgs D{};
@@ -4957,7 +4958,7 @@ int hg_jvp(hg_ctx* ctx, const double* Q0, const double* dQ0, const double* param
     t0 += ns;
   }
   if (law || (lux && !lux_fr)) pn = dn;  // the law's or network's tangent of n, rewritten every step
-  double* dfm = lux_fr ? dn : nullptr;     // the network's tangent of the friction magnitude
+  double* const dout = lux_fr ? dfmag : dn;  // the network's tangent: of the friction magnitude, or of n
   for (int64_t t = t0; t < nsteps; ++t) {
     const double* in[3] = {ctx->st[cur][0], ctx->st[cur][1], ctx->st[cur][2]};
     double* out[3] = {ctx->st[1 - cur][0], ctx->st[1 - cur][1], ctx->st[1 - cur][2]};
@@ -4973,10 +4974,10 @@ int hg_jvp(hg_ctx* ctx, const double* Q0, const double* dQ0, const double* param
       const hg::LuxArgs u = lux_args(ctx, in);
       if (ctx->lux_mw == 4)
         hipLaunchKernelGGL(k_lux_jvp<4>, dim3(grid_of(N)), dim3(kBlock), 0, ctx->stream, u, Tb[cur], Tb[cur] + N,
-                           Tb[cur] + 2 * N, pw, dn);
+                           Tb[cur] + 2 * N, pw, dout);
       else
         hipLaunchKernelGGL(k_lux_jvp<hg::kLuxMaxW>, dim3(grid_of(N)), dim3(kBlock), 0, ctx->stream, u, Tb[cur],
-                           Tb[cur] + N, Tb[cur] + 2 * N, pw, dn);
+                           Tb[cur] + N, Tb[cur] + 2 * N, pw, dout);
     }
     if (ctx->n_inlet > 0)
       hipLaunchKernelGGL(k_inlet_conveyance_jvp, dim3((ctx->n_inlet + 63) / 64), dim3(64), 0, ctx->stream,
@@ -4996,7 +4997,7 @@ int hg_jvp(hg_ctx* ctx, const double* Q0, const double* dQ0, const double* param
     J.dg_zb = pzb ? dgzb : nullptr;
     J.dinletQ = pQ;
     J.dtotalA = dtot;
-    J.dfmag = dfm;
+    J.dfmag = lux_fr ? dfmag : nullptr;
     hipLaunchKernelGGL(k_swe_step_jvp, dim3(grid_of(N)), dim3(kBlock), 0, ctx->stream, J);
     HG_TRY(hipGetLastError());
     cur = 1 - cur;
