@@ -354,12 +354,14 @@ struct hg_ctx {
   int32_t ncu = 256;      // compute units of the device
   int32_t max_items = 0;  // work items of the fullest tile
   // resident runs (hg_resident.hpp): tiles the device holds at once of each
-  // variant ([split][n mode][dual]; -1: not asked yet), off for good once a
-  // wait ran out, this run's share of the device, the exchange ring and its
+  // variant ([split][n mode][dual]; -1: not asked yet), off once a wait ran
+  // out (until hg_set_resident), this run's share of the device, the exchange ring and its
   // control word; the same for the reverse run, its rings and the sums it
   // writes, and for Tsit5, its state between launches and its frames
   int32_t res_cap[2][3][2] = {{{-1, -1}, {-1, -1}, {-1, -1}}, {{-1, -1}, {-1, -1}, {-1, -1}}};
   bool res_off = false;
+  bool res_short = false;                   // runs lack their last work-group and give up (HG_RESIDENT_SHORT)
+  int64_t res_runs = 0, res_given_up = 0;  // runs that ended, and that gave up
   int32_t res_share = 0;
   unsigned long long* res_ring = nullptr;
   size_t res_ring_n = 0;

@@ -2381,6 +2381,9 @@ bool res_claim(hg_ctx* ctx, int cap) {
   return true;
 }
 
+// Work-groups of a resident run: all tiles (HG_RESIDENT_SHORT: one less).
+int res_grid(const hg_ctx* ctx) { return ctx->ntiles - (ctx->res_short ? 1 : 0); }
+
 // After the launch of a resident run (e: its status): waits for it and gives its room back;
 // *done: every tile finished.
 int res_finish(hg_ctx* ctx, hipError_t e, bool* done) {
@@ -2391,10 +2394,12 @@ int res_finish(hg_ctx* ctx, hipError_t e, bool* done) {
   }
   HG_TRY(e);
   ctx->pin_used = 0;
-  if (ctx->flags_host[2]) {  // the device was shared with something else: one launch per step from here on
+  if (ctx->flags_host[2] || ctx->res_short) {  // the device was shared with something else: one launch per step from here on
     ctx->flags_host[2] = 0;
     ctx->res_off = true;
+    ++ctx->res_given_up;
   } else {
+    ++ctx->res_runs;
     *done = true;
   }
   return HG_OK;
@@ -2424,7 +2429,7 @@ int res_run(hg_ctx* ctx, const hg::ResKind& k, const double* const in[3], double
     R.dg_zb = T->dg_zb; R.dinletQ = T->dinletQ; R.net_dw = T->net_dw;
   }
   hipError_t e = hg::res_init(ctx->stream, int64_t(4) * words * ctx->N, ctx->res_ring, ctx->res_ctl);
-  if (e == hipSuccess) e = hg::launch_run(ctx->stream, k, ctx->ntiles, make_tile_args_p(ctx, in, out, dt), R);
+  if (e == hipSuccess && res_grid(ctx)) e = hg::launch_run(ctx->stream, k, res_grid(ctx), make_tile_args_p(ctx, in, out, dt), R);
   return res_finish(ctx, e, done);
 }
 
@@ -2956,7 +2961,7 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
     R.o_wpart = ctx->adj_wpart;
   }
   hipError_t e = hg::res_init(ctx->stream, nring, ctx->adj_ring, ctx->res_ctl);
-  if (e == hipSuccess) e = hg::launch_adj_run(ctx->stream, ctx->tileMD, k.nmode, ctx->ntiles, a, R);
+  if (e == hipSuccess && res_grid(ctx)) e = hg::launch_adj_run(ctx->stream, ctx->tileMD, k.nmode, res_grid(ctx), a, R);
   int rc = res_finish(ctx, e, done);
   if (rc || !*done) return rc;
   ArrayList take;
@@ -5057,8 +5062,8 @@ static int tsit5_resident(hg_ctx* ctx, double t0, double t1, int64_t n_save, dou
     P.out = ctx->rk_state + (launch & 1);
     if (!res_claim(ctx, cap)) return HG_OK;
     hipError_t e = hg::res_init(ctx->stream, 12 * N + 4 * hg::kResRed, ctx->res_ring, ctx->res_ctl);
-    if (e == hipSuccess)
-      e = hg::launch_tsit5(ctx->stream, k.md, k.nmode, ctx->ntiles, make_tile_args_p(ctx, in, ctx->st[1], 0.0),
+    if (e == hipSuccess && res_grid(ctx))
+      e = hg::launch_tsit5(ctx->stream, k.md, k.nmode, res_grid(ctx), make_tile_args_p(ctx, in, ctx->st[1], 0.0),
                            res_args(ctx, 0), P);
     bool ran = false;
     rc = res_finish(ctx, e, &ran);
@@ -5361,6 +5366,25 @@ int hg_get_tile_config(hg_ctx* ctx, int32_t* tile_cells, int32_t* xcd_chunk) {
   if (!ctx) return HG_ERR_ARG;
   if (tile_cells) *tile_cells = ctx->tiled ? ctx->tileT : 0;
   if (xcd_chunk) *xcd_chunk = ctx->xcd_chunk;
+  return HG_OK;
+}
+
+int hg_set_resident(hg_ctx* ctx, int32_t mode) {
+  if (!ctx) return HG_ERR_ARG;
+  if (mode < HG_RESIDENT_OFF || mode > HG_RESIDENT_SHORT) {
+    ctx->err = "hg_set_resident: unknown mode";
+    return HG_ERR_ARG;
+  }
+  ctx->res_off = mode == HG_RESIDENT_OFF;
+  ctx->res_short = mode == HG_RESIDENT_SHORT;
+  return HG_OK;
+}
+
+int hg_get_resident(const hg_ctx* ctx, int32_t* on, int64_t* runs, int64_t* given_up) {
+  if (!ctx) return HG_ERR_ARG;
+  if (on) *on = ctx->res_off ? 0 : 1;
+  if (runs) *runs = ctx->res_runs;
+  if (given_up) *given_up = ctx->res_given_up;
   return HG_OK;
 }
 

@@ -17,6 +17,7 @@ _LIB = None
 
 HG_OK, HG_ERR_ARG, HG_ERR_HIP, HG_ERR_MESH, HG_ERR_CONVEYANCE, HG_ERR_NONFINITE, HG_ERR_STATE = range(7)
 HG_PARAM_NONE, HG_PARAM_ZB, HG_PARAM_N_ZONE, HG_PARAM_N_CELL, HG_PARAM_Q, HG_PARAM_UDE = range(6)
+HG_RESIDENT_OFF, HG_RESIDENT_ON, HG_RESIDENT_SHORT = range(3)
 HG_REORDER = 1
 HG_CELL_KERNEL = 2
 HG_NLAW_OFF, HG_NLAW_POWER, HG_NLAW_SIGMOID, HG_NLAW_INVERSE, HG_NLAW_H_UMAG_KS = range(5)
@@ -36,7 +37,7 @@ EXPORTS = [
     "hg_set_params", "hg_state_upload", "hg_state_download", "hg_advance", "hg_cfl_dt", "hg_time_advance",
     "hg_info", "hg_probe_copy", "hg_rhs_vjp", "hg_adjoint", "hg_grad_probes", "hg_batch_create",
     "hg_set_tile_config", "hg_get_tile_config", "hg_set_adjoint_tile", "hg_last_checkpoint_interval", "hg_adjoint_forward",
-    "hg_adjoint_reverse", "hg_autotune", "hg_set_ude", "hg_ude_n", "hg_ude_grad",
+    "hg_adjoint_reverse", "hg_autotune", "hg_set_resident", "hg_get_resident", "hg_set_ude", "hg_ude_n", "hg_ude_grad",
     "hg_mfma_probe", "hg_tsit5_solve", "hg_tsit5_tableau", "hg_jvp", "hg_batch_set_dt", "hg_set_n_law",
     "hg_n_law_eval", "hg_cell_n", "hg_lux_n_params", "hg_set_lux_ude", "hg_lux_eval", "hg_lux_grad",
     "hg_advance_timed", "hg_advance_region", "hg_prepare_advance", "hg_cfl_dt_noalloc", "hg_fields_create",
@@ -108,6 +109,8 @@ def lib():
         L.hg_set_tile_config.argtypes = [C.c_void_p, C.c_int32, C.c_int32]
         L.hg_batch_set_dt.argtypes = [C.c_void_p, C.c_void_p]
         L.hg_get_tile_config.argtypes = [C.c_void_p, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
+        L.hg_set_resident.argtypes = [C.c_void_p, C.c_int32]
+        L.hg_get_resident.argtypes = [C.c_void_p, C.POINTER(C.c_int32), C.POINTER(C.c_int64), C.POINTER(C.c_int64)]
         L.hg_autotune.argtypes = [C.c_void_p, C.c_double, C.c_int64, C.POINTER(C.c_int32), C.POINTER(C.c_int32),
                                   C.POINTER(C.c_double)]
         L.hg_set_ude.argtypes = [C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_int32]
@@ -508,6 +511,17 @@ class Context:
         t, x = C.c_int32(), C.c_int32()
         self._chk(lib().hg_get_tile_config(self.h, C.byref(t), C.byref(x)))
         return t.value, x.value
+
+    def set_resident(self, mode):
+        """HG_RESIDENT_OFF, _ON or _SHORT: whether a small mesh advances many
+        steps per launch."""
+        self._chk(lib().hg_set_resident(self.h, int(mode)))
+
+    def resident(self):
+        """(whether resident runs are on, runs that ended, runs that gave up)."""
+        on, runs, up = C.c_int32(), C.c_int64(), C.c_int64()
+        self._chk(lib().hg_get_resident(self.h, C.byref(on), C.byref(runs), C.byref(up)))
+        return bool(on.value), runs.value, up.value
 
     def autotune(self, dt, nsteps=64):
         """Times every launch shape from the device state (restored

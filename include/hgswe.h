@@ -253,6 +253,22 @@ int hg_get_tile_config(hg_ctx* ctx, int32_t* tile_cells, int32_t* xcd_chunk);
  * bit-identical gradients. */
 int hg_set_adjoint_tile(hg_ctx* ctx, int32_t tile_cells);
 
+/* Resident runs (no reference counterpart): a mesh of up to about 130,000
+ * cells with 128-cell tiles (65,000 in reverse, 32,000 with a network in
+ * reverse or under hg_tsit5_solve) advances many steps in one launch whose
+ * work-groups wait for each other's border cells.  The library starts one only
+ * if all of its work-groups fit on the device beside the process's other
+ * runs; of other processes on the device it does not know.  A wait of more
+ * than a second ends the run: its steps are repeated with one launch each, as
+ * are all later steps of the context until this call allows runs again.
+ * HG_RESIDENT_SHORT starts every run without its last work-group, so that it
+ * gives up (to test what follows). */
+enum { HG_RESIDENT_OFF = 0, HG_RESIDENT_ON = 1, HG_RESIDENT_SHORT = 2 };
+int hg_set_resident(hg_ctx* ctx, int32_t mode);
+/* Whether resident runs are on, and how many of the context's have ended and
+ * given up so far (any of the three may be NULL). */
+int hg_get_resident(const hg_ctx* ctx, int32_t* on, int64_t* runs, int64_t* given_up);
+
 /* Autotuner: after 500 warm-up steps (the device clocks settle), times the
  * step kernel over nsteps steps of every launch shape, twice each (events on
  * each dispatch, after 16 warm-up steps), from the current device state

@@ -100,3 +100,62 @@ def test_roughness_cotangent_of_inlet_cells(n):
         lam = np.random.default_rng(seed).normal(size=3 * c.N)
         for x, y in zip(ctx.adjoint(c.Q0, c.dt, 12, 0, lam), single.adjoint(c.Q0, c.dt, 12, 0, lam)):
             assert np.array_equal(x, y)
+
+
+# ---- which path ran, and a wait that runs out
+CALLS = {
+    "step": lambda k, c, lam: [k.step(c.Q0, c.dt, 12)],
+    "adjoint": lambda k, c, lam: list(k.adjoint(c.Q0, c.dt, 12, 0, lam)),
+    "reverse": lambda k, c, lam: list(k.adjoint_reverse(lam)),
+    "jvp": lambda k, c, lam: list(k.jvp(c.Q0, c.dt, 12, dQ0=lam)),
+    "tsit5": lambda k, c, lam: [k.tsit5(c.Q0, 0.0, 12 * c.dt, 3, dt0=c.dt)[0]],
+}
+
+
+def resident_and_single(c, law, call, lam):
+    ctx, single = capi.Context(c), capi.Context(c)
+    single.set_resident(capi.HG_RESIDENT_OFF)
+    for k in (ctx, single):
+        with_law(k, c, law)
+        if call == "reverse":
+            k.adjoint_forward(c.Q0, c.dt, 12, 0)
+    return ctx, single
+
+
+@pytest.mark.parametrize("law", ["field", "sigmoid", "ManningN_h"])
+@pytest.mark.parametrize("call", sorted(CALLS))
+def test_resident_runs_are_taken(call, law):
+    c = moving(channel(1100))
+    lam = np.random.default_rng(1).normal(size=3 * c.N)
+    ctx, single = resident_and_single(c, law, call, lam)
+    before = ctx.resident()[1]
+    CALLS[call](ctx, c, lam)
+    CALLS[call](single, c, lam)
+    assert ctx.resident() == (True, before + (2 if call == "adjoint" else 1), 0)
+    assert single.resident() == (False, 0, 0)
+
+
+@pytest.mark.parametrize("law", ["field", "sigmoid", "ManningN_h"])
+@pytest.mark.parametrize("call", sorted(CALLS))
+def test_a_wait_that_runs_out(call, law):
+    """One tile is left out of the run and the others give up waiting for it (after a second); the call starts over with
+    single launches."""
+    c = moving(channel(1100))
+    lam = np.random.default_rng(1).normal(size=3 * c.N)
+    ctx, single = resident_and_single(c, law, call, lam)
+    want = CALLS[call](single, c, lam)
+    if law != "field" and call in ("adjoint", "reverse"):
+        want.append(single.lux_grad() if law == "ManningN_h" else want[0])
+    before = ctx.resident()[1]
+    ctx.set_resident(capi.HG_RESIDENT_SHORT)
+    got = CALLS[call](ctx, c, lam)
+    if law != "field" and call in ("adjoint", "reverse"):
+        got.append(ctx.lux_grad() if law == "ManningN_h" else got[0])
+    assert ctx.resident() == (False, before, 1)
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y)
+    ctx.set_resident(capi.HG_RESIDENT_ON)
+    ctx.step(c.Q0, c.dt, 12)
+    assert ctx.resident() == (True, before + 1, 1)
+    with pytest.raises(capi.HGError):
+        ctx.set_resident(3)
