@@ -335,6 +335,7 @@ struct hg_ctx {
   // cell's next face there (or -1), L^(2/3), L^(5/3) (the inlet adjoint)
   hg::InletFaceRec* in_rec = nullptr;
   bool inlets_listed = true;    // every inlet-Q ghost is in its inlet's list
+  bool inlet_empty = false;     // an inlet has no faces
   bool inlets_disjoint = true;  // no cell sits on two inlets: the inlet adjoint runs one work-group per inlet
   double *inletQ = nullptr, *inletQ0 = nullptr, *exitWSE = nullptr, *totalA = nullptr;
   int32_t* flags = nullptr;  // device address of flags_host: [0] conveyance error, [1] non-finite state, [2] a resident run's wait ran out

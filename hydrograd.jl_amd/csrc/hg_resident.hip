@@ -1008,9 +1008,6 @@ __device__ __forceinline__ bool adj_run_cells(AdjArgs a, const AdjRunArgs& R, do
     const int b = R.tile_in_list[sl];
     if (R.in_rec[R.in_off[b]].cell / T == t) R.o_Qbar[b] = qa[sl - in0];
   }
-  if (t == 0 && R.n_inlet > 0)  // an inlet without faces is on no tile's list
-    for (int b = tid; b < R.n_inlet; b += NT)
-      if (R.in_off[b] == R.in_off[b + 1]) R.o_Qbar[b] = R.Qbar[b];
   if (NM == RES_N_NET) __syncthreads();
   return true;
 }

@@ -82,7 +82,7 @@ struct AdjRunArgs {
   const int32_t* in_off;
   const InletFaceRec* in_rec;
   const double* Qbar;
-  double *o_nbar, *o_zbbar, *o_S0bar, *o_Qbar;
+  double *o_nbar, *o_zbbar, *o_S0bar, *o_Qbar;  // o_Qbar: of the inlets that have faces
   // with a law or network: what the forward run recorded of it ([ns][N]), the
   // closure (as in ResArgs), and the tiles' weight cotangents ([P][ntiles])
   const double* rec_n;

@@ -2921,6 +2921,12 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
     int rc = dalloc(ctx, &ctx->adj_wpart, size_t(hg::kAdjRunMaxP) * ctx->ntiles);
     if (rc) return rc;
   }
+  if (ctx->inlet_empty) {  // on no tile's list: its discharge cotangent stays what it is
+    ArrayList keep;
+    keep.add(ctx->adj_sums + 4 * N, ctx->adj_Qbar, ctx->n_inlet);
+    const int rc = launch_arrays(ctx, keep);
+    if (rc) return rc;
+  }
   if (!res_claim(ctx, ctx->adj_res_cap[k.nmode])) return HG_OK;
   const double* q[3] = {seg_state(ctx, 0, 0, b), seg_state(ctx, 0, 1, b), seg_state(ctx, 0, 2, b)};
   double *L = ctx->adj_lam[lam0], *O = ctx->adj_lam[1 - lam0], *sums = ctx->adj_sums;
@@ -3953,6 +3959,7 @@ int create_impl(hg_ctx** out, const hg_mesh* m, const hg_bcs* b, const hg_consts
       recs[f] = hg::InletFaceRec{gi, in_cell[f], first[f], next[f], g_L23[gi], in_L53[f]};
     }
     rc = upload(ctx, ctx->in_rec, recs.data(), ctx->n_inlet_faces);
+    for (int bi = 0; bi < b->n_inlet; ++bi) ctx->inlet_empty = ctx->inlet_empty || in_off[bi] == in_off[bi + 1];
     std::vector<uint8_t> listed(size_t(G), 0);
     for (int32_t f = 0; f < ctx->n_inlet_faces; ++f) listed[b->inlet_ghost[f]] = 1;
     for (int64_t gi = 0; gi < G; ++gi)
