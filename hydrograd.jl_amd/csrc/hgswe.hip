@@ -99,7 +99,7 @@ std::mutex g_scratch_mu;
 double* g_scratch_dev[kMaxDevices] = {};
 
 constexpr int kBlock = 256;
-constexpr int kRewarmSteps = 1024;  // graph-replayed steps the autotuner ends with (a multiple of kGraphSteps)
+constexpr int kRewarmSteps = 1024;  // steps the autotuner ends with (a multiple of kGraphSteps)
 constexpr int kGraphSteps = 16;  // steps per captured graph (even: the graph returns to buffer 0)
 // Largest state and cotangent together (bytes) that go through a context's
 // pinned block, by a host RHS both ways: 19,530 cells (0.9 MiB) 62 us through
@@ -5430,8 +5430,13 @@ int hg_autotune(hg_ctx* ctx, double dt, int64_t nsteps, int32_t* tile_cells, int
     }
     std::vector<std::pair<int, int>> shapes;
     for (int T : {128, 256, 512})
-      if (tile_lds_bytes(T, ctx->tileMD) <= ctx->lds_max)
+      if (tile_lds_bytes(T, ctx->tileMD) <= ctx->lds_max) {
         for (int x : {0, 1, 2, 4, 8, 16, 64}) shapes.emplace_back(T, x);
+        shapes.emplace_back(T, default_chunk((ctx->Nm + T - 1) / T, ctx->K));
+      }
+    shapes.emplace_back(ctx->tileT, ctx->xcd_chunk);  // what it was
+    std::sort(shapes.begin(), shapes.end());
+    shapes.erase(std::unique(shapes.begin(), shapes.end()), shapes.end());
     std::vector<double> t_best(shapes.size(), INFINITY);
     for (int pass = 0; pass < 2 && !rc; ++pass)
       for (size_t c = 0; c < shapes.size() && !rc; ++c) {
@@ -5448,12 +5453,50 @@ int hg_autotune(hg_ctx* ctx, double dt, int64_t nsteps, int32_t* tile_cells, int
         if (!rc) rc = check_flags(ctx);
         if (!rc) t_best[c] = std::min(t_best[c], ms);
       }
-    for (size_t c = 0; c < shapes.size() && !rc; ++c)
-      if (t_best[c] < best) {
-        best = t_best[c];
-        bestT = shapes[c].first;
-        bestX = shapes[c].second;
+    auto fastest = [&](int only_T) {
+      best = INFINITY;
+      for (size_t c = 0; c < shapes.size(); ++c)
+        if ((!only_T || shapes[c].first == only_T) && t_best[c] < best) {
+          best = t_best[c];
+          bestT = shapes[c].first;
+          bestX = shapes[c].second;
+        }
+    };
+    if (!rc) fastest(0);
+    // Small meshes run resident with tiles of kResT cells alone: the steps as
+    // hg_advance takes them there against the fastest single launch's kernel
+    // (39,248 cells: 4.9 us resident, 7.6 with the 256-cell tiles that the
+    // single launches alone would choose; 117,648 cells 6.6 and 9.1).  More
+    // than four tiles per CU never fit: such a mesh is not tiled for it.
+    hg::ResKind kind;
+    const int64_t rsteps = std::max<int64_t>(nsteps, 64);
+    const bool small = ctx->K == 1 && (ctx->Nm + kResT - 1) / kResT <= int64_t(4) * ctx->ncu;
+    if (!rc && small) rc = hg_set_tile_config(ctx, kResT, ctx->xcd_chunk);
+    if (!rc && small && res_kind(ctx, rsteps, false, kind)) {
+      double t_res = INFINITY;
+      hipEvent_t e[2] = {ctx->ev_pool[0], ctx->ev_pool[1]};
+      for (int pass = 0; pass < 3 && !rc; ++pass) {
+        for (int k = 0; k < 3 && !rc; ++k)
+          if (hipMemcpyAsync(ctx->st[0][k], ctx->scratch + k * N, N * sizeof(double), hipMemcpyDeviceToDevice,
+                             ctx->stream) != hipSuccess)
+            rc = HG_ERR_HIP;
+        ctx->cur = 0;
+        const int64_t runs = ctx->res_runs;
+        float ms = 0.f;
+        if (!rc) rc = clear_flags(ctx);
+        if (!rc && hipEventRecord(e[0], ctx->stream) != hipSuccess) rc = HG_ERR_HIP;
+        if (!rc) rc = advance_async(ctx, dt, rsteps);
+        if (!rc && (hipEventRecord(e[1], ctx->stream) != hipSuccess || hipEventSynchronize(e[1]) != hipSuccess ||
+                    hipEventElapsedTime(&ms, e[0], e[1]) != hipSuccess))
+          rc = HG_ERR_HIP;
+        if (!rc) rc = check_flags(ctx);
+        if (!rc && ctx->res_runs > runs) t_res = std::min(t_res, double(ms) / double(rsteps));
       }
+      if (!rc && t_res < best) {
+        fastest(kResT);  // the mapping of the launches that are left (shorter calls, the reverse step)
+        best = t_res;
+      }
+    }
     if (!rc) rc = hg_set_tile_config(ctx, bestT, bestX);
     // Re-warm with the kept shape: switching back may rebuild the tiling on
     // the host while the device idles, and a caller that times right after

@@ -273,9 +273,11 @@ int hg_get_resident(const hg_ctx* ctx, int32_t* on, int64_t* runs, int64_t* give
  * step kernel over nsteps steps of every launch shape, twice each (events on
  * each dispatch, after 16 warm-up steps), from the current device state
  * (which is restored afterwards); keeps the shape with the lowest time and
- * reports that mean kernel time in *ms_per_step.  It ends by instantiating
- * the stepping graph for dt with the kept shape and replaying it for 320
- * steps, so the device is warm and no graph is built by the next
+ * reports that mean kernel time in *ms_per_step.  Where the mesh can step
+ * resident (see hg_set_resident) and a resident run of max(nsteps, 64) steps
+ * takes less time per step, it keeps 128-cell tiles and reports that time.  It
+ * ends by instantiating the stepping graph for dt with the kept shape and
+ * advancing 1,024 steps, so the device is warm and no graph is built by the next
  * hg_advance; the state is then restored.  Needs hg_set_fields and a
  * device state (hg_state_upload). */
 int hg_autotune(hg_ctx* ctx, double dt, int64_t nsteps, int32_t* tile_cells, int32_t* xcd_chunk,

@@ -159,3 +159,19 @@ def test_a_wait_that_runs_out(call, law):
     assert ctx.resident() == (True, before + 1, 1)
     with pytest.raises(capi.HGError):
         ctx.set_resident(3)
+
+
+@pytest.mark.parametrize("n", [300, 1100, 9000, 40000, 98000])
+def test_tuned_meshes_step_resident(n):
+    """The tuner compares a resident run with the single launches, and leaves a mesh that it suits to it."""
+    c = channel(n)
+    ctx, ref = capi.Context(c), capi.Context(c)
+    ctx.upload(c.Q0)
+    T, x, ms = ctx.autotune(c.dt, 16)
+    assert (T, x) == ctx.tile_config() and T == 128 and ms > 0.0
+    assert np.array_equal(ctx.download(), c.Q0)
+    runs = ctx.resident()[1]
+    assert np.array_equal(ctx.step(c.Q0, c.dt, 40), ref.step(c.Q0, c.dt, 40))
+    assert ctx.resident() == (True, runs + 1, 0)
+    ctx.set_resident(capi.HG_RESIDENT_OFF)
+    assert np.array_equal(ctx.step(c.Q0, c.dt, 40), ref.step(c.Q0, c.dt, 40))
