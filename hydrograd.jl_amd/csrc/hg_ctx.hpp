@@ -362,6 +362,7 @@ struct hg_ctx {
   int32_t res_cap[2][3][2] = {{{-1, -1}, {-1, -1}, {-1, -1}}, {{-1, -1}, {-1, -1}, {-1, -1}}};
   bool res_off = false;
   bool res_short = false;                   // runs lack their last work-group and give up (HG_RESIDENT_SHORT)
+  bool res_nomem = false;                   // no memory is to be had for them (HG_RESIDENT_NOMEM)
   int64_t res_runs = 0, res_given_up = 0;  // runs that ended, and that gave up
   int32_t res_share = 0;
   unsigned long long* res_ring = nullptr;

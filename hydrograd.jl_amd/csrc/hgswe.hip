@@ -120,6 +120,21 @@ int dalloc(hg_ctx* ctx, T** p, size_t n) {
   return HG_OK;
 }
 
+// The same for a buffer that the call can do without: false, with nothing
+// left of the failure, when there is no memory for it.
+template <class T>
+bool dalloc_spare(hg_ctx* ctx, T** p, size_t n) {
+  T* q = nullptr;
+  const std::string err = ctx->err;
+  const bool got = !ctx->res_nomem && dalloc(ctx, &q, n) == HG_OK;
+  if (!got) {
+    (void)hipGetLastError();
+    ctx->err = err;
+  }
+  *p = got ? q : nullptr;
+  return got;
+}
+
 // Frees a buffer dalloc gave (NULL: nothing), after the context's streams
 // are idle.
 template <class T>
@@ -2354,18 +2369,18 @@ hg::ResArgs res_args(hg_ctx* ctx, int64_t nsteps) {
 }
 
 // The exchange ring for `words` values per cell and slot, behind it the
-// tiles' error sums.
-int ensure_res_ring(hg_ctx* ctx, int words) {
+// tiles' error sums.  *got: false when there is no memory for it.
+int ensure_res_ring(hg_ctx* ctx, int words, bool* got) {
   const size_t need = size_t(4) * words * ctx->N + 4 * hg::kResRed;
-  int rc = 0;
-  if (need > ctx->res_ring_n) {
-    rc = dfree(ctx, ctx->res_ring);
+  *got = ctx->res_ctl || dalloc_spare(ctx, &ctx->res_ctl, 1);
+  if (*got && need > ctx->res_ring_n) {
+    const int rc = dfree(ctx, ctx->res_ring);
     ctx->res_ring_n = 0;
-    if (!rc) rc = dalloc(ctx, &ctx->res_ring, need);
-    if (!rc) ctx->res_ring_n = need;
+    if (rc) return rc;
+    *got = dalloc_spare(ctx, &ctx->res_ring, need);
+    if (*got) ctx->res_ring_n = need;
   }
-  if (!rc && !ctx->res_ctl) rc = dalloc(ctx, &ctx->res_ctl, 1);
-  return rc;
+  return HG_OK;
 }
 
 // Takes this context's tiles out of the device's room, or false when they do
@@ -2414,9 +2429,10 @@ int res_run(hg_ctx* ctx, const hg::ResKind& k, const double* const in[3], double
             bool* done) {
   *done = false;
   const int words = k.dual ? 6 : 3;
-  int rc = ensure_res_ring(ctx, words);
+  bool ring = false;
+  const int rc = ensure_res_ring(ctx, words, &ring);
   if (rc) return rc;
-  if (!res_claim(ctx, ctx->res_cap[k.split][k.nmode][k.dual])) return HG_OK;
+  if (!ring || !res_claim(ctx, ctx->res_cap[k.split][k.nmode][k.dual])) return HG_OK;
   hg::ResArgs R = res_args(ctx, nsteps);
   R.rec = rec;
   R.rec_clamp = rec_clamp;
@@ -2830,11 +2846,10 @@ int forward_checkpointed(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck) {
         int rc = drop_graph(ctx);
         if (!rc) rc = dfree(ctx, ctx->adj_nseg[0]);
         ctx->adj_nseg_cap[0] = 0;
-        if (!rc) rc = dalloc(ctx, &ctx->adj_nseg[0], size_t(ns) * N);
         if (rc) return rc;
-        ctx->adj_nseg_cap[0] = size_t(ns);
+        if (dalloc_spare(ctx, &ctx->adj_nseg[0], size_t(ns) * N)) ctx->adj_nseg_cap[0] = size_t(ns);
       }
-      rec_n = ctx->adj_nseg[0];
+      rec_n = ctx->adj_nseg[0];  // NULL (no memory): reversed by single launches
     }
     const double* in[3] = {ctx->st[ctx->cur][0], ctx->st[ctx->cur][1], ctx->st[ctx->cur][2]};
     ArrayList copy;  // the recorded run's first state, and the segment's checkpoint
@@ -2910,17 +2925,12 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
   hg::ResKind k;
   if (!ctx->rec_resident || !adj_res_usable(ctx, ns, k)) return HG_OK;
   const int64_t N = ctx->N, G = std::max<int64_t>(ctx->G, 1), nring = 12 * N + 4 * G;
-  if (!ctx->adj_ring) {
-    int rc = dalloc(ctx, &ctx->adj_ring, size_t(nring));
-    if (!rc) rc = dalloc(ctx, &ctx->adj_sums, size_t(4) * N + std::max<int32_t>(ctx->n_inlet, 1));
-    if (!rc && !ctx->res_ctl) rc = dalloc(ctx, &ctx->res_ctl, 1);
-    if (rc) return rc;
-  }
   const int P = k.nmode == hg::RES_N_NET ? ctx->lux.P : 0;
-  if (P && !ctx->adj_wpart) {
-    int rc = dalloc(ctx, &ctx->adj_wpart, size_t(hg::kAdjRunMaxP) * ctx->ntiles);
-    if (rc) return rc;
-  }
+  if ((!ctx->adj_ring && !dalloc_spare(ctx, &ctx->adj_ring, size_t(nring))) ||
+      (!ctx->adj_sums && !dalloc_spare(ctx, &ctx->adj_sums, size_t(4) * N + std::max<int32_t>(ctx->n_inlet, 1))) ||
+      (!ctx->res_ctl && !dalloc_spare(ctx, &ctx->res_ctl, 1)) ||
+      (P && !ctx->adj_wpart && !dalloc_spare(ctx, &ctx->adj_wpart, size_t(hg::kAdjRunMaxP) * ctx->ntiles)))
+    return HG_OK;  // no memory: single launches
   if (ctx->inlet_empty) {  // on no tile's list: its discharge cotangent stays what it is
     ArrayList keep;
     keep.add(ctx->adj_sums + 4 * N, ctx->adj_Qbar, ctx->n_inlet);
@@ -3590,7 +3600,8 @@ int ensure_graph(hg_ctx* ctx, double dt) {
   return HG_OK;
 }
 
-// Advance the device state nsteps (no host sync at the end).
+// Advance the device state nsteps.  Synchronizes where a run is resident; the
+// launches are left in flight.
 int advance_async(hg_ctx* ctx, double dt, int64_t nsteps) {
   for (hg::ResKind k; res_kind(ctx, nsteps, false, k);) {  // a small mesh: runs of steps in one launch each
     const int64_t ns = std::min<int64_t>(nsteps, kResSteps);
@@ -4320,6 +4331,9 @@ int hg_prepare_advance(hg_ctx* ctx, double dt) {
   if (!ctx || !(dt > 0.0)) return HG_ERR_ARG;
   if (require_fields(ctx, "hg_prepare_advance")) return HG_ERR_STATE;
   int rc = ensure_graph(ctx, dt);
+  hg::ResKind k;
+  bool ring;
+  if (!rc && res_kind(ctx, kGraphSteps, false, k)) rc = ensure_res_ring(ctx, 3, &ring);
   if (!rc) rc = advance_timed(ctx, dt, 0, nullptr);  // the dispatch events
   if (!rc && hipStreamSynchronize(ctx->stream) != hipSuccess) rc = HG_ERR_HIP;
   return rc;
@@ -5038,15 +5052,15 @@ static int tsit5_resident(hg_ctx* ctx, double t0, double t1, int64_t n_save, dou
   int32_t& cap = ctx->tsit5_cap[k.nmode];
   if (cap < 0) cap = hg::tsit5_capacity(k.md, k.nmode, ctx->ncu);
   if (ctx->ntiles > cap) return HG_OK;
-  int rc = ensure_res_ring(ctx, 3);
-  if (!rc && frames > ctx->rk_frames_n) {
+  bool ring = false;
+  int rc = ensure_res_ring(ctx, 3, &ring);
+  if (!rc && ring && frames > ctx->rk_frames_n) {
     rc = dfree(ctx, ctx->rk_frames);
     ctx->rk_frames_n = 0;
-    if (!rc) rc = dalloc(ctx, &ctx->rk_frames, frames);
-    if (!rc) ctx->rk_frames_n = frames;
+    if (!rc && dalloc_spare(ctx, &ctx->rk_frames, frames)) ctx->rk_frames_n = frames;
   }
-  if (rc) return rc;
   if (!rc) rc = clear_flags(ctx);
+  if (rc || !ring || frames > ctx->rk_frames_n) return rc;  // no memory: the launches copy each frame out as it is reached
   hg::Tsit5Args P{};
   P.t0 = t0;
   P.t1 = t1;
@@ -5378,12 +5392,13 @@ int hg_get_tile_config(hg_ctx* ctx, int32_t* tile_cells, int32_t* xcd_chunk) {
 
 int hg_set_resident(hg_ctx* ctx, int32_t mode) {
   if (!ctx) return HG_ERR_ARG;
-  if (mode < HG_RESIDENT_OFF || mode > HG_RESIDENT_SHORT) {
+  if (mode < HG_RESIDENT_OFF || mode > HG_RESIDENT_NOMEM) {
     ctx->err = "hg_set_resident: unknown mode";
     return HG_ERR_ARG;
   }
   ctx->res_off = mode == HG_RESIDENT_OFF;
   ctx->res_short = mode == HG_RESIDENT_SHORT;
+  ctx->res_nomem = mode == HG_RESIDENT_NOMEM;
   return HG_OK;
 }
 
@@ -5573,13 +5588,15 @@ int hg_rhs_vjp(hg_ctx* ctx, const double* Q, const double* params, int64_t n_par
 
 // The checkpoint interval the library picks for kck <= 0: the whole run as
 // one stored segment (nothing recomputed) when its states, clamp flags and
-// recorded conveyances (and the closure's n) take at most half of the device
+// recorded conveyances (and the closure's n, or a small mesh's law's or network's) take at most half of the device
 // memory free for them (the context's segment buffers count as free), else
 // ceil(sqrt(nsteps)) (two segment buffers and nsteps / kck checkpoints:
 // about 3 sqrt(nsteps) states).
 int64_t auto_kck(hg_ctx* ctx, int64_t nsteps) {
   const double N = double(ctx->N);
-  const double per_step = 24.0 * N + N + 8.0 * std::max<int32_t>(ctx->n_inlet, 1) + (ctx->ude_prec ? 8.0 * N : 0.0);
+  hg::ResKind k;
+  const bool rec_n = ctx->ude_prec || (nsteps <= kResSteps && res_kind(ctx, nsteps, false, k) && k.nmode != hg::RES_N_FIELD);
+  const double per_step = 24.0 * N + N + 8.0 * std::max<int32_t>(ctx->n_inlet, 1) + (rec_n ? 8.0 * N : 0.0);
   if (int64_t(ctx->adj_seg_cap[0]) >= nsteps && (!ctx->ude_prec || int64_t(ctx->adj_nseg_cap[0]) >= nsteps))
     return nsteps;  // an earlier call took the room
   size_t fr = 0, tot = 0;

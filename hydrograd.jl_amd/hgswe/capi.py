@@ -17,7 +17,7 @@ _LIB = None
 
 HG_OK, HG_ERR_ARG, HG_ERR_HIP, HG_ERR_MESH, HG_ERR_CONVEYANCE, HG_ERR_NONFINITE, HG_ERR_STATE = range(7)
 HG_PARAM_NONE, HG_PARAM_ZB, HG_PARAM_N_ZONE, HG_PARAM_N_CELL, HG_PARAM_Q, HG_PARAM_UDE = range(6)
-HG_RESIDENT_OFF, HG_RESIDENT_ON, HG_RESIDENT_SHORT = range(3)
+HG_RESIDENT_OFF, HG_RESIDENT_ON, HG_RESIDENT_SHORT, HG_RESIDENT_NOMEM = range(4)
 HG_REORDER = 1
 HG_CELL_KERNEL = 2
 HG_NLAW_OFF, HG_NLAW_POWER, HG_NLAW_SIGMOID, HG_NLAW_INVERSE, HG_NLAW_H_UMAG_KS = range(5)
@@ -513,7 +513,7 @@ class Context:
         return t.value, x.value
 
     def set_resident(self, mode):
-        """HG_RESIDENT_OFF, _ON or _SHORT: whether a small mesh advances many
+        """HG_RESIDENT_OFF, _ON, or for tests _SHORT or _NOMEM: whether a small mesh advances many
         steps per launch."""
         self._chk(lib().hg_set_resident(self.h, int(mode)))
 

@@ -261,9 +261,11 @@ int hg_set_adjoint_tile(hg_ctx* ctx, int32_t tile_cells);
  * runs; of other processes on the device it does not know.  A wait of more
  * than a second ends the run: its steps are repeated with one launch each, as
  * are all later steps of the context until this call allows runs again.
- * HG_RESIDENT_SHORT starts every run without its last work-group, so that it
- * gives up (to test what follows). */
-enum { HG_RESIDENT_OFF = 0, HG_RESIDENT_ON = 1, HG_RESIDENT_SHORT = 2 };
+ * A call that finds no memory for what only its resident run needs does
+ * without the run.  To test what follows then, HG_RESIDENT_SHORT starts every
+ * run without its last work-group, so that it gives up, and HG_RESIDENT_NOMEM
+ * lets every such allocation fail. */
+enum { HG_RESIDENT_OFF = 0, HG_RESIDENT_ON = 1, HG_RESIDENT_SHORT = 2, HG_RESIDENT_NOMEM = 3 };
 int hg_set_resident(hg_ctx* ctx, int32_t mode);
 /* Whether resident runs are on, and how many of the context's have ended and
  * given up so far (any of the three may be NULL). */

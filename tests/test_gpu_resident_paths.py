@@ -158,7 +158,7 @@ def test_a_wait_that_runs_out(call, law):
     ctx.step(c.Q0, c.dt, 12)
     assert ctx.resident() == (True, before + 1, 1)
     with pytest.raises(capi.HGError):
-        ctx.set_resident(3)
+        ctx.set_resident(4)
 
 
 @pytest.mark.parametrize("n", [300, 1100, 9000, 40000, 98000])
@@ -175,3 +175,40 @@ def test_tuned_meshes_step_resident(n):
     assert ctx.resident() == (True, runs + 1, 0)
     ctx.set_resident(capi.HG_RESIDENT_OFF)
     assert np.array_equal(ctx.step(c.Q0, c.dt, 40), ref.step(c.Q0, c.dt, 40))
+
+
+@pytest.mark.parametrize("law", ["field", "sigmoid", "ManningN_h"])
+@pytest.mark.parametrize("call", sorted(CALLS))
+def test_no_memory_for_the_run(call, law):
+    """Where a resident run's own memory (rings, sums, Tsit5's frames, a law's recorded n) is not to be had, the call
+    takes single launches; with the memory it runs resident again."""
+    c = moving(channel(1100))
+    lam = np.random.default_rng(1).normal(size=3 * c.N)
+    ctx, single = capi.Context(c), capi.Context(c)
+    single.set_resident(capi.HG_RESIDENT_OFF)
+    ctx.set_resident(capi.HG_RESIDENT_NOMEM)
+    for k in (ctx, single):
+        with_law(k, c, law)
+        if call == "reverse":
+            k.adjoint_forward(c.Q0, c.dt, 12, 0)
+    for x, y in zip(CALLS[call](ctx, c, lam), CALLS[call](single, c, lam)):
+        assert np.array_equal(x, y)
+    assert ctx.resident() == (True, 0, 0)
+    ctx.set_resident(capi.HG_RESIDENT_ON)
+    assert np.array_equal(ctx.step(c.Q0, c.dt, 12), single.step(c.Q0, c.dt, 12))
+    assert ctx.resident() == (True, 1, 0)
+
+
+def test_reversal_without_memory_for_the_law():
+    """The forward run is resident, its law's n of each step is not recorded: the reversal takes single launches."""
+    c = moving(channel(1100))
+    lam = np.random.default_rng(1).normal(size=3 * c.N)
+    ctx, single = capi.Context(c), capi.Context(c)
+    single.set_resident(capi.HG_RESIDENT_OFF)
+    for k in (ctx, single):
+        with_law(k, c, "sigmoid")
+    ctx.step(c.Q0, c.dt, 12)  # takes the ring
+    ctx.set_resident(capi.HG_RESIDENT_NOMEM)
+    for x, y in zip(ctx.adjoint(c.Q0, c.dt, 12, 0, lam), single.adjoint(c.Q0, c.dt, 12, 0, lam)):
+        assert np.array_equal(x, y)
+    assert ctx.resident() == (True, 2, 0)
