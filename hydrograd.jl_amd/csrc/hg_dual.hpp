@@ -58,7 +58,7 @@ __device__ __forceinline__ Dual1 div_est(const Dual1& a, const Dual1& b, double 
   return Dual1(v, (a.d - v * b.d) * y);
 }
 __device__ __forceinline__ Dual1 div_est(const Dual1& a, double b, double y) {
-  return Dual1(div_est(a.v, b, y), a.d * y);
+  return Dual1(div_est(a.v, b, y), div_est(a.d, b, y));  // both as a / b gives them
 }
 __device__ __forceinline__ Dual1 sqrt_half_rcp(const Dual1& x, Dual1& o) {
   double ov;
