@@ -460,6 +460,8 @@ struct hg_ctx {
   double* lux_obar = nullptr;  // N
   double* lux_wpart = nullptr; // P x blocks
   double* lux_wbar = nullptr;  // P
+  double* lux_wcell = nullptr; // P x N, the sums over the steps (small networks on small meshes, see lux_by_cell)
+  bool lux_summed = false;     // lux_wbar is complete: a resident reversal summed its tiles
   double* lux_dw = nullptr;    // weight tangent of hg_jvp (kLuxMaxP)
   std::vector<void*> lux_allocs;
 

@@ -476,6 +476,31 @@ __device__ __forceinline__ void lux_jacobian(const LuxNet& L, const LuxPad& P, c
   df[2] = MW > 2 ? xb[MW > 2 ? 2 : 0] : 0.0;
 }
 
+// State components that the features read: ManningN_h takes the depth only.
+__device__ __forceinline__ int lux_state_inputs(const LuxNet& L) { return L.choice == LUX_MANNING_H ? 1 : 3; }
+
+// The output's derivatives cs by the cell's state (xi, q_x, q_y), from those
+// by the features: one dual pass for each of the ns components they read.
+__device__ __forceinline__ void lux_state_derivatives(const LuxNet& L, int ns, const double (&q)[3], double hs,
+                                                      double hsmall, double ks, const double (&df)[3], double* cs,
+                                                      int stride) {
+  for (int c = 0; c < ns; ++c) {
+    const Dual1 x0(q[0], c == 0 ? 1.0 : 0.0), x1(q[1], c == 1 ? 1.0 : 0.0), x2(q[2], c == 2 ? 1.0 : 0.0);
+    Dual1 fd[3];
+    lux_features<Dual1>(L, x0, x1, x2, hs, hsmall, ks, fd);
+    cs[c * stride] = df[0] * fd[0].d + df[1] * fd[1].d + df[2] * fd[2].d;
+  }
+  for (int c = ns; c < 3; ++c) cs[c * stride] = 0.0;
+}
+
+// The sum over a tile of 2 x 64 cells of v[cell], by one wave and a fixed
+// tree; N: cells of the mesh, c0: the tile's first.
+__device__ __forceinline__ double lux_tile_sum(const double* v, int c0, int N, int lane) {
+  double s = (c0 + lane < N ? v[lane] : 0.0) + (c0 + 64 + lane < N ? v[64 + lane] : 0.0);
+  for (int w = 32; w > 0; w >>= 1) s += __shfl_xor(s, w, 64);
+  return s;
+}
+
 struct LuxArgs {
   LuxNet net;
   int32_t N;
@@ -491,7 +516,8 @@ struct LuxArgs {
   double* ox;            // += state cotangent
   double* oqx;
   double* oqy;
-  double* wpart;         // [P][gridDim.x] per-block weight cotangents
+  double* wpart;         // [P][blocks] per-block weight cotangents
+  double* wcell;         // [P][N] per-cell ones (k_lux_vjp_cells)
 };
 
 __device__ __forceinline__ double lux_ks(const LuxArgs& a, int i) {

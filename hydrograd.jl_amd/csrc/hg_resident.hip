@@ -659,7 +659,7 @@ __device__ __forceinline__ bool adj_run_net(const AdjArgs& a, const AdjRunArgs& 
                                             bool own, int n_in) {
   constexpr int T = kResT;
   const int64_t N = a.N;
-  const int ns = R.net.choice == LUX_MANNING_H ? 1 : 3, P = R.net.P;
+  const int ns = lux_state_inputs(R.net), P = R.net.P;
   const double hs = own ? a.hstill[i] : 0.0, ksc = R.ks && own ? R.ks[i] : 1.0;
   double q[3] = {0.0, 0.0, 0.0}, nx[3] = {0.0, 0.0, 0.0};  // the step's recorded state, and the next one's
   auto read_ahead = [&](int64_t k) {
@@ -687,13 +687,7 @@ __device__ __forceinline__ bool adj_run_net(const AdjArgs& a, const AdjRunArgs& 
       if (r > 0) add();
       double df[3];
       lux_jacobian<4, NH>(R.net, pad, pass, J, T, df);
-      for (int c = 0; c < ns; ++c) {
-        const Dual1 x0(q[0], c == 0 ? 1.0 : 0.0), x1(q[1], c == 1 ? 1.0 : 0.0), x2(q[2], c == 2 ? 1.0 : 0.0);
-        Dual1 fd[3];
-        lux_features<Dual1>(R.net, x0, x1, x2, hs, a.hsmall, ksc, fd);
-        Cs[c * T] = df[0] * fd[0].d + df[1] * fd[1].d + df[2] * fd[2].d;
-      }
-      for (int c = ns; c < 3; ++c) Cs[c * T] = 0.0;
+      lux_state_derivatives(R.net, ns, q, hs, a.hsmall, ksc, df, Cs, T);
     }
     if (r >= 0) {
       __syncthreads();
@@ -1040,8 +1034,7 @@ __global__ __launch_bounds__(adj_run_threads(MD, NM), 2) void k_adj_run(AdjArgs 
     __syncthreads();
     for (int p = tid / 64; p < P; p += adj_run_threads(MD, NM) / 64) {  // the tile's sum per weight, by a fixed tree
       const int l = tid & 63;
-      double v = (t * T + l < a.N ? Wsum[p * T + l] : 0.0) + (t * T + 64 + l < a.N ? Wsum[p * T + 64 + l] : 0.0);
-      for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w, 64);
+      const double v = lux_tile_sum(Wsum + p * T, t * T, a.N, l);
       if (l == 0) R.o_wpart[int64_t(p) * gridDim.x + t] = v;
     }
   }

@@ -107,6 +107,8 @@ int res_capacity(const ResKind& k, int ncu);
 int adj_run_capacity(int md, int nmode, int net_P, int ncu);
 // Weights and hidden layers a resident reverse run can hold (2 LDS values per weight and cell).
 constexpr int kAdjRunMaxP = 56, kAdjRunMaxHidden = 2;
+// Tiles of a mesh on which such a network's weight cotangents are summed cell by cell, resident or not.
+constexpr int kAdjRunNetTiles = 256;
 int tsit5_capacity(int md, int nmode, int ncu);
 
 hipError_t res_init(hipStream_t stream, int64_t n, unsigned long long* ring, int32_t* ctl);

@@ -1633,7 +1633,7 @@ __global__ __launch_bounds__(64) void k_lux_vjp(hg::LuxArgs a) {
     hg::lux_backward<MW>(a.net, hg::lux_const(a.w), f, ob, acc, lane, fb);
     if (valid && ob != 0.0) {
       using hg::Dual1;
-      const int ns = a.net.choice == hg::LUX_MANNING_H ? 1 : 3;  // ManningN_h reads the depth only
+      const int ns = hg::lux_state_inputs(a.net);
       for (int st = 0; st < ns; ++st) {
         const Dual1 xi(a.xi[i], st == 0 ? 1.0 : 0.0), qx(a.qx[i], st == 1 ? 1.0 : 0.0),
             qy(a.qy[i], st == 2 ? 1.0 : 0.0);
@@ -1651,6 +1651,45 @@ __global__ __launch_bounds__(64) void k_lux_vjp(hg::LuxArgs a) {
   }
   __syncthreads();
   for (int k = lane; k < P; k += 64) a.wpart[size_t(k) * gridDim.x + blockIdx.x] += acc[k];
+}
+
+// The same for networks and meshes that a resident reversal takes (lux_by_cell),
+// with its operations in its order, so that a gradient has the same bits
+// whichever runs: a cell's weight cotangents are the output's derivatives times
+// its cotangent, and add up over the steps in memory, one value per weight and
+// cell; k_lux_tile_sums sums them per tile of kResT cells when all steps are
+// done.  The derivatives pass through LDS (J), as their place depends on the
+// layers' widths.
+template <int NH>
+__global__ __launch_bounds__(kResT) void k_lux_vjp_cells(hg::LuxArgs a) {
+  extern __shared__ double lds[];
+  const int tid = threadIdx.x, i = blockIdx.x * kResT + tid;
+  hg::lux_pad_fill(a.net, a.w, lds, tid, kResT);
+  __syncthreads();
+  if (i >= a.N) return;
+  const hg::LuxPad pad{lds, nullptr, a.net.n_hidden};
+  double* const J = lds + hg::kLuxPadN + tid;
+  const double q[3] = {a.xi[i], a.qx[i], a.qy[i]};
+  const double hs = a.hstill[i], ks = hg::lux_ks(a, i), ob = a.obar[i];
+  double f[3], df[3], cs[3];
+  hg::lux_features<double>(a.net, q[0], q[1], q[2], hs, a.hsmall, ks, f);
+  hg::LuxPass<4, NH> pass;
+  hg::lux_pass<4, NH>(a.net, pad, f, pass);
+  hg::lux_jacobian<4, NH>(a.net, pad, pass, J, kResT, df);
+  hg::lux_state_derivatives(a.net, hg::lux_state_inputs(a.net), q, hs, a.hsmall, ks, df, cs, 1);
+#pragma unroll 8
+  for (int p = 0; p < a.net.P; ++p) a.wcell[int64_t(p) * a.N + i] += ob * J[p * kResT];
+  if (ob != 0.0) {
+    a.ox[i] += ob * cs[0];
+    a.oqx[i] += ob * cs[1];
+    a.oqy[i] += ob * cs[2];
+  }
+}
+
+__global__ __launch_bounds__(64) void k_lux_tile_sums(int N, const double* wcell, double* wpart) {
+  const int t = blockIdx.x, p = blockIdx.y;
+  const double v = hg::lux_tile_sum(wcell + int64_t(p) * N + t * kResT, t * kResT, N, threadIdx.x);
+  if (threadIdx.x == 0) wpart[int64_t(p) * gridDim.x + t] = v;
 }
 
 // Layout check of the 16x16x4 matrix-core products used above: D = A B for
@@ -2236,6 +2275,14 @@ hg::LuxArgs lux_args(hg_ctx* ctx, const double* const q[3]) {
 
 int lux_vjp_blocks(const hg_ctx* ctx) { return int(std::min<int64_t>((ctx->N + 63) / 64, 1024)); }
 
+// Whether a network's weight cotangents are summed cell by cell: those that a
+// resident reversal can hold, on meshes of the size that it takes.  By these
+// sizes alone, whether or not one runs.
+bool lux_by_cell(const hg_ctx* ctx, const hg::LuxNet& L, int mw) {
+  return mw == 4 && L.P <= hg::kAdjRunMaxP && L.n_hidden <= hg::kAdjRunMaxHidden &&
+         ctx->N <= int64_t(hg::kAdjRunNetTiles) * kResT;
+}
+
 // n (or the friction magnitude) <- the reference's UDE network at state q.
 int enqueue_lux_fwd(hg_ctx* ctx, const double* const q[3]) {
   if (ctx->lux.choice == hg::LUX_OFF) return HG_OK;
@@ -2745,8 +2792,14 @@ int enqueue_adjoint(hg_ctx* ctx, const double* const q[3], const double* const l
     u.oqx = out[1];
     u.oqy = out[2];
     u.wpart = ctx->lux_wpart;
-    const int nb = lux_vjp_blocks(ctx);
-    if (ctx->lux_mw == 4)
+    u.wcell = ctx->lux_wcell;
+    const int nb = lux_vjp_blocks(ctx), nt = int((ctx->N + kResT - 1) / kResT);
+    const size_t lds = (hg::kLuxPadN + size_t(ctx->lux.P) * kResT) * sizeof(double);
+    if (ctx->lux_wcell && ctx->lux.n_hidden == 1)
+      hipLaunchKernelGGL(k_lux_vjp_cells<1>, dim3(nt), dim3(kResT), lds, ctx->stream, u);
+    else if (ctx->lux_wcell)
+      hipLaunchKernelGGL(k_lux_vjp_cells<2>, dim3(nt), dim3(kResT), lds, ctx->stream, u);
+    else if (ctx->lux_mw == 4)
       hipLaunchKernelGGL(k_lux_vjp<4>, dim3(nb), dim3(64), 0, ctx->stream, u);
     else
       hipLaunchKernelGGL(k_lux_vjp<hg::kLuxMaxW>, dim3(nb), dim3(64), 0, ctx->stream, u);
@@ -2767,9 +2820,16 @@ int finish_adjoint(hg_ctx* ctx) {
   if (ctx->ude_prec)
     hipLaunchKernelGGL(k_ude_wsum, dim3(hg::kUdeW, ctx->ude_nsets), dim3(kBlock), 0, ctx->stream, ctx->ude_nslots,
                        ctx->ude_set_start, ctx->ude_wpart, int64_t(1), int64_t(hg::kUdeW), ctx->ude_wbar);
-  if (ctx->lux.choice)
-    hipLaunchKernelGGL(k_ude_wsum, dim3(ctx->lux.P), dim3(kBlock), 0, ctx->stream, lux_vjp_blocks(ctx), nullptr,
-                       ctx->lux_wpart, int64_t(lux_vjp_blocks(ctx)), int64_t(1), ctx->lux_wbar);
+  if (ctx->lux.choice && !ctx->lux_summed) {
+    int nb = lux_vjp_blocks(ctx);
+    if (ctx->lux_wcell) {
+      nb = int((ctx->N + kResT - 1) / kResT);
+      hipLaunchKernelGGL(k_lux_tile_sums, dim3(nb, ctx->lux.P), dim3(64), 0, ctx->stream, int(ctx->N), ctx->lux_wcell,
+                         ctx->lux_wpart);
+    }
+    hipLaunchKernelGGL(k_ude_wsum, dim3(ctx->lux.P), dim3(kBlock), 0, ctx->stream, nb, nullptr, ctx->lux_wpart,
+                       int64_t(nb), int64_t(1), ctx->lux_wbar);
+  }
   HG_TRY(hipGetLastError());
   return HG_OK;
 }
@@ -2782,7 +2842,11 @@ int zero_adj_accumulators(hg_ctx* ctx) {
   }
   if (ctx->lux.choice) {
     z.add(ctx->lux_wbar, nullptr, ctx->lux.P);
-    z.add(ctx->lux_wpart, nullptr, int64_t(ctx->lux.P) * lux_vjp_blocks(ctx));
+    if (ctx->lux_wcell)
+      z.add(ctx->lux_wcell, nullptr, int64_t(ctx->lux.P) * ctx->N);
+    else
+      z.add(ctx->lux_wpart, nullptr, int64_t(ctx->lux.P) * lux_vjp_blocks(ctx));
+    ctx->lux_summed = false;
   }
   if (ctx->adj_want_zb) {
     z.add(ctx->adj_S0bar, nullptr, 2 * ctx->N);
@@ -2910,8 +2974,7 @@ int recompute_segment(hg_ctx* ctx, double dt, int64_t nsteps, int64_t kck, int64
 // Whether a recorded run of ns steps can be reversed resident.
 bool adj_res_usable(hg_ctx* ctx, int64_t ns, hg::ResKind& k) {
   if (!res_kind(ctx, ns, false, k) || ns > kResSteps || !ctx->inlets_disjoint || ctx->adj_T != kResT) return false;
-  if (k.nmode == hg::RES_N_NET && (ctx->lux.P > hg::kAdjRunMaxP || ctx->lux.n_hidden > hg::kAdjRunMaxHidden))
-    return false;
+  if (k.nmode == hg::RES_N_NET && !ctx->lux_wcell) return false;
   int32_t& cap = ctx->adj_res_cap[k.nmode];  // asked again when a network is set
   if (cap < 0) cap = hg::adj_run_capacity(ctx->tileMD, k.nmode, ctx->lux.P, ctx->ncu);
   return ctx->ntiles <= cap;
@@ -2993,6 +3056,7 @@ int adj_res_run(hg_ctx* ctx, double dt, int64_t ns, int b, int lam0, bool* done)
     hipLaunchKernelGGL(k_ude_wsum, dim3(P), dim3(kBlock), 0, ctx->stream, ctx->ntiles, nullptr, ctx->adj_wpart,
                        int64_t(ctx->ntiles), int64_t(1), ctx->lux_wbar);
     HG_TRY(hipGetLastError());
+    ctx->lux_summed = true;
   }
   return HG_OK;
 }
@@ -4748,7 +4812,7 @@ int hg_set_lux_ude(hg_ctx* ctx, const hg_lux_net* net, const double* params, con
   }
   ctx->lux_allocs.clear();
   ctx->lux = hg::LuxNet{};
-  ctx->lux_w = ctx->lux_ks = ctx->lux_fmag = ctx->lux_obar = ctx->lux_wpart = ctx->lux_wbar = nullptr;
+  ctx->lux_w = ctx->lux_ks = ctx->lux_fmag = ctx->lux_obar = ctx->lux_wpart = ctx->lux_wbar = ctx->lux_wcell = nullptr;
   ctx->lux_mw = 0;
   if (ctx->active == HG_PARAM_UDE) ctx->active = HG_PARAM_NONE;
   if (!net) {  // off: back to the per-cell n of hg_set_fields
@@ -4791,16 +4855,18 @@ int hg_set_lux_ude(hg_ctx* ctx, const hg_lux_net* net, const double* params, con
   if (!rc) rc = dalloc(ctx, &ctx->lux_obar, N);
   if (!rc) rc = dalloc(ctx, &ctx->lux_wpart, size_t(L.P) * lux_vjp_blocks(ctx));
   if (!rc) rc = dalloc(ctx, &ctx->lux_wbar, size_t(L.P));
+  int maxw = 0;
+  for (int l = 0; l < L.n_hidden; ++l) maxw = std::max(maxw, int(L.width[l]));
+  const int mw = maxw <= 4 ? 4 : hg::kLuxMaxW;
+  if (!rc && lux_by_cell(ctx, L, mw)) rc = dalloc(ctx, &ctx->lux_wcell, size_t(L.P) * N);
   ctx->lux_allocs.assign(ctx->allocs.begin() + nalloc0, ctx->allocs.end());
   if (rc) {
-    ctx->lux_w = ctx->lux_ks = ctx->lux_fmag = ctx->lux_obar = ctx->lux_wpart = ctx->lux_wbar = nullptr;
+    ctx->lux_w = ctx->lux_ks = ctx->lux_fmag = ctx->lux_obar = ctx->lux_wpart = ctx->lux_wbar = ctx->lux_wcell = nullptr;
     return rc;
   }
   HG_TRY(hipMemsetAsync(ctx->lux_wbar, 0, size_t(L.P) * sizeof(double), ctx->stream));
   HG_TRY(hipStreamSynchronize(ctx->stream));
-  int maxw = 0;
-  for (int l = 0; l < L.n_hidden; ++l) maxw = std::max(maxw, int(L.width[l]));
-  ctx->lux_mw = maxw <= 4 ? 4 : hg::kLuxMaxW;
+  ctx->lux_mw = mw;
   ctx->lux = L;
   ctx->adj_res_cap[hg::RES_N_NET] = -1;  // its LDS depends on the number of weights
   return HG_OK;

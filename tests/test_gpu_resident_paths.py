@@ -239,3 +239,30 @@ def test_forward_mode_has_the_same_bits(name, law):
             out.append(k.jvp(c.Q0, c.dt, 24, dQ0=d0, params=p, dparams=dp))
         for x, y in zip(*out):  # (the power law has no finite value on dry cells)
             assert np.any(np.isfinite(y)) and np.array_equal(x, y, equal_nan=True), kind
+
+
+@pytest.mark.parametrize("law", ["sigmoid", "power_law", "h_Umag_ks", "ManningN_h", "ManningN_h_Umag_ks",
+                                 "FlowResistance", "one_layer", "three_layers"])
+@pytest.mark.parametrize("name", ["one_tile", "tile_and_one", "tiny_channel", "channel", "mixed", "two_inlets", "quads",
+                                  "batch"])
+def test_gradients_through_closures_have_the_same_bits(name, law):
+    """Whole, by segments, and by single launches under another tiling: every cotangent, the weights' among them."""
+    c = moving(REVERSE[name]())
+    lam = np.random.default_rng(1).normal(size=3 * c.N)
+    out = []
+    for mode, tile, kck in ((capi.HG_RESIDENT_ON, 128, 0), (capi.HG_RESIDENT_ON, 128, 5), (capi.HG_RESIDENT_OFF, 256, 3)):
+        ctx = capi.Context(c)
+        ctx.set_resident(mode)
+        ctx.set_tile_config(tile)
+        net = law in ("one_layer", "three_layers")
+        if net:
+            hidden, acts = ([4], ["sigmoid"]) if law == "one_layer" else ([3, 2, 4], ["tanh", "leakyrelu", "softplus"])
+            n = capi.lux_net("ManningN_h", hidden, acts, (0.02, 0.06), (0.1, 4.0))
+            ctx.set_lux_ude(n, 0.5 * np.random.default_rng(2).normal(size=capi.lux_n_params(n)))
+        else:
+            net = with_law(ctx, c, law) is not None
+        out.append(list(ctx.adjoint(c.Q0, c.dt, 12, kck, lam)) + ([ctx.lux_grad()] if net else []))
+        assert (ctx.resident()[1] > 0) == (mode == capi.HG_RESIDENT_ON)
+    for other in out[1:]:
+        for x, y in zip(out[0], other):
+            assert np.all(np.isfinite(y)) and np.array_equal(x, y)
