@@ -586,7 +586,7 @@ __global__ __launch_bounds__(res_threads(MD, true), 2) void k_tsit5_run(TileArgs
       st.code = HG_ERR_NONFINITE;
       break;
     }
-    const double fac = err > 0.0 ? 0.9 * ::pow(err, -0.2) : 10.0;
+    const double fac = tsit5::step_factor(err);
     if (err <= 1.0) {  // accept: the new solution and its derivative (first same as last)
       st.t = last ? tt : st.t + h;
       for (int c = 0; c < 3; ++c) {

@@ -1,5 +1,9 @@
 // hg_tsit5.hpp -- the coefficients of the adaptive integrator.
 #pragma once
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+
 
 namespace hg {
 
@@ -20,6 +24,10 @@ constexpr double a[7][6] = {
 constexpr double btilde[7] = {-0.00178001105222577714, -0.0008164344596567469, 0.007880878010261995,
                               -0.1447110071732629,     0.5823571654525552,    -0.45808210592918697,
                               0.015151515151515152};
+// The factor (before its limits) that the step changes by after error norm err.
+__host__ __device__ __forceinline__ double step_factor(double err) {
+  return err > 0.0 ? 0.9 * ::pow(err, -0.2) : 10.0;
+}
 }  // namespace tsit5
 
 }  // namespace hg

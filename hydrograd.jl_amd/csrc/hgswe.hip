@@ -1746,6 +1746,40 @@ __global__ __launch_bounds__(kBlock) void k_rk_err(RkArgs a, const double* ynew,
   if (threadIdx.x == 0) part[blockIdx.x] = s[0];
 }
 
+// The same on meshes that k_tsit5_run takes (at most kResRed tiles of kResT
+// cells), grouped as it groups the sums, so that the step sizes have the same
+// bits whichever runs: per tile of kResT cells, one cell per work-item ...
+__global__ __launch_bounds__(kResT) void k_rk_err_tiles(RkArgs a, int N, const double* ynew, double abstol,
+                                                        double reltol, double* part) {
+  static_assert(kResT == 128, "two waves to a tile");
+  __shared__ double red[2];
+  const int tid = threadIdx.x, i = blockIdx.x * kResT + tid;
+  double v = 0.0;
+  if (i < N)
+    for (int c = 0; c < 3; ++c) {
+      const int64_t x = int64_t(c) * N + i;
+      double e = 0.0;
+      for (int j = 0; j < a.nk; ++j) e += a.coef[j] * a.k[j][x];
+      const double sc = abstol + reltol * fmax(fabs(a.y[x]), fabs(ynew[x]));
+      v += (e / sc) * (e / sc);
+    }
+  for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w, 64);
+  if ((tid & 63) == 0) red[tid >> 6] = v;
+  __syncthreads();
+  if (tid == 0) part[blockIdx.x] = red[0] + red[1];
+}
+
+// ... then over the tiles, with the norm (out[0]) and the step's factor (out[1]).
+__global__ __launch_bounds__(64) void k_rk_norm(int nt, int64_t n3, const double* part, double* out) {
+  double ss = 0.0;
+  for (int w = threadIdx.x; w < hg::kResRed; w += 64) ss += w < nt ? part[w] : 0.0;
+  for (int w = 32; w > 0; w >>= 1) ss += __shfl_xor(ss, w, 64);
+  if (threadIdx.x) return;
+  const double err = ::sqrt(ss / double(n3));
+  out[0] = err;
+  out[1] = hg::tsit5::step_factor(err);
+}
+
 // out[0] = sum of part[0 .. n) by one work-group (fixed tree).
 __global__ __launch_bounds__(kBlock) void k_sum(int n, const double* part, double* out) {
   __shared__ double s[kBlock];
@@ -5204,7 +5238,7 @@ int hg_tsit5_solve(hg_ctx* ctx, const double* Q0, const double* params, int64_t 
   if (rc) return rc;
   if (!ctx->rk) {
     rc = dalloc(ctx, &ctx->rk, size_t(10) * n3);
-    if (!rc) rc = dalloc(ctx, &ctx->rk_part, size_t((n3 + kBlock - 1) / kBlock) + 1);
+    if (!rc) rc = dalloc(ctx, &ctx->rk_part, size_t((n3 + kBlock - 1) / kBlock) + 2);
     if (rc) return rc;
   }
   double* K[7];
@@ -5282,21 +5316,30 @@ int hg_tsit5_solve(hg_ctx* ctx, const double* Q0, const double* params, int64_t 
         r.k[j] = K[j];
         r.coef[j] = h * tsit5::btilde[j];
       }
-      hipLaunchKernelGGL(k_rk_err, dim3(grid), dim3(kBlock), 0, ctx->stream, r, ynew, abstol, reltol,
-                         ctx->rk_part);
-      hipLaunchKernelGGL(k_sum, dim3(1), dim3(kBlock), 0, ctx->stream, grid, ctx->rk_part, errv);
-      double ss = 0.0;
-      if (hipMemcpyAsync(&ss, errv, sizeof(double), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+      const int64_t tiles = (N + kResT - 1) / kResT;
+      const bool small = tiles <= hg::kResRed;
+      if (small) {
+        hipLaunchKernelGGL(k_rk_err_tiles, dim3(int(tiles)), dim3(kResT), 0, ctx->stream, r, int(N), ynew, abstol,
+                           reltol, ctx->rk_part);
+        hipLaunchKernelGGL(k_rk_norm, dim3(1), dim3(64), 0, ctx->stream, int(tiles), n3, ctx->rk_part, errv);
+      } else {
+        hipLaunchKernelGGL(k_rk_err, dim3(grid), dim3(kBlock), 0, ctx->stream, r, ynew, abstol, reltol,
+                           ctx->rk_part);
+        hipLaunchKernelGGL(k_sum, dim3(1), dim3(kBlock), 0, ctx->stream, grid, ctx->rk_part, errv);
+      }
+      double ev[2] = {0.0, 0.0};
+      if (hipMemcpyAsync(ev, errv, (small ? 2 : 1) * sizeof(double), hipMemcpyDeviceToHost, ctx->stream) !=
+              hipSuccess ||
           hipStreamSynchronize(ctx->stream) != hipSuccess) {
         ctx->err = "hg_tsit5_solve: HIP error";
         return HG_ERR_HIP;
       }
-      const double err = std::sqrt(ss / double(n3));
+      const double err = small ? ev[0] : std::sqrt(ev[0] / double(n3));
       if (!std::isfinite(err)) {
         ctx->err = "hg_tsit5_solve: non-finite error estimate";
         return HG_ERR_NONFINITE;
       }
-      const double fac = err > 0.0 ? 0.9 * std::pow(err, -0.2) : 10.0;
+      const double fac = small ? ev[1] : tsit5::step_factor(err);
       if (err <= 1.0) {  // accept: the new solution and its derivative (first same as last)
         t = last ? tt : t + h;
         std::swap(y, ynew);

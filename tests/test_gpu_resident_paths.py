@@ -6,7 +6,7 @@ import dataclasses
 import numpy as np
 import pytest
 
-from hgswe import capi
+from hgswe import capi, cases
 from hgswe import mesh as hm
 
 from test_gpu_resident import LAWS, REVERSE, channel, moving, two_inlets, with_law
@@ -266,3 +266,28 @@ def test_gradients_through_closures_have_the_same_bits(name, law):
     for other in out[1:]:
         for x, y in zip(out[0], other):
             assert np.all(np.isfinite(y)) and np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("law", ["field", "sigmoid", "ManningN_h", "FlowResistance"])
+@pytest.mark.parametrize("name", ["one_tile", "tile_and_one", "quads", "tiny_channel", "channel", "mixed", "two_inlets",
+                                  "two_inlets_large"])
+def test_tsit5_has_the_same_bits(name, law):
+    """The adaptive integrator takes the same steps: frames and counts, over a few steps and over several launches."""
+    c = REVERSE[name]()
+    ctx, single = capi.Context(c), capi.Context(c)
+    single.set_resident(capi.HG_RESIDENT_OFF)
+    for k in (ctx, single):
+        with_law(k, c, law)
+    for T, frames, tol in ((12 * c.dt, 3, 1e-3), (60 * c.dt, 7, 1e-4)):
+        (F, n), (G, m) = [k.tsit5(c.Q0, 0.0, T, frames, dt0=0.1 * c.dt, reltol=tol) for k in (ctx, single)]
+        assert n == m and np.all(np.isfinite(G)) and np.array_equal(F, G)
+    assert ctx.resident()[1] >= 2
+
+
+def test_tsit5_has_the_same_bits_over_many_launches():
+    c = cases.dam_break(nx=40, ny=5)
+    ctx, single = capi.Context(c), capi.Context(c)
+    single.set_resident(capi.HG_RESIDENT_OFF)
+    (F, n), (G, m) = [k.tsit5(c.Q0, 0.0, 120.0, 3, abstol=1e-13, reltol=1e-12, dt0=1e-3) for k in (ctx, single)]
+    assert n == m and n[0] + n[1] > 1024 and np.array_equal(F, G)
+    assert ctx.resident()[1] >= 2
