@@ -1703,6 +1703,20 @@ __global__ __launch_bounds__(64) void k_mfma_probe(const T* A, const T* B, T* D)
   for (int r = 0; r < 4; ++r) D[M::row(kq, r) * 16 + col] = acc[r];
 }
 
+// The shared-part quotients and roots of hg_device.hpp at a and b > 0: a / b,
+// sqrt(b), 0.5 over that root, 1 / sqrt(b), 1 / b (rows of n).
+__global__ __launch_bounds__(kBlock) void k_rounding_probe(int64_t n, const double* a, const double* b, double* out) {
+  const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const double y = hg::rcp_est(b[i]);
+  double o;
+  out[i] = hg::div_est(a[i], b[i], y);
+  out[n + i] = hg::sqrt_half_rcp(b[i], o);
+  out[2 * n + i] = o;
+  out[3 * n + i] = hg::rsq_est(b[i]);
+  out[4 * n + i] = y;
+}
+
 // ---- Tsit5 (hg_tsit5.hpp): stage combinations and the error norm
 namespace tsit5 = hg::tsit5;
 
@@ -4969,6 +4983,22 @@ int hg_mfma_probe(int32_t precision, const double* A, const double* B, double* D
   (void)hipFree(dA);
   (void)hipFree(dB);
   (void)hipFree(dD);
+  return e == hipSuccess ? HG_OK : HG_ERR_HIP;
+}
+
+int hg_rounding_probe(int64_t n, const double* a, const double* b, double* out) {
+  if (!a || !b || !out || n <= 0 || n > (int64_t(1) << 28)) return HG_ERR_ARG;
+  const size_t bytes = size_t(n) * sizeof(double);
+  double* d = nullptr;
+  if (hipMalloc(reinterpret_cast<void**>(&d), 7 * bytes) != hipSuccess) return HG_ERR_HIP;
+  hipError_t e = hipMemcpy(d, a, bytes, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(d + n, b, bytes, hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(k_rounding_probe, dim3(grid_of(n)), dim3(kBlock), 0, 0, n, d, d + n, d + 2 * n);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpy(out, d + 2 * n, 5 * bytes, hipMemcpyDeviceToHost);
+  (void)hipFree(d);
   return e == hipSuccess ? HG_OK : HG_ERR_HIP;
 }
 

@@ -38,7 +38,7 @@ EXPORTS = [
     "hg_info", "hg_probe_copy", "hg_rhs_vjp", "hg_adjoint", "hg_grad_probes", "hg_batch_create",
     "hg_set_tile_config", "hg_get_tile_config", "hg_set_adjoint_tile", "hg_last_checkpoint_interval", "hg_adjoint_forward",
     "hg_adjoint_reverse", "hg_autotune", "hg_set_resident", "hg_get_resident", "hg_set_ude", "hg_ude_n", "hg_ude_grad",
-    "hg_mfma_probe", "hg_tsit5_solve", "hg_tsit5_tableau", "hg_jvp", "hg_batch_set_dt", "hg_set_n_law",
+    "hg_mfma_probe", "hg_rounding_probe", "hg_tsit5_solve", "hg_tsit5_tableau", "hg_jvp", "hg_batch_set_dt", "hg_set_n_law",
     "hg_n_law_eval", "hg_cell_n", "hg_lux_n_params", "hg_set_lux_ude", "hg_lux_eval", "hg_lux_grad",
     "hg_advance_timed", "hg_advance_region", "hg_prepare_advance", "hg_cfl_dt_noalloc", "hg_fields_create",
 ]
@@ -125,6 +125,7 @@ def lib():
         L.hg_lux_eval.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p]
         L.hg_lux_grad.argtypes = [C.c_void_p, C.c_void_p]
         L.hg_mfma_probe.argtypes = [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p]
+        L.hg_rounding_probe.argtypes = [C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]
         L.hg_tsit5_solve.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_double, C.c_double,
                                      C.c_int64, C.c_double, C.c_double, C.c_double, C.c_void_p, C.c_void_p]
         L.hg_tsit5_tableau.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p]
@@ -540,6 +541,17 @@ def mfma_probe(precision, A, B):
     if rc:
         raise HGError(rc, "hg_mfma_probe failed")
     return D
+
+
+def rounding_probe(a, b):
+    """(a / b, sqrt(b), 0.5 over that root, 1 / sqrt(b), 1 / b) as the step kernels form them."""
+    a = np.ascontiguousarray(a, dtype=np.float64)
+    b = np.ascontiguousarray(b, dtype=np.float64)
+    out = np.empty((5, a.size))
+    rc = lib().hg_rounding_probe(a.size, _ptr(a), _ptr(b), _ptr(out))
+    if rc:
+        raise HGError(rc, "hg_rounding_probe failed")
+    return tuple(out)
 
 
 def tsit5_tableau():

@@ -497,6 +497,11 @@ int hg_lux_grad(hg_ctx* ctx, double* params_bar);
  * given precision (32 or 64); verifies the lane layout the closure uses. */
 int hg_mfma_probe(int32_t precision, const double* A, const double* B, double* D);
 
+/* Self-check with no counterpart in the reference: a / b, sqrt(b),
+ * 0.5 over that root, 1 / sqrt(b) and 1 / b (five rows of n in out) as the
+ * step kernels form them, for n values a and b > 0. */
+int hg_rounding_probe(int64_t n, const double* a, const double* b, double* out);
+
 /* Measurement helper with no counterpart in the reference: copies nbytes
  * between two scratch device buffers `reps` times with a plain streaming
  * kernel and reports the achieved bandwidth (read + write bytes / time).  Its
