@@ -3206,11 +3206,6 @@ int check_flags(hg_ctx* ctx) {
   return HG_OK;
 }
 
-// Finiteness check of the device state (one reduction, at the end of a call).
-
-// Host 3N state (caller order) -> device state `slot` (library order).
-// The staging buffer and device permutation of the transfers below
-// (allocated on first use).
 // ---- host <-> device copies of caller arrays.  A caller's array is ordinary
 // (pageable) host memory, which the GPU cannot address.  It goes through
 // pinned memory, which the permutation kernels read and write directly: they
@@ -3434,6 +3429,8 @@ int device_to_host(hg_ctx* ctx, double* dst, const double* const s[3], const int
   return HG_OK;
 }
 
+// The staging buffer and device permutations of the transfers (allocated on
+// first use).
 int ensure_xfer(hg_ctx* ctx) {
   if (ctx->stage) return HG_OK;
   int rc = dalloc(ctx, &ctx->d_perm, size_t(ctx->N));
@@ -3501,6 +3498,7 @@ int perm_out(hg_ctx* ctx, const double* const s[3], int ncomp, double* dst) {
   return perm_out_all(ctx, &o, 1);
 }
 
+// Host 3N state (caller order) -> device state `slot` (library order).
 int state_in(hg_ctx* ctx, const double* Q, int slot) {
   double* const d[3] = {ctx->st[slot][0], ctx->st[slot][1], ctx->st[slot][2]};
   return perm_in(ctx, Q, 3, d);
@@ -3745,8 +3743,6 @@ int advance_async(hg_ctx* ctx, double dt, int64_t nsteps) {
   return HG_OK;
 }
 
-// nsteps single-launch steps, each step kernel with its own start / stop
-// events on its dispatch; *kernel_ms = their mean duration.  Synchronous.
 // Entry points that launch kernels over the fields refuse to run before
 // hg_set_fields has uploaded them (the kernels would read null pointers).
 int require_fields(hg_ctx* ctx, const char* who) {
@@ -3762,6 +3758,8 @@ int refuse_fields(hg_ctx* ctx, const char* who) {
   return HG_ERR_STATE;
 }
 
+// nsteps single-launch steps, each step kernel with its own start / stop
+// events on its dispatch; *kernel_ms = their mean duration.  Synchronous.
 int advance_timed(hg_ctx* ctx, double dt, int64_t nsteps, double* kernel_ms) {
   std::vector<hipEvent_t>& ev = ctx->ev_pool;  // grown once (at least 2 x 2048), reused by later calls
   int rc = HG_OK;
