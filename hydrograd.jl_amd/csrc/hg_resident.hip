@@ -55,7 +55,9 @@ constexpr int kBlock = 256;
 // (few tiles): the cells' work-items take no items, so the friction is off the
 // step's critical path; else they take the items that the rest leave.
 constexpr unsigned long long kResEmpty = 0x7ff4c0de5ea1ed01ull;
-constexpr long long kResTicks = 100000000;  // wall_clock64 ticks (100 MHz): 1 s
+// wall_clock64 ticks (100 MHz) that a wait may take: 1 s.  A constant: from memory or scalar registers the bound cost 2
+// to 3 % of a step of 1,000 cells, through the code around the polling loop.
+constexpr long long kResTicks = 100000000;
 constexpr int kResIn = 128;                 // inlet faces whose constants a tile keeps in LDS
 constexpr int res_threads(int MD, bool split) { return res_items(MD) + (split ? kResT : 0); }
 
